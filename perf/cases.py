@@ -23,7 +23,7 @@ import math
 import numpy as np
 import torch
 
-from spinterps_amd import configs, cyth
+from spinterps_amd import _lib, configs, cyth
 from spinterps_amd.interp.steps import (DeviceProblem, interp_neb_steps,
                                         interp_steps)
 from spinterps_amd.variograms.fitvgs import BatchVariogramFitter
@@ -44,6 +44,10 @@ def listed():
         # steps: latency and launches
         _steps('ok_small_fp64', stns=100, nx=50, ny=50, extent=1e5, steps=24,
                method='OK', values='daily', vg='small'),
+        # one time step of a small domain, as a forecast loop interpolates
+        # it when its observations arrive
+        _steps('idw_one_step', stns=100, nx=50, ny=50, extent=1e5, steps=1,
+               method='IDW', values='daily'),
         # a week of daily fields in the default (plain FP64) precision
         _steps('ok_daily_fp64', stns=1000, nx=500, ny=500, extent=5e5,
                steps=7, method='OK', values='daily', vg='daily'),
@@ -133,9 +137,9 @@ def draw(rng):
                       rng.choice(['hourly', 'daily']), vg=vg,
                       precision='mixed')
     if kind == 'idw':
-        nx, ny = _grid(rng, 20000, 400000)
-        return _steps(None, _log(rng, 50, 2000), nx, ny, extent,
-                      _log(rng, 8, 365), rng.choice(['IDW', 'IDW', 'NNB']),
+        nx, ny = _grid(rng, 1000, 400000)
+        return _steps(None, _log(rng, 20, 2000), nx, ny, extent,
+                      _log(rng, 1, 365), rng.choice(['IDW', 'IDW', 'NNB']),
                       'daily', idw_exp=rng.choice([1.0, 2.0, 3.5]))
     if kind == 'neb':
         nebs = rng.randint(8, 50)
@@ -268,6 +272,7 @@ def _class_inputs(case, seed):
 
 def prepare(case, seed):
     kind = case['kind']
+    _lib.lib()  # loaded once, before the first context is made
     if kind in ('steps', 'neb'):
         w, vals, vgs = _workload(case, seed)
         return dict(case=case, prob=DeviceProblem.from_workload(w),
