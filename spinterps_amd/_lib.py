@@ -182,7 +182,9 @@ SIGNATURES = {
 }
 
 _lib = None
-_lock = threading.Lock()
+# re-entrant: context() makes a Context under it, whose first library call
+# loads the library under it too
+_lock = threading.RLock()
 
 
 def lib():

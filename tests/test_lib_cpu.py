@@ -2,6 +2,8 @@
 host-only parts (variogram parsing, nugget check) work without a GPU."""
 import ctypes
 import re
+import subprocess
+import sys
 from pathlib import Path
 
 import numpy as np
@@ -71,3 +73,15 @@ def test_f32_out_struct_layout():
     assert S.est32.offset == 0 and S.var32.offset == 8
     assert S.has_min.offset == 16 and S.has_max.offset == 20
     assert S.min_cut.offset == 24 and S.max_cut.offset == 32
+
+
+def test_first_context_loads_the_library():
+    """A process whose first library call makes a context (as an IDW call
+    or a variogram fit does) does not wait on its own lock: context() holds
+    it while the library is loaded under it.  Without a GPU the context
+    itself is refused."""
+    code = ('from spinterps_amd import _lib\n'
+            'try:\n    _lib.context(0)\nexcept Exception:\n    pass\n'
+            'assert _lib._lib is not None\n')
+    subprocess.run([sys.executable, '-c', code], check=True, timeout=60,
+                   cwd=Path(__file__).resolve().parents[1])
