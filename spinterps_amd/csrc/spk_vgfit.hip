@@ -11,8 +11,11 @@
 //  spk_vgfit_de_dev    : differential evolution (best1bin, dither
 //                        U(0.5, 1) per generation, CR 0.7, Latin-hypercube
 //                        start, stop when std(E) <= tol |mean(E)|) of every
-//                        (step, candidate model) pair, one workgroup each;
-//                        the objective is vgs.py:661-678 without weights.
+//                        (step, candidate model) pair over the whole
+//                        device; the objective is vgs.py:661-678 without
+//                        weights.
+#include <algorithm>
+
 #include <hipcub/hipcub.hpp>
 
 #include "spk_internal.h"
@@ -61,89 +64,193 @@ __global__ void k_pair_unpack(const unsigned long long *__restrict__ key,
 }
 
 // ---- empirical variograms ----------------------------------------------------
-// One workgroup per step.  list: per-step scratch of M int32 (indices into
-// the sorted pair arrays of the kept pairs).
-__global__ __launch_bounds__(256) void k_evg(
-    const int32_t *__restrict__ pi, const int32_t *__restrict__ pj,
-    const double *__restrict__ pd, int64_t M, const double *__restrict__ vals,
-    int64_t N, double mdr, int nk, int classic, int max_bins,
-    int32_t *__restrict__ list, double *__restrict__ bh,
-    double *__restrict__ bg, int32_t *__restrict__ bn,
-    int32_t *__restrict__ nbins) {
-  const int s = blockIdx.x;
-  const double *z = vals + (int64_t)s * N;
-  int32_t *L = list + (int64_t)s * M;
-  __shared__ int wcnt[4];
-  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
-  int64_t base = 0;
-  for (int64_t b0 = 0; b0 < M; b0 += 256) {
-    const int64_t e = b0 + tid;
-    bool act = false;
-    if (e < M) act = !isnan(z[pi[e]]) && !isnan(z[pj[e]]);
-    const unsigned long long m = __ballot(act);
-    const int pre = __popcll(m & ((1ull << lane) - 1ull));
-    if (lane == 0) wcnt[wave] = __popcll(m);
-    __syncthreads();
-    int off = 0;
-    for (int w = 0; w < wave; ++w) off += wcnt[w];
-    if (act) L[base + off + pre] = (int32_t)e;
-    const int tot = wcnt[0] + wcnt[1] + wcnt[2] + wcnt[3];
-    __syncthreads();
-    base += tot;
+// list: per-step scratch of M int32 (indices into the sorted pair arrays of
+// the step's active pairs, in their order).  Written by (chunk, step)
+// workgroups in three passes: counts per chunk of kEvgChunk pairs, their
+// exclusive scan, then the list; the distance clip and the bins follow.
+// One workgroup per step that walked all pairs by itself took 7.2 ms for 24
+// steps of 1 500 stations (1.1 million pairs), bound by its serial chain of
+// loads; this split takes 0.56 ms.
+constexpr int kEvgChunk = 4096;
+
+// Active pairs of one chunk: bit u of the result is set when pair
+// b0 + tid + 256 u has both values.
+__device__ inline unsigned evg_active(const int32_t *pi, const int32_t *pj,
+                                      const double *z, int64_t b0, int64_t M) {
+  unsigned m = 0;
+#pragma unroll
+  for (int u = 0; u < kEvgChunk / 256; ++u) {
+    const int64_t e = b0 + threadIdx.x + 256 * u;
+    if (e < M && !isnan(z[pi[e]]) && !isnan(z[pj[e]])) m |= 1u << u;
   }
-  // base = active pairs.  Distance clip: argmin |d - mdr max| (first
-  // occurrence) over the sorted active distances.
-  __shared__ int64_t keep_s;
-  if (tid == 0) {
-    int64_t keep = base;
-    if (base > 0) {
-      const double act_max = pd[L[base - 1]];
-      const double md = act_max * mdr;
-      // first active position with d > md
-      int64_t lo = 0, hi = base;
-      while (lo < hi) {
-        const int64_t mid = (lo + hi) / 2;
-        if (pd[L[mid]] > md) hi = mid; else lo = mid + 1;
-      }
-      int64_t idx;
-      if (lo == 0) {
-        idx = 0;
-      } else if (lo == base) {
-        idx = base - 1;
-      } else {
-        const double da = md - pd[L[lo - 1]], db = pd[L[lo]] - md;
-        idx = (da <= db) ? lo - 1 : lo;
-      }
-      // first occurrence of that distance value
-      const double dv = pd[L[idx]];
-      {
-        int64_t a = 0, b2 = idx;
-        while (a < b2) {
-          const int64_t mid = (a + b2) / 2;
-          if (pd[L[mid]] < dv) a = mid + 1; else b2 = mid;
-        }
-        idx = a;
-      }
-      double clip_ul = pd[L[idx]];
-      if (!(clip_ul - md > 0)) clip_ul = md;
-      if (idx != base - 1) {
-        // keep d < clip_ul
-        int64_t a = 0, b2 = base;
-        while (a < b2) {
-          const int64_t mid = (a + b2) / 2;
-          if (pd[L[mid]] < clip_ul) a = mid + 1; else b2 = mid;
-        }
-        keep = a;
-      }
+  return m;
+}
+
+// grid (chunks, steps): cnt[step][chunk]
+__global__ __launch_bounds__(256) void k_evg_count(
+    const int32_t *__restrict__ pi, const int32_t *__restrict__ pj, int64_t M,
+    const double *__restrict__ vals, int64_t N, int64_t *__restrict__ cnt) {
+  const double *z = vals + (int64_t)blockIdx.y * N;
+  int c = __popc(evg_active(pi, pj, z, (int64_t)blockIdx.x * kEvgChunk, M));
+  for (int off = 32; off > 0; off >>= 1) c += __shfl_xor(c, off, 64);
+  __shared__ int w[4];
+  if ((threadIdx.x & 63) == 0) w[threadIdx.x >> 6] = c;
+  __syncthreads();
+  if (threadIdx.x == 0)
+    cnt[(int64_t)blockIdx.y * gridDim.x + blockIdx.x] =
+        w[0] + w[1] + w[2] + w[3];
+}
+
+// One workgroup per step: cnt becomes the chunks' start positions,
+// act[step] the number of active pairs.
+__global__ __launch_bounds__(256) void k_evg_scan(int64_t *__restrict__ cnt,
+                                                  int nchunk,
+                                                  int64_t *__restrict__ act) {
+  int64_t *c = cnt + (int64_t)blockIdx.x * nchunk;
+  __shared__ int64_t sh[256];
+  int64_t base = 0;
+  for (int k0 = 0; k0 < nchunk; k0 += 256) {
+    const int k = k0 + (int)threadIdx.x;
+    const int64_t v = k < nchunk ? c[k] : 0;
+    sh[threadIdx.x] = v;
+    __syncthreads();
+    for (int w = 1; w < 256; w <<= 1) {
+      const int64_t o = (int)threadIdx.x >= w ? sh[threadIdx.x - w] : 0;
+      __syncthreads();
+      sh[threadIdx.x] += o;
+      __syncthreads();
     }
-    keep_s = keep;
+    if (k < nchunk) c[k] = base + sh[threadIdx.x] - v;
+    base += sh[255];
+    __syncthreads();
+  }
+  if (threadIdx.x == 0) act[blockIdx.x] = base;
+}
+
+// grid (chunks, steps): the active pairs in their order.
+__global__ __launch_bounds__(256) void k_evg_list(
+    const int32_t *__restrict__ pi, const int32_t *__restrict__ pj, int64_t M,
+    const double *__restrict__ vals, int64_t N,
+    const int64_t *__restrict__ cnt, int32_t *__restrict__ list) {
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int64_t b0 = (int64_t)blockIdx.x * kEvgChunk;
+  const unsigned m =
+      evg_active(pi, pj, vals + (int64_t)blockIdx.y * N, b0, M);
+  int32_t *L = list + (int64_t)blockIdx.y * M;
+  __shared__ int wcnt[kEvgChunk / 64];  // active pairs per run of 64
+#pragma unroll
+  for (int u = 0; u < kEvgChunk / 256; ++u) {
+    const unsigned long long bm = __ballot((m >> u) & 1u);
+    if (lane == 0) wcnt[u * 4 + wave] = __popcll(bm);
   }
   __syncthreads();
-  const int64_t keep = keep_s;
-  int nb = (int)((keep + nk - 1) / nk);
-  if (nb > max_bins) nb = max_bins;
-  if (tid == 0) nbins[s] = nb;
-  for (int b = tid; b < nb; b += 256) {
+  if (threadIdx.x < 64) {  // exclusive scan of the 64 runs
+    const int v = wcnt[lane];
+    int x = v;
+    for (int w = 1; w < 64; w <<= 1) {
+      const int o = __shfl_up(x, w, 64);
+      if (lane >= w) x += o;
+    }
+    wcnt[lane] = x - v;
+  }
+  __syncthreads();
+  const int64_t base =
+      cnt[(int64_t)blockIdx.y * gridDim.x + blockIdx.x];
+#pragma unroll
+  for (int u = 0; u < kEvgChunk / 256; ++u) {
+    const bool act = (m >> u) & 1u;
+    const unsigned long long bm = __ballot(act);
+    if (act)
+      L[base + wcnt[u * 4 + wave] + __popcll(bm & ((1ull << lane) - 1ull))] =
+          (int32_t)(b0 + threadIdx.x + 256 * u);
+  }
+}
+
+// First position p in [0, hi) of a step's ascending active distances with
+// d > v (strict) or not d < v, hi if there is none: 64 probes per round, so
+// that a million pairs take four dependent loads.  Run by one wave; every
+// lane returns the position.
+__device__ inline int64_t evg_first(const double *pd, const int32_t *L,
+                                    int64_t hi, double v, bool strict) {
+  const int lane = threadIdx.x & 63;
+  int64_t lo = 0;
+  while (lo < hi) {
+    // probes lo, lo + st, ..., each below hi or ignored
+    const int64_t st = (hi - lo + 63) / 64;
+    const int64_t p = lo + st * lane;
+    bool t = false;
+    if (p < hi) {
+      const double d = pd[L[p]];
+      t = strict ? d > v : !(d < v);
+    }
+    const unsigned long long bm = __ballot(t);
+    const unsigned long long in = __ballot(p < hi);
+    if (bm == 0) {
+      // false at every probe: the answer lies after the last one
+      lo += st * (__popcll(in) - 1) + 1;
+    } else {
+      const int f = __ffsll((long long)bm) - 1;
+      hi = lo + st * f;  // true there
+      if (f > 0) lo += st * (f - 1) + 1;
+    }
+  }
+  return lo;
+}
+
+// One wave per step: the distance clip (vgs.py:597-659), argmin
+// |d - mdr max| (first occurrence) over the sorted active distances, and
+// the number of bins.  keep[step]: pairs kept.
+__global__ __launch_bounds__(64) void k_evg_clip(
+    const double *__restrict__ pd, int64_t M, double mdr, int nk,
+    int max_bins, const int32_t *__restrict__ list,
+    const int64_t *__restrict__ act, int64_t *__restrict__ keep_out,
+    int32_t *__restrict__ nbins) {
+  const int s = blockIdx.x;
+  const int32_t *L = list + (int64_t)s * M;
+  const int64_t base = act[s];
+  int64_t keep = base;
+  if (base > 0) {
+    const double act_max = pd[L[base - 1]];
+    const double md = act_max * mdr;
+    const int64_t lo = evg_first(pd, L, base, md, true);
+    int64_t idx;
+    if (lo == 0) {
+      idx = 0;
+    } else if (lo == base) {
+      idx = base - 1;
+    } else {
+      const double da = md - pd[L[lo - 1]], db = pd[L[lo]] - md;
+      idx = (da <= db) ? lo - 1 : lo;
+    }
+    // first occurrence of that distance value
+    idx = evg_first(pd, L, idx, pd[L[idx]], false);
+    double clip_ul = pd[L[idx]];
+    if (!(clip_ul - md > 0)) clip_ul = md;
+    // keep d < clip_ul
+    if (idx != base - 1) keep = evg_first(pd, L, base, clip_ul, false);
+  }
+  if (threadIdx.x == 0) {
+    keep_out[s] = keep;
+    nbins[s] = (int)min((keep + nk - 1) / nk, (int64_t)max_bins);
+  }
+}
+
+// grid (ceil(max bins / 256), steps): one thread per bin, its pairs summed
+// in their order.
+__global__ __launch_bounds__(256) void k_evg_bins(
+    const int32_t *__restrict__ pi, const int32_t *__restrict__ pj,
+    const double *__restrict__ pd, int64_t M, const double *__restrict__ vals,
+    int64_t N, int nk, int classic, int max_bins,
+    const int32_t *__restrict__ list, const int64_t *__restrict__ keep_in,
+    const int32_t *__restrict__ nbins, double *__restrict__ bh,
+    double *__restrict__ bg, int32_t *__restrict__ bn) {
+  const int s = blockIdx.y;
+  const double *z = vals + (int64_t)s * N;
+  const int32_t *L = list + (int64_t)s * M;
+  const int64_t keep = keep_in[s];
+  const int nb = nbins[s];
+  const int b = blockIdx.x * 256 + threadIdx.x;
+  if (b < nb) {
     const int64_t p0 = (int64_t)b * nk;
     const int cntb = (int)min((int64_t)nk, keep - p0);
     double sd = 0.0, sr = 0.0;
@@ -511,6 +618,345 @@ __global__ __launch_bounds__(256) void k_de(
   }
 }
 
+// ---- differential evolution over the whole device ------------------------------
+// The same evolution as k_de, generation by generation in two launches: the
+// energies of all candidates' trials over (member groups, bin chunks), then
+// one workgroup per candidate that selects, tests convergence and draws the
+// next trials.  k_de keeps a candidate on one CU, and its time is the
+// largest candidate's: 800 members x 16 000 bins x 2 components of exp() per
+// generation, 1 200 ms for a day of 24 steps x 7 candidates with 168 of 256
+// CUs in use and most of them early idle.  Spread over the device the same
+// day takes 11 ms (energies 9.1, selection and trials 1.3), bound by FP64
+// VALU issue: 21 instructions per member and bin for the exponential, 0.2 ms
+// per generation of the day's 430 million model values.  The random streams, the order of the draws and the
+// selection are k_de's; an energy's sum over bins is taken in kDeSplit
+// parts, whose bounds depend on the step's bins only.
+constexpr int kDeSplit = 16;
+constexpr int kDeMinBins = 64;
+
+__host__ __device__ inline int de_part_bins(int nb) {
+  const int l = (nb + kDeSplit - 1) / kDeSplit;
+  return l < kDeMinBins ? kDeMinBins : l;
+}
+
+// Bounds of component c's (range, sill) of candidate cd (vgs.py:735-757).
+__device__ inline void de_bounds(const int32_t *cd, int c, double h0,
+                                 double g0, double v, double range_ub,
+                                 double *lb, double *ub) {
+  if (cd[1 + c] == SPK_VG_POW) {
+    lb[0] = 1e-5;
+    ub[0] = 2.0;
+    lb[1] = 1e-5;
+    ub[1] = 2.0 * v;
+  } else if (cd[5] && c == 0) {
+    lb[0] = ub[0] = h0;
+    lb[1] = ub[1] = g0;
+  } else {
+    lb[0] = h0;
+    ub[0] = range_ub;
+    lb[1] = 1e-5;
+    ub[1] = 2.0 * v;
+  }
+}
+
+// 2^y for y <= 0: the nearest integer goes to the exponent, the rest f
+// (|f| <= 1/2) through a degree-11 Chebyshev interpolant of 2^f (largest
+// relative error 2e-17).
+__device__ inline double de_exp2(double y) {
+  y = fmax(y, -1100.0);  // 2^-1100 is zero; keeps -inf out of y - k
+  const double k = rint(y);
+  const double f = y - k;
+  double p = 4.4558179083360645e-10;
+  p = fma(p, f, 7.074194297288521e-09);
+  p = fma(p, f, 1.0178057087733941e-07);
+  p = fma(p, f, 1.3215432535912375e-06);
+  p = fma(p, f, 1.5252733841556773e-05);
+  p = fma(p, f, 0.00015403530463724353);
+  p = fma(p, f, 0.001333355814640647);
+  p = fma(p, f, 0.009618129107587256);
+  p = fma(p, f, 0.055504108664821625);
+  p = fma(p, f, 0.24022650695910158);
+  p = fma(p, f, 0.6931471805599453);
+  p = fma(p, f, 1.0);
+  return ldexp(p, (int)k);
+}
+
+// sum over bins [b0, b1) of (g - c - s f(h))^2, f per model
+template <typename F>
+__device__ inline double de_sum(const double *__restrict__ h,
+                                const double *__restrict__ g, int b0, int b1,
+                                F res) {
+  double acc = 0.0;
+#pragma unroll 4
+  for (int b = b0; b < b1; ++b) {
+    const double d = res(h[b], g[b]);
+    acc = fma(d, d, acc);
+  }
+  return acc;
+}
+
+// One wave: 64 members of one candidate over one chunk of its step's bins.
+// grid (waves / 4, candidates); q = step * ncand + candidate within the
+// batch, list (optional) the batch's candidates still evolving.
+__global__ __launch_bounds__(256) void k_de_energy(
+    const double *__restrict__ bh, const double *__restrict__ bg,
+    const int32_t *__restrict__ nbins, int max_bins,
+    const double *__restrict__ var, const int32_t *__restrict__ cand,
+    int ncand, int popmul, double range_ub, int pcap, int ds,
+    const double *__restrict__ mem, const int32_t *__restrict__ list,
+    const int32_t *__restrict__ done, double *__restrict__ part) {
+  const int q = list ? list[blockIdx.y] : (int)blockIdx.y;
+  if (done[q]) return;
+  const int s = q / ncand, ci = q - s * ncand;
+  const int32_t *cd = cand + ci * 6;
+  const int ncomp = cd[0], P = de_pop(popmul, 2 * ncomp);
+  const int nb = nbins[s];
+  const int mgs = (P + 63) / 64;
+  const int wv = __builtin_amdgcn_readfirstlane(
+      (int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+  const int ch = wv / mgs, mg = wv - ch * mgs;
+  const int len = de_part_bins(nb);
+  const int b0 = ch * len, b1 = min(nb, b0 + len);
+  if (ch >= kDeSplit || b0 >= b1) return;
+  const double *h = bh + (int64_t)s * max_bins;
+  const double *g = bg + (int64_t)s * max_bins;
+  const int i = mg * 64 + (int)(threadIdx.x & 63);
+  const double *x = mem + ((int64_t)q * pcap + min(i, P - 1)) * ds;
+  double acc;
+  // the constant (nugget) components and the one other component
+  int one = -1, others = 0;
+  for (int c = 0; c < ncomp; ++c)
+    if (cd[1 + c] != SPK_VG_NUG) {
+      one = c;
+      ++others;
+    }
+  const int ty = one >= 0 ? cd[1 + one] : SPK_VG_NUG;
+  double nug = 0.0, rg = 1.0, sl = 0.0;
+  for (int c = 0; c < ncomp; ++c) {
+    double lb[2], ub[2];
+    de_bounds(cd, c, h[0], g[0], var[s], range_ub, lb, ub);
+    const double cs = lb[1] + x[2 * c + 1] * (ub[1] - lb[1]);
+    if (cd[1 + c] == SPK_VG_NUG) {
+      nug += cs;
+    } else if (c == one) {
+      rg = lb[0] + x[2 * c] * (ub[0] - lb[0]);
+      sl = cs;
+    }
+  }
+  const double kLog2e = 1.4426950408889634;
+  if (others == 0) {
+    acc = de_sum(h, g, b0, b1, [&](double, double gb) { return gb - nug; });
+  } else if (others == 1 && ty == SPK_VG_EXP) {
+    const double c = (-3.0 / rg) * kLog2e, top = nug + sl;
+    acc = de_sum(h, g, b0, b1, [&](double hb, double gb) {
+      return fma(sl, de_exp2(hb * c), gb - top);
+    });
+  } else if (others == 1 && ty == SPK_VG_GAU) {
+    const double c = (-3.0 / (rg * rg)) * kLog2e, top = nug + sl;
+    acc = de_sum(h, g, b0, b1, [&](double hb, double gb) {
+      return fma(sl, de_exp2((hb * hb) * c), gb - top);
+    });
+  } else if (others == 1 && ty == SPK_VG_SPH) {
+    const double c = 1.0 / rg;
+    acc = de_sum(h, g, b0, b1, [&](double hb, double gb) {
+      const double u = fmin(hb * c, 1.0);  // the sill at h >= r
+      return fma(-sl, u * fma(u * u, -0.5, 1.5), gb - nug);
+    });
+  } else {
+    acc = 0.0;
+    for (int b = b0; b < b1; ++b) {
+      const double hb = h[b];
+      double v = 0.0;
+      for (int c = 0; c < ncomp; ++c) {
+        double lb[2], ub[2];
+        de_bounds(cd, c, h[0], g[0], var[s], range_ub, lb, ub);
+        v += fit_model(cd[1 + c], hb, lb[0] + x[2 * c] * (ub[0] - lb[0]),
+                       lb[1] + x[2 * c + 1] * (ub[1] - lb[1]));
+      }
+      const double r = g[b] - v;
+      acc += r * r;
+    }
+  }
+  if (i < P) part[((int64_t)q * kDeSplit + ch) * pcap + i] = acc;
+}
+
+// The start population of every candidate of a batch (k_de's
+// Latin-hypercube or seeded start); s0: the batch's first step within the
+// launch sequence's numbering, which keys the random streams.
+__global__ __launch_bounds__(256) void k_de_init(
+    const double *__restrict__ bh, const double *__restrict__ bg,
+    const int32_t *__restrict__ nbins, int max_bins,
+    const double *__restrict__ var, const int32_t *__restrict__ cand,
+    int ncand, int popmul, double range_ub, unsigned long long seed, int s0,
+    const double *__restrict__ init, double spread, int pcap, int ds,
+    double *__restrict__ pop, unsigned long long *__restrict__ rngs,
+    int32_t *__restrict__ done, double *__restrict__ out_fun,
+    int32_t *__restrict__ out_nit) {
+  const int s = blockIdx.y, ci = blockIdx.x, q = s * ncand + ci;
+  const int tid = threadIdx.x;
+  const int32_t *cd = cand + ci * 6;
+  const int D = 2 * cd[0], P = de_pop(popmul, D);
+  const bool none = nbins[s] <= 0 || P > pcap || D > ds;
+  if (tid == 0) done[q] = none ? 1 : 0;
+  if (none) {
+    if (tid == 0) {
+      out_fun[q] = NAN;
+      out_nit[q] = 0;
+    }
+    return;
+  }
+  __shared__ int perm[kDeMaxPop];
+  Rng rng(mix64(seed ^ mix64(((unsigned long long)(s0 + s) << 20) ^
+                             ((unsigned long long)ci << 8) ^ tid)));
+  pop += (int64_t)q * pcap * ds;
+  for (int d = 0; d < D; ++d) {
+    if (tid == 0) {
+      for (int i = 0; i < P; ++i) perm[i] = i;
+      for (int i = P - 1; i > 0; --i) {
+        const int j = (int)(rng.uni() * (i + 1));
+        const int t = perm[i];
+        perm[i] = perm[j];
+        perm[j] = t;
+      }
+    }
+    __syncthreads();
+    if (!init) {
+      for (int i = tid; i < P; i += 256)
+        pop[i * ds + d] = (perm[i] + rng.uni()) / P;
+    } else {
+      double lb[2], ub[2];
+      de_bounds(cd, d >> 1, bh[(int64_t)s * max_bins],
+                bg[(int64_t)s * max_bins], var[s], range_ub, lb, ub);
+      const double l = lb[d & 1], u1 = ub[d & 1], w = u1 - l;
+      const double c = fmin(fmax(init[(int64_t)q * kDeMaxD + d], l), u1);
+      for (int i = tid; i < P; i += 256) {
+        double u = 0.0;
+        if (w > 0.0) {
+          double v = c;
+          if (i > 0)
+            v = c * exp(spread * (2.0 * (perm[i] + rng.uni()) / P - 1.0));
+          v = fmin(fmax(v, l), u1);
+          u = (v - l) / w;
+        }
+        pop[i * ds + d] = u;
+      }
+    }
+    __syncthreads();
+  }
+  rngs[(int64_t)q * 256 + tid] = rng.s;
+}
+
+// One workgroup per candidate: takes the energies of generation `it`'s
+// trials (0: of the start population), selects, stops the candidate on
+// convergence or at maxiter, else draws the trials of generation it + 1.
+// The population is staged in LDS (pcap x ds doubles).
+__global__ __launch_bounds__(256) void k_de_step(
+    const double *__restrict__ bh, const double *__restrict__ bg,
+    const int32_t *__restrict__ nbins, int max_bins,
+    const double *__restrict__ var, const int32_t *__restrict__ cand,
+    int ncand, int it, int maxiter, int popmul, double tol, double range_ub,
+    int pcap, int ds, double *__restrict__ pop, double *__restrict__ trial,
+    double *__restrict__ energy, const double *__restrict__ part,
+    unsigned long long *__restrict__ rngs, const int32_t *__restrict__ list,
+    int32_t *__restrict__ done, double *__restrict__ out_par,
+    double *__restrict__ out_fun, int32_t *__restrict__ out_nit) {
+  const int q = list ? list[blockIdx.x] : (int)blockIdx.x;
+  if (done[q]) return;
+  const int s = q / ncand, ci = q - s * ncand;
+  const int tid = threadIdx.x;
+  const int32_t *cd = cand + ci * 6;
+  const int D = 2 * cd[0], P = de_pop(popmul, D);
+  const int nb = nbins[s];
+  const int nch = (nb + de_part_bins(nb) - 1) / de_part_bins(nb);
+  extern __shared__ double de_lds[];  // the population
+  __shared__ double red[4], redv[4], e0s, Fs;
+  __shared__ int redi[4];
+  pop += (int64_t)q * pcap * ds;
+  trial += (int64_t)q * pcap * ds;
+  energy += (int64_t)q * pcap;
+  part += (int64_t)q * kDeSplit * pcap;
+  double en[kDeOwn];
+#pragma unroll
+  for (int k = 0; k < kDeOwn; ++k) en[k] = 0.0;
+  for (int k = 0; tid + 256 * k < P; ++k) {
+    const int i = tid + 256 * k;
+    double e = 0.0;
+    for (int c = 0; c < nch; ++c) e += part[(int64_t)c * pcap + i];
+    const double old = it > 0 ? energy[i] : 0.0;
+    const bool take = it == 0 || e <= old;
+    const double *src = it > 0 && take ? trial : pop;
+    for (int d = 0; d < D; ++d) {
+      const double v = src[i * ds + d];
+      de_lds[i * ds + d] = v;
+      if (it > 0 && take) pop[i * ds + d] = v;
+    }
+    if (take) energy[i] = e;
+    set_own(en, k, take ? e : old);
+  }
+  __syncthreads();
+  bool stop = false;
+  if (it > 0) {
+    // convergence: std(E) <= tol * |mean(E)|
+    double sm = 0.0;
+#pragma unroll
+    for (int k = 0; k < kDeOwn; ++k)
+      if (tid + 256 * k < P) sm += en[k];
+    const double mean = blk_sum(sm, red) / P;
+    double sq = 0.0;
+#pragma unroll
+    for (int k = 0; k < kDeOwn; ++k) {
+      if (tid + 256 * k < P) {
+        const double dv = en[k] - mean;
+        sq += dv * dv;
+      }
+    }
+    const double sd = sqrt(blk_sum(sq, red) / P);
+    stop = sd <= tol * fabs(mean) || it >= maxiter;
+  }
+  double best;
+  const int bi = blk_argmin(en, P, redv, redi, &e0s, best);
+  if (stop) {
+    if (tid == 0) {
+      for (int c = 0; c < kDeMaxD / 2; ++c) {
+        double lb[2] = {0.0, 0.0}, ub[2] = {0.0, 0.0};
+        if (c < cd[0])
+          de_bounds(cd, c, bh[(int64_t)s * max_bins],
+                    bg[(int64_t)s * max_bins], var[s], range_ub, lb, ub);
+        for (int e = 0; e < 2; ++e)
+          out_par[(int64_t)q * kDeMaxD + 2 * c + e] =
+              c < cd[0]
+                  ? lb[e] + de_lds[bi * ds + 2 * c + e] * (ub[e] - lb[e])
+                  : 0.0;
+      }
+      out_fun[q] = best;
+      out_nit[q] = it;
+      done[q] = 1;
+    }
+    return;
+  }
+  Rng rng(1);
+  rng.s = rngs[(int64_t)q * 256 + tid];
+  if (tid == 0) Fs = 0.5 + 0.5 * rng.uni();
+  __syncthreads();
+  const double F = Fs;
+  for (int i = tid; i < P; i += 256) {
+    int r0, r1;
+    do { r0 = (int)(rng.uni() * P); } while (r0 == i);
+    do { r1 = (int)(rng.uni() * P); } while (r1 == i || r1 == r0);
+    const int fill = (int)(rng.uni() * D);
+    for (int d = 0; d < D; ++d) {
+      double v = de_lds[i * ds + d];
+      if (d == fill || rng.uni() < 0.7) {
+        v = de_lds[bi * ds + d] +
+            F * (de_lds[r0 * ds + d] - de_lds[r1 * ds + d]);
+        if (v < 0.0 || v > 1.0) v = rng.uni();
+      }
+      trial[i * ds + d] = v;
+    }
+  }
+  rngs[(int64_t)q * 256 + tid] = rng.s;
+}
+
 // ---- spatial order of cells -------------------------------------------------
 // Morton (Z-order) keys of the cells' coordinates quantised to 2^20 levels
 // per axis over their bounding box; sorting by key makes runs of 64 / 256
@@ -673,15 +1119,123 @@ int spk_vgfit_evg_dev(spk_ctx *ctx, const int32_t *pi, const int32_t *pj,
   if (T <= 0) return SPK_OK;
   SPK_HIP(hipSetDevice(ctx->device));
   const int64_t S = std::min<int64_t>(T, 256);
+  const int nch = (int)ceil_div(std::max<int64_t>(M, 1), kEvgChunk);
+  // bins that a step can have, so that the grid covers every step's
+  const int64_t nbm = std::min<int64_t>(max_bins, ceil_div(M, nk));
   int32_t *list;
+  int64_t *cnt;
   SPK_TRY(ws_get(ctx, "vglist", S * M * 4, (void **)&list));
+  SPK_TRY(ws_get(ctx, "vgcnt", S * (nch + 2) * 8, (void **)&cnt));
+  int64_t *act = cnt + S * nch, *keep = act + S;
   for (int64_t t0 = 0; t0 < T; t0 += S) {
     const int Sb = (int)std::min<int64_t>(S, T - t0);
-    hipLaunchKernelGGL(k_evg, dim3(Sb), dim3(256), 0, ctx->stream, pi, pj, pd,
-                       M, vals + t0 * N, N, mdr, nk, classic, max_bins, list,
-                       bin_h + t0 * max_bins, bin_g + t0 * max_bins,
-                       bin_n + t0 * max_bins, nbins + t0);
+    const double *v = vals + t0 * N;
+    hipLaunchKernelGGL(k_evg_count, dim3(nch, Sb), dim3(256), 0, ctx->stream,
+                       pi, pj, M, v, N, cnt);
+    hipLaunchKernelGGL(k_evg_scan, dim3(Sb), dim3(256), 0, ctx->stream, cnt,
+                       nch, act);
+    hipLaunchKernelGGL(k_evg_list, dim3(nch, Sb), dim3(256), 0, ctx->stream,
+                       pi, pj, M, v, N, (const int64_t *)cnt, list);
+    hipLaunchKernelGGL(k_evg_clip, dim3(Sb), dim3(64), 0, ctx->stream, pd, M,
+                       mdr, nk, max_bins, (const int32_t *)list,
+                       (const int64_t *)act, keep, nbins + t0);
+    if (nbm > 0)
+      hipLaunchKernelGGL(k_evg_bins, dim3((unsigned)ceil_div(nbm, 256), Sb),
+                         dim3(256), 0, ctx->stream, pi, pj, pd, M, v, N, nk,
+                         classic, max_bins, (const int32_t *)list,
+                         (const int64_t *)keep, (const int32_t *)nbins + t0,
+                         bin_h + t0 * max_bins, bin_g + t0 * max_bins,
+                         bin_n + t0 * max_bins);
     SPK_TRY(check_launch("k_evg"));
+  }
+  return SPK_OK;
+}
+
+// Whether a caller is capturing the stream into a graph.
+static bool stream_capturing(hipStream_t st) {
+  if (!st) return false;  // the null stream cannot be captured
+  hipStreamCaptureStatus cs = hipStreamCaptureStatusNone;
+  if (hipStreamIsCapturing(st, &cs) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return cs != hipStreamCaptureStatusNone;
+}
+
+// The evolution over the whole device (k_de_energy, k_de_step) in batches
+// of at most kDeBatch (step, candidate) pairs, whose scratch is 150 KB
+// (two components) to 260 KB each.  The host reads the pairs still
+// evolving every kDePoll generations (fits take 1 to 45).
+constexpr int kDeBatch = 2048;
+constexpr int kDePoll = 4;
+
+static int de_device(spk_ctx *ctx, const double *bin_h, const double *bin_g,
+                     const int32_t *nbins, int max_bins, const double *var,
+                     int64_t T, const int32_t *dc, int n_cands, int maxiter,
+                     int popmul, double tol, double range_ub, uint64_t seed,
+                     const double *init, double spread, int pcap, int ds,
+                     double *params, double *fun, int32_t *nit) {
+  hipStream_t st = ctx->stream;
+  const int64_t S =
+      std::min<int64_t>(T, std::max<int64_t>(1, kDeBatch / n_cands));
+  const int64_t nq = S * n_cands;
+  double *pop, *trial, *energy, *part;
+  unsigned long long *rngs;
+  int32_t *done;
+  SPK_TRY(ws_get(ctx, "vgde_pop", nq * pcap * ds * 8, (void **)&pop));
+  SPK_TRY(ws_get(ctx, "vgde_trial", nq * pcap * ds * 8, (void **)&trial));
+  SPK_TRY(ws_get(ctx, "vgde_energy", nq * pcap * 8, (void **)&energy));
+  SPK_TRY(ws_get(ctx, "vgde_part", nq * kDeSplit * pcap * 8,
+                 (void **)&part));
+  SPK_TRY(ws_get(ctx, "vgde_rng", nq * 256 * 8, (void **)&rngs));
+  SPK_TRY(ws_get(ctx, "vgde_done", 2 * nq * 4, (void **)&done));
+  int32_t *list = done + nq;
+  const size_t lds = (size_t)pcap * ds * sizeof(double);
+  std::vector<int32_t> h_done(nq), h_list(nq);
+  const unsigned gx =
+      (unsigned)ceil_div(ceil_div(pcap, 64) * kDeSplit, 4);
+  for (int64_t t0 = 0; t0 < T;) {
+    // k_de's launches cover 65 535 steps and number them from zero
+    const int64_t s0 = t0 % 65535;
+    const int Sb =
+        (int)std::min<int64_t>(std::min<int64_t>(S, T - t0), 65535 - s0);
+    const double *h = bin_h + t0 * max_bins, *g = bin_g + t0 * max_bins;
+    const int32_t *nbs = nbins + t0;
+    const double *vr = var + t0;
+    double *par = params + t0 * n_cands * kDeMaxD;
+    double *fn = fun + t0 * n_cands;
+    int32_t *ni = nit + t0 * n_cands;
+    hipLaunchKernelGGL(k_de_init, dim3(n_cands, Sb), dim3(256), 0, st, h, g,
+                       nbs, max_bins, vr, dc, n_cands, popmul, range_ub,
+                       (unsigned long long)seed, (int)s0,
+                       init ? init + t0 * n_cands * kDeMaxD : nullptr, spread,
+                       pcap, ds, pop, rngs, done, fn, ni);
+    int na = Sb * n_cands;
+    const int32_t *lst = nullptr;
+    auto generation = [&](int it) {
+      hipLaunchKernelGGL(k_de_energy, dim3(gx, na), dim3(256), 0, st, h, g,
+                         nbs, max_bins, vr, dc, n_cands, popmul, range_ub,
+                         pcap, ds, (const double *)(it ? trial : pop), lst,
+                         (const int32_t *)done, part);
+      hipLaunchKernelGGL(k_de_step, dim3(na), dim3(256), lds, st, h, g, nbs,
+                         max_bins, vr, dc, n_cands, it, maxiter, popmul, tol,
+                         range_ub, pcap, ds, pop, trial, energy,
+                         (const double *)part, rngs, lst, done, par, fn, ni);
+    };
+    generation(0);
+    for (int it = 1; it <= maxiter && na > 0; ++it) {
+      generation(it);
+      if (it % kDePoll && it < maxiter) continue;
+      SPK_TRY(check_launch("k_de_step"));
+      SPK_TRY(d2h(ctx, h_done.data(), done, (size_t)Sb * n_cands * 4));
+      na = 0;
+      for (int k = 0; k < Sb * n_cands; ++k)
+        if (!h_done[k]) h_list[na++] = k;
+      if (na > 0) SPK_TRY(h2d(ctx, list, h_list.data(), (size_t)na * 4));
+      lst = list;
+    }
+    SPK_TRY(check_launch("k_de_energy"));
+    t0 += Sb;
   }
   return SPK_OK;
 }
@@ -714,6 +1268,12 @@ static int de_launch(spk_ctx *ctx, const double *bin_h, const double *bin_g,
     ds = std::max(ds, D);
     pcap = std::max(pcap, de_pop(popmul, D));
   }
+  if (!stream_capturing(ctx->stream))
+    return de_device(ctx, bin_h, bin_g, nbins, max_bins, var, T, dc, n_cands,
+                     maxiter, popmul, tol, range_ub, seed, init, spread, pcap,
+                     ds, params, fun, nit);
+  // captured launches cannot be followed by host reads: one workgroup per
+  // (step, candidate) evolves by itself
   const size_t lds = de_lds_bytes(pcap, ds);
   if (lds > 64 * 1024)
     SPK_HIP(hipFuncSetAttribute((const void *)k_de,

@@ -175,3 +175,87 @@ def test_de_three_component_objective_matches_scipy(gpu):
                                  polish=False, seed=np.random.default_rng(2))
     fg = det['fun'][0, c]
     assert fg <= res.fun * (1 + 1e-3) + 1e-12, (fg, res.fun)
+
+
+@pytest.mark.parametrize('n,nk', [(24, 50), (130, 10), (400, 7)])
+def test_de_every_model_and_bin_count(gpu, n, nk):
+    """The device-wide evolution sums an energy in parts of max(64,
+    bins / 16) bins (fewer than 64 bins, a few parts, 16 ragged parts) with
+    loops of its own for Nug, Sph, Exp and Gau: every candidate's objective
+    is the oracle's at its parameters, and a step gives the same bits alone
+    as among others."""
+    from spinterps_amd.variograms.fitvgs import BatchVariogramFitter
+    rng = np.random.default_rng(n)
+    x, y = rng.uniform(0, 2e5, n), rng.uniform(0, 2e5, n)
+    vals = rng.gamma(2.0, 3.0, (3, n))
+    vals[1, rng.choice(n, n // 3, replace=False)] = np.nan
+    f = BatchVariogramFitter(x, y)
+    kw = dict(mdr=0.5, nk=nk, perm_r_list=[1, 2], fit_vgs=['all'],
+              fil_nug_vg='Nug', range_ub=2e5, opt_iters=60, seed=3,
+              return_details=True)
+    _, det = f.fit(vals, **kw)
+    _, one = f.fit(vals[:1], **kw)
+    np.testing.assert_array_equal(one['params'][0], det['params'][0])
+    np.testing.assert_array_equal(one['nit'][0], det['nit'][0])
+    bh, bg, nb = (det['bins'][k].cpu().numpy() for k in (0, 1, 3))
+    for k in range(3):
+        h, g = bh[k, :nb[k]], bg[k, :nb[k]]
+        for c, o in enumerate(det['cands']):
+            p = det['params'][k, c, :2 * len(o)]
+            ref = V.objective(p, list(o), h, g)
+            # a residual carries some 16 roundings of the size of g, which
+            # is what is left where few bins are fitted almost exactly:
+            # d(sum r^2) <= 2 sqrt(sum r^2) sqrt(sum (16 u g)^2)
+            np.testing.assert_allclose(
+                det['fun'][k, c], ref, rtol=1e-9,
+                atol=2 * np.sqrt(ref) * 16 * 1.2e-16 * np.linalg.norm(g))
+
+
+def test_de_captured_matches_eager(gpu):
+    """A captured launch cannot be followed by the host's reads and evolves
+    each candidate in one workgroup: the same random streams, so the same
+    generations, and objectives equal to the order of the energy sums."""
+    import ctypes
+    import torch
+    from spinterps_amd import _lib
+    from spinterps_amd.variograms.fitvgs import (TYPE_ID, BatchVariogramFitter,
+                                                 candidate_sets)
+    x, y, _ = _field(0)
+    vals = np.stack([_field(s)[2] for s in (0, 1)])
+    f = BatchVariogramFitter(x, y)
+    bh, _, _, nb = bins = f.empirical(vals)
+    cands = candidate_sets(['Sph', 'Exp', 'Gau'], [1, 2], 'Nug')
+    var = np.nanvar(vals, axis=1)
+    _, fun, nit = f.de(bins, var, cands, 'Nug', seed=4, range_ub=2e5)
+    spec = np.zeros((len(cands), 6), np.int32)
+    for c, o in enumerate(cands):
+        spec[c, 0] = len(o)
+        spec[c, 1:1 + len(o)] = [TYPE_ID[m] for m in o]
+        spec[c, 5] = 1 if len(o) > 1 and o[0] == 'Nug' else 0
+    ctx, st = _lib.Context(0), torch.cuda.Stream()
+    ctx.set_stream(st.cuda_stream)
+    vd = torch.as_tensor(var, device='cuda')
+    par2 = torch.zeros((2, len(cands), 8), dtype=torch.float64, device='cuda')
+    fun2, nit2 = torch.zeros_like(fun), torch.zeros_like(nit)
+
+    def call():
+        _lib.check(_lib.lib().spk_vgfit_de_dev(
+            ctx.h, bh.data_ptr(), bins[1].data_ptr(), nb.data_ptr(),
+            bh.shape[1], vd.data_ptr(), 2,
+            spec.ctypes.data_as(ctypes.POINTER(ctypes.c_int32)), len(cands),
+            10000, 50, 0.01, 2e5, 4, par2.data_ptr(), fun2.data_ptr(),
+            nit2.data_ptr()))
+    torch.cuda.synchronize()
+    call()  # sizes the context's scratch
+    st.synchronize()
+    g = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(g, stream=st):
+        call()
+    for _ in range(3):
+        fun2.zero_()
+        nit2.zero_()
+        g.replay()
+        torch.cuda.synchronize()
+        np.testing.assert_array_equal(nit2.cpu().numpy(), nit.cpu().numpy())
+        np.testing.assert_allclose(fun2.cpu().numpy(), fun.cpu().numpy(),
+                                   rtol=1e-11)
