@@ -61,7 +61,7 @@ int spk_ctx_set_graphs(spk_ctx *ctx, int on);
  * multiplied).  With SPK_TUNE_AUTO a context times every variant on the
  * first launch of each size class (the system's rows in classes of 1024)
  * on the real operands and keeps the fastest; SPK_TUNE_OFF launches the
- * library's defaults (1 and 0).  The reference's per-step loop
+ * library's defaults (0 and 0).  The reference's per-step loop
  * (interp/steps.py:315-401) has no counterpart: its tiles are numpy's. */
 #define SPK_TUNE_OFF   0
 #define SPK_TUNE_AUTO  1   /* default */

@@ -1,21 +1,16 @@
 // Cell-side kernels of the step interpolation and the batch driver behind
 // spk_interp_steps_dev.
 //
-//  k_rhs_plain   station-cell distance -> semivariogram/covariance, written
-//                as the reference's right-hand sides R [(n+p) x cells]
-//                (interp/steps.py:203-234), plus the nearest active station
-//  k_gemm<..>    MFMA contraction over all cells of a step:
-//                PLAIN: Lambda = K^-1 R (interp/steps.py:416) with the
-//                       estimate / sum-of-weights / variance epilogue of
-//                       interp/steps.py:418-434 fused in
-//                TRI  : W = L^-1 K, q = |W|^2 per cell (variance term)
-//  k_tri64       the TRI contraction in FP64, 128 x 128 tiles
+//  k_gemm<..>    W = L^-1 K, q = |W|^2 per cell (variance term) on FP32
+//                MFMA
+//  k_tri64       the same contraction in FP64, 128 x 128 tiles
 //  k_nearest     each cell's nearest active station (batched variance)
 //  k_kgen<..>    fused distance -> covariance for the batched path, with
 //                the dual-form estimate k.alpha accumulated in FP64 and the
 //                locally deflated covariances delta for the variance
 //  k_var_reduce  variance from the FP64 terms and the partial norms
-//  (the int8 plane-product contraction is in spk_int8.hip)
+//  (the int8 plane-product contraction is in spk_int8.hip, the plain FP64
+//  path's kernels are in spk_plain.hip)
 //  k_idw_nnb     interp/steps.py:285-313 (nearest neighbour; IDW runs as
 //                a masked FP64 MFMA contraction, k_idw_mfma in spk_idw.hip)
 //  k_special     one-station, mean-fill and failed-system steps
@@ -37,14 +32,6 @@ struct Mfma;
 // Result row held in slot r by lane group g = lane / 16 (column lane % 16):
 // f64 16x16x4 interleaves rows (g + 4 r), f32 16x16x4 keeps blocks (4 g + r)
 // (checked on gfx950 against a host matmul).
-template <>
-struct Mfma<double> {
-  using V = d4_t;
-  __device__ static inline V op(double a, double b, V c) {
-    return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
-  }
-  __device__ static constexpr int row(int g, int r) { return g + 4 * r; }
-};
 template <>
 struct Mfma<float> {
   using V = f4_t;
@@ -88,61 +75,9 @@ __global__ void k_recenter(const double *__restrict__ in,
     out[i] = in[i] - o;
 }
 
-// ---- plain path right-hand sides ---------------------------------------------
-__global__ __launch_bounds__(256) void k_rhs_plain(
-    const double *__restrict__ sx, const double *__restrict__ sy,
-    const int32_t *__restrict__ idx, const StepSc *__restrict__ sc,
-    const spk_vg *__restrict__ vgp, const double *__restrict__ cx,
-    const double *__restrict__ cy, int64_t Cs, int64_t C,
-    const double *__restrict__ cell_drift, int method, int m, int covar_flag,
-    double min_vg_val, double *__restrict__ R, int64_t ldr,
-    int32_t *__restrict__ nnb, const int *__restrict__ ccount) {
-  if (sc->status) return;
-  const int n = sc->n;
-  // ccount (device, optional): the cells of this launch, at most Cs
-  if (ccount) Cs = min(Cs, (int64_t)*ccount);
-  if (blockIdx.x * (int64_t)256 >= Cs) return;
-  __shared__ double stx[256], sty[256];
-  __shared__ spk_vg vg;
-  const int tid = threadIdx.x;
-  const int64_t c = blockIdx.x * (int64_t)256 + tid;
-  const bool valid = c < Cs;
-  const double x = valid ? cx[c] : 0.0, y = valid ? cy[c] : 0.0;
-  if (tid == 0) vg = *vgp;
-  double best = INFINITY;
-  int bi = 0;
-  for (int base = 0; base < n; base += 256) {
-    __syncthreads();
-    if (base + tid < n) {
-      stx[tid] = sx[idx[base + tid]];
-      sty[tid] = sy[idx[base + tid]];
-    }
-    __syncthreads();
-    const int cnt = min(256, n - base);
-    if (valid) {
-      for (int j = 0; j < cnt; ++j) {
-        const double d = dist2(x, y, stx[j], sty[j]);
-        // ties go to the lower station index (np.argmin), whatever order
-        // the step's stations are compacted in
-        if (d < best || (d == best && idx[base + j] < idx[bi])) {
-          best = d;
-          bi = base + j;
-        }
-        R[(int64_t)(base + j) * ldr + c] =
-            vg_entry(vg, d, covar_flag, min_vg_val);
-      }
-    }
-  }
-  if (!valid) return;
-  if (method != SPK_M_SK) R[(int64_t)n * ldr + c] = 1.0;
-  if (method == SPK_M_EDK)
-    for (int k = 0; k < m; ++k)
-      R[(int64_t)(n + 1 + k) * ldr + c] = cell_drift[(int64_t)k * C + c];
-  nnb[c] = bi;
-}
-
 // ---- MFMA contraction --------------------------------------------------------
-// Block tile: 64 rows x 128 cells, k in chunks of BK, 256 threads = 4 waves;
+// W = L^-1 delta, |W|^2 per cell and 64-row block, on FP32 operands
+// (SPK_P_MIXED_F32, and SPK_P_MIXED above 8 192 rows).  Block tile: 64 rows x 128 cells, k in chunks of BK, 256 threads = 4 waves;
 // wave w owns cells [32 w, 32 w + 32) of the tile over all 64 rows as 4 x 2
 // MFMA 16x16 tiles, so the per-cell row reductions of the epilogue need no
 // cross-wave step.  The next k chunk is loaded into registers while the
@@ -157,42 +92,24 @@ template <>
 struct Vec4<float> {
   using type = float4;
 };
-template <>
-struct Vec4<double> {
-  using type = double2;  // 16-byte loads: two doubles
-};
 
-template <typename T, bool PLAIN, int BK>
-__global__ __launch_bounds__(256, PLAIN ? 1 : 3) void k_gemm(
+template <typename T, int BK>
+__global__ __launch_bounds__(256, 3) void k_gemm(
     const T *__restrict__ A, int64_t lda, int64_t strideA,
     const T *__restrict__ B, int64_t ldb, int64_t strideB,
-    StepSc *__restrict__ sc, int p, int method, int want_var, int skm,
-    const double *__restrict__ zact, int64_t ldz,
-    const int32_t *__restrict__ nnb, int64_t ldn,
-    const double *__restrict__ abuf, int64_t ldab, int64_t Cs,
-    double *__restrict__ est, double *__restrict__ var, int64_t ldo,
-    int sel, double *__restrict__ qpart, int nrb,
-    const uint8_t *__restrict__ nzb, int64_t nzk,
-    unsigned long long *__restrict__ nexec,
-    const int *__restrict__ ccount, const int32_t *__restrict__ cmap) {
+    const StepSc *__restrict__ sc, int64_t ldab, int64_t Cs, int sel,
+    double *__restrict__ qpart, int nrb, const uint8_t *__restrict__ nzb,
+    int64_t nzk, unsigned long long *__restrict__ nexec) {
   using MF = Mfma<T>;
-  // ccount (device, optional): the cells of this launch, at most Cs;
-  // cmap (PLAIN, optional): output index of each cell
-  if (ccount) Cs = min(Cs, (int64_t)*ccount);
   using V = typename MF::V;
   constexpr int BM = 64, BN = 128;
-  // PLAIN: grid (cell tiles, steps), each block walks all row blocks.
-  // TRI: grid (row blocks, cell tiles, steps), one row block per block;
+  // grid (row blocks, cell tiles, steps), one row block per block;
   // blocks on the same XCD (linear id mod 8) take consecutive row blocks of
   // one cell tile so that the tile's K rows stay in that XCD's L2.
-  int rbi = 0, cti = blockIdx.x;
-  if (!PLAIN) {
-    const int G = gridDim.x * gridDim.y;
-    int lin = blockIdx.x + blockIdx.y * gridDim.x;
-    if ((G & 7) == 0) lin = (lin & 7) * (G >> 3) + (lin >> 3);
-    rbi = lin % gridDim.x;
-    cti = lin / gridDim.x;
-  }
+  const int G = gridDim.x * gridDim.y;
+  int lin = blockIdx.x + blockIdx.y * gridDim.x;
+  if ((G & 7) == 0) lin = (lin & 7) * (G >> 3) + (lin >> 3);
+  const int rbi = lin % gridDim.x, cti = lin / gridDim.x;
   constexpr int VW = 16 / sizeof(T);         // elements per 16-byte load
   // row padding: FP32 rows 16 banks apart, so the four 16-lane groups of a
   // 32-bit LDS read (one row each) fall on distinct banks
@@ -201,7 +118,7 @@ __global__ __launch_bounds__(256, PLAIN ? 1 : 3) void k_gemm(
   constexpr int B_LD = BN * BK / VW / 256;
   static_assert(A_LD >= 1 && B_LD >= 1, "tile too small");
   using VT = typename Vec4<T>::type;
-  const int sl = PLAIN ? blockIdx.y : blockIdx.z;
+  const int sl = blockIdx.z;
   const StepSc st = sc[sl];
   if (st.status) return;
   // sel 1: only the FP32 steps (neither SPK_ST_FP64VAR nor SPK_ST_INT8VAR),
@@ -209,29 +126,27 @@ __global__ __launch_bounds__(256, PLAIN ? 1 : 3) void k_gemm(
   if (sel == 1 && (st.flags & (SPK_ST_FP64VAR | SPK_ST_INT8VAR))) return;
   if (sel == 2 && !(st.flags & SPK_ST_FP64VAR)) return;
   const int n = st.n;
-  const int P = PLAIN ? n + p : n;
+  const int P = n;
   const int64_t c0 = cti * (int64_t)BN;
   if (c0 >= Cs) return;
-  const int r_lo = PLAIN ? 0 : rbi * BM;
+  const int r_lo = rbi * BM;
   if (r_lo >= P) return;
-  const int r_hi = PLAIN ? P : min(P, r_lo + BM);
+  const int r_hi = min(P, r_lo + BM);
   A += (int64_t)sl * strideA;
   B += (int64_t)sl * strideB;
-  const double *z = zact + (int64_t)sl * ldz;
   __shared__ __align__(16) T As[2][BK][BM + PAD];
   __shared__ __align__(16) T Bs[2][BK][BN + PAD];
-  __shared__ int s_list[256];  // nonzero chunks (TRI with a chunk map)
+  __shared__ int s_list[256];  // nonzero chunks (with a chunk map)
   __shared__ int s_cnt[4];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int li = lane & 15, lg = lane >> 4;
 
-  double acc_e[2] = {0.0, 0.0}, acc_l[2] = {0.0, 0.0};
-  double acc_v[2] = {0.0, 0.0}, acc_m[2] = {0.0, 0.0};
+  double acc_v[2] = {0.0, 0.0};
 
   // register stages of the next chunks' tiles; the FP32 contraction keeps
   // two chunks in flight, which covers an L2 miss behind the chunk being
   // multiplied
-  constexpr bool PF2 = !PLAIN && sizeof(T) == 4;
+  constexpr bool PF2 = sizeof(T) == 4;
   VT ra[A_LD], rb[B_LD], ra2[PF2 ? A_LD : 1], rb2[PF2 ? B_LD : 1];
   // A tile element group q: rows r..r+VW-1 of column k
   auto load_tiles = [&](auto &ra, auto &rb, int r0, int k0, int kend) {
@@ -296,12 +211,12 @@ __global__ __launch_bounds__(256, PLAIN ? 1 : 3) void k_gemm(
 #pragma unroll
           for (int r = 0; r < 4; ++r) acc64[a][b][r] = 0.0;
     }
-    const int kend = PLAIN ? P : min(P, r0 + BM);
+    const int kend = min(P, r0 + BM);
     int nch = (kend + BK - 1) / BK;
-    // TRI with a map of the 16-row chunks of delta that hold a nonzero
+    // with a map of the 16-row chunks of delta that hold a nonzero
     // value in this cell tile: only those chunks are multiplied (a zero
     // chunk adds exactly nothing)
-    const bool skip = !PLAIN && BK == 16 && nzb != nullptr && nch <= 256;
+    const bool skip = BK == 16 && nzb != nullptr && nch <= 256;
     if (skip) {
       const uint8_t *nz = nzb + ((int64_t)sl * gridDim.y + cti) * nzk;
       const bool f = tid < nch && nz[tid] != 0;
@@ -316,7 +231,7 @@ __global__ __launch_bounds__(256, PLAIN ? 1 : 3) void k_gemm(
       nch = tot;
     }
     // executed chunks, counted when profiling
-    if (!PLAIN && nexec && tid == 0)
+    if (nexec && tid == 0)
       atomicAdd(nexec, (unsigned long long)nch);
     auto kchunk = [&](int ch) { return skip ? s_list[ch] * BK : ch * BK; };
     // multiply chunk ch out of LDS buffer ch & 1 (FP32: then add to FP64)
@@ -391,17 +306,7 @@ __global__ __launch_bounds__(256, PLAIN ? 1 : 3) void k_gemm(
           const int row = r0 + ti * 16 + MF::row(lg, r);
           const double v = ACC64 ? acc64[ACC64 ? ti : 0][tj][r]
                                  : (double)acc[ti][tj][r];
-          if (PLAIN) {
-            if (row < n) {
-              acc_e[tj] += v * z[row];
-              acc_l[tj] += v;
-            }
-            if (want_var && row <= n)
-              acc_v[tj] += v * (double)B[(int64_t)row * ldb + col];
-            if (want_var && row == n) acc_m[tj] += v;
-          } else {
-            if (row < n) acc_v[tj] += v * v;
-          }
+          if (row < n) acc_v[tj] += v * v;
         }
       }
     }
@@ -409,47 +314,17 @@ __global__ __launch_bounds__(256, PLAIN ? 1 : 3) void k_gemm(
   // the four lane groups of a wave share each column
 #pragma unroll
   for (int tj = 0; tj < 2; ++tj) {
-    acc_e[tj] += __shfl_xor(acc_e[tj], 16, 64);
-    acc_e[tj] += __shfl_xor(acc_e[tj], 32, 64);
-    acc_l[tj] += __shfl_xor(acc_l[tj], 16, 64);
-    acc_l[tj] += __shfl_xor(acc_l[tj], 32, 64);
     acc_v[tj] += __shfl_xor(acc_v[tj], 16, 64);
     acc_v[tj] += __shfl_xor(acc_v[tj], 32, 64);
-    acc_m[tj] += __shfl_xor(acc_m[tj], 16, 64);
-    acc_m[tj] += __shfl_xor(acc_m[tj], 32, 64);
   }
   if (lg != 0) return;
-  double *eo = est + (int64_t)sl * ldo;
-  double *vo = var ? var + (int64_t)sl * ldo : nullptr;
-  bool ill = false;
 #pragma unroll
   for (int tj = 0; tj < 2; ++tj) {
     const int64_t col = c0 + wave * 32 + tj * 16 + li;
-    if (col >= Cs) continue;
-    if (PLAIN) {
-      // residual check: the weights of an OK / EDK system sum to one
-      // exactly, so their sum's distance from one is rounding of the
-      // explicit inverse
-      if (method != SPK_M_SK && fabs(acc_l[tj] - 1.0) > kSumTol) ill = true;
-      const int64_t oc = cmap ? (int64_t)cmap[col] : col;
-      if (skm) {
-        // SK with the step mean m as known mean: m + lambda^T (z - m)
-        eo[oc] = acc_e[tj] + st.mean * (1.0 - acc_l[tj]);
-      } else if (isclose1(acc_l[tj])) {
-        eo[oc] = acc_e[tj];
-        if (want_var) vo[oc] = acc_v[tj] + acc_m[tj];
-      } else {
-        eo[oc] = z[nnb[(int64_t)sl * ldn + col]];
-        if (want_var) vo[oc] = 0.0;
-      }
-    } else {
-      // this row block's share of |L^-1 delta|^2
+    // this row block's share of |L^-1 delta|^2
+    if (col < Cs)
       qpart[((int64_t)sl * nrb + rbi) * ldab + col] = acc_v[tj];
-    }
   }
-  if (PLAIN && __ballot(ill) != 0ull && li == 0 &&
-      !(st.flags & SPK_ST_ILLCOND))
-    atomicOr(&sc[sl].flags, SPK_ST_ILLCOND);
 }
 
 // OK variance lambda.g + 2 mu (interp/steps.py:432-434): the FP64 base
@@ -1930,8 +1805,12 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
       rhs_budget = std::min<size_t>(std::max<size_t>(rhs_budget, tot / 8),
                                     (size_t)48 << 30);
   }
+  // plain path: right-hand sides of at most 4 GiB per launch (several steps
+  // where a step's fit, so that small grids fill the device)
+  const int64_t rowsR = N + p + 64;
+  const int64_t plain_budget = (int64_t)4 << 30;
   if (!batched) {
-    Cs = std::min<int64_t>(C, (int64_t)(rhs_budget / ((N + p + 64) * 8)));
+    Cs = std::min<int64_t>(C, plain_budget / (rowsR * 8));
   } else if (want_var) {
     // bytes per (step, station, cell): FP64 delta, plus the FP32 delta
     // or its three bfloat16 planes and the int8 planes in the mixed path
@@ -1941,16 +1820,23 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
   // whole 256-cell blocks of k_kgen: a block's cells share a table of
   // nearest stations for their local fits, so with stripes of whole blocks
   // a cell's block, and its results, do not depend on the stripe length
-  Cs = std::max<int64_t>(256, Cs / 256 * 256);
+  // (a stripe that takes all cells stays whole: a remainder of less than a
+  // block used to cost launches of its own)
+  if (Cs < C) Cs = std::max<int64_t>(256, Cs / 256 * 256);
   if (Cs > C) Cs = C;
   const int64_t ldk = round_up(Cs, 128);
+  const int gsteps =
+      batched ? 1
+              : (int)std::max<int64_t>(
+                    1, std::min<int64_t>(S, plain_budget / (rowsR * ldk * 8)));
   const int nrb = (int)ceil_div(N, 64);
   double *R = nullptr, *abuf = nullptr, *K64 = nullptr, *qpart = nullptr;
   double *kap_lam = nullptr;  // the condition estimate's two eigenvalues
   double *dual_ds = nullptr;  // per-step scratch of the dual-vector kernels
   float *K32 = nullptr;
   uint4 *Kb = nullptr;
-  int32_t *nnb = nullptr, *nrst = nullptr;
+  double *qplain = nullptr;  // plain path: shares per row tile
+  int32_t *nrst = nullptr;
   int8_t *B8 = nullptr;
   int *eb8 = nullptr;
   double *dmax = nullptr;
@@ -1972,8 +1858,10 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
     SPK_TRY(ws_get(ctx, "dual_ds", S * kDualSc * 8, (void **)&dual_ds));
   }
   if (!batched) {
-    SPK_TRY(ws_get(ctx, "R", (N + p + 64) * ldk * 8, (void **)&R));
-    SPK_TRY(ws_get(ctx, "nnb", ldk * 4, (void **)&nnb));
+    SPK_TRY(ws_get(ctx, "R", (size_t)gsteps * rowsR * ldk * 8, (void **)&R));
+    SPK_TRY(ws_get(ctx, "qplain",
+                   (size_t)gsteps * 3 * ceil_div(N + p, 64) * ldk * 8,
+                   (void **)&qplain));
   } else if (want_var) {
     // FP64 buffer for the batched FP64 path and for the steps the mixed
     // path promotes to FP64 (SPK_ST_FP64VAR)
@@ -2321,53 +2209,74 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
     double *eb = est + t0 * C;
     double *vbo = want_var ? var + t0 * C : nullptr;
     if (!batched) {
-      for (int s = 0; s < Sb; ++s) {
-        if (std::find(q.pinv.begin(), q.pinv.end(), s) != q.pinv.end())
-          hipLaunchKernelGGL(k_mark_pinv, dim3(1), dim3(64), 0, sm, q.sc + s);
+      for (int s : q.pinv)
+        hipLaunchKernelGGL(k_mark_pinv, dim3(1), dim3(64), 0, sm, q.sc + s);
+      for (int s0 = 0; s0 < Sb; s0 += gsteps) {
+        const int ns = std::min(gsteps, Sb - s0);
+        // row tiles of the group's largest system
+        int nm = 1;
+        for (int s = s0; s < s0 + ns; ++s) nm = std::max(nm, h_sc[s].n);
+        const int nrt = (int)ceil_div(nm + p, 64);
         for (int64_t cb = 0; cb < C; cb += Cs) {
           const int64_t cn = std::min<int64_t>(Cs, C - cb);
+          const unsigned gc = (unsigned)ceil_div(cn, 256);
           {
             ProfScope ps(ctx, "rhs_plain");
             hipLaunchKernelGGL(
-                k_rhs_plain, dim3((unsigned)ceil_div(cn, 256)), dim3(256), 0,
-                sm, sx, sy, q.idx + s * N, q.sc + s, gb + s, cx + cb, cy + cb,
-                cn, C, prob->cell_drift ? prob->cell_drift + cb : nullptr,
-                method, m, method == SPK_M_SK ? 1 : 0, mvg, R, ldk, nnb,
-                (const int *)nullptr);
+                k_plain_rhs,
+                dim3(gc, (unsigned)ceil_div(nm, kPlainStn), (unsigned)ns),
+                dim3(256), 0, sm, sx, sy, q.idx + s0 * N, N, q.sc + s0,
+                gb + s0, cx + cb, cy + cb, cn, C,
+                prob->cell_drift ? prob->cell_drift + cb : nullptr, method, m,
+                mvg, R, ldk, rowsR * ldk, (const int *)nullptr);
           }
-          SPK_TRY(check_launch("k_rhs_plain"));
+          SPK_TRY(check_launch("k_plain_rhs"));
           {
             ProfScope ps(ctx, "gemm_plain_f64");
             // k depth per LDS stage 8, 16 or 32 (the same products in the
-            // same order); a tuning run takes the first 1 024 cell tiles,
-            // whole waves of blocks at one, two or four blocks per CU
+            // same order); a tuning run takes the first 1 024 cell tiles
+            // of the group's largest system
             auto run = [&](int v, bool timing) -> int {
-              const int64_t cr =
-                  timing ? std::min<int64_t>(cn, 1024 * 128) : cn;
-              auto k = v == 0   ? k_gemm<double, true, 8>
-                       : v == 2 ? k_gemm<double, true, 32>
-                                : k_gemm<double, true, 16>;
+              int s1 = s0, n1 = ns;
+              int64_t cr = cn;
+              if (timing) {
+                for (int s = s0; s < s0 + ns; ++s)
+                  if (h_sc[s].n == nm) s1 = s;
+                n1 = 1;
+                cr = std::min<int64_t>(cn, 1024 * 128);
+              }
+              auto k = v == 0   ? k_plain_gemm<8>
+                       : v == 2 ? k_plain_gemm<32>
+                                : k_plain_gemm<16>;
               hipLaunchKernelGGL(
-                  k, dim3((unsigned)ceil_div(cr, 128), 1), dim3(256), 0, sm,
-                  q.M + s * strideM, ld, (int64_t)0, R, ldk, (int64_t)0,
-                  q.sc + s, p, method, want_var ? 1 : 0, skm,
-                  q.zact + s * ldz, ldz, nnb, ldk, (const double *)nullptr,
-                  (int64_t)0, cr, eb + s * C + cb,
-                  vbo ? vbo + s * C + cb : nullptr, C, 0, (double *)nullptr,
-                  0, (const uint8_t *)nullptr, (int64_t)0,
-                  (unsigned long long *)nullptr, (const int *)nullptr,
-                  (const int32_t *)nullptr);
-              return check_launch("k_gemm<double,plain>");
+                  k, dim3((unsigned)(nrt * ceil_div(cr, 128)), 1, (unsigned)n1),
+                  dim3(256), 0, sm, (const double *)(q.M + s1 * strideM), ld,
+                  strideM, (const double *)(R + (s1 - s0) * rowsR * ldk), ldk,
+                  rowsR * ldk, (const StepSc *)(q.sc + s1), p,
+                  want_var ? 1 : 0, (const double *)(q.zact + s1 * ldz), ldz,
+                  nrt, cr, qplain + (int64_t)(s1 - s0) * 3 * nrt * ldk, ldk,
+                  (const int *)nullptr);
+              return check_launch("k_plain_gemm");
             };
-            // steps the kernel skips (no system) are not timed
-            const int hs = h_sc[s].status;
-            if (hs != 0 && hs != SPK_ST_FAILED)
-              SPK_TRY(run(1, false));
-            else
+            // a group without a system to contract is not timed
+            bool any = false;
+            for (int s = s0; s < s0 + ns; ++s)
+              any = any || (h_sc[s].n == nm && (h_sc[s].status == 0 ||
+                                                h_sc[s].status == SPK_ST_FAILED));
+            if (any)
               SPK_TRY(tune_launch(ctx, "gemm_plain_f64",
-                                  (int)ceil_div(h_sc[s].n + p, 1024), sm, 3,
-                                  1, run));
+                                  (int)ceil_div(nm + p, 1024), sm, 3, 0, run));
+            else
+              SPK_TRY(run(0, false));
           }
+          hipLaunchKernelGGL(
+              k_plain_fin, dim3(gc, (unsigned)ns), dim3(256), 0, sm, sx, sy,
+              q.idx + s0 * N, N, q.sc + s0, p, method, want_var ? 1 : 0, skm,
+              q.zact + s0 * ldz, ldz, cx + cb, cy + cb,
+              (const double *)qplain, ldk, nrt, cn, eb + s0 * C + cb,
+              vbo ? vbo + s0 * C + cb : nullptr, C, kSumTol,
+              (const int *)nullptr, (const int32_t *)nullptr);
+          SPK_TRY(check_launch("k_plain_fin"));
         }
       }
     } else {
@@ -2467,14 +2376,11 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
         } else if (mixed) {
           ProfScope ps(ctx, "gemm_tri_f32");
           // k chunks of 16: FP32 sums of 32 products, 3 waves per SIMD
-          hipLaunchKernelGGL((k_gemm<float, false, 16>), grid, dim3(256), 0, sm,
+          hipLaunchKernelGGL((k_gemm<float, 16>), grid, dim3(256), 0, sm,
                              q.L32, ld, strideM, (const float *)K32, ldk,
-                             ld * ldk, q.sc, p, method, 1, 0, q.zact, ldz,
-                             (const int32_t *)nullptr, (int64_t)0, abuf, ldk,
-                             cn, eb + cb, vbo + cb, C, 1, qpart, nrb,
+                             ld * ldk, q.sc, ldk, cn, 1, qpart, nrb,
                              (const uint8_t *)nzb, nzk,
-                             prof_of(ctx).on ? prof_of(ctx).work : nullptr,
-                             (const int *)nullptr, (const int32_t *)nullptr);
+                             prof_of(ctx).on ? prof_of(ctx).work : nullptr);
         }
         {
           ProfScope ps(ctx, "gemm_tri_f64");
@@ -2511,8 +2417,9 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
         const int64_t ldkp = round_up(Csp, 128);
         const int nstr = (int)ceil_div(C, Csp);
         const int want_list = (method == SPK_M_OK && want_var) ? 1 : 0;
-        double *bwp, *gxy = nullptr, *Rp = nullptr;
-        int32_t *plist, *nnbp = nullptr;
+        const int nrtp = (int)ceil_div(N + p, 64);
+        double *bwp, *gxy = nullptr, *Rp = nullptr, *qp = nullptr;
+        int32_t *plist;
         int *pcnt;
         SPK_TRY(ws_get(ctx, "pinv_bw", 2 * ld * 8, (void **)&bwp));
         SPK_TRY(ws_get(ctx, "pinv_list", C * 4, (void **)&plist));
@@ -2520,7 +2427,8 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
         if (want_list) {
           SPK_TRY(ws_get(ctx, "pinv_gxy", 2 * C * 8, (void **)&gxy));
           SPK_TRY(ws_get(ctx, "R", (N + p + 64) * ldkp * 8, (void **)&Rp));
-          SPK_TRY(ws_get(ctx, "nnb", ldkp * 4, (void **)&nnbp));
+          SPK_TRY(ws_get(ctx, "qplain", (size_t)3 * nrtp * ldkp * 8,
+                         (void **)&qp));
         }
         for (int s : q.pinv) {
           ProfScope ps(ctx, "pinv_contract");
@@ -2547,21 +2455,27 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
           for (int k2 = 0; k2 < nstr; ++k2) {
             const int64_t off = (int64_t)k2 * Csp;
             const int64_t cn = std::min<int64_t>(Csp, C - off);
+            const int *cc = pcnt + 1 + k2;
             hipLaunchKernelGGL(
-                k_rhs_plain, dim3((unsigned)ceil_div(cn, 256)), dim3(256), 0,
-                sm, sx, sy, q.idx + s * N, q.sc + s, gb + s, gxy + off,
-                gxy + C + off, cn, C, (const double *)nullptr, method, m, 0,
-                mvg, Rp, ldkp, nnbp, (const int *)(pcnt + 1 + k2));
-            hipLaunchKernelGGL((k_gemm<double, true, 16>),
-                               dim3((unsigned)ceil_div(cn, 128), 1), dim3(256),
-                               0, sm, Ms, ld, (int64_t)0, Rp, ldkp, (int64_t)0,
-                               q.sc + s, p, method, 1, skm, q.zact + s * ldz,
-                               ldz, nnbp, ldkp, (const double *)nullptr,
-                               (int64_t)0, cn, eb + s * C, vbo + s * C, C, 0,
-                               (double *)nullptr, 0, (const uint8_t *)nullptr,
-                               (int64_t)0, (unsigned long long *)nullptr,
-                               (const int *)(pcnt + 1 + k2),
-                               (const int32_t *)(plist + off));
+                k_plain_rhs,
+                dim3((unsigned)ceil_div(cn, 256),
+                     (unsigned)ceil_div(N, kPlainStn), 1),
+                dim3(256), 0, sm, sx, sy, q.idx + s * N, N, q.sc + s, gb + s,
+                gxy + off, gxy + C + off, cn, C, (const double *)nullptr,
+                method, m, mvg, Rp, ldkp, (int64_t)0, cc);
+            hipLaunchKernelGGL(
+                k_plain_gemm<8>,
+                dim3((unsigned)(nrtp * ceil_div(cn, 128)), 1, 1), dim3(256), 0,
+                sm, Ms, ld, (int64_t)0, (const double *)Rp, ldkp, (int64_t)0,
+                (const StepSc *)(q.sc + s), p, 1,
+                (const double *)(q.zact + s * ldz), ldz, nrtp, cn, qp, ldkp,
+                cc);
+            hipLaunchKernelGGL(
+                k_plain_fin, dim3((unsigned)ceil_div(cn, 256), 1), dim3(256),
+                0, sm, sx, sy, q.idx + s * N, N, q.sc + s, p, method, 1, skm,
+                q.zact + s * ldz, ldz, gxy + off, gxy + C + off,
+                (const double *)qp, ldkp, nrtp, cn, eb + s * C, vbo + s * C, C,
+                kSumTol, cc, (const int32_t *)(plist + off));
           }
           SPK_TRY(check_launch("pinv contraction"));
         }

@@ -57,6 +57,32 @@ __global__ void k_idw_mfma(const double *sx, const double *sy, int64_t N,
                            int64_t ldz, const double *cx, const double *cy,
                            int64_t C, double p, double *est, int *bad);
 
+// ---- plain FP64 contraction (spk_plain.hip) ---------------------------------
+// stations per block of k_plain_rhs (grid.y = ceil(stations / kPlainStn))
+constexpr int kPlainStn = 128;
+__global__ void k_plain_rhs(const double *sx, const double *sy,
+                            const int32_t *idx, int64_t N, const StepSc *sc,
+                            const spk_vg *vgs, const double *cx,
+                            const double *cy, int64_t Cs, int64_t ldd,
+                            const double *cell_drift, int method, int m,
+                            double min_vg_val, double *R, int64_t ldr,
+                            int64_t strideR, const int *ccount);
+template <int BK>
+__global__ void k_plain_gemm(const double *M, int64_t lda, int64_t strideM,
+                             const double *R, int64_t ldr, int64_t strideR,
+                             const StepSc *sc, int p, int want_var,
+                             const double *zact, int64_t ldz, int nrt,
+                             int64_t Cs, double *part, int64_t ldq,
+                             const int *ccount);
+__global__ void k_plain_fin(const double *sx, const double *sy,
+                            const int32_t *idx, int64_t N, StepSc *sc, int p,
+                            int method, int want_var, int skm,
+                            const double *zact, int64_t ldz, const double *cx,
+                            const double *cy, const double *part, int64_t ldq,
+                            int nrt, int64_t Cs, double *est, double *var,
+                            int64_t ldo, double sum_tol, const int *ccount,
+                            const int32_t *cmap);
+
 // ---- pseudo-inverse fallback of failed steps (spk_pinv.hip) ----------------
 // For the steps `steps` of a batch (step records sc on the device, their
 // host copies h_sc): builds each bordered system, zero-padded to the

@@ -570,3 +570,49 @@ def test_int8_plane_contraction_matches_fp64(gpu):
     assert rv[sel & (k <= 1e6)].max(initial=0.0) < 1e-7
     assert rv[sel & (k <= 1e8)].max(initial=0.0) < 1e-5
     assert rv[sel].max() < 1e-4
+
+
+@pytest.mark.parametrize('n,cells,method', [
+    (2, 1, 'OK'), (63, 129, 'OK'), (64, 257, 'EDK'), (129, 300, 'SKM'),
+    (130, 127, 'SK'), (191, 513, 'OK')])
+def test_plain_tiles_edges(gpu, n, cells, method):
+    """The plain contraction's 64-row x 128-cell tiles, 128-station chunks
+    of right-hand sides and several steps per launch at their edges: steps
+    of different station counts in one call, with the systems' rows (n + the
+    constraint rows) below, at and above a tile, against the exact solution
+    (1e-9 as for every well-conditioned system; the reference's SK against
+    the oracle, which shares its sum-of-weights test)."""
+    from spinterps_amd.interp.steps import DeviceProblem, interp_steps
+    rng = np.random.default_rng(n * 1000 + cells)
+    sx, sy = rng.uniform(0, 1e5, n), rng.uniform(0, 1e5, n)
+    cx, cy = rng.uniform(0, 1e5, cells), rng.uniform(0, 1e5, cells)
+    sd = (sx / 1e5 + np.sin(sy / 2e4))[:, None]
+    cd = (cx / 1e5 + np.sin(cy / 2e4))[None]
+    vals = rng.gamma(2.0, 3.0, (5, n))
+    vals[1, :n // 3] = np.nan
+    vals[3, n // 2:] = np.nan
+    vgs = ['0.1 Nug(0.0) + 0.9 Sph(30000.0)', '1.2 Exp(20000.0)',
+           '0.3 Nug(0.0) + 2.0 Gau(4000.0)', '0.5 Sph(9e3) + 0.5 Exp(3e4)',
+           '0.1 Nug(0.0) + 0.7 Exp(5e4) + 0.2 Lin(4e3)']
+    prob = DeviceProblem(sx, sy, cx, cy, sd if method == 'EDK' else None,
+                         cd if method == 'EDK' else None)
+    est, var, info = interp_steps(prob, vals, vgs, method)
+    est = est.cpu().numpy()
+    for t in range(5):
+        a = ~np.isnan(vals[t])
+        if a.sum() < 2 or int(info[t]) & (4 | 8 | 128):
+            continue
+        dd = O.dists_2d(sx[a], sy[a], sx[a], sy[a])
+        rd = O.dists_2d(cx, cy, sx[a], sy[a])
+        z = vals[t, a]
+        if method == 'SK':
+            K, R = O.krig_system('SK', vgs[t], dd, rd, None, None, 0.0)
+            ref, v = O.krige_solve(K, R, z, rd, False)[:2]
+        else:
+            ref, v, _ = O.krige_exact(method, vgs[t], dd, rd, z, sd[a], cd,
+                                      want_var=method == 'OK')
+        sc = np.abs(z).mean()
+        assert np.abs(est[t] - ref).max() <= 1e-9 * max(1.0, sc), (t, method)
+        if method == 'OK':
+            np.testing.assert_allclose(var[t].cpu().numpy(), v, rtol=1e-9,
+                                       atol=1e-9 * np.abs(v).mean())
