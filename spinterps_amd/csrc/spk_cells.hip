@@ -2017,23 +2017,8 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
       ProfScope ps(ctx, "potrf", sf);
       SPK_TRY(graph_run(ctx, "potrf", gk.v, sf, [&]() -> int {
         // the systems have at most N rows: the panels of the largest
-        if (method != SPK_M_SK)
-          hipLaunchKernelGGL(k_chol_shift, dim3(Sb), dim3(256), 0, sf, q.A,
-                             ld, strideM, q.sc, (const spk_vg *)q.vg);
-        for (int k0 = 0; k0 < N; k0 += 32) {
-          hipLaunchKernelGGL(k_chol_diag, dim3(1, Sb), dim3(256), 0, sf, q.A,
-                             ld, strideM, q.sc, k0);
-          const int64_t below = N - (k0 + 32);
-          if (below <= 0) break;
-          hipLaunchKernelGGL(k_chol_solve,
-                             dim3((unsigned)ceil_div(below, 256), Sb),
-                             dim3(256), 0, sf, q.A, ld, strideM, q.sc, k0);
-          const int64_t nt = ceil_div(below, 64);
-          hipLaunchKernelGGL(k_chol_trail,
-                             dim3((unsigned)(nt * (nt + 1) / 2), Sb),
-                             dim3(256), 0, sf, q.A, ld, strideM, q.sc, k0);
-        }
-        return check_launch("k_potrf");
+        return chol_steps(sf, q.A, ld, strideM, q.sc, (const spk_vg *)q.vg,
+                          method != SPK_M_SK ? 1 : 0, N, Sb);
       }));
     }
     // which steps failed the Cholesky (the host waits for this batch's
@@ -2046,23 +2031,17 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
       if (h_sc[s2].status == SPK_ST_FAILED) q.pinv.push_back(s2);
     {
       ProfScope ps(ctx, "trtri", sf);
-      const dim3 gt((unsigned)ceil_div(N, 64), Sb);
-      hipLaunchKernelGGL(k_trtri_diag, gt, dim3(256), 0, sf, q.A, q.Li, ld,
-                         strideM, q.sc);
-      hipLaunchKernelGGL(k_trtri_cols, gt, dim3(256), 0, sf, q.A, q.Li, ld,
-                         strideM, q.sc);
+      SPK_TRY(trtri_steps(sf, q.A, q.Li, ld, strideM, q.sc, N, Sb));
     }
-    SPK_TRY(check_launch("k_trtri"));
     if (!batched) {
       ProfScope ps(ctx, "minv", sf);
-      hipLaunchKernelGGL(k_minv, dim3(Sb), dim3(256), 0, sf, q.Li, ld, strideM,
-                         q.sc, q.idx, N, prob->stn_drift, m, method, q.M, q.T0,
-                         gb, mvg);
+      SPK_TRY(minv_steps(sf, q.Li, ld, strideM, q.sc, q.idx, N,
+                         prob->stn_drift, m, method, q.M, q.T0, gb, mvg, Sb));
     } else {
       {
         // condition estimate (power iteration over (row blocks, steps))
         ProfScope ps(ctx, "kappa", sf);
-        const unsigned gl = (unsigned)ceil_div(N, 256);
+        const unsigned gl = (unsigned)ceil_div(N, 64);
         const unsigned gu = (unsigned)ceil_div(N, 4);
         GraphKey kk = gk;
         kk << kap_lam << fp64var_thr << fp64var_thr_gau << int8var_thr;
@@ -2098,7 +2077,7 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
       }
       {
         ProfScope ps(ctx, "dual", sf);
-        const unsigned gl = (unsigned)ceil_div(N, 256);
+        const unsigned gl = (unsigned)ceil_div(N, 64);
         const unsigned gu = (unsigned)ceil_div(N, 4);
         const int pq = method == SPK_M_EDK ? 1 + m : 1;
         GraphKey dk = gk;

@@ -2,13 +2,15 @@
 // Cholesky, triangular inverse, the dual-form vectors of the batched path
 // and the explicit inverse operator of the plain path.
 //
-// Every kernel here runs one workgroup per time step (blockIdx.x = step),
-// so a launch factorises a whole batch of uneven systems at once.  Matrices
-// are column-major with a common leading dimension `ld`.
+// Every launch covers a whole batch of uneven systems, over (blocks, steps)
+// or one workgroup per step for the small parts.  Matrices are column-major
+// with a common leading dimension `ld`.
 //
 // Reference: interp/steps.py:170-243 (system layout), :350-371 (inverse),
 // misc.py:1074-1105 (nugget-only check), interp/steps.py:276, :760-765
 // (step means and interpolation flags).
+#include <algorithm>
+
 #include "spk_krige.h"
 
 namespace spk {
@@ -162,220 +164,33 @@ __global__ __launch_bounds__(256) void k_assemble(
 // largest entry plus the sill sum).  The constant shift leaves the kriging
 // weights unchanged because they sum to one, which is also why the
 // reference's nugget (added to every entry, pyx:192-201) cancels.  Then
-// C = L L^T, right-looking, 32-wide panels, 64x64 trailing tiles.  A failed
-// pivot marks the step SPK_ST_FAILED, which interp/steps.py:363-384 answers
-// with the nearest station's value.
-__global__ __launch_bounds__(256) void k_potrf(double *__restrict__ A,
-                                               int64_t ld, int64_t strideA,
-                                               StepSc *__restrict__ sc,
-                                               const spk_vg *__restrict__ vgs,
-                                               int shift) {
-  const int s = blockIdx.x;
-  if (sc[s].status) return;
-  const int n = sc[s].n;
-  double *As = A + (int64_t)s * strideA;
-  const int tid = threadIdx.x;
-  __shared__ double D[32][33];
-  __shared__ double Pa[64][33];
-  __shared__ double Pb[64][33];
-  __shared__ int fail;
-  __shared__ double red[256];
-  __shared__ double c0s;
+// C = L L^T, right-looking, in 64-wide panels: k_chol_diag factors the
+// panel's diagonal block, k_chol_solve solves the rows below it,
+// k_chol_trail subtracts the panel's outer product from the trailing
+// triangle on FP64 MFMA.  A failed pivot marks the step SPK_ST_FAILED
+// (interp/steps.py:363-384), after which its later launches return at once.
+// 32-wide panels on the vector ALU read and wrote the trailing triangle
+// twice as often and multiplied out of LDS at two reads per four products:
+// 16 steps of up to 2 000 stations took 13 ms (shift 4.9 with one workgroup
+// per step, diagonal 1.5, solve 0.6, trailing 6.2), now 2.2 (0.05, 0.7, 0.6,
+// 0.8).
 
-  if (shift) {
-    const spk_vg &vg = vgs[s];
-    bool bounded = true;
-    for (int k = 0; k < vg.n; ++k) {
-      const int ty = vg.type[k];
-      if (ty == SPK_VG_RNG || ty == SPK_VG_POW || ty == SPK_VG_HOL)
-        bounded = false;
-    }
-    if (bounded) {
-      if (tid == 0) c0s = vg.sill_sum;
-    } else {
-      double mx = 0.0;
-      for (int64_t e = tid; e < (int64_t)n * n; e += 256) {
-        const int i = (int)(e % n), j = (int)(e / n);
-        if (i >= j) mx = fmax(mx, fabs(As[i + (int64_t)j * ld]));
-      }
-      red[tid] = mx;
-      __syncthreads();
-      for (int w = 128; w > 0; w >>= 1) {
-        if (tid < w) red[tid] = fmax(red[tid], red[tid + w]);
-        __syncthreads();
-      }
-      if (tid == 0) c0s = 2.0 * red[0] + fabs(vg.sill_sum);
-    }
-    __syncthreads();
-    const double c0 = c0s;
-    for (int64_t e = tid; e < (int64_t)n * n; e += 256) {
-      const int i = (int)(e % n), j = (int)(e / n);
-      if (i >= j) As[i + (int64_t)j * ld] = c0 - As[i + (int64_t)j * ld];
-    }
-    if (tid == 0) sc[s].c0 = c0;
-  }
-  if (tid == 0) fail = 0;
-  __syncthreads();
-
-  for (int k0 = 0; k0 < n; k0 += 32) {
-    const int jb = min(32, n - k0);
-    for (int e = tid; e < 32 * 32; e += 256) {
-      const int i = e & 31, j = e >> 5;
-      D[i][j] = (i < jb && j < jb && i >= j)
-                    ? As[(k0 + i) + (int64_t)(k0 + j) * ld]
-                    : 0.0;
-    }
-    __syncthreads();
-    for (int j = 0; j < jb; ++j) {
-      if (tid == 0) {
-        const double d = D[j][j];
-        if (!(d > 0.0) || !isfinite(d))
-          fail = k0 + j + 1;
-        else
-          D[j][j] = sqrt(d);
-      }
-      __syncthreads();
-      if (fail) break;
-      if (tid > j && tid < jb) D[tid][j] /= D[j][j];
-      __syncthreads();
-      for (int e = tid; e < 32 * 32; e += 256) {
-        const int i = e & 31, c = e >> 5;
-        if (c > j && i >= c && i < jb) D[i][c] -= D[i][j] * D[c][j];
-      }
-      __syncthreads();
-    }
-    if (fail) break;
-    for (int e = tid; e < 32 * 32; e += 256) {
-      const int i = e & 31, j = e >> 5;
-      if (i < jb && j < jb && i >= j)
-        As[(k0 + i) + (int64_t)(k0 + j) * ld] = D[i][j];
-    }
-    // panel: rows r >= k0 + jb solve x L_kk^T = a
-    for (int r = k0 + jb + tid; r < n; r += 256) {
-      double x[32];
-#pragma unroll
-      for (int c = 0; c < 32; ++c)
-        x[c] = c < jb ? As[r + (int64_t)(k0 + c) * ld] : 0.0;
-#pragma unroll
-      for (int c = 0; c < 32; ++c) {
-        if (c < jb) {
-          double v = x[c];
-#pragma unroll
-          for (int q = 0; q < c; ++q) v -= x[q] * D[c][q];
-          x[c] = v / D[c][c];
-        }
-      }
-#pragma unroll
-      for (int c = 0; c < 32; ++c)
-        if (c < jb) As[r + (int64_t)(k0 + c) * ld] = x[c];
-    }
-    __syncthreads();
-    // trailing update of rows/cols >= m0
-    const int m0 = k0 + jb;
-    const int mt = n - m0;
-    if (mt <= 0) break;
-    const int nt = (mt + 63) / 64;
-    const int ty = tid >> 4, tx = tid & 15;
-    // tiles (bi, bj <= bi) in order; the next tile's panel rows are loaded
-    // into registers while this tile is updated (the panel columns are not
-    // written by the trailing update)
-    double qa[8], qb[8], qc[4][4];
-    auto fetch = [&](int bi, int bj) {
-      const int i0 = m0 + bi * 64, j0 = m0 + bj * 64;
-#pragma unroll
-      for (int q = 0; q < 8; ++q) {
-        const int e = tid + q * 256;
-        const int r = e & 63, c = e >> 6;
-        qa[q] = (i0 + r < n && c < jb) ? As[(i0 + r) + (int64_t)(k0 + c) * ld]
-                                       : 0.0;
-        qb[q] = (j0 + r < n && c < jb) ? As[(j0 + r) + (int64_t)(k0 + c) * ld]
-                                       : 0.0;
-      }
-      // the tile's own entries (tiles are disjoint)
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const int i = i0 + ty * 4 + a, j = j0 + tx * 4 + b;
-          qc[a][b] = (i < n && j < n && i >= j) ? As[i + (int64_t)j * ld] : 0.0;
-        }
-    };
-    fetch(0, 0);
-    for (int bi = 0; bi < nt; ++bi) {
-      for (int bj = 0; bj <= bi; ++bj) {
-        const int i0 = m0 + bi * 64, j0 = m0 + bj * 64;
-#pragma unroll
-        for (int q = 0; q < 8; ++q) {
-          const int e = tid + q * 256;
-          Pa[e & 63][e >> 6] = qa[q];
-          Pb[e & 63][e >> 6] = qb[q];
-        }
-        double cur[4][4];
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-          for (int b = 0; b < 4; ++b) cur[a][b] = qc[a][b];
-        __syncthreads();
-        if (bj < bi)
-          fetch(bi, bj + 1);
-        else if (bi + 1 < nt)
-          fetch(bi + 1, 0);
-        double acc[4][4];
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-          for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-        for (int c = 0; c < jb; ++c) {
-          double pa[4], pb[4];
-#pragma unroll
-          for (int a = 0; a < 4; ++a) pa[a] = Pa[ty * 4 + a][c];
-#pragma unroll
-          for (int b = 0; b < 4; ++b) pb[b] = Pb[tx * 4 + b][c];
-#pragma unroll
-          for (int a = 0; a < 4; ++a)
-#pragma unroll
-            for (int b = 0; b < 4; ++b) acc[a][b] += pa[a] * pb[b];
-        }
-#pragma unroll
-        for (int a = 0; a < 4; ++a) {
-          const int i = i0 + ty * 4 + a;
-#pragma unroll
-          for (int b = 0; b < 4; ++b) {
-            const int j = j0 + tx * 4 + b;
-            if (i < n && j < n && i >= j)
-              As[i + (int64_t)j * ld] = cur[a][b] - acc[a][b];
-          }
-        }
-        __syncthreads();
-      }
-    }
-  }
-  __syncthreads();
-  if (tid == 0 && fail) sc[s].status = SPK_ST_FAILED;
+typedef double f4d_t __attribute__((ext_vector_type(4)));
+__device__ inline f4d_t mfma64(double a, double b, f4d_t c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// ---- Cholesky over (block, step) workgroups ------------------------------------
-// The same factorisation as k_potrf, with the same operations in the same
-// order (bit-identical results), spread over many workgroups: k_chol_shift
-// forms C = c0 - G (one workgroup per step); then per 32-wide panel k0,
-// k_chol_diag factors the panel's diagonal block, k_chol_solve solves 256
-// of the rows below it per workgroup, and k_chol_trail updates the
-// trailing triangle, one 64 x 64 tile per workgroup.  A failed pivot sets
-// SPK_ST_FAILED, after which the step's later launches return at once.
-// (Panels of 32 rows only: a panel shorter than 32 is the last one and
-// leaves nothing below it.)
-__global__ __launch_bounds__(256) void k_chol_shift(double *__restrict__ A,
-                                                    int64_t ld,
-                                                    int64_t strideA,
-                                                    StepSc *__restrict__ sc,
-                                                    const spk_vg *__restrict__ vgs) {
+// c0 of every step (grid (steps)).
+__global__ __launch_bounds__(256) void k_chol_c0(const double *__restrict__ A,
+                                                 int64_t ld, int64_t strideA,
+                                                 StepSc *__restrict__ sc,
+                                                 const spk_vg *__restrict__ vgs) {
   const int s = blockIdx.x;
   if (sc[s].status) return;
   const int n = sc[s].n;
-  double *As = A + (int64_t)s * strideA;
+  const double *As = A + (int64_t)s * strideA;
   const int tid = threadIdx.x;
   __shared__ double red[256];
-  __shared__ double c0s;
   const spk_vg &vg = vgs[s];
   bool bounded = true;
   for (int k = 0; k < vg.n; ++k) {
@@ -384,68 +199,100 @@ __global__ __launch_bounds__(256) void k_chol_shift(double *__restrict__ A,
       bounded = false;
   }
   if (bounded) {
-    if (tid == 0) c0s = vg.sill_sum;
-  } else {
-    double mx = 0.0;
-    for (int64_t e = tid; e < (int64_t)n * n; e += 256) {
-      const int i = (int)(e % n), j = (int)(e / n);
-      if (i >= j) mx = fmax(mx, fabs(As[i + (int64_t)j * ld]));
-    }
-    red[tid] = mx;
-    __syncthreads();
-    for (int w = 128; w > 0; w >>= 1) {
-      if (tid < w) red[tid] = fmax(red[tid], red[tid + w]);
-      __syncthreads();
-    }
-    if (tid == 0) c0s = 2.0 * red[0] + fabs(vg.sill_sum);
+    if (tid == 0) sc[s].c0 = vg.sill_sum;
+    return;
   }
-  __syncthreads();
-  const double c0 = c0s;
+  double mx = 0.0;
   for (int64_t e = tid; e < (int64_t)n * n; e += 256) {
     const int i = (int)(e % n), j = (int)(e / n);
-    if (i >= j) As[i + (int64_t)j * ld] = c0 - As[i + (int64_t)j * ld];
+    if (i >= j) mx = fmax(mx, fabs(As[i + (int64_t)j * ld]));
   }
-  if (tid == 0) sc[s].c0 = c0;
+  red[tid] = mx;
+  __syncthreads();
+  for (int w = 128; w > 0; w >>= 1) {
+    if (tid < w) red[tid] = fmax(red[tid], red[tid + w]);
+    __syncthreads();
+  }
+  if (tid == 0) sc[s].c0 = 2.0 * red[0] + fabs(vg.sill_sum);
 }
 
-// the panel's 32 x 32 diagonal block, factored in LDS and written back;
-// grid (1, steps)
+// A <- c0 - A on the lower triangle; grid (column groups, steps), block x
+// takes columns x, x + gridDim.x, ...
+__global__ __launch_bounds__(256) void k_chol_shift(double *__restrict__ A,
+                                                    int64_t ld,
+                                                    int64_t strideA,
+                                                    const StepSc *__restrict__ sc) {
+  const int s = blockIdx.y;
+  if (sc[s].status) return;
+  const int n = sc[s].n;
+  const double c0 = sc[s].c0;
+  double *As = A + (int64_t)s * strideA;
+  for (int j = blockIdx.x; j < n; j += gridDim.x)
+    for (int i = j + (int)threadIdx.x; i < n; i += 256)
+      As[i + (int64_t)j * ld] = c0 - As[i + (int64_t)j * ld];
+}
+
+__device__ inline double lane_value(double v, int src) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_readlane((int)b, src);
+  const int hi = __builtin_amdgcn_readlane((int)(b >> 32), src);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
+}
+
+// The panel's 64 x 64 diagonal block in LDS, 16 columns at a time: the first
+// wave factors the 16 columns with row i in lane i's registers (pivots and
+// multipliers by readlane, no barrier inside), then all waves update the
+// columns to their right.  Bound by the chain of 64 reciprocal square roots;
+// 32 columns with three barriers each took 24 us, 64 now 22 us.
+// grid (steps)
 __global__ __launch_bounds__(256) void k_chol_diag(double *__restrict__ A,
                                                    int64_t ld, int64_t strideA,
                                                    StepSc *__restrict__ sc,
                                                    int k0) {
-  const int s = blockIdx.y;
+  const int s = blockIdx.x;
   if (sc[s].status) return;
   const int n = sc[s].n;
   if (k0 >= n) return;
-  const int jb = min(32, n - k0);
+  const int jb = min(64, n - k0);
   double *As = A + (int64_t)s * strideA;
-  const int tid = threadIdx.x;
-  __shared__ double D[32][33];
+  const int tid = threadIdx.x, lane = tid & 63;
+  __shared__ double D[64][65];  // D[column][row]
   __shared__ int fail;
   if (tid == 0) fail = 0;
-  for (int e = tid; e < 32 * 32; e += 256) {
-    const int i = e & 31, j = e >> 5;
-    D[i][j] = (i < jb && j < jb && i >= j)
+  for (int e = tid; e < 64 * 64; e += 256) {
+    const int i = e & 63, j = e >> 6;
+    D[j][i] = (i < jb && j < jb && i >= j)
                   ? As[(k0 + i) + (int64_t)(k0 + j) * ld]
-                  : 0.0;
+                  : (i == j ? 1.0 : 0.0);
   }
   __syncthreads();
-  for (int j = 0; j < jb; ++j) {
-    if (tid == 0) {
-      const double d = D[j][j];
-      if (!(d > 0.0) || !isfinite(d))
-        fail = k0 + j + 1;
-      else
-        D[j][j] = sqrt(d);
+  for (int b = 0; b < jb; b += 16) {
+    if (tid < 64) {
+      double a[16];
+#pragma unroll
+      for (int c = 0; c < 16; ++c) a[c] = D[b + c][lane];
+      bool bad = false;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) {
+        const double d = lane_value(a[j], b + j);
+        bad = bad || !(d > 0.0) || !isfinite(d);
+        const double l = a[j] * rsqrt(d);  // d / sqrt(d) at the pivot
+        a[j] = l;
+#pragma unroll
+        for (int c = j + 1; c < 16; ++c) a[c] -= l * lane_value(l, b + c);
+      }
+#pragma unroll
+      for (int c = 0; c < 16; ++c) D[b + c][lane] = a[c];
+      if (bad && lane == 0) fail = 1;
     }
     __syncthreads();
     if (fail) break;
-    if (tid > j && tid < jb) D[tid][j] /= D[j][j];
-    __syncthreads();
-    for (int e = tid; e < 32 * 32; e += 256) {
-      const int i = e & 31, c = e >> 5;
-      if (c > j && i >= c && i < jb) D[i][c] -= D[i][j] * D[c][j];
+    // columns b + 16 .. 63, rows from the diagonal down
+    for (int c = b + 16 + (tid >> 6); c < 64; c += 4) {
+      double v = D[c][lane];
+#pragma unroll
+      for (int j = 0; j < 16; ++j) v -= D[b + j][lane] * D[b + j][c];
+      D[c][lane] = v;
     }
     __syncthreads();
   }
@@ -453,59 +300,95 @@ __global__ __launch_bounds__(256) void k_chol_diag(double *__restrict__ A,
     if (tid == 0) sc[s].status = SPK_ST_FAILED;
     return;
   }
-  for (int e = tid; e < 32 * 32; e += 256) {
-    const int i = e & 31, j = e >> 5;
+  for (int e = tid; e < 64 * 64; e += 256) {
+    const int i = e & 63, j = e >> 6;
     if (i < jb && j < jb && i >= j)
-      As[(k0 + i) + (int64_t)(k0 + j) * ld] = D[i][j];
+      As[(k0 + i) + (int64_t)(k0 + j) * ld] = D[j][i];
   }
 }
 
-// rows r >= k0 + 32 solve x L_kk^T = a, 256 rows per workgroup;
-// grid (rows below the panel / 256, steps)
-__global__ __launch_bounds__(256) void k_chol_solve(double *__restrict__ A,
-                                                    int64_t ld,
-                                                    int64_t strideA,
-                                                    const StepSc *__restrict__ sc,
-                                                    int k0) {
-  const int s = blockIdx.y;
-  if (sc[s].status) return;
-  const int n = sc[s].n;
-  if (k0 + 32 >= n) return;
-  const int jb = 32, m0 = k0 + 32;
-  const int rbase = m0 + (int)blockIdx.x * 256;
-  if (rbase >= n) return;
-  double *As = A + (int64_t)s * strideA;
-  const int tid = threadIdx.x;
-  __shared__ double D[32][33];
-  for (int e = tid; e < 32 * 32; e += 256) {
-    const int i = e & 31, j = e >> 5;
-    D[i][j] = (i >= j) ? As[(k0 + i) + (int64_t)(k0 + j) * ld] : 0.0;
-  }
-  __syncthreads();
-  const int r = rbase + tid;
-  if (r < n) {
-    double x[32];
+// Forward substitution L x = a for 64 right-hand sides, one per lane of a
+// wave: 16 unknowns at a time in registers, first reduced by the earlier ones
+// (kept in LDS, as many FMAs as 16-byte broadcasts of L allow), then solved
+// among themselves.  Lt[q][c] = L[c][q], dinv[c] = 1 / L[c][c], a(c) the
+// lane's right-hand side, done(c, x) takes the results.  The loops over the
+// blocks stay rolled: fully unrolled, with all 64 unknowns in registers, the
+// 35 KB of code took 50 to 78 us per launch, bound by instruction fetch; this
+// takes 18 to 33.
+template <typename A, typename D>
+__device__ inline void wave_fwd_subst(const double (*Lt)[64],
+                                      const double *dinv, double (*Xs)[64],
+                                      A a, D done) {
+  const int lane = threadIdx.x & 63;
+#pragma unroll 1
+  for (int b = 0; b < 64; b += 16) {
+    double x[16];
 #pragma unroll
-    for (int c = 0; c < 32; ++c)
-      x[c] = c < jb ? As[r + (int64_t)(k0 + c) * ld] : 0.0;
+    for (int c = 0; c < 16; ++c) x[c] = a(b + c);
+#pragma unroll 2
+    for (int k = 0; k < b; ++k) {
+      const double xk = Xs[k][lane];
 #pragma unroll
-    for (int c = 0; c < 32; ++c) {
-      if (c < jb) {
-        double v = x[c];
-#pragma unroll
-        for (int q = 0; q < c; ++q) v -= x[q] * D[c][q];
-        x[c] = v / D[c][c];
-      }
+      for (int c = 0; c < 16; ++c) x[c] -= Lt[k][b + c] * xk;
     }
 #pragma unroll
-    for (int c = 0; c < 32; ++c)
-      if (c < jb) As[r + (int64_t)(k0 + c) * ld] = x[c];
+    for (int c = 0; c < 16; ++c) {
+#pragma unroll
+      for (int q = 0; q < c; ++q) x[c] -= x[q] * Lt[b + q][b + c];
+      x[c] *= dinv[b + c];
+    }
+#pragma unroll
+    for (int c = 0; c < 16; ++c) {
+      if (b < 48) Xs[b + c][lane] = x[c];
+      done(b + c, x[c]);
+    }
   }
 }
 
+// rows r >= k0 + 64 solve x L_kk^T = a, one row per lane, 64 rows per
+// workgroup (one wave: few rows are left in most panels);
+// grid (rows below the panel / 64, steps)
+__global__ __launch_bounds__(64) void k_chol_solve(double *__restrict__ A,
+                                                   int64_t ld,
+                                                   int64_t strideA,
+                                                   const StepSc *__restrict__ sc,
+                                                   int k0) {
+  const int s = blockIdx.y;
+  if (sc[s].status) return;
+  const int n = sc[s].n;
+  const int rbase = k0 + 64 + (int)blockIdx.x * 64;
+  if (rbase >= n) return;
+  double *As = A + (int64_t)s * strideA;
+  const int lane = threadIdx.x;
+  __shared__ __align__(16) double Lt[64][64];
+  __shared__ double Xs[48][64];
+  __shared__ double dinv[64];
+#pragma unroll 16
+  for (int j = 0; j < 64; ++j)
+    Lt[j][lane] = As[(k0 + lane) + (int64_t)(k0 + j) * ld];
+  __syncthreads();
+  dinv[lane] = 1.0 / Lt[lane][lane];
+  __syncthreads();
+  const int r = rbase + lane;
+  const double *in = As + min(r, n - 1) + (int64_t)k0 * ld;
+  double *out = As + r + (int64_t)k0 * ld;
+  wave_fwd_subst(
+      Lt, dinv, Xs, [&](int c) { return in[(int64_t)c * ld]; },
+      [&](int c, double x) {
+        if (r < n) out[(int64_t)c * ld] = x;
+      });
+}
+
+// Trailing triangle -= P P^T, one 64 x 64 tile per workgroup, each wave
+// 32 x 32 of it as 2 x 2 MFMA tiles; the panel's fragments come straight
+// from memory (16 consecutive rows per lane group).  The product is formed
+// transposed, so that a lane group's results are 16 consecutive rows too.
+// Bound by the triangle's read and write.  Rows from n to the tile's end lie
+// inside the slab (ld is a multiple of 64); what they hold only reaches
+// entries that are not stored.
 // grid (tiles of the largest trailing triangle, steps): tile t = (bi, bj),
-// bj <= bi, t = bi (bi + 1) / 2 + bj, of the rows / columns >= k0 + 32
-__global__ __launch_bounds__(256) void k_chol_trail(double *__restrict__ A,
+// bj <= bi, t = bi (bi + 1) / 2 + bj, of the rows / columns >= k0 + 64
+__global__ __launch_bounds__(256, 2) void k_chol_trail(double *__restrict__ A,
                                                     int64_t ld,
                                                     int64_t strideA,
                                                     const StepSc *__restrict__ sc,
@@ -513,8 +396,8 @@ __global__ __launch_bounds__(256) void k_chol_trail(double *__restrict__ A,
   const int s = blockIdx.y;
   if (sc[s].status) return;
   const int n = sc[s].n;
-  if (k0 + 32 >= n) return;
-  const int jb = 32, m0 = k0 + 32;
+  const int m0 = k0 + 64;
+  if (m0 >= n) return;
   const int nt = (n - m0 + 63) / 64;
   const int t = blockIdx.x;
   if (t >= nt * (nt + 1) / 2) return;
@@ -523,55 +406,58 @@ __global__ __launch_bounds__(256) void k_chol_trail(double *__restrict__ A,
   while ((bi + 1) * (bi + 2) / 2 <= t) ++bi;
   const int bj = t - bi * (bi + 1) / 2;
   double *As = A + (int64_t)s * strideA;
-  const int tid = threadIdx.x;
-  const int ty = tid >> 4, tx = tid & 15;
-  __shared__ double Pa[64][33];
-  __shared__ double Pb[64][33];
-  const int i0 = m0 + bi * 64, j0 = m0 + bj * 64;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int li = lane & 15, lg = lane >> 4;
+  const int i0 = m0 + bi * 64 + (wave & 1) * 32;
+  const int j0 = m0 + bj * 64 + (wave >> 1) * 32;
+  const double *Pi = As + i0 + li + (int64_t)(k0 + lg) * ld;
+  const double *Pj = As + j0 + li + (int64_t)(k0 + lg) * ld;
+  f4d_t acc[2][2];
 #pragma unroll
-  for (int q = 0; q < 8; ++q) {
-    const int e = tid + q * 256;
-    const int r = e & 63, c = e >> 6;
-    Pa[r][c] = (i0 + r < n && c < jb) ? As[(i0 + r) + (int64_t)(k0 + c) * ld]
-                                      : 0.0;
-    Pb[r][c] = (j0 + r < n && c < jb) ? As[(j0 + r) + (int64_t)(k0 + c) * ld]
-                                      : 0.0;
-  }
-  double cur[4][4];
+  for (int a = 0; a < 2; ++a)
 #pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const int i = i0 + ty * 4 + a, j = j0 + tx * 4 + b;
-      cur[a][b] = (i < n && j < n && i >= j) ? As[i + (int64_t)j * ld] : 0.0;
-    }
-  __syncthreads();
-  double acc[4][4];
-#pragma unroll
-  for (int a = 0; a < 4; ++a)
-#pragma unroll
-    for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-  for (int c = 0; c < jb; ++c) {
-    double pa[4], pb[4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a) pa[a] = Pa[ty * 4 + a][c];
-#pragma unroll
-    for (int b = 0; b < 4; ++b) pb[b] = Pb[tx * 4 + b][c];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) acc[a][b] += pa[a] * pb[b];
+    for (int b = 0; b < 2; ++b) acc[a][b] = f4d_t{0, 0, 0, 0};
+#pragma unroll 8
+  for (int k = 0; k < 64; k += 4) {
+    const double a0 = Pj[(int64_t)k * ld], a1 = Pj[16 + (int64_t)k * ld];
+    const double b0 = Pi[(int64_t)k * ld], b1 = Pi[16 + (int64_t)k * ld];
+    acc[0][0] = mfma64(a0, b0, acc[0][0]);
+    acc[0][1] = mfma64(a0, b1, acc[0][1]);
+    acc[1][0] = mfma64(a1, b0, acc[1][0]);
+    acc[1][1] = mfma64(a1, b1, acc[1][1]);
   }
 #pragma unroll
-  for (int a = 0; a < 4; ++a) {
-    const int i = i0 + ty * 4 + a;
+  for (int a = 0; a < 2; ++a)
 #pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const int j = j0 + tx * 4 + b;
-      if (i < n && j < n && i >= j)
-        As[i + (int64_t)j * ld] = cur[a][b] - acc[a][b];
-    }
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = i0 + b * 16 + li, j = j0 + a * 16 + lg + 4 * r;
+        if (i < n && i >= j) As[i + (int64_t)j * ld] -= acc[a][b][r];
+      }
+}
+
+int chol_steps(hipStream_t st, double *A, int64_t ld, int64_t stride,
+               StepSc *sc, const spk_vg *vgs, int shift, int64_t N, int S) {
+  if (shift) {
+    hipLaunchKernelGGL(k_chol_c0, dim3(S), dim3(256), 0, st,
+                       (const double *)A, ld, stride, sc, vgs);
+    hipLaunchKernelGGL(k_chol_shift,
+                       dim3((unsigned)std::min<int64_t>(N, 256), S), dim3(256),
+                       0, st, A, ld, stride, (const StepSc *)sc);
   }
+  for (int k0 = 0; k0 < N; k0 += 64) {
+    hipLaunchKernelGGL(k_chol_diag, dim3(S), dim3(256), 0, st, A, ld, stride,
+                       sc, k0);
+    const int64_t nt = ceil_div(N - k0, 64) - 1;
+    if (nt <= 0) break;
+    hipLaunchKernelGGL(k_chol_solve, dim3((unsigned)nt, S), dim3(64), 0, st, A,
+                       ld, stride, (const StepSc *)sc, k0);
+    hipLaunchKernelGGL(k_chol_trail, dim3((unsigned)(nt * (nt + 1) / 2), S),
+                       dim3(256), 0, st, A, ld, stride, (const StepSc *)sc,
+                       k0);
+  }
+  return check_launch("k_chol");
 }
 
 // ---- triangular inverse ----------------------------------------------------------
@@ -583,7 +469,11 @@ __global__ __launch_bounds__(256) void k_chol_trail(double *__restrict__ A,
 // blocks (grid (blocks, steps)), then k_trtri_cols runs one column block's
 // chain per workgroup (grid (blocks, steps)).  The n x n region of X is
 // fully written (upper part zero).
-__global__ __launch_bounds__(256) void k_trtri_diag(
+
+// Lane j: column j of the block's inverse by forward substitution from the
+// unit vector (the column-by-column form with two barriers per column took
+// 105 us, this 21).
+__global__ __launch_bounds__(64) void k_trtri_diag(
     const double *__restrict__ L, double *__restrict__ X, int64_t ld,
     int64_t stride, const StepSc *__restrict__ sc) {
   const int s = blockIdx.y;
@@ -594,35 +484,45 @@ __global__ __launch_bounds__(256) void k_trtri_diag(
   const int rn = min(64, n - r0);
   const double *Ls = L + (int64_t)s * stride;
   double *Xs = X + (int64_t)s * stride;
-  const int tid = threadIdx.x;
-  __shared__ double Di[64][65];
-  for (int e = tid; e < 64 * 64; e += 256) {
-    const int i = e & 63, j = e >> 6;
-    Di[i][j] = (i < rn && j < rn && i >= j)
-                   ? Ls[(r0 + i) + (int64_t)(r0 + j) * ld]
-                   : 0.0;
+  const int lane = threadIdx.x;
+  __shared__ __align__(16) double Lt[64][64];
+  __shared__ double Xc[48][64];
+  __shared__ double T[16][65];  // results of 16 rows, [row][column]
+  __shared__ double dinv[64];
+  const double *Lp = Ls + r0 + min(lane, rn - 1) + (int64_t)r0 * ld;
+#pragma unroll 16
+  for (int j = 0; j < 64; ++j) {
+    const double v = Lp[(int64_t)min(j, rn - 1) * ld];
+    Lt[j][lane] = lane < rn && j < rn && lane >= j ? v : lane == j ? 1.0 : 0.0;
   }
   __syncthreads();
-  // in-place inverse, last column first:
-  // X_jj = 1/L_jj, X[i, j] = -X_jj sum_{j<k<=i} X[i, k] L[k, j]
-  for (int j = rn - 1; j >= 0; --j) {
-    double v = 0.0;
-    const double djj = 1.0 / Di[j][j];
-    if (tid > j && tid < rn)
-      for (int k = j + 1; k <= tid; ++k) v += Di[tid][k] * Di[k][j];
-    __syncthreads();
-    if (tid > j && tid < rn) Di[tid][j] = -v * djj;
-    if (tid == j) Di[j][j] = djj;
-    __syncthreads();
-  }
-  for (int e = tid; e < 64 * 64; e += 256) {
-    const int i = e & 63, j = e >> 6;
-    if (i < rn && j < rn)
-      Xs[(r0 + i) + (int64_t)(r0 + j) * ld] = (i >= j) ? Di[i][j] : 0.0;
-  }
+  dinv[lane] = 1.0 / Lt[lane][lane];
+  __syncthreads();
+  wave_fwd_subst(
+      Lt, dinv, Xc, [&](int c) { return lane == c ? 1.0 : 0.0; },
+      [&](int c, double x) {
+        T[c & 15][lane] = x;
+        if ((c & 15) != 15) return;
+        // 16 rows done: four columns per pass, 16 consecutive rows each
+        __syncthreads();
+        const int i = (c & ~15) + (lane & 15);
+#pragma unroll 4
+        for (int j = lane >> 4; j < rn; j += 4)
+          if (i < rn) Xs[(r0 + i) + (int64_t)(r0 + j) * ld] = T[lane & 15][j];
+        __syncthreads();
+      });
 }
 
-__global__ __launch_bounds__(256) void k_trtri_cols(
+// Products on FP64 MFMA, each wave 32 x 32 of the 64 x 64 block as 2 x 2
+// tiles, formed transposed (rows: columns of X, columns: rows of X) so that
+// a lane group's results are 16 consecutive rows in memory.  k in chunks of
+// 32, the next chunk loaded into registers while the current one is
+// multiplied out of LDS (two buffers, one barrier per chunk).  X's chunk is
+// kept by columns (36 doubles apart: conflict-free writes of 32 rows and
+// reads of 16 columns x 4 rows).  The longest chain (block 0) bounds a
+// launch of few steps: 16 steps of up to 2 000 stations took 7.1 ms on the
+// vector ALU, now 2.3 (64 hourly steps: 20.8, now 6.3).
+__global__ __launch_bounds__(256, 2) void k_trtri_cols(
     const double *__restrict__ L, double *__restrict__ X, int64_t ld,
     int64_t stride, const StepSc *__restrict__ sc) {
   const int s = blockIdx.y;
@@ -633,16 +533,13 @@ __global__ __launch_bounds__(256) void k_trtri_cols(
   if (c0 >= n) return;
   const double *Ls = L + (int64_t)s * stride;
   double *Xs = X + (int64_t)s * stride;
-  const int tid = threadIdx.x;
-  const int ty = tid >> 4, tx = tid & 15;
-  __shared__ double Di[64][65];  // X[r, r]
-  __shared__ union {
-    struct {
-      double a[64][33];
-      double b[32][65];
-    } t;
-    double acc[64][65];
-  } sm;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int li = lane & 15, lg = lane >> 4;
+  const int wi = (wave & 1) * 32, wj = (wave >> 1) * 32;
+  __shared__ double La[2][32][80];  // [k][row of L]
+  __shared__ double Xt[2][64][36];  // [column of X][k]
+  // the sums, [column of X][row], in La's space once its chunks are read
+  double (*At)[68] = reinterpret_cast<double (*)[68]>(&La[0][0][0]);
   const int nb = (n + 63) / 64;
   const int cn = min(64, n - c0);
   // the strictly-upper blocks of this column block
@@ -650,92 +547,108 @@ __global__ __launch_bounds__(256) void k_trtri_cols(
     const int i = (int)(e % c0), j = (int)(e / c0);
     Xs[i + (int64_t)(c0 + j) * ld] = 0.0;
   }
+  double pa[8], pb[8];
   for (int rb = cb + 1; rb < nb; ++rb) {
     const int r0 = rb * 64;
     const int rn = min(64, n - r0);
-    for (int e = tid; e < 64 * 64; e += 256) {
-      const int i = e & 63, j = e >> 6;
-      Di[i][j] = (i < rn && j < rn) ? Xs[(r0 + i) + (int64_t)(r0 + j) * ld]
-                                    : 0.0;
-    }
-    double acc[4][4];
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-    // acc -= L[r, k] X[k, c] for k in [c0, r0); the next chunk's tiles
-    // are loaded into registers while this one is multiplied
-    double pa_[8], pb_[8];
     auto fetch = [&](int k0) {
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const int e = tid + q * 256;
         const int r = e & 63, k = e >> 6;
-        pa_[q] = (r < rn) ? Ls[(r0 + r) + (int64_t)(k0 + k) * ld] : 0.0;
+        pa[q] = r < rn ? Ls[(r0 + r) + (int64_t)(k0 + k) * ld] : 0.0;
       }
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const int e = tid + q * 256;
         const int k = e & 31, c = e >> 5;
-        pb_[q] = (c0 + c < n) ? Xs[(k0 + k) + (int64_t)(c0 + c) * ld] : 0.0;
+        pb[q] = c < cn ? Xs[(k0 + k) + (int64_t)(c0 + c) * ld] : 0.0;
       }
     };
-    fetch(c0);
-    for (int k0 = c0; k0 < r0; k0 += 32) {
+    auto put = [&](int buf) {
 #pragma unroll
       for (int q = 0; q < 8; ++q) {
         const int e = tid + q * 256;
-        sm.t.a[e & 63][e >> 6] = pa_[q];
-        sm.t.b[e & 31][e >> 5] = pb_[q];
+        La[buf][e >> 6][e & 63] = pa[q];
+        Xt[buf][e >> 5][e & 31] = pb[q];
       }
-      __syncthreads();
-      if (k0 + 32 < r0) fetch(k0 + 32);
-      for (int k = 0; k < 32; ++k) {
-        double pa[4], pb[4];
+    };
+    f4d_t acc[2][2];
 #pragma unroll
-        for (int a = 0; a < 4; ++a) pa[a] = sm.t.a[ty * 4 + a][k];
+    for (int a = 0; a < 2; ++a)
 #pragma unroll
-        for (int b = 0; b < 4; ++b) pb[b] = sm.t.b[k][tx * 4 + b];
-#pragma unroll
-        for (int a = 0; a < 4; ++a)
-#pragma unroll
-          for (int b = 0; b < 4; ++b) acc[a][b] -= pa[a] * pb[b];
-      }
-      __syncthreads();
-    }
-    // X[r, c] = X[r, r] acc
-#pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) sm.acc[ty * 4 + a][tx * 4 + b] = acc[a][b];
+      for (int b = 0; b < 2; ++b) acc[a][b] = f4d_t{0, 0, 0, 0};
+    fetch(c0);
+    put(0);
     __syncthreads();
-    double out[4][4];
+    const int nch = (r0 - c0) / 32;
+    for (int ch = 0; ch < nch; ++ch) {
+      const int buf = ch & 1;
+      if (ch + 1 < nch) fetch(c0 + (ch + 1) * 32);
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
-#pragma unroll
-      for (int b = 0; b < 4; ++b) out[a][b] = 0.0;
-    for (int k = 0; k < 64; ++k) {
-      double pa[4], pb[4];
-#pragma unroll
-      for (int a = 0; a < 4; ++a) pa[a] = Di[ty * 4 + a][k];
-#pragma unroll
-      for (int b = 0; b < 4; ++b) pb[b] = sm.acc[k][tx * 4 + b];
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) out[a][b] += pa[a] * pb[b];
-    }
-#pragma unroll
-    for (int a = 0; a < 4; ++a) {
-      const int i = r0 + ty * 4 + a;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int j = c0 + tx * 4 + b;
-        if (i < n && j < n) Xs[i + (int64_t)j * ld] = out[a][b];
+      for (int kk = 0; kk < 32; kk += 4) {
+        const double a0 = Xt[buf][wj + li][kk + lg];
+        const double a1 = Xt[buf][wj + 16 + li][kk + lg];
+        const double b0 = La[buf][kk + lg][wi + li];
+        const double b1 = La[buf][kk + lg][wi + 16 + li];
+        acc[0][0] = mfma64(a0, b0, acc[0][0]);
+        acc[0][1] = mfma64(a0, b1, acc[0][1]);
+        acc[1][0] = mfma64(a1, b0, acc[1][0]);
+        acc[1][1] = mfma64(a1, b1, acc[1][1]);
       }
+      if (ch + 1 < nch) put(buf ^ 1);
+      __syncthreads();
     }
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r)
+          At[wj + a * 16 + lg + 4 * r][wi + b * 16 + li] = acc[a][b][r];
+    __syncthreads();
+    // X[r, c] = - X[r, r] sums; X[r, r] (zero above its diagonal) straight
+    // from memory
+    f4d_t out[2][2];
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b) out[a][b] = f4d_t{0, 0, 0, 0};
+#pragma unroll 4
+    for (int k = 0; k < 64; k += 4) {
+      const double a0 = At[wj + li][k + lg], a1 = At[wj + 16 + li][k + lg];
+      double b0 = 0.0, b1 = 0.0;
+      if (k + lg < rn) {
+        const double *Dp = Xs + r0 + wi + li + (int64_t)(r0 + k + lg) * ld;
+        if (wi + li < rn) b0 = Dp[0];
+        if (wi + 16 + li < rn) b1 = Dp[16];
+      }
+      out[0][0] = mfma64(a0, b0, out[0][0]);
+      out[0][1] = mfma64(a0, b1, out[0][1]);
+      out[1][0] = mfma64(a1, b0, out[1][0]);
+      out[1][1] = mfma64(a1, b1, out[1][1]);
+    }
+#pragma unroll
+    for (int a = 0; a < 2; ++a)
+#pragma unroll
+      for (int b = 0; b < 2; ++b)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int i = wi + b * 16 + li, j = wj + a * 16 + lg + 4 * r;
+          if (i < rn && j < cn)
+            Xs[(r0 + i) + (int64_t)(c0 + j) * ld] = -out[a][b][r];
+        }
+    // the next row block reads this one's rows (same workgroup), and At
     __syncthreads();
   }
+}
+
+int trtri_steps(hipStream_t st, const double *L, double *X, int64_t ld,
+                int64_t stride, const StepSc *sc, int64_t N, int S) {
+  const dim3 g((unsigned)ceil_div(N, 64), S);
+  hipLaunchKernelGGL(k_trtri_diag, g, dim3(64), 0, st, L, X, ld, stride, sc);
+  hipLaunchKernelGGL(k_trtri_cols, g, dim3(256), 0, st, L, X, ld, stride, sc);
+  return check_launch("k_trtri");
 }
 
 // ---- dual-form vectors (batched path) -----------------------------------------
@@ -799,43 +712,44 @@ __device__ void small_inverse(double *B, int p, double *Binv) {
     for (int j = 0; j < p; ++j) Binv[i * p + j] = a[i][p + j];
 }
 
-// Y[:, r] = Li X[:, r] (r < nr), X and Y column-major with leading dim ld.
-// The k loops are unrolled so that a thread's loads of the next entries are
-// in flight while it adds up the current ones (in the same order).
-__device__ void tri_lower_mv(const double *__restrict__ Li, int64_t ld, int n,
-                             const double *__restrict__ X,
-                             double *__restrict__ Y, int nr) {
-  for (int i = threadIdx.x; i < n; i += blockDim.x) {
-    double acc[kMaxP + 1];
-    for (int r = 0; r < nr; ++r) acc[r] = 0.0;
-#pragma unroll 8
-    for (int k = 0; k <= i; ++k) {
-      const double l = Li[i + (int64_t)k * ld];
-      for (int r = 0; r < nr; ++r) acc[r] += l * X[k + (int64_t)r * ld];
-    }
-    for (int r = 0; r < nr; ++r) Y[i + (int64_t)r * ld] = acc[r];
-  }
-}
+// Rows per workgroup of the triangular products L x: lane = row, the four
+// waves take a quarter of the columns each, and their sums are added in
+// wave order.  (One row per thread over all columns kept 16 steps of 2 000
+// rows on 128 workgroups: 83 us per product, now 33; two columns 642, now
+// 70.)
+constexpr int kLmvRows = 64;
 
-// Y[:, r] = Li^T X[:, r]: one wave per output entry, lanes over rows.
-__device__ void tri_lower_tmv(const double *__restrict__ Li, int64_t ld,
-                              int n, const double *__restrict__ X,
-                              double *__restrict__ Y, int nr) {
+// This wave's share of (T X[:, r])[i], r < NR, for the block's rows i0 ..
+// i0 + 63 (T lower, column-major), summed over the block's waves into red
+// and returned to the first wave.
+template <int NR>
+__device__ inline void block_lmv(const double *__restrict__ T, int64_t ld,
+                                 int n, int i0, const double *__restrict__ X,
+                                 int64_t ldx, double (*red)[4][64],
+                                 double *acc) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int nw = blockDim.x >> 6;
-  for (int k = wave; k < n; k += nw) {
-    double acc[kMaxP + 1];
-    for (int r = 0; r < nr; ++r) acc[r] = 0.0;
-#pragma unroll 4
-    for (int i = k + lane; i < n; i += 64) {
-      const double l = Li[i + (int64_t)k * ld];
-      for (int r = 0; r < nr; ++r) acc[r] += l * X[i + (int64_t)r * ld];
-    }
-    for (int r = 0; r < nr; ++r) {
-      const double v = wave_sum(acc[r]);
-      if (lane == 0) Y[k + (int64_t)r * ld] = v;
-    }
+  const int i = i0 + lane;
+  const double *Ti = T + min(i, n - 1);
+  const int kend = min(n, i0 + kLmvRows);
+  const int len = (kend + 3) / 4;
+  const int k1 = min(kend, (wave + 1) * len);
+#pragma unroll
+  for (int r = 0; r < NR; ++r) acc[r] = 0.0;
+#pragma unroll 8
+  for (int k = wave * len; k < k1; ++k) {
+    // (what lies above the diagonal is loaded and not used)
+    const double t = Ti[(int64_t)k * ld];
+    const double l = k <= i ? t : 0.0;
+#pragma unroll
+    for (int r = 0; r < NR; ++r) acc[r] += l * X[k + (int64_t)r * ldx];
   }
+#pragma unroll
+  for (int r = 0; r < NR; ++r) red[r][wave][lane] = acc[r];
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < NR; ++r)
+    acc[r] = red[r][0][lane] + red[r][1][lane] + red[r][2][lane] +
+             red[r][3][lane];
 }
 
 // ---- condition estimate over (block, step) workgroups --------------------------
@@ -845,10 +759,9 @@ __device__ void tri_lower_tmv(const double *__restrict__ Li, int64_t ld,
 // two scratch columns of the step's T0 (X and U of k_dual).  Launch order
 // per which: k_kap_start, then 12 x (k_kap_norm, product into u,
 // k_kap_rq, product back into x); then k_kap_flags.  The products run over
-// (row blocks, steps), one row per thread (k_kap_lmv, y = T x) or one
-// column per wave (k_kap_umv, y = T^T x), with the sums in the order of
-// tri_lower_mv / tri_lower_tmv, and the norms as one workgroup per step with
-// block_sum, so the estimate is the one a single workgroup per step gives.
+// (row blocks, steps), 64 rows per workgroup (k_kap_lmv, y = T x) or one
+// column per wave (k_kap_umv, y = T^T x), and the norms as one workgroup per
+// step.
 __device__ inline double *kap_x(double *T0, int64_t ldt, int s) {
   return T0 + (int64_t)s * ldt * kT0Cols;
 }
@@ -907,7 +820,7 @@ __global__ __launch_bounds__(256) void k_kap_rq(const StepSc *__restrict__ sc,
 }
 
 // y = T v (T lower, column-major, ld), v and y the step's x / u columns
-// (to_u: v = x, y = u; else v = u, y = x); grid (ceil(n_max / 256), steps)
+// (to_u: v = x, y = u; else v = u, y = x); grid (ceil(n_max / 64), steps)
 __global__ __launch_bounds__(256) void k_kap_lmv(const double *__restrict__ T,
                                                  int64_t ld, int64_t stride,
                                                  const StepSc *__restrict__ sc,
@@ -916,18 +829,14 @@ __global__ __launch_bounds__(256) void k_kap_lmv(const double *__restrict__ T,
   const int s = blockIdx.y;
   if (sc[s].status) return;
   const int n = sc[s].n;
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
-  const double *Ts = T + (int64_t)s * stride;
+  const int i0 = blockIdx.x * kLmvRows;
+  if (i0 >= n) return;
   const double *v = to_u ? kap_x(T0, ldt, s) : kap_u(T0, ldt, s);
   double *y = to_u ? kap_u(T0, ldt, s) : kap_x(T0, ldt, s);
-  double acc = 0.0;
-#pragma unroll 8
-  for (int k = 0; k <= i; ++k) {
-    const double l = Ts[i + (int64_t)k * ld];
-    acc += l * v[k];
-  }
-  y[i] = acc;
+  __shared__ double red[1][4][64];
+  double acc[1];
+  block_lmv<1>(T + (int64_t)s * stride, ld, n, i0, v, 0, red, acc);
+  if (threadIdx.x < 64 && i0 + (int)threadIdx.x < n) y[i0 + threadIdx.x] = acc[0];
 }
 
 // y = T^T v, one wave per entry k (lanes over rows i >= k);
@@ -995,9 +904,6 @@ __global__ void k_kap_flags(StepSc *__restrict__ sc,
 //   then twice: k_dual_resid (r1 = z - C alpha - F h, rw = 1 - C w;
 //   row blocks, steps), k_dual_lmv / k_dual_umv on [r1 rw], k_dual_upd
 //   (the corrections of h, alpha and w; steps); then k_dual_fin (steps).
-// Every sum runs in the order of the one-workgroup-per-step form (a row per
-// thread, a column per wave, one workgroup per step for the small
-// reductions), so the results are the ones that form gives.
 constexpr int kDsG = 0;                                  // (p+1)^2
 constexpr int kDsBi = kDsG + (kMaxP + 1) * (kMaxP + 1);  // p^2
 constexpr int kDsH = kDsBi + kMaxP * kMaxP;              // hcoef
@@ -1058,8 +964,8 @@ __device__ inline double *t0_col(double *T0, int64_t ldt, int s, int col) {
   }
 }
 
-// Y[:, r] = Li X[:, r] (r < nr), one row per thread; grid (ceil(n_max /
-// 256), steps)
+// Y[:, r] = Li X[:, r] (r < nr), 64 rows per workgroup; grid (ceil(n_max /
+// 64), steps)
 __global__ __launch_bounds__(256) void k_dual_lmv(
     const double *__restrict__ Li, int64_t ld, int64_t stride,
     const StepSc *__restrict__ sc, double *__restrict__ T0, int64_t ldt,
@@ -1067,19 +973,26 @@ __global__ __launch_bounds__(256) void k_dual_lmv(
   const int s = blockIdx.y;
   if (sc[s].status) return;
   const int n = sc[s].n;
-  const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i >= n) return;
+  const int i0 = blockIdx.x * kLmvRows;
+  if (i0 >= n) return;
   const double *L = Li + (int64_t)s * stride;
   const double *X = t0_col(T0, ldt, s, src);
   double *Y = t0_col(T0, ldt, s, dst);
-  double acc[kMaxP + 1];
-  for (int r = 0; r < nr; ++r) acc[r] = 0.0;
-#pragma unroll 8
-  for (int k = 0; k <= i; ++k) {
-    const double l = L[i + (int64_t)k * ld];
-    for (int r = 0; r < nr; ++r) acc[r] += l * X[k + (int64_t)r * ldt];
+  __shared__ double red[2][4][64];
+  const int i = i0 + (int)threadIdx.x;
+  // two columns at a time ([1 z] and [r1 rw] are two)
+  for (int r = 0; r < nr; r += 2) {
+    double acc[2];
+    if (r > 0) __syncthreads();
+    if (r + 1 < nr)
+      block_lmv<2>(L, ld, n, i0, X + (int64_t)r * ldt, ldt, red, acc);
+    else
+      block_lmv<1>(L, ld, n, i0, X + (int64_t)r * ldt, ldt, red, acc);
+    if (threadIdx.x < 64 && i < n) {
+      Y[i + (int64_t)r * ldt] = acc[0];
+      if (r + 1 < nr) Y[i + (int64_t)(r + 1) * ldt] = acc[1];
+    }
   }
-  for (int r = 0; r < nr; ++r) Y[i + (int64_t)r * ldt] = acc[r];
 }
 
 // Y[:, r] = Li^T X[:, r], one wave per output entry (lanes over rows);
@@ -1174,7 +1087,11 @@ __global__ __launch_bounds__(256) void k_dual_mid(
 // Two steps: the first removes the error of the explicit-inverse solve,
 // the second's correction is of the size of the error left, which the
 // cell kernel turns into each cell's error indicator.
-// One row per thread; grid (ceil(n_max / 256), steps).
+// 64 rows per workgroup, a lane per row, each wave a quarter of the stations
+// of every pass of 256; the waves' sums are added in wave order (one row per
+// thread over all stations took 1.3 ms for 16 steps of up to 2 000 rows,
+// this 0.37).
+// grid (ceil(n_max / 64), steps).
 __global__ __launch_bounds__(256) void k_dual_resid(
     const StepSc *__restrict__ sc, const double *__restrict__ zact,
     int64_t ldz, const int32_t *__restrict__ idx, int64_t N,
@@ -1185,19 +1102,20 @@ __global__ __launch_bounds__(256) void k_dual_resid(
   const int s = blockIdx.y;
   if (sc[s].status) return;
   const int n = sc[s].n;
-  const int i0 = blockIdx.x * 256;
+  const int i0 = blockIdx.x * kLmvRows;
   if (i0 >= n) return;
   const DualPtrs d = dual_ptrs(T0, ldt, V, ldv, DS, s);
   const double *z = zact + (int64_t)s * ldz;
   const int32_t *my = idx + (int64_t)s * N;
   const int p = (method == SPK_M_EDK) ? 1 + m : 1;
-  const int tid = threadIdx.x;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   __shared__ double stx[256], sty[256], sal[256], sw[256];
+  __shared__ double red[2][4][64];
   __shared__ spk_vg vg;
   if (tid == 0) vg = vgs[s];
   const bool sk = method == SPK_M_SK;
   const double c0 = sc[s].c0;
-  const int i = i0 + tid;
+  const int i = i0 + lane;
   double xi = 0.0, yi = 0.0;
   if (i < n) {
     xi = sx[my[i]];
@@ -1214,17 +1132,21 @@ __global__ __launch_bounds__(256) void k_dual_resid(
       sw[tid] = d.w[j0 + tid];
     }
     __syncthreads();
-    const int cnt = min(256, n - j0);
-    if (i < n)
-      for (int j = 0; j < cnt; ++j) {
-        const double dd = dist2(xi, yi, stx[j], sty[j]);
-        const double e = vg_entry(vg, dd, sk ? 1 : 0, min_vg_val);
-        const double c = sk ? e : c0 - e;
-        ca += c * sal[j];
-        cw += c * sw[j];
-      }
+    const int j1 = min(wave * 64 + 64, n - j0);
+    for (int j = wave * 64; j < j1; ++j) {
+      const double dd = dist2(xi, yi, stx[j], sty[j]);
+      const double e = vg_entry(vg, dd, sk ? 1 : 0, min_vg_val);
+      const double c = sk ? e : c0 - e;
+      ca += c * sal[j];
+      cw += c * sw[j];
+    }
   }
-  if (i < n) {
+  red[0][wave][lane] = ca;
+  red[1][wave][lane] = cw;
+  __syncthreads();
+  if (wave == 0 && i < n) {
+    ca = red[0][0][lane] + red[0][1][lane] + red[0][2][lane] + red[0][3][lane];
+    cw = red[1][0][lane] + red[1][1][lane] + red[1][2][lane] + red[1][3][lane];
     double r1 = z[i] - ca;
     if (!sk) {
       r1 -= d.ds[kDsHc + 0];
@@ -1323,109 +1245,169 @@ __global__ void k_dual_fin(StepSc *__restrict__ sc, int m, int method,
 // The reference's K = [[G, F], [F^T, 0]] with G = c0 11^T - C has the
 // inverse [[-P, Q], [Q^T, B^-1 - c0 e0 e0^T]], written to M (ld rows).
 // SK has no constraint rows: M = Cinv.
-__global__ __launch_bounds__(256) void k_minv(
+// Launches over (tiles or row blocks, steps): k_minv_tiles, k_minv_w,
+// k_minv_mid, k_minv_fin (minv_steps).  One workgroup per step for all of it
+// took 11.8 ms for systems of 900 rows; the four take 0.24 ms for seven.
+
+// Cinv[i, j] = sum over k >= i of Li[k, i] Li[k, j], a 64 x 64 tile (bi >=
+// bj) per workgroup and its mirror image, on FP64 MFMA (32 x 32 per wave).
+// Both operands are read down columns of Li and kept by columns in LDS (36
+// doubles apart).  grid (tiles of the lower triangle, steps)
+__global__ __launch_bounds__(256, 2) void k_minv_tiles(
     const double *__restrict__ Li, int64_t ld, int64_t stride,
+    const StepSc *__restrict__ sc, double *__restrict__ M) {
+  const int s = blockIdx.y;
+  if (sc[s].status) return;
+  const int n = sc[s].n;
+  const int nb = (n + 63) / 64;
+  const int t = blockIdx.x;
+  if (t >= nb * (nb + 1) / 2) return;
+  int bi = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
+  while (bi * (bi + 1) / 2 > t) --bi;
+  while ((bi + 1) * (bi + 2) / 2 <= t) ++bi;
+  const int bj = t - bi * (bi + 1) / 2;
+  const double *L = Li + (int64_t)s * stride;
+  double *Ms = M + (int64_t)s * stride;
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int li = lane & 15, lg = lane >> 4;
+  const int wi = (wave & 1) * 32, wj = (wave >> 1) * 32;
+  __shared__ double Ti[2][64][36], Tj[2][64][36];  // [column][k]
+  double pi_[8], pj_[8];
+  auto fetch = [&](int k0) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int e = tid + q * 256;
+      const int k = k0 + (e & 31), c = e >> 5;
+      pi_[q] = k < n && bi * 64 + c < n
+                   ? L[k + (int64_t)(bi * 64 + c) * ld] : 0.0;
+      pj_[q] = k < n && bj * 64 + c < n
+                   ? L[k + (int64_t)(bj * 64 + c) * ld] : 0.0;
+    }
+  };
+  auto put = [&](int buf) {
+#pragma unroll
+    for (int q = 0; q < 8; ++q) {
+      const int e = tid + q * 256;
+      Ti[buf][e >> 5][e & 31] = pi_[q];
+      Tj[buf][e >> 5][e & 31] = pj_[q];
+    }
+  };
+  f4d_t acc[2][2];
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b) acc[a][b] = f4d_t{0, 0, 0, 0};
+  fetch(bi * 64);
+  put(0);
+  __syncthreads();
+  const int nch = (n - bi * 64 + 31) / 32;
+  for (int ch = 0; ch < nch; ++ch) {
+    const int buf = ch & 1;
+    if (ch + 1 < nch) fetch(bi * 64 + (ch + 1) * 32);
+#pragma unroll
+    for (int kk = 0; kk < 32; kk += 4) {
+      const double a0 = Tj[buf][wj + li][kk + lg];
+      const double a1 = Tj[buf][wj + 16 + li][kk + lg];
+      const double b0 = Ti[buf][wi + li][kk + lg];
+      const double b1 = Ti[buf][wi + 16 + li][kk + lg];
+      acc[0][0] = mfma64(a0, b0, acc[0][0]);
+      acc[0][1] = mfma64(a0, b1, acc[0][1]);
+      acc[1][0] = mfma64(a1, b0, acc[1][0]);
+      acc[1][1] = mfma64(a1, b1, acc[1][1]);
+    }
+    if (ch + 1 < nch) put(buf ^ 1);
+    __syncthreads();
+  }
+#pragma unroll
+  for (int a = 0; a < 2; ++a)
+#pragma unroll
+    for (int b = 0; b < 2; ++b)
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int i = bi * 64 + wi + b * 16 + li;
+        const int j = bj * 64 + wj + a * 16 + lg + 4 * r;
+        if (i < n && j < n) {
+          Ms[i + (int64_t)j * ld] = acc[a][b][r];
+          Ms[j + (int64_t)i * ld] = acc[a][b][r];
+        }
+      }
+}
+
+// W = Cinv F (columns 0 .. p-1 of the step's work area T0), 64 rows per
+// workgroup, each wave a quarter of the columns; grid (ceil(n_max / 64),
+// steps)
+__global__ __launch_bounds__(256) void k_minv_w(
+    const double *__restrict__ M, int64_t ld, int64_t stride,
+    const StepSc *__restrict__ sc, const int32_t *__restrict__ idx, int64_t N,
+    const double *__restrict__ stn_drift, int m, int p,
+    double *__restrict__ T0, int64_t ldt) {
+  const int s = blockIdx.y;
+  if (sc[s].status) return;
+  const int n = sc[s].n;
+  const int i0 = blockIdx.x * 64;
+  if (i0 >= n) return;
+  const double *Ms = M + (int64_t)s * stride;
+  const int32_t *my = idx + (int64_t)s * N;
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int i = min(i0 + lane, n - 1);
+  __shared__ double red[kMaxP][4][64];
+  double acc[kMaxP];
+#pragma unroll
+  for (int r = 0; r < kMaxP; ++r) acc[r] = 0.0;
+  const int len = (n + 3) / 4;
+  const int k1 = min(n, (wave + 1) * len);
+  for (int k = wave * len; k < k1; ++k) {
+    const double c = Ms[i + (int64_t)k * ld];
+    acc[0] += c;
+#pragma unroll
+    for (int r = 1; r < kMaxP; ++r)
+      if (r < p) acc[r] += c * stn_drift[(int64_t)my[k] * m + (r - 1)];
+  }
+#pragma unroll
+  for (int r = 0; r < kMaxP; ++r) red[r][wave][lane] = acc[r];
+  __syncthreads();
+  double *W = T0 + (int64_t)s * ldt * kT0Cols;
+  for (int r = wave; r < p; r += 4)
+    if (i0 + lane < n)
+      W[i0 + lane + (int64_t)r * ldt] = red[r][0][lane] + red[r][1][lane] +
+                                        red[r][2][lane] + red[r][3][lane];
+}
+
+// The condition estimate max diag(Cinv) max diag(C), then B = F^T W, its
+// inverse (M's corner) and Q = W B^-1 (columns p .. 2p-1 of T0); grid
+// (steps)
+__global__ __launch_bounds__(256) void k_minv_mid(
+    double *__restrict__ M, int64_t ld, int64_t stride,
     StepSc *__restrict__ sc, const int32_t *__restrict__ idx, int64_t N,
-    const double *__restrict__ stn_drift, int m, int method,
-    double *__restrict__ M, double *__restrict__ T0,
-    const spk_vg *__restrict__ vgs, double min_vg_val) {
-  const int64_t ldt = ld;
+    const double *__restrict__ stn_drift, int m, int method, int p,
+    double *__restrict__ T0, int64_t ldt, const spk_vg *__restrict__ vgs,
+    double min_vg_val) {
   const int s = blockIdx.x;
   if (sc[s].status) return;
   const int n = sc[s].n;
-  const double *L = Li + (int64_t)s * stride;
   double *Ms = M + (int64_t)s * stride;
   const int32_t *my = idx + (int64_t)s * N;
-  const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
-  __shared__ double Ta[32][65];
-  __shared__ double Tb[32][65];
-  const int nb = (n + 63) / 64;
-  // Cinv tiles (bi >= bj): sum over k >= bi*64 of L[k, i] L[k, j]
-  for (int bi = 0; bi < nb; ++bi) {
-    for (int bj = 0; bj <= bi; ++bj) {
-      double acc[4][4];
-#pragma unroll
-      for (int a = 0; a < 4; ++a)
-#pragma unroll
-        for (int b = 0; b < 4; ++b) acc[a][b] = 0.0;
-      for (int k0 = bi * 64; k0 < n; k0 += 32) {
-        for (int e = tid; e < 32 * 64; e += 256) {
-          const int k = e & 31, c = e >> 5;
-          const int kk = k0 + k;
-          Ta[k][c] = (kk < n && bi * 64 + c < n)
-                         ? L[kk + (int64_t)(bi * 64 + c) * ld]
-                         : 0.0;
-          Tb[k][c] = (kk < n && bj * 64 + c < n)
-                         ? L[kk + (int64_t)(bj * 64 + c) * ld]
-                         : 0.0;
-        }
-        __syncthreads();
-        for (int k = 0; k < 32; ++k) {
-          double pa[4], pb[4];
-#pragma unroll
-          for (int a = 0; a < 4; ++a) pa[a] = Ta[k][ty * 4 + a];
-#pragma unroll
-          for (int b = 0; b < 4; ++b) pb[b] = Tb[k][tx * 4 + b];
-#pragma unroll
-          for (int a = 0; a < 4; ++a)
-#pragma unroll
-            for (int b = 0; b < 4; ++b) acc[a][b] += pa[a] * pb[b];
-        }
-        __syncthreads();
-      }
-#pragma unroll
-      for (int a = 0; a < 4; ++a) {
-        const int i = bi * 64 + ty * 4 + a;
-#pragma unroll
-        for (int b = 0; b < 4; ++b) {
-          const int j = bj * 64 + tx * 4 + b;
-          if (i < n && j < n) {
-            Ms[i + (int64_t)j * ld] = acc[a][b];
-            Ms[j + (int64_t)i * ld] = acc[a][b];
-          }
-        }
-      }
-    }
-  }
+  const int tid = threadIdx.x;
+  __shared__ double red[256];
+  double mx = 0.0;
+  for (int i = tid; i < n; i += 256) mx = fmax(mx, Ms[i + (int64_t)i * ld]);
+  red[tid] = mx;
   __syncthreads();
-  {
-    __shared__ double red[256];
-    double mx = 0.0;
-    for (int i = tid; i < n; i += 256) mx = fmax(mx, Ms[i + (int64_t)i * ld]);
-    red[tid] = mx;
+  for (int w2 = 128; w2 > 0; w2 >>= 1) {
+    if (tid < w2) red[tid] = fmax(red[tid], red[tid + w2]);
     __syncthreads();
-    for (int w2 = 128; w2 > 0; w2 >>= 1) {
-      if (tid < w2) red[tid] = fmax(red[tid], red[tid + w2]);
-      __syncthreads();
-    }
-    if (tid == 0) {
-      const spk_vg &vg = vgs[s];
-      const double cii = (method == SPK_M_SK)
-                             ? vg_entry(vg, 0.0, 1, min_vg_val)
-                             : sc[s].c0 - vg_entry(vg, 0.0, 0, min_vg_val);
-      const double kap = red[0] * fabs(cii);
-      sc[s].kappa = kap;
-      sc[s].flags = (kap <= 1e12) ? 0 : SPK_ST_ILLCOND;
-    }
-    __syncthreads();
+  }
+  if (tid == 0) {
+    const spk_vg &vg = vgs[s];
+    const double cii = (method == SPK_M_SK)
+                           ? vg_entry(vg, 0.0, 1, min_vg_val)
+                           : sc[s].c0 - vg_entry(vg, 0.0, 0, min_vg_val);
+    const double kap = red[0] * fabs(cii);
+    sc[s].kappa = kap;
+    sc[s].flags = (kap <= 1e12) ? 0 : SPK_ST_ILLCOND;
   }
   if (method == SPK_M_SK) return;
-  const int p = (method == SPK_M_EDK) ? 1 + m : 1;
-  // per-step work area: kT0Cols columns of ld (W, then Q)
   double *W = T0 + (int64_t)s * ldt * kT0Cols;
-  // W = Cinv F
-  for (int i = tid; i < n; i += 256) {
-    double acc[kMaxP];
-    for (int r = 0; r < p; ++r) acc[r] = 0.0;
-    for (int k = 0; k < n; ++k) {
-      const double c = Ms[i + (int64_t)k * ld];
-      acc[0] += c;
-      for (int r = 1; r < p; ++r)
-        acc[r] += c * stn_drift[(int64_t)my[k] * m + (r - 1)];
-    }
-    for (int r = 0; r < p; ++r) W[i + (int64_t)r * ldt] = acc[r];
-  }
-  __syncthreads();
   __shared__ double Bs[kMaxP * kMaxP], Bi[kMaxP * kMaxP];
   for (int e = tid >> 6; e < p * p; e += 4) {
     const int a = e / p, b = e % p;
@@ -1440,7 +1422,6 @@ __global__ __launch_bounds__(256) void k_minv(
   __syncthreads();
   if (tid == 0) small_inverse(Bs, p, Bi);
   __syncthreads();
-  // Q = W B^-1 (into columns p..2p-1 of the work array)
   double *Q = W + (int64_t)p * ldt;
   for (int i = tid; i < n; i += 256)
     for (int a = 0; a < p; ++a) {
@@ -1448,26 +1429,61 @@ __global__ __launch_bounds__(256) void k_minv(
       for (int b = 0; b < p; ++b) v += W[i + (int64_t)b * ldt] * Bi[b * p + a];
       Q[i + (int64_t)a * ldt] = v;
     }
-  __syncthreads();
-  const double c0 = sc[s].c0;
-  for (int64_t e = tid; e < (int64_t)n * n; e += 256) {
-    const int i = (int)(e % n), j = (int)(e / n);
-    double v = Ms[i + (int64_t)j * ld];
-    for (int a = 0; a < p; ++a)
-      v -= Q[i + (int64_t)a * ldt] * W[j + (int64_t)a * ldt];
-    Ms[i + (int64_t)j * ld] = -v;
-  }
-  for (int i = tid; i < n; i += 256)
-    for (int a = 0; a < p; ++a) {
-      const double q = Q[i + (int64_t)a * ldt];
-      Ms[i + (int64_t)(n + a) * ld] = q;
-      Ms[(n + a) + (int64_t)i * ld] = q;
-    }
   if (tid < p * p) {
     const int a = tid / p, b = tid % p;
     Ms[(n + a) + (int64_t)(n + b) * ld] =
-        Bi[a * p + b] - ((a == 0 && b == 0) ? c0 : 0.0);
+        Bi[a * p + b] - ((a == 0 && b == 0) ? sc[s].c0 : 0.0);
   }
+}
+
+// M <- -(Cinv - Q W^T) and the border rows; grid (column groups, steps),
+// block x takes columns x, x + gridDim.x, ...
+__global__ __launch_bounds__(256) void k_minv_fin(
+    double *__restrict__ M, int64_t ld, int64_t stride,
+    const StepSc *__restrict__ sc, int p, const double *__restrict__ T0,
+    int64_t ldt) {
+  const int s = blockIdx.y;
+  if (sc[s].status) return;
+  const int n = sc[s].n;
+  double *Ms = M + (int64_t)s * stride;
+  const double *W = T0 + (int64_t)s * ldt * kT0Cols;
+  const double *Q = W + (int64_t)p * ldt;
+  for (int j = blockIdx.x; j < n; j += gridDim.x) {
+    for (int i = threadIdx.x; i < n; i += 256) {
+      double v = Ms[i + (int64_t)j * ld];
+      for (int a = 0; a < p; ++a)
+        v -= Q[i + (int64_t)a * ldt] * W[j + (int64_t)a * ldt];
+      Ms[i + (int64_t)j * ld] = -v;
+    }
+    if ((int)threadIdx.x < p) {
+      const int a = threadIdx.x;
+      const double q = Q[j + (int64_t)a * ldt];
+      Ms[j + (int64_t)(n + a) * ld] = q;
+      Ms[(n + a) + (int64_t)j * ld] = q;
+    }
+  }
+}
+
+int minv_steps(hipStream_t st, const double *Li, int64_t ld, int64_t stride,
+               StepSc *sc, const int32_t *idx, int64_t N,
+               const double *stn_drift, int m, int method, double *M,
+               double *T0, const spk_vg *vgs, double min_vg_val, int S) {
+  const int64_t nb = ceil_div(N, 64);
+  const int p = method == SPK_M_SK ? 0 : method == SPK_M_EDK ? 1 + m : 1;
+  hipLaunchKernelGGL(k_minv_tiles, dim3((unsigned)(nb * (nb + 1) / 2), S),
+                     dim3(256), 0, st, Li, ld, stride, (const StepSc *)sc, M);
+  if (p > 0)
+    hipLaunchKernelGGL(k_minv_w, dim3((unsigned)nb, S), dim3(256), 0, st,
+                       (const double *)M, ld, stride, (const StepSc *)sc, idx,
+                       N, stn_drift, m, p, T0, ld);
+  hipLaunchKernelGGL(k_minv_mid, dim3(S), dim3(256), 0, st, M, ld, stride, sc,
+                     idx, N, stn_drift, m, method, p, T0, ld, vgs, min_vg_val);
+  if (p > 0)
+    hipLaunchKernelGGL(k_minv_fin,
+                       dim3((unsigned)std::min<int64_t>(N, 256), S), dim3(256),
+                       0, st, M, ld, stride, (const StepSc *)sc, p,
+                       (const double *)T0, ld);
+  return check_launch("k_minv");
 }
 
 // Li as float (column-major) for the FP32 contraction.

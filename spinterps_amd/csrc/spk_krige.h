@@ -143,26 +143,15 @@ __global__ void k_assemble(const double *sx, const double *sy,
                            const spk_vg *vgs, int covar_flag, double min_vg_val,
                            double *A, int64_t ld, int64_t strideA,
                            double *Gfull);
-__global__ void k_potrf(double *A, int64_t ld, int64_t strideA, StepSc *sc,
-                        const spk_vg *vgs, int shift);
-// Cholesky over (block, step) workgroups: k_chol_shift (grid (steps)),
-// then per 32-wide panel k0: k_chol_diag (grid (1, steps)), k_chol_solve
-// (grid (rows below / 256, steps)), k_chol_trail (grid (trailing 64 x 64
-// tiles, steps)).  chol_steps launches the sequence.
-__global__ void k_chol_shift(double *A, int64_t ld, int64_t strideA,
-                             StepSc *sc, const spk_vg *vgs);
-__global__ void k_chol_diag(double *A, int64_t ld, int64_t strideA,
-                            StepSc *sc, int k0);
-__global__ void k_chol_solve(double *A, int64_t ld, int64_t strideA,
-                             const StepSc *sc, int k0);
-__global__ void k_chol_trail(double *A, int64_t ld, int64_t strideA,
-                             const StepSc *sc, int k0);
-// X = L^-1: k_trtri_diag then k_trtri_cols, each with grid
-// (ceil(n_max / 64), steps)
-__global__ void k_trtri_diag(const double *L, double *X, int64_t ld,
-                             int64_t stride, const StepSc *sc);
-__global__ void k_trtri_cols(const double *L, double *X, int64_t ld,
-                             int64_t stride, const StepSc *sc);
+// C = c0 - G (shift) or A as it is, then the Cholesky factor in the lower
+// triangle, of S systems of at most N rows: k_chol_c0, k_chol_shift, then
+// per 64-wide panel k_chol_diag, k_chol_solve, k_chol_trail.  N <= ld, ld a
+// multiple of 64.
+int chol_steps(hipStream_t st, double *A, int64_t ld, int64_t stride,
+               StepSc *sc, const spk_vg *vgs, int shift, int64_t N, int S);
+// X = L^-1 of the same systems
+int trtri_steps(hipStream_t st, const double *L, double *X, int64_t ld,
+                int64_t stride, const StepSc *sc, int64_t N, int S);
 // condition estimate: k_kap_start, 12 x (k_kap_norm, k_kap_umv / k_kap_lmv,
 // k_kap_rq, k_kap_lmv / k_kap_umv) per power iteration, then k_kap_flags
 // (spk_factor.hip)
@@ -205,10 +194,11 @@ __global__ void k_dual_upd(const StepSc *sc, const int32_t *idx, int64_t N,
                            double *T0, int64_t ldt, double *V, int64_t ldv,
                            double *DS);
 __global__ void k_dual_fin(StepSc *sc, int m, int method, const double *DS);
-__global__ void k_minv(const double *Li, int64_t ld, int64_t stride,
-                       StepSc *sc, const int32_t *idx, int64_t N,
-                       const double *stn_drift, int m, int method, double *M,
-                       double *T0, const spk_vg *vgs, double min_vg_val);
+// the plain path's K^-1 of S systems of at most N stations
+int minv_steps(hipStream_t st, const double *Li, int64_t ld, int64_t stride,
+               StepSc *sc, const int32_t *idx, int64_t N,
+               const double *stn_drift, int m, int method, double *M,
+               double *T0, const spk_vg *vgs, double min_vg_val, int S);
 __global__ void k_recenter(const double *in, double *out, int64_t n, double o);
 __global__ void k_status_out(const StepSc *sc, int S, int32_t *info,
                              double *kappa);

@@ -456,8 +456,7 @@ int spk_simulate_fields_dev(spk_ctx *ctx, const spk_problem *prob, int64_t T,
                        strideM, (double *)nullptr);
     hipLaunchKernelGGL(k_sim_diag, dim3(8, Sb), dim3(256), 0, sm, A, ld,
                        strideM, sc, vgs + t0);
-    hipLaunchKernelGGL(k_potrf, dim3(Sb), dim3(256), 0, sm, A, ld, strideM, sc,
-                       vgs + t0, 0);
+    SPK_TRY(chol_steps(sm, A, ld, strideM, sc, vgs + t0, 0, N, Sb));
     hipLaunchKernelGGL(k_sim_apply, dim3(Sb), dim3(256), 0, sm, A, ld, strideM,
                        sc, idx, N, means, (unsigned long long)seed, t0,
                        out + t0 * N);

@@ -616,3 +616,35 @@ def test_plain_tiles_edges(gpu, n, cells, method):
         if method == 'OK':
             np.testing.assert_allclose(var[t].cpu().numpy(), v, rtol=1e-9,
                                        atol=1e-9 * np.abs(v).mean())
+
+
+@pytest.mark.parametrize('n', [15, 16, 64, 65, 127, 128, 129, 192, 257])
+def test_factor_panels_edges(gpu, n):
+    """The factorisation's 64-wide panels (16 columns at a time), 64-row
+    products and 64 x 64 MFMA tiles at their edges: dual-form estimates and
+    the batched FP64 variance against the exact solution, for steps of n and
+    of fewer stations in one call."""
+    from spinterps_amd.interp.steps import DeviceProblem, interp_steps
+    rng = np.random.default_rng(n)
+    sx, sy = rng.uniform(0, 1e5, n), rng.uniform(0, 1e5, n)
+    cx, cy = rng.uniform(0, 1e5, 70), rng.uniform(0, 1e5, 70)
+    vals = rng.gamma(2.0, 3.0, (3, n))
+    vals[1, : n // 2] = np.nan
+    vals[2, n - 1:] = np.nan
+    vgs = ['0.1 Nug(0.0) + 0.9 Sph(30000.0)', '1.2 Exp(20000.0)',
+           '0.3 Nug(0.0) + 2.0 Gau(4000.0)']
+    prob = DeviceProblem(sx, sy, cx, cy)
+    for prec in ('fp64b', 'fp64'):
+        est, var, info = interp_steps(prob, vals, vgs, 'OK', precision=prec)
+        est, var = est.cpu().numpy(), var.cpu().numpy()
+        for t in range(3):
+            a = ~np.isnan(vals[t])
+            dd = O.dists_2d(sx[a], sy[a], sx[a], sy[a])
+            rd = O.dists_2d(cx, cy, sx[a], sy[a])
+            ref, v, _ = O.krige_exact('OK', vgs[t], dd, rd, vals[t, a],
+                                      want_var=True)
+            assert int(info[t]) & (4 | 16 | 128) == 0
+            np.testing.assert_allclose(est[t], ref, rtol=0,
+                                       atol=1e-9 * np.abs(vals[t, a]).mean())
+            np.testing.assert_allclose(var[t], v, rtol=1e-9,
+                                       atol=1e-9 * np.abs(v).mean())
