@@ -5,9 +5,10 @@
 //                MFMA
 //  k_tri64       the same contraction in FP64, 128 x 128 tiles
 //  k_nearest     each cell's nearest active station (batched variance)
-//  k_kgen<..>    fused distance -> covariance for the batched path, with
-//                the dual-form estimate k.alpha accumulated in FP64 and the
-//                locally deflated covariances delta for the variance
+//  k_kgen<..>    fused distance -> covariance for the batched path with the
+//                OK variance: the dual-form estimate k.alpha accumulated in
+//                FP64 and the locally deflated covariances delta (estimates
+//                alone: spk_est.hip)
 //  k_var_reduce  variance from the FP64 terms and the partial norms
 //  (the int8 plane-product contraction is in spk_int8.hip, the plain FP64
 //  path's kernels are in spk_plain.hip)
@@ -52,21 +53,10 @@ constexpr double kSumTol = 1e-9;
 // magnitude), while pinv drops the eigenvalues under 1e-15 of the largest
 // as the reference does.
 constexpr double kPinvKappa = 1e14;
-// Relative change of a cell's estimate by the second refinement step above
-// which the step is flagged SPK_ST_ILLCOND (the change is of the size of
-// the error left by the first step; the refined estimate is at least as
-// good), so unflagged steps stay well inside 1e-6.
-constexpr double kRefineTol = 1e-7;
 // L^-1 of the split-BF16 contraction: 1 = FP32 octets split into the
 // bfloat16 planes as k_tri_bf stages them (4 bytes per value read from
 // memory instead of 6), 0 = the planes themselves.
 constexpr int kBfA32 = 1;
-
-// np.isclose(x, 1.0) with rtol 1e-5, atol 1e-8 (interp/steps.py:418)
-__device__ inline bool isclose1(double x) {
-  const double tol = 1e-8 + 1e-5 * 1.0;
-  return fabs(x - 1.0) <= tol;
-}
 
 __global__ void k_recenter(const double *__restrict__ in,
                            double *__restrict__ out, int64_t n, double o) {
@@ -737,14 +727,11 @@ template <bool GEN>
 __global__ __launch_bounds__(256, 4) void k_kgen(
     const double *__restrict__ sx, const double *__restrict__ sy,
     const int32_t *__restrict__ idx, int64_t N,
-    const double *__restrict__ zact, int64_t ldz,
-    StepSc *__restrict__ sc, const spk_vg *__restrict__ vgs,
+    const StnRec *__restrict__ recs, StepSc *__restrict__ sc,
+    const spk_vg *__restrict__ vgs,
     const double *__restrict__ cx, const double *__restrict__ cy, int64_t Cs,
-    int64_t C, const double *__restrict__ cell_drift,
     const int32_t *__restrict__ perm, const int32_t *__restrict__ nrst,
-    int64_t ldn,
-    const double *__restrict__ V, int64_t ldv, int64_t ld, int method, int m,
-    double min_vg_val, int want_var, int all64, int skm,
+    int64_t ldn, int64_t ld, double min_vg_val, int all64,
     float *__restrict__ K32,
     double *__restrict__ K64, int64_t ldk, uint4 *__restrict__ Kb,
     const double *__restrict__ Gfull,
@@ -756,11 +743,9 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
   if (stp->status) return;
   const int n = stp->n;
   const int32_t *my = idx + (int64_t)sl * N;
-  const double *alpha = V + (int64_t)sl * ldv;
-  const double *w = alpha + ld;
-  const double *dal = w + ld;   // refinement correction of alpha (k_dual)
-  __shared__ double stx[kChunk], sty[kChunk], sal[kChunk], sw[kChunk];
-  __shared__ double sdal[kChunk];
+  // station records of the step, read at uniform addresses (scalar loads)
+  const StnRec *rec = recs + (int64_t)sl * N;
+  __shared__ double stx[kChunk], sty[kChunk];
   // one double of padding per slot row: lanes reading different slots at
   // the same station hit different banks
   __shared__ double sG[kSlots][kChunk + 1];
@@ -770,27 +755,31 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
   const int tid = threadIdx.x;
   const int64_t c = blockIdx.x * (int64_t)256 + tid;
   const bool valid = c < Cs;
-  const double x = valid ? cx[c] : 0.0, y = valid ? cy[c] : 0.0;
+  const double x = valid ? coord_fast(cx[c]) : 0.0;
+  const double y = valid ? coord_fast(cy[c]) : 0.0;
   if (tid == 0) {
     vg_fast_init(vgs[sl], vf);
     n_slots = 0;
   }
   if (tid < kSlots) slot_j[tid] = -1;
-  const int cflag = method == SPK_M_SK ? 1 : 0;
   const double c0 = stp->c0;
-  const bool var_on = want_var && method == SPK_M_OK;
+  // the distance of the lags: dist_fast, or dist2 where a power or
+  // hole-effect component wants exact zeros
+  const bool simp = !GEN || vg_simple(vgs[sl]);
+  auto lag = [&](double sxj, double syj) {
+    return simp ? dist_fast(x - sxj, y - syj) : dist2(x, y, sxj, syj);
+  };
   // FP64 delta for the FP64 and the int8 contractions
   const bool use64 =
       all64 || (stp->flags & (SPK_ST_FP64VAR | SPK_ST_INT8VAR));
   // FP32-tier delta: FP32 (K32), or its three bfloat16 planes (Kb: octet
   // o of cell c of plane p at (p ld / 8 + o) ldk + c)
-  float *K32s = (var_on && !use64 && !Kb) ? K32 + (int64_t)sl * ld * ldk
-                                          : nullptr;
-  uint4 *Kbs = (var_on && !use64 && Kb) ? Kb + (int64_t)sl * 3 * (ld / 8) * ldk + c
-                                        : nullptr;
+  float *K32s = !use64 && !Kb ? K32 + (int64_t)sl * ld * ldk : nullptr;
+  uint4 *Kbs = !use64 && Kb ? Kb + (int64_t)sl * 3 * (ld / 8) * ldk + c
+                            : nullptr;
   const int64_t kbp = (ld / 8) * ldk;  // plane stride of Kbs
-  double *K64s = (var_on && use64) ? K64 + (int64_t)sl * ld * ldk : nullptr;
-  const double *Gs = var_on ? Gfull + (int64_t)sl * ld * ld : nullptr;
+  double *K64s = use64 ? K64 + (int64_t)sl * ld * ldk : nullptr;
+  const double *Gs = Gfull + (int64_t)sl * ld * ld;
   double beta[kJ];
   int slt[kJ];
 #pragma unroll
@@ -799,7 +788,7 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
     slt[q] = -1;
   }
   double qloc = 0.0;
-  if (var_on) {
+  {
     // the cell's nearest active station, from k_nearest
     const int bj = valid ? nrst[(int64_t)sl * ldn + c] : -1;
     __syncthreads();  // slot_j and n_slots initialised
@@ -818,8 +807,8 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
     const int ns = n_slots;
     if (tid < ns) {
       const int g = my[slot_j[tid]];
-      stx[tid] = sx[g];
-      sty[tid] = sy[g];
+      stx[tid] = coord_fast(sx[g]);
+      sty[tid] = coord_fast(sy[g]);
     }
     __syncthreads();
     // J: the cell's kJ nearest stations among the table (ascending)
@@ -880,8 +869,8 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
           if (t2 < q) v -= Lj[q][t2] * Lj[q][t2];
         if (v > 1e-8 * dq && dq > 0.0) {
           Lj[q][q] = sqrt(v);
-          kJv[q] = c0 - kg_vg<GEN>(vf, dist2(x, y, stx[slt[q]], sty[slt[q]]),
-                                   0, min_vg_val);
+          kJv[q] = c0 - kg_vg<GEN>(vf, lag(stx[slt[q]], sty[slt[q]]), 0,
+                                   min_vg_val);
           mm = q + 1;
         } else {
           ok = false;
@@ -930,8 +919,8 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
   const int one = vg_one_of(vf, vo);
   // Culling.  For a single bounded model whose far value nug + s equals c0
   // (and is above min_vg_val), k = c0 - gamma(h) is exactly 0 beyond a
-  // distance: h >= r (spherical), h c1 <= -42 (exponential) or h^2 c1 <= -42
-  // (Gaussian), where exp() < 2^-54 so that 1 - exp() rounds to 1.  A
+  // distance: h >= r (spherical), h c1 <= -61 (exponential) or h^2 c1 <= -61
+  // (Gaussian), where 2^y < 2^-54 so that 1 - 2^y rounds to 1.  A
   // sub-chunk of 16 stations whose bounding box is that far from every cell
   // of the block (the gap measured by dist2 itself, so that by monotone
   // rounding no cell-station distance the loop computes is below it), and
@@ -943,7 +932,7 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
   // step); otherwise zeros are written.
   __shared__ double s_bb[4][4];  // per wave, then the block's in row 0
   __shared__ int s_cull[kChunk / 16];
-  const bool cull_on = var_on && one >= 0 && c0 == vo.nug + vo.s &&
+  const bool cull_on = one >= 0 && c0 == vo.nug + vo.s &&
                        vo.nug + vo.s > min_vg_val;
   const bool zwrite = !(zskip && !all64 && !(stp->flags & SPK_ST_FP64VAR));
   if (cull_on) {
@@ -974,8 +963,6 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
     }
     // read after the station loop's first barrier
   }
-  double best = INFINITY;
-  int bi = 0;
   double e = 0.0, a = 0.0;
   // the estimate's change by the last refinement step
   double ke = 0.0;
@@ -983,15 +970,11 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
   for (int base = 0; base < n; base += kChunk) {
     __syncthreads();
     if (tid < kChunk && base + tid < n) {
-      const int g = my[base + tid];
-      stx[tid] = sx[g];
-      sty[tid] = sy[g];
-      sal[tid] = alpha[base + tid];
-      sw[tid] = w[base + tid];
-      sdal[tid] = dal[base + tid];
+      stx[tid] = rec[base + tid].x;
+      sty[tid] = rec[base + tid].y;
     }
     const int cnt = min(kChunk, n - base);
-    if (var_on) {
+    {
       const int ns = n_slots;
       for (int e2 = tid; e2 < ns * kChunk; e2 += 256) {
         const int k = e2 / kChunk, u = e2 % kChunk;
@@ -1029,9 +1012,9 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
           if (one == SPK_VG_SPH)
             far = D >= vo.r;
           else if (one == SPK_VG_EXP)
-            far = D * vo.c1 <= -42.0;
+            far = D * vo.c1 <= -61.0;
           else
-            far = (D * D) * vo.c1 <= -42.0;
+            far = (D * D) * vo.c1 <= -61.0;
           s_cull[tid >> 4] = (z && far) ? 1 : 0;
         }
       }
@@ -1039,23 +1022,23 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
     }
     unsigned nzf = 0;  // 16-station chunks of this pass with delta != 0
     if (valid) {
-      if (var_on) {
+      {
         // the station loop, specialised on a single bounded model, over
         // sub-chunks of 16 stations
         auto var_loop = [&](auto tag) {
           constexpr int MT = decltype(tag)::value;
           // delta of station j of the pass (and its estimate terms)
           auto eval = [&](int j) {
-            const double d = dist2(x, y, stx[j], sty[j]);
+            const StnRec &r = rec[base + j];
             double g;
             if constexpr (MT < 0)
-              g = kg_vg<GEN>(vf, d, 0, min_vg_val);
+              g = kg_vg<GEN>(vf, lag(r.x, r.y), 0, min_vg_val);
             else
-              g = vg_one<MT>(vo, d, min_vg_val);
+              g = vg_one<MT>(vo, dist_fast(x - r.x, y - r.y), min_vg_val);
             const double k = c0 - g;
-            e += k * sal[j];
-            a += k * sw[j];
-            ke += k * sdal[j];
+            e += k * r.alpha;
+            a += k * r.w;
+            ke += k * r.dalpha;
             double delta = k;
 #pragma unroll
             for (int q = 0; q < kJ; ++q)
@@ -1132,24 +1115,11 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
           default:
             var_loop(std::integral_constant<int, -1>{});
         }
-      } else {
-        for (int j = 0; j < cnt; ++j) {
-          const double d = dist2(x, y, stx[j], sty[j]);
-          if (d < best || (d == best && my[base + j] < my[bi])) {
-            best = d;
-            bi = base + j;
-          }
-          const double g = kg_vg<GEN>(vf, d, cflag, min_vg_val);
-          const double k = cflag ? g : c0 - g;
-          e += k * sal[j];
-          a += k * sw[j];
-          ke += k * sdal[j];
-        }
       }
     }
     // the chunk map of this wave's 64 cells (one 128-cell tile of the
     // contraction): any lane's nonzero delta marks the chunk
-    if (var_on && nzb) {
+    if (nzb) {
       unsigned m = nzf;
 #pragma unroll
       for (int off = 32; off >= 1; off >>= 1) m |= __shfl_xor(m, off, 64);
@@ -1165,7 +1135,6 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
   if (!valid) return;
   const int64_t oc = perm ? (int64_t)perm[c] : c;
   double *eo = est + (int64_t)sl * ldo;
-  const double *z = zact + (int64_t)sl * ldz;
   // Residual check: the second refinement step changed this cell's
   // estimate by de, of the size of the error the first one left, and the
   // result is at least as good; a change above kRefineTol of the cell's
@@ -1173,36 +1142,15 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
   // the step ill-conditioned: no FP64 solve of it is reproducible to 1e-6.
   // (The variance is far less sensitive: in the dual form its error stays
   // near 1e-9 where the estimate's reaches 1e-6.)
-  double de = ke;
-  double ev;
-  if (method == SPK_M_OK) {
-    ev = e + stp->a0;
-    de += stp->dh[0];
-  } else if (method == SPK_M_EDK) {
-    ev = e + stp->h[0];
-    de += stp->dh[0];
-    for (int k = 0; k < m; ++k) {
-      const double f = cell_drift[(int64_t)k * C + oc];
-      ev += stp->h[1 + k] * f;
-      de += stp->dh[1 + k] * f;
-    }
-  } else if (skm) {
-    // SK with the step mean m as known mean: m + k^T C^-1 (z - m 1)
-    // = k.alpha + m (1 - k.w)
-    ev = e + stp->mean * (1.0 - a);
-  } else {  // the reference's SK
-    ev = isclose1(a) ? e : z[bi];
-  }
+  const double de = ke + stp->dh[0];
+  const double ev = e + stp->a0;
   const bool ill = fabs(de) > kRefineTol * fmax(fabs(ev), 1e-3 * stp->zabs);
   if (ill && !(stp->flags & SPK_ST_ILLCOND))
     atomicOr(&sc[sl].flags, SPK_ST_ILLCOND);
   eo[oc] = ev;
-  if (method == SPK_M_OK) {
-    if (var_on)
-      abuf[(int64_t)sl * ldk + c] =
-          c0 - qloc + (a - 1.0) * (a - 2.0) / stp->b;
-    if (var_on && dmax) dmax[(int64_t)sl * ldk + c] = dm;
-  }
+  abuf[(int64_t)sl * ldk + c] =
+      c0 - qloc + (a - 1.0) * (a - 2.0) / stp->b;
+  if (dmax) dmax[(int64_t)sl * ldk + c] = dm;
 }
 
 // ---- IDW and nearest neighbour -------------------------------------------------
@@ -1725,6 +1673,7 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
   struct Set {
     int32_t *idx;
     double *zact, *A, *Li, *M, *V, *T0, *Gm;
+    StnRec *rec;  // the steps' station records (batched path)
     float *L32;
     uint4 *Lb;   // split-BF16 planes of L^-1 (bfop)
     int8_t *L8;  // int8 planes of L^-1 rows (mixed path)
@@ -1781,6 +1730,7 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
       SPK_TRY(get("M", S * strideM * 8, (void **)&q.M));
     } else {
       SPK_TRY(get("V", S * 4 * ld * 8, (void **)&q.V));
+      SPK_TRY(get("rec", S * N * sizeof(StnRec), (void **)&q.rec));
       if (want_var) SPK_TRY(get("Gm", S * strideM * 8, (void **)&q.Gm));
       if (mixed && want_var) {
         if (bfop)
@@ -2114,6 +2064,8 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
           return check_launch("k_dual");
         }));
       }
+      SPK_TRY(stn_records(sf, sx, sy, q.idx, N, q.sc, q.V, 4 * ld, ld, Sb,
+                          q.rec));
       // Steps whose Cholesky succeeded with a condition estimate above
       // kPinvKappa take the pseudo-inverse route too: their solve is
       // rounding noise, where the reference's pinv truncates the
@@ -2283,18 +2235,24 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
           SPK_HIP(hipMemsetAsync(nzb, 0, (size_t)Sb * nzt * nzk, sm));
         {
           ProfScope ps(ctx, "kgen");
-          hipLaunchKernelGGL(simple ? k_kgen<false> : k_kgen<true>,
-                             dim3((unsigned)ceil_div(cn, 256), Sb),
-                             dim3(256), 0, sm, sx, sy, q.idx, N, q.zact, ldz,
-                             q.sc, gb, (perm ? pcx : cx) + cb,
-                             (perm ? pcy : cy) + cb, cn, C, cd,
-                             perm ? perm + cb : (const int32_t *)nullptr,
-                             (const int32_t *)nrst, ldk, q.V,
-                             4 * ld, ld, method, m, mvg, want_var ? 1 : 0,
-                             mixed ? 0 : 1, skm, K32, K64, ldk, Kb,
-                             q.Gm,
-                             abuf, perm ? eb : eb + cb, C, dmax, nzb,
-                             nzt, nzk, zskip);
+          if (want_var)
+            hipLaunchKernelGGL(simple ? k_kgen<false> : k_kgen<true>,
+                               dim3((unsigned)ceil_div(cn, 256), Sb),
+                               dim3(256), 0, sm, sx, sy, q.idx, N,
+                               (const StnRec *)q.rec, q.sc, gb,
+                               (perm ? pcx : cx) + cb, (perm ? pcy : cy) + cb,
+                               cn, perm ? perm + cb : (const int32_t *)nullptr,
+                               (const int32_t *)nrst, ldk, ld, mvg,
+                               mixed ? 0 : 1, K32, K64, ldk, Kb, q.Gm, abuf,
+                               perm ? eb : eb + cb, C, dmax, nzb, nzt, nzk,
+                               zskip);
+          else
+            SPK_TRY(est_steps(sm, sx, sy, q.idx, N, (const StnRec *)q.rec,
+                              q.zact, ldz, q.sc, gb, Sb, simple,
+                              (perm ? pcx : cx) + cb, (perm ? pcy : cy) + cb,
+                              cn, C, cd,
+                              perm ? perm + cb : (const int32_t *)nullptr,
+                              method, m, skm, mvg, perm ? eb : eb + cb, C));
         }
         SPK_TRY(check_launch("k_kgen"));
         if (!want_var) continue;

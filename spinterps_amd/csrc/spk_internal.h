@@ -155,6 +155,57 @@ __host__ __device__ inline double dist2(double x1, double y1, double x2,
   return sqrt(s);
 }
 
+// A coordinate for dist_fast: infinite ones (a station or cell beyond every
+// range) become so large that every bounded model is at its sill and the
+// square stays finite; NaN stays NaN.
+__device__ inline double coord_fast(double x) {
+  return isinf(x) ? copysign(1e140, x) : x;
+}
+
+// dist2's value for the cell kernels' inner loops: sqrt(s) from the
+// hardware's reciprocal square root (relative error 5e-8) and two coupled
+// Newton steps, which gave sqrt()'s bits on 32 million arguments, without
+// its handling of tiny, zero and infinite arguments (8 instructions instead
+// of about 16).  The constant keeps coincident points off 0 * inf (their
+// distance becomes 1e-150); it vanishes in any other sum of squares of
+// coordinates.
+__device__ inline double dist_fast(double dx, double dy) {
+  double s;
+  {
+#pragma clang fp contract(off)
+    s = (dx * dx) + (dy * dy) + 1e-300;
+  }
+  const double y = __builtin_amdgcn_rsq(s);
+  double g = s * y, h = 0.5 * y;
+  const double r = fma(-g, h, 0.5);
+  g = fma(g, r, g);
+  h = fma(h, r, h);
+  return fma(fma(-g, g, s), h, g);
+}
+
+// 2^y for finite y <= 0: the nearest integer goes to the exponent, the rest
+// f (|f| <= 1/2) through a degree-11 Chebyshev interpolant of 2^f (largest
+// relative error 2e-17).  15 instructions, without the range tests of
+// exp(); NaN stays NaN.
+__device__ inline double exp2_neg(double y) {
+  const double k = rint(y);
+  const double f = y - k;
+  double p = 4.4558179083360645e-10;
+  p = fma(p, f, 7.074194297288521e-09);
+  p = fma(p, f, 1.0178057087733941e-07);
+  p = fma(p, f, 1.3215432535912375e-06);
+  p = fma(p, f, 1.5252733841556773e-05);
+  p = fma(p, f, 0.00015403530463724353);
+  p = fma(p, f, 0.001333355814640647);
+  p = fma(p, f, 0.009618129107587256);
+  p = fma(p, f, 0.055504108664821625);
+  p = fma(p, f, 0.24022650695910158);
+  p = fma(p, f, 0.6931471805599453);
+  p = fma(p, f, 1.0);
+  return ldexp(p, (int)k);
+}
+constexpr double kLog2e = 1.4426950408889634;
+
 // One variogram component gamma(h; r, s), pyx:38-83 (same operation order).
 // PH = false leaves out the Pow and Hol models (NaN for them), whose pow and
 // sin cost registers in kernels that never see them.
@@ -225,15 +276,15 @@ __host__ __device__ inline double vg_entry(const spk_vg &vg, double h,
 }
 
 // A variogram with per-component constants folded in (reciprocals instead
-// of divisions) for the batched path's bulk cell evaluation.  Values agree
-// with vg_entry to a few ulp; the plain FP64 path keeps vg_entry.
+// of divisions, exponents to base two) for the bulk cell evaluation.  Values
+// agree with vg_entry to a few ulp.
 struct VgFast {
   int n;
   int type[SPK_VG_MAX];
   double s[SPK_VG_MAX], r[SPK_VG_MAX], c1[SPK_VG_MAX], c2[SPK_VG_MAX];
 };
 
-__host__ __device__ inline void vg_fast_init(const spk_vg &vg, VgFast &f) {
+__device__ inline void vg_fast_init(const spk_vg &vg, VgFast &f) {
   f.n = vg.n;
   for (int k = 0; k < vg.n; ++k) {
     const double r = vg.range[k];
@@ -248,10 +299,10 @@ __host__ __device__ inline void vg_fast_init(const spk_vg &vg, VgFast &f) {
         f.c2[k] = 0.5 / (r * r * r);
         break;
       case SPK_VG_EXP:
-        f.c1[k] = -3.0 / r;
+        f.c1[k] = (-3.0 / r) * kLog2e;
         break;
       case SPK_VG_GAU:
-        f.c1[k] = -3.0 / (r * r);
+        f.c1[k] = (-3.0 / (r * r)) * kLog2e;
         break;
       case SPK_VG_LIN:
         f.c1[k] = 1.0 / r;
@@ -278,8 +329,8 @@ __device__ inline double vg_fast_entry(const VgFast &f, double h,
       case SPK_VG_SPH:
         g = (h >= f.r[k]) ? s : s * (h * f.c1[k] - (h * h * h) * f.c2[k]);
         break;
-      case SPK_VG_EXP: g = s * (1.0 - exp(h * f.c1[k])); break;
-      case SPK_VG_GAU: g = s * (1.0 - exp((h * h) * f.c1[k])); break;
+      case SPK_VG_EXP: g = s * (1.0 - exp2_neg(h * f.c1[k])); break;
+      case SPK_VG_GAU: g = s * (1.0 - exp2_neg((h * h) * f.c1[k])); break;
       case SPK_VG_LIN: g = (h > f.r[k]) ? s : s * (h * f.c1[k]); break;
       case SPK_VG_POW: g = s * pow(h, f.r[k]); break;
       case SPK_VG_HOL: {
@@ -315,8 +366,8 @@ __device__ inline double vg_simple_entry(const VgFast &f, double h,
       case SPK_VG_SPH:
         g = (h >= f.r[k]) ? s : s * (h * f.c1[k] - (h * h * h) * f.c2[k]);
         break;
-      case SPK_VG_EXP: g = s * (1.0 - exp(h * f.c1[k])); break;
-      case SPK_VG_GAU: g = s * (1.0 - exp((h * h) * f.c1[k])); break;
+      case SPK_VG_EXP: g = s * (1.0 - exp2_neg(h * f.c1[k])); break;
+      case SPK_VG_GAU: g = s * (1.0 - exp2_neg((h * h) * f.c1[k])); break;
       case SPK_VG_LIN: g = (h > f.r[k]) ? s : s * (h * f.c1[k]); break;
       default: g = NAN;
     }
@@ -365,9 +416,9 @@ __device__ inline double vg_one(const VgOne &o, double h, double min_vg_val) {
   if constexpr (MT == SPK_VG_SPH)
     g = (h >= o.r) ? o.s : o.s * (h * o.c1 - (h * h * h) * o.c2);
   else if constexpr (MT == SPK_VG_EXP)
-    g = o.s * (1.0 - exp(h * o.c1));
+    g = o.s * (1.0 - exp2_neg(h * o.c1));
   else
-    g = o.s * (1.0 - exp((h * h) * o.c1));
+    g = o.s * (1.0 - exp2_neg((h * h) * o.c1));
   double acc = o.nug + g;
   if (acc <= min_vg_val) acc = 0.0;
   return acc;

@@ -23,6 +23,17 @@ __device__ inline int xcd_remap(int lin, int G) {
   return x * q + min(x, r) + (lin >> 3);
 }
 
+// Relative change of a cell's estimate by the second refinement step above
+// which the step is flagged SPK_ST_ILLCOND (the change is of the size of
+// the error left by the first step; the refined estimate is at least as
+// good), so unflagged steps stay well inside 1e-6.
+constexpr double kRefineTol = 1e-7;
+
+// np.isclose(x, 1.0) with rtol 1e-5, atol 1e-8 (interp/steps.py:418)
+__device__ inline bool isclose1(double x) {
+  return fabs(x - 1.0) <= 1e-8 + 1e-5;
+}
+
 // The steps of a batch one contraction launch takes (blockIdx.z indexes
 // s[]), chosen on the host from the step records after the factorisation:
 // blocks of the other steps would only exit.
@@ -56,6 +67,26 @@ __global__ void k_idw_mfma(const double *sx, const double *sy, int64_t N,
                            const int32_t *idx, const double *zact,
                            int64_t ldz, const double *cx, const double *cy,
                            int64_t C, double p, double *est, int *bad);
+
+// ---- batched estimates (spk_est.hip) -----------------------------------------
+// What the cell kernels read of one active station of a step, in one cache
+// line's half: position, dual vectors alpha and w, last refinement
+// correction of alpha.
+struct alignas(64) StnRec {
+  double x, y, alpha, w, dalpha, pad_[3];
+};
+// rec[s * N + j] of every step's active stations (after the dual vectors)
+int stn_records(hipStream_t st, const double *sx, const double *sy,
+                const int32_t *idx, int64_t N, const StepSc *sc,
+                const double *V, int64_t ldv, int64_t ld, int S, StnRec *rec);
+// dual-form estimates of the cells [0, Cs) of S steps, without a variance
+int est_steps(hipStream_t st, const double *sx, const double *sy,
+              const int32_t *idx, int64_t N, const StnRec *rec,
+              const double *zact, int64_t ldz, StepSc *sc, const spk_vg *vgs,
+              int S, bool simple, const double *cx, const double *cy,
+              int64_t Cs, int64_t C, const double *cell_drift,
+              const int32_t *perm, int method, int m, int skm,
+              double min_vg_val, double *est, int64_t ldo);
 
 // ---- plain FP64 contraction (spk_plain.hip) ---------------------------------
 // stations per block of k_plain_rhs (grid.y = ceil(stations / kPlainStn))

@@ -16,11 +16,6 @@ namespace spk {
 
 typedef double p4_t __attribute__((ext_vector_type(4)));
 
-// np.isclose(x, 1.0) with rtol 1e-5, atol 1e-8 (interp/steps.py:418)
-__device__ inline bool plain_isclose1(double x) {
-  return fabs(x - 1.0) <= 1e-8 + 1e-5;
-}
-
 // One column of a station chunk: value of every station of the chunk at
 // the thread's cell, stored row by row.
 template <typename F>
@@ -28,7 +23,7 @@ __device__ inline void plain_col(const double2 *st, int cnt, double x,
                                  double y, double *R, int64_t ldr, F val) {
 #pragma unroll 4
   for (int j = 0; j < cnt; ++j)
-    R[(int64_t)j * ldr] = val(dist2(x, y, st[j].x, st[j].y));
+    R[(int64_t)j * ldr] = val(dist_fast(x - st[j].x, y - st[j].y));
 }
 
 // grid (cells / 256, stations / 128, steps).  One bounded model with or
@@ -60,9 +55,10 @@ __global__ __launch_bounds__(256) void k_plain_rhs(
   __shared__ int model;
   const int tid = threadIdx.x;
   const int covar = method == SPK_M_SK ? 1 : 0;
+  const int32_t *my = idx + (int64_t)s * N + j0;
   if (tid < kPlainStn && j0 + tid < n) {
-    const int g = idx[(int64_t)s * N + j0 + tid];
-    st[tid] = double2{sx[g], sy[g]};
+    const int g = my[tid];
+    st[tid] = double2{coord_fast(sx[g]), coord_fast(sy[g])};
   }
   if (tid == kPlainStn) {
     vg = vgs[s];
@@ -76,7 +72,7 @@ __global__ __launch_bounds__(256) void k_plain_rhs(
   const int64_t c = blockIdx.x * (int64_t)256 + tid;
   if (c >= Cs) return;
   const int cnt = min(kPlainStn, n - j0);
-  const double x = cx[c], y = cy[c];
+  const double x = coord_fast(cx[c]), y = coord_fast(cy[c]);
   double *Rs = R + (int64_t)s * strideR;
   double *Rc = Rs + (int64_t)j0 * ldr + c;
   const VgOne o = one;
@@ -116,9 +112,10 @@ __global__ __launch_bounds__(256) void k_plain_rhs(
         return vg_one<SPK_VG_GAU>(o, h, min_vg_val);
       });
   } else {
-    plain_col(st, cnt, x, y, Rc, ldr, [&](double h) {
-      return vg_entry(vg, h, covar, min_vg_val);
-    });
+    for (int j = 0; j < cnt; ++j)
+      Rc[(int64_t)j * ldr] =
+          vg_entry(vg, dist2(cx[c], cy[c], sx[my[j]], sy[my[j]]), covar,
+                   min_vg_val);
   }
   if (j0 > 0) return;
   if (method != SPK_M_SK) Rs[(int64_t)n * ldr + c] = 1.0;
@@ -324,7 +321,7 @@ __global__ __launch_bounds__(256) void k_plain_fin(
       !(sc[sl].flags & SPK_ST_ILLCOND))
     atomicOr(&sc[sl].flags, SPK_ST_ILLCOND);
   const double *z = zact + (int64_t)sl * ldz;
-  const bool far = valid && !skm && !plain_isclose1(l);
+  const bool far = valid && !skm && !isclose1(l);
   int bi = 0;
   if (__syncthreads_or(far ? 1 : 0)) {
     __shared__ double2 st[256];

@@ -659,28 +659,6 @@ __device__ inline void de_bounds(const int32_t *cd, int c, double h0,
   }
 }
 
-// 2^y for y <= 0: the nearest integer goes to the exponent, the rest f
-// (|f| <= 1/2) through a degree-11 Chebyshev interpolant of 2^f (largest
-// relative error 2e-17).
-__device__ inline double de_exp2(double y) {
-  y = fmax(y, -1100.0);  // 2^-1100 is zero; keeps -inf out of y - k
-  const double k = rint(y);
-  const double f = y - k;
-  double p = 4.4558179083360645e-10;
-  p = fma(p, f, 7.074194297288521e-09);
-  p = fma(p, f, 1.0178057087733941e-07);
-  p = fma(p, f, 1.3215432535912375e-06);
-  p = fma(p, f, 1.5252733841556773e-05);
-  p = fma(p, f, 0.00015403530463724353);
-  p = fma(p, f, 0.001333355814640647);
-  p = fma(p, f, 0.009618129107587256);
-  p = fma(p, f, 0.055504108664821625);
-  p = fma(p, f, 0.24022650695910158);
-  p = fma(p, f, 0.6931471805599453);
-  p = fma(p, f, 1.0);
-  return ldexp(p, (int)k);
-}
-
 // sum over bins [b0, b1) of (g - c - s f(h))^2, f per model
 template <typename F>
 __device__ inline double de_sum(const double *__restrict__ h,
@@ -743,18 +721,18 @@ __global__ __launch_bounds__(256) void k_de_energy(
       sl = cs;
     }
   }
-  const double kLog2e = 1.4426950408889634;
   if (others == 0) {
     acc = de_sum(h, g, b0, b1, [&](double, double gb) { return gb - nug; });
   } else if (others == 1 && ty == SPK_VG_EXP) {
+    // (the bound keeps a range of zero, -inf, out of exp2_neg)
     const double c = (-3.0 / rg) * kLog2e, top = nug + sl;
     acc = de_sum(h, g, b0, b1, [&](double hb, double gb) {
-      return fma(sl, de_exp2(hb * c), gb - top);
+      return fma(sl, exp2_neg(fmax(hb * c, -1100.0)), gb - top);
     });
   } else if (others == 1 && ty == SPK_VG_GAU) {
     const double c = (-3.0 / (rg * rg)) * kLog2e, top = nug + sl;
     acc = de_sum(h, g, b0, b1, [&](double hb, double gb) {
-      return fma(sl, de_exp2((hb * hb) * c), gb - top);
+      return fma(sl, exp2_neg(fmax((hb * hb) * c, -1100.0)), gb - top);
     });
   } else if (others == 1 && ty == SPK_VG_SPH) {
     const double c = 1.0 / rg;
