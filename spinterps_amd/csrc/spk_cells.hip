@@ -723,8 +723,14 @@ __global__ __launch_bounds__(256) void k_nearest(
   if (tid == 0 && ovf) atomicOr(&stp->flags, SPK_ST_FP64VAR);
 }
 
+// Bound: FP64 VALU issue and latency (about 80 instructions per station and
+// cell), and the write of delta (6 bytes per value, 195 GB for the hourly
+// batch's 46 % of stations that culling leaves: 41 of 110 ms at the copy
+// rate).  Three waves per SIMD with 168 registers: 3.24 ms per stripe of the
+// hourly batch, against 3.42 with four waves and more spills, and 4.34 with
+// one station evaluated at a time.
 template <bool GEN>
-__global__ __launch_bounds__(256, 4) void k_kgen(
+__global__ __launch_bounds__(256, 3) void k_kgen(
     const double *__restrict__ sx, const double *__restrict__ sy,
     const int32_t *__restrict__ idx, int64_t N,
     const StnRec *__restrict__ recs, StepSc *__restrict__ sc,
@@ -744,7 +750,7 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
   const int n = stp->n;
   const int32_t *my = idx + (int64_t)sl * N;
   // station records of the step, read at uniform addresses (scalar loads)
-  const StnRec *rec = recs + (int64_t)sl * N;
+  const StnRec *rec = recs + sl * rec_stride(N);
   __shared__ double stx[kChunk], sty[kChunk];
   // one double of padding per slot row: lanes reading different slots at
   // the same station hit different banks
@@ -916,7 +922,10 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
   for (int q = 0; q < kJ; ++q) slq[q] = slt[q] >= 0 ? slt[q] : 0;
   double dm = 0.0;  // max |delta| of the cell (int8 plane scaling)
   VgOne vo;
-  const int one = vg_one_of(vf, vo);
+  int one = vg_one_of(vf, vo);
+  // with min_vg_val <= 0 and nonnegative sills the cut at min_vg_val
+  // (pyx:217) changes nothing and the specialised loop leaves it out
+  if (!(min_vg_val <= 0.0 && vo.s >= 0.0 && vo.nug >= 0.0)) one = -1;
   // Culling.  For a single bounded model whose far value nug + s equals c0
   // (and is above min_vg_val), k = c0 - gamma(h) is exactly 0 beyond a
   // distance: h >= r (spherical), h c1 <= -61 (exponential) or h^2 c1 <= -61
@@ -980,7 +989,8 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
         const int k = e2 / kChunk, u = e2 % kChunk;
         // staged as covariances c0 - G: a station out of range of the cell
         // and of every J station then gives delta = 0 exactly
-        if (u < cnt) sG[k][u] = c0 - Gs[(int64_t)slot_j[k] * ld + base + u];
+        sG[k][u] =
+            u < cnt ? c0 - Gs[(int64_t)slot_j[k] * ld + base + u] : 0.0;
       }
     }
     __syncthreads();
@@ -1027,25 +1037,83 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
         // sub-chunks of 16 stations
         auto var_loop = [&](auto tag) {
           constexpr int MT = decltype(tag)::value;
-          // delta of station j of the pass (and its estimate terms)
-          auto eval = [&](int j) {
-            const StnRec &r = rec[base + j];
-            double g;
-            if constexpr (MT < 0)
-              g = kg_vg<GEN>(vf, lag(r.x, r.y), 0, min_vg_val);
-            else
-              g = vg_one<MT>(vo, dist_fast(x - r.x, y - r.y), min_vg_val);
-            const double k = c0 - g;
-            e += k * r.alpha;
-            a += k * r.w;
-            ke += k * r.dalpha;
-            double delta = k;
+          // delta of stations j .. j + 3 of the pass and their estimate
+          // terms.  Four at once, with no branch between them, so that the
+          // chains of one station (about 40 dependent FP64 instructions)
+          // overlap.  FULL: stations past the step's last one are records
+          // out of every range with zero vectors (stn_records) and zero
+          // slot entries, whose k and delta are exactly zero for a single
+          // bounded model; else those from j1 on are set to zero.
+          auto eval4 = [&](auto full, int j, int j1, double (&dl)[4]) {
+            constexpr bool FULL = decltype(full)::value;
 #pragma unroll
-            for (int q = 0; q < kJ; ++q)
-              delta -= sG[slq[q]][j] * beta[q];
-            dm = fmax(dm, fabs(delta));
-            if (delta != 0.0) nzf |= 1u << (j >> 4);
-            return delta;
+            for (int u = 0; u < 4; ++u) {
+              const int ju = FULL ? j + u : min(j + u, j1 - 1);
+              const StnRec &r = rec[base + ju];
+              double g;
+              if constexpr (MT < 0)
+                g = kg_vg<GEN>(vf, lag(r.x, r.y), 0, min_vg_val);
+              else
+                g = vg_one_pos<MT>(vo, dist_fast(x - r.x, y - r.y));
+              double k = c0 - g;
+              if (!FULL && j + u >= j1) k = 0.0;
+              dl[u] = k;
+            }
+#pragma unroll
+            for (int u = 0; u < 4; ++u) {
+              const int ju = FULL ? j + u : min(j + u, j1 - 1);
+              const StnRec &r = rec[base + ju];
+              e += dl[u] * r.alpha;
+              a += dl[u] * r.w;
+              ke += dl[u] * r.dalpha;
+#pragma unroll
+              for (int q = 0; q < kJ; ++q)
+                dl[u] -= sG[slq[q]][ju] * beta[q];
+              if (!FULL && j + u >= j1) dl[u] = 0.0;
+            }
+          };
+          // 16 stations from j0 of a step whose delta goes to bfloat16
+          // planes: both octets, zero beyond the pass
+          auto planes16 = [&](auto full, int j0, int j1) {
+            uint32_t any = 0;
+            for (int h = 0; h < 2; ++h) {
+              uint32_t hw[4], mw[4], lw[4];
+#pragma unroll
+              for (int v = 0; v < 2; ++v) {
+                double dl[4];
+                eval4(full, j0 + 8 * h + 4 * v, j1, dl);
+#pragma unroll
+                for (int u = 0; u < 2; ++u)
+                  split3f2((float)dl[2 * u], (float)dl[2 * u + 1],
+                           hw[2 * v + u], mw[2 * v + u], lw[2 * v + u]);
+              }
+              const int64_t o = (base + j0 + 8 * h) >> 3;
+              Kbs[o * ldk] = uint4{hw[0], hw[1], hw[2], hw[3]};
+              Kbs[kbp + o * ldk] = uint4{mw[0], mw[1], mw[2], mw[3]};
+              Kbs[2 * kbp + o * ldk] = uint4{lw[0], lw[1], lw[2], lw[3]};
+              // a value whose leading term is +-0 has no others
+              any |= hw[0] | hw[1] | hw[2] | hw[3];
+            }
+            if (any & 0x7fff7fffu) nzf |= 1u << (j0 >> 4);
+          };
+          // the same for FP32 or FP64 delta
+          auto rows16 = [&](auto full, int j0, int j1) {
+            bool any = false;
+            for (int j = j0; j < j1; j += 4) {
+              double dl[4];
+              eval4(full, j, j1, dl);
+#pragma unroll
+              for (int u = 0; u < 4; ++u) {
+                if (!decltype(full)::value && j + u >= j1) break;
+                dm = fmax(dm, fabs(dl[u]));
+                any = any || dl[u] != 0.0;
+                if (K32s)
+                  K32s[(int64_t)(base + j + u) * ldk + c] = (float)dl[u];
+                else
+                  K64s[(int64_t)(base + j + u) * ldk + c] = dl[u];
+              }
+            }
+            if (any) nzf |= 1u << (j0 >> 4);
           };
           for (int j0 = 0; j0 < cnt; j0 += 16) {
             const int j1 = min(cnt, j0 + 16);
@@ -1069,37 +1137,11 @@ __global__ __launch_bounds__(256, 4) void k_kgen(
               }
               continue;
             }
-            if (Kbs) {
-              // both octets of the 16 stations, zero beyond the pass
-              for (int h = 0; h < 2; ++h) {
-                const int jb = j0 + 8 * h;
-                uint32_t hw[4], mw[4], lw[4];
-#pragma unroll
-                for (int u = 0; u < 8; ++u) {
-                  const int j = jb + u;
-                  const float df = j < j1 ? (float)eval(j) : 0.0f;
-                  uint16_t hh, mm2, ll;
-                  split3f(df, hh, mm2, ll);
-                  const int sh = (u & 1) * 16;
-                  if (!(u & 1)) hw[u / 2] = mw[u / 2] = lw[u / 2] = 0u;
-                  hw[u / 2] |= (uint32_t)hh << sh;
-                  mw[u / 2] |= (uint32_t)mm2 << sh;
-                  lw[u / 2] |= (uint32_t)ll << sh;
-                }
-                const int64_t o = (base + jb) >> 3;
-                Kbs[o * ldk] = uint4{hw[0], hw[1], hw[2], hw[3]};
-                Kbs[kbp + o * ldk] = uint4{mw[0], mw[1], mw[2], mw[3]};
-                Kbs[2 * kbp + o * ldk] = uint4{lw[0], lw[1], lw[2], lw[3]};
-              }
-            } else {
-              for (int j = j0; j < j1; ++j) {
-                const double delta = eval(j);
-                if (K32s)
-                  K32s[(int64_t)(base + j) * ldk + c] = (float)delta;
-                else
-                  K64s[(int64_t)(base + j) * ldk + c] = delta;
-              }
-            }
+            using Full = std::integral_constant<bool, (MT >= 0)>;
+            if (Kbs)
+              planes16(Full{}, j0, j1);
+            else
+              rows16(Full{}, j0, j1);
           }
         };
         switch (one) {
@@ -1730,7 +1772,8 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
       SPK_TRY(get("M", S * strideM * 8, (void **)&q.M));
     } else {
       SPK_TRY(get("V", S * 4 * ld * 8, (void **)&q.V));
-      SPK_TRY(get("rec", S * N * sizeof(StnRec), (void **)&q.rec));
+      SPK_TRY(get("rec", S * rec_stride(N) * sizeof(StnRec),
+                  (void **)&q.rec));
       if (want_var) SPK_TRY(get("Gm", S * strideM * 8, (void **)&q.Gm));
       if (mixed && want_var) {
         if (bfop)

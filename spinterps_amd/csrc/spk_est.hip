@@ -6,7 +6,7 @@
 
 namespace spk {
 
-// grid (ceil(n_max / 256), steps)
+// grid (ceil(rec_stride(N) / 256), steps)
 __global__ __launch_bounds__(256) void k_stn_rec(
     const double *__restrict__ sx, const double *__restrict__ sy,
     const int32_t *__restrict__ idx, int64_t N, const StepSc *__restrict__ sc,
@@ -15,24 +15,26 @@ __global__ __launch_bounds__(256) void k_stn_rec(
   const int s = blockIdx.y;
   if (sc[s].status) return;
   const int j = blockIdx.x * 256 + threadIdx.x;
-  if (j >= sc[s].n) return;
-  const int g = idx[(int64_t)s * N + j];
-  const double *v = V + (int64_t)s * ldv + j;  // alpha, w, dalpha: ld apart
-  StnRec r;
-  r.x = coord_fast(sx[g]);
-  r.y = coord_fast(sy[g]);
-  r.alpha = v[0];
-  r.w = v[ld];
-  r.dalpha = v[2 * ld];
-  r.pad_[0] = r.pad_[1] = r.pad_[2] = 0.0;
-  rec[(int64_t)s * N + j] = r;
+  const int n = sc[s].n;
+  if (j >= (n + 15) / 16 * 16) return;
+  StnRec r = {1e140, 1e140, 0.0, 0.0, 0.0, {0.0, 0.0, 0.0}};
+  if (j < n) {
+    const int g = idx[(int64_t)s * N + j];
+    const double *v = V + (int64_t)s * ldv + j;  // alpha, w, dalpha: ld apart
+    r.x = coord_fast(sx[g]);
+    r.y = coord_fast(sy[g]);
+    r.alpha = v[0];
+    r.w = v[ld];
+    r.dalpha = v[2 * ld];
+  }
+  rec[s * rec_stride(N) + j] = r;
 }
 
 int stn_records(hipStream_t st, const double *sx, const double *sy,
                 const int32_t *idx, int64_t N, const StepSc *sc,
                 const double *V, int64_t ldv, int64_t ld, int S, StnRec *rec) {
-  hipLaunchKernelGGL(k_stn_rec, dim3((unsigned)ceil_div(N, 256), S), dim3(256),
-                     0, st, sx, sy, idx, N, sc, V, ldv, ld, rec);
+  hipLaunchKernelGGL(k_stn_rec, dim3((unsigned)ceil_div(rec_stride(N), 256), S),
+                     dim3(256), 0, st, sx, sy, idx, N, sc, V, ldv, ld, rec);
   return check_launch("k_stn_rec");
 }
 
@@ -85,7 +87,7 @@ __global__ __launch_bounds__(256) void k_est(
   const bool valid = c < Cs;
   const double xr = valid ? cx[c] : 0.0, yr = valid ? cy[c] : 0.0;
   const double x = coord_fast(xr), y = coord_fast(yr);
-  const StnRec *rec = recs + (int64_t)sl * N;
+  const StnRec *rec = recs + sl * rec_stride(N);
   const bool sk = method == SPK_M_SK;
   const double c0 = stp->c0;
   VgOne o;

@@ -410,7 +410,7 @@ __device__ inline int vg_one_of(const VgFast &f, VgOne &o) {
   return f.type[model];
 }
 template <int MT>
-__device__ inline double vg_one(const VgOne &o, double h, double min_vg_val) {
+__device__ inline double vg_one_pos(const VgOne &o, double h) {
 #pragma clang fp contract(off)
   double g;
   if constexpr (MT == SPK_VG_SPH)
@@ -419,9 +419,13 @@ __device__ inline double vg_one(const VgOne &o, double h, double min_vg_val) {
     g = o.s * (1.0 - exp2_neg(h * o.c1));
   else
     g = o.s * (1.0 - exp2_neg((h * h) * o.c1));
-  double acc = o.nug + g;
-  if (acc <= min_vg_val) acc = 0.0;
-  return acc;
+  return o.nug + g;
+}
+// with the cut at min_vg_val
+template <int MT>
+__device__ inline double vg_one(const VgOne &o, double h, double min_vg_val) {
+  const double acc = vg_one_pos<MT>(o, h);
+  return acc <= min_vg_val ? 0.0 : acc;
 }
 
 __host__ __device__ inline bool vg_simple(const spk_vg &vg) {

@@ -75,7 +75,13 @@ __global__ void k_idw_mfma(const double *sx, const double *sy, int64_t N,
 struct alignas(64) StnRec {
   double x, y, alpha, w, dalpha, pad_[3];
 };
-// rec[s * N + j] of every step's active stations (after the dual vectors)
+// Records per step: the active stations and up to 15 records out of every
+// range with zero vectors, to the end of a group of 16.
+__host__ __device__ inline int64_t rec_stride(int64_t N) {
+  return (N + 15) / 16 * 16;
+}
+// rec[s * rec_stride(N) + j] of every step's active stations (after the dual
+// vectors)
 int stn_records(hipStream_t st, const double *sx, const double *sy,
                 const int32_t *idx, int64_t N, const StepSc *sc,
                 const double *V, int64_t ldv, int64_t ld, int S, StnRec *rec);
