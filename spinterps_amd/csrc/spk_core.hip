@@ -530,6 +530,9 @@ int spk_ctx_destroy(spk_ctx *ctx) {
 int spk_ctx_set_stream(spk_ctx *ctx, void *s) {
   if (!ctx) return set_error(SPK_EARG, "null ctx");
   SPK_HIP(hipSetDevice(ctx->device));
+  // callers set their current stream before every call: the same stream
+  // needs no wait, its work is in order
+  if (!ctx->own_stream && ctx->stream == (hipStream_t)s) return SPK_OK;
   SPK_HIP(hipStreamSynchronize(ctx->stream));
   if (ctx->own_stream) SPK_HIP(hipStreamDestroy(ctx->stream));
   ctx->stream = (hipStream_t)s;
