@@ -193,7 +193,7 @@ __host__ __device__ constexpr int64_t b_off(int l) {
   return w_off(l) + (int64_t)mlp_dim(l) * mlp_dim(l - 1);
 }
 constexpr int64_t kNParams = w_off(5);
-constexpr int kMaxBatch = 1 << 21;  // 32-row tiles in grid.y <= 65535
+constexpr int kMaxBatch = 1 << 21;
 
 __device__ inline float gelu(float x) {
   return 0.5f * x * (1.0f + erff(x * 0.70710678118654752f));
@@ -204,122 +204,251 @@ __device__ inline float gelu_d(float x) {
   return cdf + x * pdf;
 }
 
-// C[r][c] = sum_k A(r, k) B(k, c) over LDS tiles of 32.  A(r, k) =
-// A[r * lda + k] (TA = 0) or A[k * lda + r] (TA = 1); B(k, c) likewise.
-// beta = 0 overwrites, 1 accumulates.  16 x 16 threads, 2 x 2 outputs each.
-template <int TA, int TB>
-__global__ __launch_bounds__(256) void k_sgemm(int R, int Cc, int K,
-                                               const float *__restrict__ A,
-                                               int lda,
-                                               const float *__restrict__ B,
-                                               int ldb, float *__restrict__ Cm,
-                                               int ldc, int beta) {
-  __shared__ float As[32][33], Bs[32][33];
-  const int ty = threadIdx.x >> 4, tx = threadIdx.x & 15;
-  const int r0 = blockIdx.y * 32, c0 = blockIdx.x * 32;
-  float acc[2][2] = {{0.f, 0.f}, {0.f, 0.f}};
-  for (int k0 = 0; k0 < K; k0 += 32) {
-    for (int e = threadIdx.x; e < 32 * 32; e += 256) {
-      const int i = e >> 5, k = e & 31;
-      const int r = r0 + i, kk = k0 + k;
-      As[i][k] = (r < R && kk < K) ? (TA ? A[(int64_t)kk * lda + r]
-                                         : A[(int64_t)r * lda + kk])
-                                   : 0.f;
-      const int c = c0 + i;
-      Bs[i][k] = (c < Cc && kk < K) ? (TB ? B[(int64_t)c * ldb + kk]
-                                          : B[(int64_t)kk * ldb + c])
-                                    : 0.f;
-    }
-    __syncthreads();
-    for (int k = 0; k < 32; ++k) {
-      const float a0 = As[ty * 2][k], a1 = As[ty * 2 + 1][k];
-      const float b0 = Bs[tx * 2][k], b1 = Bs[tx * 2 + 1][k];
-      acc[0][0] += a0 * b0;
-      acc[0][1] += a0 * b1;
-      acc[1][0] += a1 * b0;
-      acc[1][1] += a1 * b1;
-    }
-    __syncthreads();
-  }
-  for (int a = 0; a < 2; ++a)
-    for (int b = 0; b < 2; ++b) {
-      const int r = r0 + ty * 2 + a, c = c0 + tx * 2 + b;
-      if (r < R && c < Cc) {
-        float *p = &Cm[(int64_t)r * ldc + c];
-        *p = beta ? *p + acc[a][b] : acc[a][b];
-      }
-    }
+typedef float mf4_t __attribute__((ext_vector_type(4)));
+__device__ inline mf4_t mfma32(float a, float b, mf4_t c) {
+  return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
 }
+// four consecutive floats at any float's alignment
+struct __attribute__((packed, aligned(4))) F4 {
+  float v[4];
+};
 
-// Z[b][o] += bias[o]; H = gelu(Z) (act) or H = Z
-__global__ void k_bias_act(float *__restrict__ Z, float *__restrict__ H,
-                           const float *__restrict__ bias, int B, int O,
-                           int act) {
-  for (int64_t e = blockIdx.x * 256 + threadIdx.x; e < (int64_t)B * O;
-       e += (int64_t)gridDim.x * 256) {
-    const float z = Z[e] + bias[e % O];
-    Z[e] = z;
-    H[e] = act ? gelu(z) : z;
-  }
-}
-
-// dZ = dH * gelu'(Z)
-__global__ void k_act_bwd(const float *__restrict__ Z, float *__restrict__ dH,
-                          int64_t n) {
-  for (int64_t e = blockIdx.x * 256 + threadIdx.x; e < n;
-       e += (int64_t)gridDim.x * 256)
-    dH[e] *= gelu_d(Z[e]);
-}
-
-// db[o] = sum_b dZ[b][o]
-__global__ void k_bias_grad(const float *__restrict__ dZ, int B, int O,
-                            float *__restrict__ db) {
-  const int o = blockIdx.x * 256 + threadIdx.x;
-  if (o >= O) return;
-  float acc = 0.f;
-  for (int b = 0; b < B; ++b) acc += dZ[(int64_t)b * O + o];
-  db[o] = acc;
-}
-
-// Mean loss over the batch and its gradient w.r.t. the outputs:
+// Forward pass of 16 samples per workgroup through all layers on FP32 MFMA,
+// activations in LDS; with TRAIN also the loss, its gradient with respect to
+// the outputs and the backward pass to every layer's dZ:
 // L = CE(softmax(y[0:3]), cls) + reg_w * sum_k (y[3+k] - t[k])^2 * m[k]
-// where m masks regression targets that are NaN; a class outside 0..2
-// drops the cross-entropy term of that sample.
-__global__ void k_loss(const float *__restrict__ Y, const int32_t *__restrict__ cls,
-                       const float *__restrict__ tgt, int B, float reg_w,
-                       float *__restrict__ dY, float *__restrict__ loss) {
-  __shared__ float red[256];
-  float acc = 0.f;
-  for (int b = threadIdx.x; b < B; b += 256) {
-    const float *y = Y + (int64_t)b * kOut;
-    float *g = dY + (int64_t)b * kOut;
-    float mx = fmaxf(fmaxf(y[0], y[1]), y[2]);
-    float e0 = expf(y[0] - mx), e1 = expf(y[1] - mx), e2 = expf(y[2] - mx);
-    const float se = e0 + e1 + e2;
-    const int c = cls[b];
-    const float p[3] = {e0 / se, e1 / se, e2 / se};
-    const bool has_c = c >= 0 && c < kNCls;  // other labels: no class term
-    if (has_c) acc += -(y[c] - mx - logf(se));
-    for (int k = 0; k < kNCls; ++k)
-      g[k] = has_c ? (p[k] - (k == c ? 1.f : 0.f)) / B : 0.f;
-    for (int k = 0; k < kNReg; ++k) {
-      const float t = tgt[(int64_t)b * kNReg + k];
-      if (isnan(t)) {
-        g[kNCls + k] = 0.f;
-        continue;
-      }
-      const float r = y[kNCls + k] - t;
-      acc += reg_w * r * r;
-      g[kNCls + k] = 2.f * reg_w * r / B;
-    }
+// where m masks regression targets that are NaN; a class outside 0..2 drops
+// the cross-entropy term of that sample.  The weights (150 KB) come from L2.
+// A layer's product runs k = kb + 4 lg + j for MFMA j of a group of 16, so
+// that a lane reads four consecutive weights.  One launch in place of 8
+// (forward) or 16 (with the backward pass): those were bound by their
+// launches and, at 256 samples, by 16 to 64 workgroups each (about 110 us
+// with the backward pass, now 25).
+// hbuf: H_1 .. H_3 [B x 128] each; dbuf: dZ_1 .. dZ_3 [B x 128], dZ_4 [B x 6];
+// lossp: one partial sum per workgroup.
+template <bool TRAIN>
+__global__ __launch_bounds__(256) void k_mlp(
+    const float *__restrict__ P, const float *__restrict__ X, int B,
+    float *__restrict__ out, const int32_t *__restrict__ cls,
+    const float *__restrict__ tgt, float reg_w, float *__restrict__ hbuf,
+    float *__restrict__ dbuf, float *__restrict__ lossp) {
+  constexpr int LD = kH + 4;
+  __shared__ __align__(16) float Hs[2][16][LD];  // layer in / out, dZ in / out
+  __shared__ float Zs[3][16][LD];                // Z_1 .. Z_3
+  __shared__ float lsum[16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int li = lane & 15, lg = lane >> 4;
+  const int r0 = blockIdx.x * 16;
+  for (int e = tid; e < 16 * 48; e += 256) {
+    const int i = e / 48, k = e % 48;
+    Hs[0][i][k] = r0 + i < B && k < kIn ? X[(int64_t)(r0 + i) * kIn + k] : 0.f;
   }
-  red[threadIdx.x] = acc;
+  __syncthreads();
+#pragma unroll
+  for (int l = 1; l <= 4; ++l) {
+    const int I = mlp_dim(l - 1), O = mlp_dim(l);
+    const float *W = P + w_off(l), *bias = P + b_off(l);
+    const float (*in)[LD] = Hs[(l - 1) & 1];
+    float (*ou)[LD] = Hs[l & 1];
+    for (int t = wave; t < (O + 15) / 16; t += 4) {
+      const int col = t * 16 + li;
+      mf4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+      for (int kb = 0; kb < I; kb += 16) {
+        const int k = kb + 4 * lg;
+        F4 w = {{0.f, 0.f, 0.f, 0.f}};
+        if (col < O && k < I)
+          w = *reinterpret_cast<const F4 *>(W + (int64_t)col * I + k);
+        const float4 h = *reinterpret_cast<const float4 *>(&in[li][k]);
+        acc = mfma32(h.x, w.v[0], acc);
+        acc = mfma32(h.y, w.v[1], acc);
+        acc = mfma32(h.z, w.v[2], acc);
+        acc = mfma32(h.w, w.v[3], acc);
+      }
+      if (col < O) {
+        const float bc = bias[col];
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          const int row = 4 * lg + r;
+          const float z = acc[r] + bc;
+          if (l < 4) {
+            const float h = gelu(z);
+            ou[row][col] = h;
+            if (TRAIN) {
+              Zs[l - 1][row][col] = z;
+              if (r0 + row < B)
+                hbuf[((int64_t)(l - 1) * B + r0 + row) * kH + col] = h;
+            }
+          } else {
+            ou[row][col] = z;
+            if (!TRAIN && r0 + row < B)
+              out[(int64_t)(r0 + row) * kOut + col] = z;
+          }
+        }
+      }
+    }
+    __syncthreads();
+  }
+  if (!TRAIN) return;
+  // the outputs are in Hs[0]; dZ_4 goes to Hs[1], zero beyond its 6 columns
+  // (to the group of 16) and beyond the batch
+  {
+    const int i = tid >> 4, k = tid & 15;
+    Hs[1][i][k] = 0.f;
+  }
+  __syncthreads();
+  if (tid < 16) {
+    float acc = 0.f;
+    const int b = r0 + tid;
+    if (b < B) {
+      const float *y = Hs[0][tid];
+      float *g = Hs[1][tid];
+      const float mx = fmaxf(fmaxf(y[0], y[1]), y[2]);
+      const float e0 = expf(y[0] - mx), e1 = expf(y[1] - mx),
+                  e2 = expf(y[2] - mx);
+      const float se = e0 + e1 + e2;
+      const int c = cls[b];
+      const float p[3] = {e0 / se, e1 / se, e2 / se};
+      const bool has_c = c >= 0 && c < kNCls;  // other labels: no class term
+      if (has_c) acc += -(y[c] - mx - logf(se));
+      for (int k = 0; k < kNCls; ++k)
+        g[k] = has_c ? (p[k] - (k == c ? 1.f : 0.f)) / B : 0.f;
+      for (int k = 0; k < kNReg; ++k) {
+        const float t = tgt[(int64_t)b * kNReg + k];
+        if (isnan(t)) {
+          g[kNCls + k] = 0.f;
+          continue;
+        }
+        const float r = y[kNCls + k] - t;
+        acc += reg_w * r * r;
+        g[kNCls + k] = 2.f * reg_w * r / B;
+      }
+      for (int k = 0; k < kOut; ++k)
+        dbuf[(int64_t)3 * B * kH + (int64_t)b * kOut + k] = g[k];
+    }
+    lsum[tid] = acc;
+  }
+  __syncthreads();
+  if (tid == 0) {
+    float acc = 0.f;
+    for (int i = 0; i < 16; ++i) acc += lsum[i];
+    lossp[blockIdx.x] = acc;
+  }
+  // dZ_{l-1} = (dZ_l W_l) * gelu'(Z_{l-1})
+#pragma unroll
+  for (int l = 4; l >= 2; --l) {
+    const int O = mlp_dim(l);
+    const float *W = P + w_off(l);
+    const float (*in)[LD] = Hs[(l - 1) & 1];
+    float (*ou)[LD] = Hs[l & 1];
+    for (int t = wave; t < kH / 16; t += 4) {
+      const int col = t * 16 + li;
+      mf4_t acc = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll 4
+      for (int kb = 0; kb < O; kb += 16) {
+        const int k = kb + 4 * lg;
+        float w[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j)
+          w[j] = k + j < O ? W[(int64_t)(k + j) * kH + col] : 0.f;
+        const float4 d = *reinterpret_cast<const float4 *>(&in[li][k]);
+        acc = mfma32(d.x, w[0], acc);
+        acc = mfma32(d.y, w[1], acc);
+        acc = mfma32(d.z, w[2], acc);
+        acc = mfma32(d.w, w[3], acc);
+      }
+#pragma unroll
+      for (int r = 0; r < 4; ++r) {
+        const int row = 4 * lg + r;
+        const float d = acc[r] * gelu_d(Zs[l - 2][row][col]);
+        ou[row][col] = d;
+        if (r0 + row < B)
+          dbuf[((int64_t)(l - 2) * B + r0 + row) * kH + col] = d;
+      }
+    }
+    __syncthreads();
+  }
+}
+
+// Weight and bias gradients dW_l = dZ_l^T H_{l-1}, db_l = sum dZ_l of all
+// layers: one 16 x 16 tile per workgroup (kGradTiles over the layers), its
+// batch rows [blockIdx.y * rows, ...) dealt to the four waves, whose sums are
+// added in wave order.  part: the gradients themselves (one row chunk) or one
+// copy per chunk for k_grad_sum.  The first workgroup also sums the loss.
+// (Four products, each with 8 to 64 workgroups that walked all rows, and four
+// bias sums with one thread per output took 250 us at 256 samples, this 7.5.)
+constexpr int kGradTiles = 8 * 3 + 8 * 8 + 8 * 8 + 8;
+__global__ __launch_bounds__(256) void k_mlp_grad(
+    const float *__restrict__ X, int B, const float *__restrict__ hbuf,
+    const float *__restrict__ dbuf, int rows, float *__restrict__ part,
+    const float *__restrict__ lossp, int nloss, float *__restrict__ loss) {
+  __shared__ float red[4][17][16];
+  const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
+  const int li = lane & 15, lg = lane >> 4;
+  int t = blockIdx.x, l = 1;
+  if (t < 24) {
+    l = 1;
+  } else if ((t -= 24) < 64) {
+    l = 2;
+  } else if ((t -= 64) < 64) {
+    l = 3;
+  } else {
+    t -= 64;
+    l = 4;
+  }
+  const int I = mlp_dim(l - 1), O = mlp_dim(l);
+  const int nti = (I + 15) / 16;
+  const int o = (t / nti) * 16 + li, i = (t % nti) * 16 + li;
+  const float *dZ = dbuf + (int64_t)(l - 1) * B * kH;
+  const float *H = l == 1 ? X : hbuf + (int64_t)(l - 2) * B * kH;
+  const int b0 = blockIdx.y * rows, b1 = min(B, b0 + rows);
+  mf4_t acc = {0.f, 0.f, 0.f, 0.f};
+  float db = 0.f;
+#pragma unroll 4
+  for (int b = b0 + 4 * wave + lg; b - lg < b1; b += 16) {
+    const bool in = b < b1;
+    const float d = in && o < O ? dZ[(int64_t)b * O + o] : 0.f;
+    const float h = in && i < I ? H[(int64_t)b * I + i] : 0.f;
+    db += d;
+    acc = mfma32(d, h, acc);
+  }
+#pragma unroll
+  for (int r = 0; r < 4; ++r) red[wave][4 * lg + r][li] = acc[r];
+  db += __shfl_xor(db, 16, 64);
+  db += __shfl_xor(db, 32, 64);
+  if (lg == 0) red[wave][16][li] = db;
+  __syncthreads();
+  float *g = part + (int64_t)blockIdx.y * kNParams;
+  {
+    const int r = tid >> 4, c = tid & 15;
+    const int oo = (t / nti) * 16 + r, ii = (t % nti) * 16 + c;
+    if (oo < O && ii < I)
+      g[w_off(l) + (int64_t)oo * I + ii] =
+          red[0][r][c] + red[1][r][c] + red[2][r][c] + red[3][r][c];
+  }
+  if (t % nti == 0 && tid < 16 && o < O)
+    g[b_off(l) + o] =
+        red[0][16][li] + red[1][16][li] + red[2][16][li] + red[3][16][li];
+  if (blockIdx.x || blockIdx.y) return;
+  __shared__ float ls[256];
+  float v = 0.f;
+  for (int e = tid; e < nloss; e += 256) v += lossp[e];
+  ls[tid] = v;
   __syncthreads();
   for (int w = 128; w > 0; w >>= 1) {
-    if ((int)threadIdx.x < w) red[threadIdx.x] += red[threadIdx.x + w];
+    if (tid < w) ls[tid] += ls[tid + w];
     __syncthreads();
   }
-  if (threadIdx.x == 0) loss[0] = red[0] / B;
+  if (tid == 0) loss[0] = ls[0] / B;
+}
+
+__global__ __launch_bounds__(256) void k_grad_sum(
+    const float *__restrict__ part, int n, float *__restrict__ grads) {
+  const int64_t e = blockIdx.x * (int64_t)256 + threadIdx.x;
+  if (e >= kNParams) return;
+  float v = 0.f;
+  for (int k = 0; k < n; ++k) v += part[k * kNParams + e];
+  grads[e] = v;
 }
 
 __global__ void k_adam(float *__restrict__ p, const float *__restrict__ g,
@@ -350,53 +479,6 @@ __global__ void k_init_params(float *__restrict__ p, unsigned long long seed) {
     const float lim = 1.0f / sqrtf((float)mlp_dim(l - 1));
     p[e] = (float)((2.0 * u - 1.0) * lim) * (is_w ? 1.0f : 0.5f);
   }
-}
-
-static int sgemm(hipStream_t st, int ta, int tb, int R, int Cc, int K,
-                 const float *A, int lda, const float *B, int ldb, float *Cm,
-                 int ldc, int beta) {
-  const dim3 g((unsigned)ceil_div(Cc, 32), (unsigned)ceil_div(R, 32));
-  if (!ta && tb)
-    hipLaunchKernelGGL((k_sgemm<0, 1>), g, dim3(256), 0, st, R, Cc, K, A, lda,
-                       B, ldb, Cm, ldc, beta);
-  else if (ta && !tb)
-    hipLaunchKernelGGL((k_sgemm<1, 0>), g, dim3(256), 0, st, R, Cc, K, A, lda,
-                       B, ldb, Cm, ldc, beta);
-  else if (!ta && !tb)
-    hipLaunchKernelGGL((k_sgemm<0, 0>), g, dim3(256), 0, st, R, Cc, K, A, lda,
-                       B, ldb, Cm, ldc, beta);
-  else
-    hipLaunchKernelGGL((k_sgemm<1, 1>), g, dim3(256), 0, st, R, Cc, K, A, lda,
-                       B, ldb, Cm, ldc, beta);
-  return check_launch("k_sgemm");
-}
-
-// Activations workspace per layer: Z_l and H_l [B x dim(l)], l = 1..4.
-static int64_t act_floats(int B) {
-  int64_t t = 0;
-  for (int l = 1; l <= 4; ++l) t += 2 * (int64_t)B * mlp_dim(l);
-  return t;
-}
-
-static int mlp_forward(spk_ctx *ctx, const float *P, const float *X, int B,
-                       float *acts) {
-  hipStream_t st = ctx->stream;
-  const float *Hprev = X;
-  float *a = acts;
-  for (int l = 1; l <= 4; ++l) {
-    const int I = mlp_dim(l - 1), O = mlp_dim(l);
-    float *Z = a, *H = a + (int64_t)B * O;
-    // Z = H_prev W^T
-    SPK_TRY(sgemm(st, 0, 1, B, O, I, Hprev, I, P + w_off(l), I, Z, O, 0));
-    const int64_t n = (int64_t)B * O;
-    hipLaunchKernelGGL(k_bias_act, dim3((unsigned)std::min<int64_t>(ceil_div(n, 256), 4096)),
-                       dim3(256), 0, st, Z, H, P + b_off(l), B, O,
-                       l < 4 ? 1 : 0);
-    SPK_TRY(check_launch("k_bias_act"));
-    Hprev = H;
-    a += 2 * n;
-  }
-  return SPK_OK;
 }
 
 }  // namespace spk
@@ -502,16 +584,11 @@ int spk_mlp_forward_dev(spk_ctx *ctx, const float *params, const float *X,
   if (B <= 0) return SPK_OK;
   if (B > kMaxBatch) return set_error(SPK_ESHAPE, "batch above %d", kMaxBatch);
   SPK_HIP(hipSetDevice(ctx->device));
-  float *acts;
-  SPK_TRY(ws_get(ctx, "mlp_acts", act_floats(B) * 4, (void **)&acts));
-  SPK_TRY(mlp_forward(ctx, params, X, B, acts));
-  // the last H is the output
-  int64_t off = 0;
-  for (int l = 1; l < 4; ++l) off += 2 * (int64_t)B * mlp_dim(l);
-  const float *H4 = acts + off + (int64_t)B * kOut;
-  SPK_HIP(hipMemcpyAsync(out, H4, (size_t)B * kOut * 4,
-                         hipMemcpyDeviceToDevice, ctx->stream));
-  return SPK_OK;
+  hipLaunchKernelGGL((k_mlp<false>), dim3((unsigned)ceil_div(B, 16)),
+                     dim3(256), 0, ctx->stream, params, X, B, out,
+                     (const int32_t *)nullptr, (const float *)nullptr, 0.f,
+                     (float *)nullptr, (float *)nullptr, (float *)nullptr);
+  return check_launch("k_mlp");
 }
 
 int spk_mlp_loss_grad_dev(spk_ctx *ctx, const float *params, const float *X,
@@ -523,48 +600,27 @@ int spk_mlp_loss_grad_dev(spk_ctx *ctx, const float *params, const float *X,
   if (B > kMaxBatch) return set_error(SPK_ESHAPE, "batch above %d", kMaxBatch);
   SPK_HIP(hipSetDevice(ctx->device));
   hipStream_t st = ctx->stream;
-  float *acts, *dbuf;
-  SPK_TRY(ws_get(ctx, "mlp_acts", act_floats(B) * 4, (void **)&acts));
-  SPK_TRY(ws_get(ctx, "mlp_d", 2 * (int64_t)B * kH * 4, (void **)&dbuf));
-  SPK_TRY(mlp_forward(ctx, params, X, B, acts));
-  // layer activation pointers
-  float *Z[5], *H[5];
-  {
-    float *a = acts;
-    for (int l = 1; l <= 4; ++l) {
-      Z[l] = a;
-      H[l] = a + (int64_t)B * mlp_dim(l);
-      a += 2 * (int64_t)B * mlp_dim(l);
-    }
-  }
-  float *dA = dbuf, *dB = dbuf + (int64_t)B * kH;
-  // dY = dL/dH4
-  hipLaunchKernelGGL(k_loss, dim3(1), dim3(256), 0, st, H[4], cls, reg, B,
-                     reg_w, dA, loss);
-  SPK_TRY(check_launch("k_loss"));
-  for (int l = 4; l >= 1; --l) {
-    const int I = mlp_dim(l - 1), O = mlp_dim(l);
-    const float *Hprev = l > 1 ? H[l - 1] : X;
-    // dA holds dZ_l (the output layer has no activation)
-    if (l < 4) {
-      hipLaunchKernelGGL(k_act_bwd, dim3((unsigned)std::min<int64_t>(ceil_div((int64_t)B * O, 256), 4096)),
-                         dim3(256), 0, st, Z[l], dA, (int64_t)B * O);
-      SPK_TRY(check_launch("k_act_bwd"));
-    }
-    // dW_l = dZ^T H_prev  [O x I]
-    SPK_TRY(sgemm(st, 1, 0, O, I, B, dA, O, Hprev, I, grads + w_off(l), I, 0));
-    hipLaunchKernelGGL(k_bias_grad, dim3((unsigned)ceil_div(O, 256)),
-                       dim3(256), 0, st, dA, B, O, grads + b_off(l));
-    SPK_TRY(check_launch("k_bias_grad"));
-    if (l > 1) {
-      // dH_prev = dZ W  [B x I]
-      SPK_TRY(sgemm(st, 0, 0, B, I, O, dA, O, params + w_off(l), I, dB, I, 0));
-      float *t = dA;
-      dA = dB;
-      dB = t;
-    }
-  }
-  return SPK_OK;
+  const int nblk = (int)ceil_div(B, 16);
+  // row chunks of at least 256 samples, at most 32 of them
+  const int nch = (int)std::min<int64_t>(32, ceil_div(B, 256));
+  const int rows = (int)ceil_div(ceil_div(B, nch), 16) * 16;
+  float *hbuf, *dbuf, *lossp, *part = grads;
+  SPK_TRY(ws_get(ctx, "mlp_h", 3 * (int64_t)B * kH * 4, (void **)&hbuf));
+  SPK_TRY(ws_get(ctx, "mlp_d", (int64_t)B * (3 * kH + kOut) * 4,
+                 (void **)&dbuf));
+  SPK_TRY(ws_get(ctx, "mlp_loss", (int64_t)nblk * 4, (void **)&lossp));
+  if (nch > 1)
+    SPK_TRY(ws_get(ctx, "mlp_part", nch * kNParams * 4, (void **)&part));
+  hipLaunchKernelGGL((k_mlp<true>), dim3((unsigned)nblk), dim3(256), 0, st,
+                     params, X, B, (float *)nullptr, cls, reg, reg_w, hbuf,
+                     dbuf, lossp);
+  hipLaunchKernelGGL(k_mlp_grad, dim3(kGradTiles, (unsigned)nch), dim3(256), 0,
+                     st, X, B, (const float *)hbuf, (const float *)dbuf, rows,
+                     part, (const float *)lossp, nblk, loss);
+  if (nch > 1)
+    hipLaunchKernelGGL(k_grad_sum, dim3((unsigned)ceil_div(kNParams, 256)),
+                       dim3(256), 0, st, (const float *)part, nch, grads);
+  return check_launch("k_mlp_grad");
 }
 
 int spk_mlp_adam_dev(spk_ctx *ctx, float *params, const float *grads,

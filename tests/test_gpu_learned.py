@@ -202,3 +202,26 @@ def test_training_reduces_loss(gpu):
     pred = net.forward(X).cpu().numpy()
     acc = np.mean(np.argmax(pred[:, :3], axis=1) == cls)
     assert acc > 0.9
+
+
+@pytest.mark.parametrize('B', [1, 15, 16, 17, 255, 257, 513, 8200])
+def test_loss_grad_tiles_and_chunks(gpu, B):
+    """16 samples per workgroup in the forward and backward pass, row chunks
+    of 256 and more (at most 32) in the weight gradients: below, at and above
+    their edges, with classes that drop out and NaN targets, against the
+    FP64 oracle (tolerance: FP32 sums over B samples and up to 128 inputs)."""
+    from spinterps_amd.variograms.learned import VariogramProposalNet
+    rng = np.random.default_rng(B)
+    net = VariogramProposalNet(seed=3)
+    X = rng.standard_normal((B, 40)).astype(np.float32)
+    cls = rng.integers(-1, 3, B).astype(np.int32)
+    reg = rng.standard_normal((B, 3)).astype(np.float32)
+    reg[rng.random((B, 3)) < 0.2] = np.nan
+    p = net.state()
+    np.testing.assert_allclose(net.forward(X).cpu().numpy(),
+                               M.mlp_forward(p, X)[0], rtol=0, atol=2e-5)
+    for _ in range(2):
+        loss, g = net.loss_grad(X, cls, reg, reg_w=0.8)
+        lr, gr = M.mlp_loss_grad(p, X, cls, reg, 0.8)
+        assert abs(float(loss) - lr) <= 1e-5 * max(1.0, abs(lr))
+        assert np.abs(g.cpu().numpy() - gr).max() <= 1e-5 * np.abs(gr).max()
