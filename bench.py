@@ -719,8 +719,8 @@ def stress_leg(args, log):
 def idw_leg(args, log):
     """IDW cell-estimates/s on the daily workload (1 000 stations, 0-20 %
     missing per step, 500 x 500 cells at 1 km, p = 2), inputs resident in
-    HBM; one k_idw_nnb launch per batch of steps (for p = 2 one pass over
-    the active stations per cell, weights 1 / d^2: the reference's
+    HBM (spk_idw.hip: numerator and denominator as two products over
+    the stations on FP64 MFMA, weights 1 / d^2: the reference's
     normalisation by the max distance cancels in the ratio).  The
     oracle's IDW (interp/steps.py:293-313 vectorised with NumPy, one BLAS
     thread) on a cell sample is the CPU baseline and the reference values

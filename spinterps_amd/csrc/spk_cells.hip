@@ -12,8 +12,7 @@
 //  k_var_reduce  variance from the FP64 terms and the partial norms
 //  (the int8 plane-product contraction is in spk_int8.hip, the plain FP64
 //  path's kernels are in spk_plain.hip)
-//  k_idw_nnb     interp/steps.py:285-313 (nearest neighbour; IDW runs as
-//                a masked FP64 MFMA contraction, k_idw_mfma in spk_idw.hip)
+//  k_nnb         nearest neighbour (interp/steps.py:285-313; IDW: spk_idw.hip)
 //  k_special     one-station, mean-fill and failed-system steps
 //                (interp/steps.py:280-283, 325-331, 372-384)
 #include <algorithm>
@@ -58,11 +57,35 @@ constexpr double kPinvKappa = 1e14;
 // memory instead of 6), 0 = the planes themselves.
 constexpr int kBfA32 = 1;
 
-__global__ void k_recenter(const double *__restrict__ in,
-                           double *__restrict__ out, int64_t n, double o) {
-  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < n;
-       i += (int64_t)gridDim.x * blockDim.x)
-    out[i] = in[i] - o;
+// Coordinates less the problem's origin, stations and cells in one launch
+// (four launches were a tenth of a one-step IDW call).
+__global__ void k_recenter(const double *__restrict__ sx,
+                           const double *__restrict__ sy, int64_t N,
+                           const double *__restrict__ cx,
+                           const double *__restrict__ cy, int64_t C, double ox,
+                           double oy, double *__restrict__ osx,
+                           double *__restrict__ osy, double *__restrict__ ocx,
+                           double *__restrict__ ocy) {
+  for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < N + C;
+       i += (int64_t)gridDim.x * blockDim.x) {
+    if (i < N) {
+      osx[i] = sx[i] - ox;
+      osy[i] = sy[i] - oy;
+    } else {
+      ocx[i - N] = cx[i - N] - ox;
+      ocy[i - N] = cy[i - N] - oy;
+    }
+  }
+}
+
+int recenter(hipStream_t st, const spk_problem *prob, double *sx, double *sy,
+             double *cx, double *cy) {
+  const int64_t N = prob->n_stns, C = cx ? prob->n_cells : 0;
+  const int64_t g = std::min<int64_t>(ceil_div(N + C, 256), 65536);
+  hipLaunchKernelGGL(k_recenter, dim3((unsigned)g), dim3(256), 0, st,
+                     prob->stn_x, prob->stn_y, N, prob->cell_x, prob->cell_y,
+                     C, prob->origin_x, prob->origin_y, sx, sy, cx, cy);
+  return check_launch("k_recenter");
 }
 
 // ---- MFMA contraction --------------------------------------------------------
@@ -1195,14 +1218,13 @@ __global__ __launch_bounds__(256, 3) void k_kgen(
   if (dmax) dmax[(int64_t)sl * ldk + c] = dm;
 }
 
-// ---- IDW and nearest neighbour -------------------------------------------------
-__global__ __launch_bounds__(256) void k_idw_nnb(
+// ---- nearest neighbour -----------------------------------------------------------
+__global__ __launch_bounds__(256) void k_nnb(
     const double *__restrict__ sx, const double *__restrict__ sy,
     const int32_t *__restrict__ idx, int64_t N,
     const double *__restrict__ zact, int64_t ldz,
     const StepSc *__restrict__ sc, const double *__restrict__ cx,
-    const double *__restrict__ cy, int64_t C, int method, double p,
-    double *__restrict__ est, int *__restrict__ bad) {
+    const double *__restrict__ cy, int64_t C, double *__restrict__ est) {
 #pragma clang fp contract(off)
   const int sl = blockIdx.y;
   const StepSc st = sc[sl];
@@ -1210,96 +1232,32 @@ __global__ __launch_bounds__(256) void k_idw_nnb(
   const int n = st.n;
   const int32_t *my = idx + (int64_t)sl * N;
   const double *z = zact + (int64_t)sl * ldz;
-  __shared__ double stx[256], sty[256], sz[256];
+  __shared__ double stx[256], sty[256];
   const int tid = threadIdx.x;
   const int64_t c = blockIdx.x * (int64_t)256 + tid;
   const bool valid = c < C;
   const double x = valid ? cx[c] : 0.0, y = valid ? cy[c] : 0.0;
-  double *eo = est + (int64_t)sl * C;
-  if (method != SPK_M_NNB && p == 2.0) {
-    // p = 2: the reference's weights 1 / (d / dmax)^2 are dmax^2 / s with
-    // s = dx^2 + dy^2, and the per-cell factor dmax^2 cancels in
-    // sum(w z) / sum(w); one pass with w = 1 / s (no square root, one
-    // division).  The weight-sum check is made on the normalised sum
-    // max(s) sum(1 / s).
-    double ws = 0.0, wz = 0.0, smax = 0.0;
-    for (int base = 0; base < n; base += 256) {
-      __syncthreads();
-      if (base + tid < n) {
-        const int g = my[base + tid];
-        stx[tid] = sx[g];
-        sty[tid] = sy[g];
-        sz[tid] = z[base + tid];
-      }
-      __syncthreads();
-      const int cnt = min(256, n - base);
-      if (valid)
-        for (int j = 0; j < cnt; ++j) {
-          const double dx = x - stx[j], dy = y - sty[j];
-          const double s2 = (dx * dx) + (dy * dy);
-          smax = fmax(smax, s2);
-          const double wj = 1.0 / s2;
-          ws = ws + wj;
-          wz = wz + wj * sz[j];
-        }
-    }
-    if (!valid) return;
-    const double wn = smax > 0.0 ? ws * smax : ws;
-    if (!(wn >= 1e-14)) atomicOr(bad, 1);  // interp/steps.py:305
-    eo[c] = wz / ws;
-    return;
-  }
-  double dmax = 0.0, best = INFINITY;
+  double best = INFINITY;
   int bi = 0;
-  // pass 1: max distance (IDW) / nearest station (NNB)
   for (int base = 0; base < n; base += 256) {
     __syncthreads();
     if (base + tid < n) {
       const int g = my[base + tid];
       stx[tid] = sx[g];
       sty[tid] = sy[g];
-      sz[tid] = z[base + tid];
     }
     __syncthreads();
     const int cnt = min(256, n - base);
     if (valid)
       for (int j = 0; j < cnt; ++j) {
         const double d = dist2(x, y, stx[j], sty[j]);
-        dmax = fmax(dmax, d);
         if (d < best) {
           best = d;
           bi = base + j;
         }
       }
   }
-  if (method == SPK_M_NNB) {
-    if (valid) eo[c] = z[bi];
-    return;
-  }
-  // pass 2: w = 1 / (d / dmax)^p, sums in station order (pyx:784-808)
-  double ws = 0.0, wz = 0.0;
-  for (int base = 0; base < n; base += 256) {
-    __syncthreads();
-    if (base + tid < n) {
-      const int g = my[base + tid];
-      stx[tid] = sx[g];
-      sty[tid] = sy[g];
-      sz[tid] = z[base + tid];
-    }
-    __syncthreads();
-    const int cnt = min(256, n - base);
-    if (valid)
-      for (int j = 0; j < cnt; ++j) {
-        double d = dist2(x, y, stx[j], sty[j]);
-        if (dmax > 0) d = d / dmax;
-        const double wj = 1.0 / (p == 2.0 ? d * d : pow(d, p));
-        ws = ws + wj;
-        wz = wz + wj * sz[j];
-      }
-  }
-  if (!valid) return;
-  if (!(ws >= 1e-14)) atomicOr(bad, 1);  // interp/steps.py:305
-  eo[c] = wz / ws;
+  if (valid) est[(int64_t)sl * C + c] = z[bi];
 }
 
 // ---- special steps ---------------------------------------------------------------
@@ -1465,23 +1423,18 @@ static int idw_nnb_steps(spk_ctx *ctx, const spk_opts *opts, int64_t T,
                        (const int32_t *)nullptr);
     {
       ProfScope ps(ctx, "idw_nnb");
-      if (method == SPK_M_IDW)
-        // num = (Z . M) W^T and den = M W^T on FP64 MFMA, W = d^-p
-        hipLaunchKernelGGL(k_idw_mfma,
-                           dim3((unsigned)ceil_div(C, 128),
-                                (unsigned)ceil_div(Sb, 32)),
-                           dim3(256), 0, sm, sx, sy, N, vals + t0 * N, Sb,
-                           (const StepSc *)sc, (const int32_t *)idx,
-                           (const double *)zact, ldz, cx, cy, C,
-                           opts->idw_exp, eb, bad);
-      else
-        hipLaunchKernelGGL(k_idw_nnb, dim3((unsigned)ceil_div(C, 256), Sb),
+      if (method == SPK_M_IDW) {
+        SPK_TRY(idw_steps(sm, sx, sy, N, vals + t0 * N, Sb, sc, idx, zact,
+                          ldz, cx, cy, C, opts->idw_exp, eb, bad));
+      } else {
+        hipLaunchKernelGGL(k_nnb, dim3((unsigned)ceil_div(C, 256), Sb),
                            dim3(256), 0, sm, sx, sy, idx, N, zact, ldz, sc,
-                           cx, cy, C, method, opts->idw_exp, eb, bad);
+                           cx, cy, C, eb);
+        hipLaunchKernelGGL(k_special, dim3((unsigned)ceil_div(C, 256), Sb),
+                           dim3(256), 0, sm, sx, sy, idx, N, zact, ldz, sc,
+                           cx, cy, C, eb, (double *)nullptr);
+      }
     }
-    hipLaunchKernelGGL(k_special, dim3((unsigned)ceil_div(C, 256), Sb),
-                       dim3(256), 0, sm, sx, sy, idx, N, zact, ldz, sc, cx,
-                       cy, C, eb, (double *)nullptr);
     hipLaunchKernelGGL(k_status_out, dim3((unsigned)ceil_div(Sb, 256)),
                        dim3(256), 0, sm, sc, Sb, info + t0,
                        kappa ? kappa + t0 : nullptr);
@@ -1646,19 +1599,7 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
   sy = sx + N;
   SPK_TRY(ws_get(ctx, "cell_xy", 2 * C * sizeof(double), (void **)&cx));
   cy = cx + C;
-  {
-    const unsigned gs = (unsigned)std::min<int64_t>(ceil_div(N, 256), 4096);
-    const unsigned gc = (unsigned)std::min<int64_t>(ceil_div(C, 256), 65536);
-    hipLaunchKernelGGL(k_recenter, dim3(gs), dim3(256), 0, sm, prob->stn_x, sx,
-                       N, prob->origin_x);
-    hipLaunchKernelGGL(k_recenter, dim3(gs), dim3(256), 0, sm, prob->stn_y, sy,
-                       N, prob->origin_y);
-    hipLaunchKernelGGL(k_recenter, dim3(gc), dim3(256), 0, sm, prob->cell_x, cx,
-                       C, prob->origin_x);
-    hipLaunchKernelGGL(k_recenter, dim3(gc), dim3(256), 0, sm, prob->cell_y, cy,
-                       C, prob->origin_y);
-    SPK_TRY(check_launch("k_recenter"));
-  }
+  SPK_TRY(recenter(sm, prob, sx, sy, cx, cy));
   const int64_t ldz = round_up(N, 64);
   const int p = method == SPK_M_OK ? 1 : method == SPK_M_EDK ? 1 + m : 0;
   const int64_t ld = round_up(N + (p > 0 ? p : 1), 64);
@@ -2596,17 +2537,7 @@ int spk_idw_steps_noalloc_dev(spk_ctx *ctx, const spk_problem *prob,
   StepSc *sc = reinterpret_cast<StepSc *>(base + kNaOffSc);
   const int64_t ldz = round_up(N, 64);  // <= kNaMaxStns
   hipStream_t sm = ctx->stream;
-  const unsigned gs = (unsigned)std::min<int64_t>(ceil_div(N, 256), 4096);
-  const unsigned gc = (unsigned)std::min<int64_t>(ceil_div(C, 256), 65536);
-  hipLaunchKernelGGL(k_recenter, dim3(gs), dim3(256), 0, sm, prob->stn_x, sx,
-                     N, prob->origin_x);
-  hipLaunchKernelGGL(k_recenter, dim3(gs), dim3(256), 0, sm, prob->stn_y, sy,
-                     N, prob->origin_y);
-  hipLaunchKernelGGL(k_recenter, dim3(gc), dim3(256), 0, sm, prob->cell_x, cx,
-                     C, prob->origin_x);
-  hipLaunchKernelGGL(k_recenter, dim3(gc), dim3(256), 0, sm, prob->cell_y, cy,
-                     C, prob->origin_y);
-  SPK_TRY(check_launch("k_recenter"));
+  SPK_TRY(recenter(sm, prob, sx, sy, cx, cy));
   return idw_nnb_steps(ctx, opts, T, N, C, vals, sx, sy, cx, cy, idx, zact,
                        ldz, sc, std::min<int64_t>(T, kNaSteps), bad, est,
                        info, kappa);

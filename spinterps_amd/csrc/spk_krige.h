@@ -61,12 +61,12 @@ struct StepSc {
 };
 
 // ---- IDW as a masked contraction on FP64 MFMA (spk_idw.hip) ----------------
-// grid (ceil(C / 128), ceil(S / 32)), 256 threads.
-__global__ void k_idw_mfma(const double *sx, const double *sy, int64_t N,
-                           const double *vals, int S, const StepSc *sc,
-                           const int32_t *idx, const double *zact,
-                           int64_t ldz, const double *cx, const double *cy,
-                           int64_t C, double p, double *est, int *bad);
+// The fields est [S x C] of the S steps vals [S x N], special steps included;
+// idx, zact and sc are theirs (k_compact).
+int idw_steps(hipStream_t st, const double *sx, const double *sy, int64_t N,
+              const double *vals, int S, const StepSc *sc, const int32_t *idx,
+              const double *zact, int64_t ldz, const double *cx,
+              const double *cy, int64_t C, double p, double *est, int *bad);
 
 // ---- batched estimates (spk_est.hip) -----------------------------------------
 // What the cell kernels read of one active station of a step, in one cache
@@ -236,7 +236,9 @@ int minv_steps(hipStream_t st, const double *Li, int64_t ld, int64_t stride,
                StepSc *sc, const int32_t *idx, int64_t N,
                const double *stn_drift, int m, int method, double *M,
                double *T0, const spk_vg *vgs, double min_vg_val, int S);
-__global__ void k_recenter(const double *in, double *out, int64_t n, double o);
+// The problem's stations and (cx not null) cells less its origin.
+int recenter(hipStream_t st, const spk_problem *prob, double *sx, double *sy,
+             double *cx, double *cy);
 __global__ void k_status_out(const StepSc *sc, int S, int32_t *info,
                              double *kappa);
 // Spatially compact order of the cells (Morton keys over the bounding box,

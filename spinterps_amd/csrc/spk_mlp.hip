@@ -507,13 +507,7 @@ int spk_simulate_fields_dev(spk_ctx *ctx, const spk_problem *prob, int64_t T,
   double *sx;
   SPK_TRY(ws_get(ctx, "stn_xy", 2 * N * sizeof(double), (void **)&sx));
   double *sy = sx + N;
-  {
-    const unsigned gs = (unsigned)std::min<int64_t>(ceil_div(N, 256), 4096);
-    hipLaunchKernelGGL(k_recenter, dim3(gs), dim3(256), 0, sm,
-                       prob->stn_x, sx, N, prob->origin_x);
-    hipLaunchKernelGGL(k_recenter, dim3(gs), dim3(256), 0, sm,
-                       prob->stn_y, sy, N, prob->origin_y);
-  }
+  SPK_TRY(recenter(sm, prob, sx, sy, nullptr, nullptr));
   const int64_t ld = ((N + 63) / 64) * 64;
   const int64_t strideM = ld * ld;
   const int64_t ldz = ld;

@@ -1311,15 +1311,7 @@ int spk_interp_neb_steps_dev(spk_ctx *ctx, const spk_problem *prob,
   auto g1 = [](int64_t n) {
     return dim3((unsigned)std::max<int64_t>(1, std::min<int64_t>(ceil_div(n, 256), 65536)));
   };
-  hipLaunchKernelGGL(k_recenter, g1(N), dim3(256), 0, sm, prob->stn_x, sx, N,
-                     prob->origin_x);
-  hipLaunchKernelGGL(k_recenter, g1(N), dim3(256), 0, sm, prob->stn_y, sy, N,
-                     prob->origin_y);
-  hipLaunchKernelGGL(k_recenter, g1(C), dim3(256), 0, sm, prob->cell_x, cx, C,
-                     prob->origin_x);
-  hipLaunchKernelGGL(k_recenter, g1(C), dim3(256), 0, sm, prob->cell_y, cy, C,
-                     prob->origin_y);
-  SPK_TRY(check_launch("k_recenter"));
+  SPK_TRY(recenter(sm, prob, sx, sy, cx, cy));
 
   // batch size: selections [S C K] int32 plus about 40 bytes per cell
   const int64_t per_step = C * (int64_t)K * 4 + C * 40 + N * 20;

@@ -159,6 +159,55 @@ def test_idw_nnb_steps(gpu, method, p):
         np.testing.assert_allclose(got, f64[method], rtol=1e-12)
 
 
+@pytest.mark.parametrize('p', [2.0, 0.5, 1.0, 1.5, 3.0, 2.3])
+@pytest.mark.parametrize('steps,side', [(1, 1), (17, 11), (16, 257),
+                                        (47, 257), (66, 257)])
+def test_idw_block_shapes(gpu, steps, side, p):
+    """Every block shape of the IDW kernel and exponent form, with a cell at
+    a station, a step of one station, one without and one below the
+    threshold: positive values, so sum(w z) and sum(w) of N terms differ
+    from NumPy's by N ulp each, the weights by a few p ulp."""
+    from spinterps_amd.interp.steps import DeviceProblem, interp_steps
+    rng = np.random.default_rng(steps * 10 + side)
+    N = 37
+    sx, sy = rng.uniform(0, 1e4, (2, N))
+    gx, gy = np.meshgrid(np.linspace(5.0, 9995.0, side),
+                         np.linspace(5.0, 9995.0, side))
+    cx, cy = gx.ravel(), gy.ravel()
+    k = len(cx) // 2
+    cx[k], cy[k] = sx[3], sy[3]
+    vals = rng.uniform(1.0, 10.0, (steps, N))
+    vals[rng.random(vals.shape) < 0.1] = np.nan
+    vals[:, :2] = 5.0
+    if steps > 3:
+        vals[1, :] = np.nan
+        vals[2, 1:] = np.nan
+        vals[3] *= 0.01
+    vals[0, 3] = 7.0
+    prob = DeviceProblem(sx, sy, cx, cy)
+    est, _, info = interp_steps(prob, vals, None, 'IDW', idw_exp=p,
+                                min_var_thr=0.5)
+    got = est.cpu().numpy()
+    at = np.unique(np.r_[np.arange(0, len(cx), max(1, len(cx) // 400)), k,
+                         len(cx) - 1])
+    d = np.hypot(cx[at, None] - sx, cy[at, None] - sy)
+    for t in range(steps):
+        m = ~np.isnan(vals[t])
+        z = vals[t][m]
+        if len(z) == 0:
+            assert np.isnan(got[t]).all()
+            continue
+        if len(z) == 1 or z.max() < 0.5:
+            ref = np.full(len(at), z.mean())
+        else:
+            dm = d[:, m] / d[:, m].max(axis=1, keepdims=True)
+            with np.errstate(divide='ignore', invalid='ignore'):
+                w = 1.0 / dm ** p
+                ref = (w * z).sum(1) / w.sum(1)
+        np.testing.assert_allclose(
+            got[t][at], ref, rtol=(2 * N + 8 * p + 40) * 2.0 ** -53)
+
+
 @pytest.mark.parametrize('precision', ['fp64', 'fp64b', 'mixed'])
 def test_ok_small_all_precisions(gpu, precision):
     from spinterps_amd.interp.steps import DeviceProblem, interp_steps
