@@ -16,9 +16,12 @@
 //                  share a set become adjacent
 //   k_neb_mark ... groups of identical sets (interp/grps.py:103-139), cut
 //                  into chunks of at most 64 cells
-//   k_neb_krige    one wavefront per chunk: the set's covariance system,
-//                  its Cholesky factor and triangular inverse in LDS, the
-//                  dual-form vectors, then every cell of the chunk
+//   k_neb_mfma     one wavefront per chunk: stations, values, border and
+//                  cells as the rows of one matrix, Cholesky sweep over the
+//                  stations' columns, results from dot products of rows
+//   k_neb_krige    the same chunks, where that matrix has too few rows, and
+//                  the methods without a system: factor in LDS, dual-form
+//                  vectors, then every cell of the chunk
 //   k_neb_pinv_*   chunks whose Cholesky fails (or whose condition estimate
 //                  exceeds 1e14) are solved as the reference solves every
 //                  group: pinv of the bordered system (rocSOLVER eigen-
@@ -680,10 +683,61 @@ __device__ inline NebChunk neb_chunk(const NebArgs &a, int ch, int nch) {
   NebChunk q;
   q.p0 = a.cstart[ch];
   q.p1 = ch + 1 < nch ? a.cstart[ch + 1] : a.total;
-  q.t = (int)(q.p0 / a.C);
+  q.t = (int)((unsigned)q.p0 / (unsigned)a.C);  // both below 2^31
   q.n = a.sc[q.t].n;
   q.k = neb_set_size(a.K, a.kfix, q.n);
   return q;
+}
+
+// Chunks that need no system (kriging): a single station, its value
+// everywhere and the variance untouched (NaN) (interp/steps.py:280-283); a
+// set whose values are all below the threshold or whose variogram is, the
+// group's mean and variance 0 (interp/steps.py:760-765, 325-331).
+__device__ inline bool neb_no_system(const NebArgs &a, const NebChunk &q,
+                                     int lane, int np, int cell, double zl) {
+  const double mean = wave_sum(lane < q.k ? zl : 0.0) / q.k;
+  const bool anyhi = __ballot(lane < q.k && zl >= a.thr) != 0;
+  const spk_vg &vg = a.vgs[q.t];
+  const bool one = q.k == 1;
+  if (!one && anyhi && !(vg.sill_sum <= a.mvg) && !(vg.range_max_raw <= a.mvg))
+    return false;
+  if (lane < np) {
+    a.est[(int64_t)q.t * a.C + cell] = one ? bcast(zl, 0) : mean;
+    if (a.var && a.want_var)
+      a.var[(int64_t)q.t * a.C + cell] = one ? NAN : 0.0;
+  }
+  if (lane == 0)
+    atomicOr(&a.sflags[q.t], one ? SPK_ST_ONESTN : SPK_ST_MEANFILL);
+  return true;
+}
+
+// beta = B^-1 g by Cholesky of the p x p matrix B; false where B is not
+// positive definite.
+template <int PA>
+__device__ inline bool neb_beta(int p, double (&B)[PA][PA],
+                                const double (&g)[PA], double (&beta)[PA]) {
+  for (int j = 0; j < p; ++j) {
+    double d = B[j][j];
+    for (int l = 0; l < j; ++l) d -= B[j][l] * B[j][l];
+    if (!(d > 0.0) || !isfinite(d)) return false;
+    B[j][j] = sqrt(d);
+    for (int i = j + 1; i < p; ++i) {
+      double s = B[i][j];
+      for (int l = 0; l < j; ++l) s -= B[i][l] * B[j][l];
+      B[i][j] = s / B[j][j];
+    }
+  }
+  for (int i = 0; i < p; ++i) {
+    double s = g[i];
+    for (int l = 0; l < i; ++l) s -= B[i][l] * beta[l];
+    beta[i] = s / B[i][i];
+  }
+  for (int i = p - 1; i >= 0; --i) {
+    double s = beta[i];
+    for (int l = i + 1; l < p; ++l) s -= B[l][i] * beta[l];
+    beta[i] = s / B[i][i];
+  }
+  return true;
 }
 
 // One 64-thread workgroup per chunk (grid-stride over the chunks).  Lane j
@@ -932,32 +986,7 @@ __global__ __launch_bounds__(64) void k_neb_krige(NebArgs a) {
         for (int j = 0; j <= i; ++j) B[i][j] = wave_sum(gl[i] * gl[j]);
       }
       bsc = B[0][0];
-      for (int j = 0; j < p && !bfail; ++j) {
-        double d = B[j][j];
-        for (int l = 0; l < j; ++l) d -= B[j][l] * B[j][l];
-        if (!(d > 0.0) || !isfinite(d)) {
-          bfail = true;
-          break;
-        }
-        B[j][j] = sqrt(d);
-        for (int i = j + 1; i < p; ++i) {
-          double s = B[i][j];
-          for (int l = 0; l < j; ++l) s -= B[i][l] * B[j][l];
-          B[i][j] = s / B[j][j];
-        }
-      }
-      if (!bfail) {
-        for (int i = 0; i < p; ++i) {
-          double s = g[i];
-          for (int l = 0; l < i; ++l) s -= B[i][l] * beta[l];
-          beta[i] = s / B[i][i];
-        }
-        for (int i = p - 1; i >= 0; --i) {
-          double s = beta[i];
-          for (int l = i + 1; l < p; ++l) s -= B[l][i] * beta[l];
-          beta[i] = s / B[i][i];
-        }
-      }
+      bfail = !neb_beta<PA>(p, B, g, beta);
     }
     if (bfail) {
       if (lane == 0) a.fail_list[atomicAdd(a.fail_cnt, 1)] = ch;
@@ -1069,6 +1098,402 @@ __global__ __launch_bounds__(64) void k_neb_krige(NebArgs a) {
     }
     }  // KRIG
   }
+}
+
+// ---- chunks on the matrix cores ----------------------------------------------
+// One wavefront per chunk, as k_neb_krige, for sets that leave room for cells
+// in a matrix of at most 64 rows: the k stations, one row of values, P1 border
+// rows (ones, drifts), then as many cells as fit.  With the
+// stations' covariance matrix in the first k columns, a Cholesky sweep over
+// these columns turns every other row r into L^-1 r, and every result is a
+// dot product of such rows: with u, G, y of the values, border and cell,
+//   beta = (G^T G)^-1 G^T u,  estimate = y . u + beta . (f - y . G),
+//   OK variance = c0 - y . y + (a - 1)(a - 2) / b, a = y . w, b = w . w
+// (w = G's column of ones), so no backward substitution is needed.  The
+// products with u and G are minus what the sweep leaves in columns k .. k + P1
+// (zero before), which belong to the rows of the values and the border.
+//
+// Layouts: between panels the matrix is in 16 x 16 blocks in registers, lane
+// (c, g) = (lane % 16, lane / 16) and register r holding row c, column
+// g + 4 r: what an FP64 MFMA of two blocks of L yields when the block of
+// the columns is its first operand, so that updates need no transposition.  A
+// panel of 16 columns goes through LDS to one row per lane, is eliminated
+// there (a column's values for the other lanes arrive by readlane), and goes
+// back through LDS as operands.  LDS rows are 18 doubles apart: free of bank
+// conflicts in both layouts.
+//
+// Bound: FP64 VALU issue (entries and panels; the products of the blocks are
+// a tenth).  12 steps x 250 000 cells, 1 000 stations, 50 per set: 6.4 ms; 24.6
+// with k_neb_krige, which factorises a packed triangle in LDS by columns with
+// two LDS reads per multiply-add, and substitutes for four cells at a time.
+// That kernel keeps what does not fit here: sets of more than 58 stations,
+// Pow and Hol models, and the methods without a system.
+constexpr int kNebRows = 64;
+// Row blocks of 16 for nbc column blocks (stations, values, border).
+__host__ __device__ constexpr int neb_row_blocks(int nbc) {
+  return nbc < 4 ? nbc + 1 : 4;
+}
+constexpr int kNebLd = 18;
+
+typedef double neb_d4 __attribute__((ext_vector_type(4)));
+
+__global__ void k_neb_vf(const spk_vg *__restrict__ vgs, int S,
+                         VgFast *__restrict__ vf) {
+  const int s = blockIdx.x * blockDim.x + threadIdx.x;
+  if (s < S) vg_fast_init(vgs[s], vf[s]);
+}
+
+// Rows besides stations and cells.
+__host__ __device__ inline int neb_extra(int p) { return 1 + (p > 0 ? p : 1); }
+
+template <int NBC, int PT>
+__global__ __launch_bounds__(64, 2) void k_neb_mfma(
+    NebArgs a, const VgFast *__restrict__ vfs) {
+  constexpr int PA = PT > 0 ? PT : 1;
+  constexpr int NBR = neb_row_blocks(NBC), NR = 16 * NBR;
+  __shared__ double T[kNebRows * kNebLd];
+  __shared__ double rx[kNebRows], ry[kNebRows];
+  __shared__ double sp[(1 + PA) * kNebRows];
+  const int lane = threadIdx.x, c = lane & 15, g = lane >> 4;
+  const int nch = *a.nch;
+  const int p = min(neb_p(a.method, a.m), PT);
+  const int P1 = p > 0 ? p : 1;
+  const bool sk = a.method == SPK_M_SK;
+  for (int ch = blockIdx.x; ch < nch; ch += gridDim.x) {
+    const NebChunk q = neb_chunk(a, ch, nch);
+    if (q.n <= 0) continue;
+    const int k = q.k, t = q.t;
+    const int np = (int)(q.p1 - q.p0);  // at most kNebChunk
+    __syncthreads();  // the previous chunk's readers are done
+    const int cme = lane < np ? a.cells[q.p0 + lane] : 0;
+    const int32_t *list =
+        a.nb + ((int64_t)t * a.C + bcast_i(cme, 0)) * a.K;
+    double zl = 0.0, zx = 0.0, zy = 0.0;
+    int s = 0;
+    if (lane < k) {
+      // positions are below n by construction; the clamp keeps a
+      // selection that met NaN coordinates inside the step's list
+      const int pos = min(max(list[lane], 0), q.n - 1);
+      s = a.idx[(int64_t)t * a.N + pos];
+      zx = a.sx[s];
+      zy = a.sy[s];
+      zl = a.zact[(int64_t)t * a.ldz + pos];
+    }
+    if (neb_no_system(a, q, lane, np, cme, zl)) continue;
+    const double mean = wave_sum(lane < k ? zl : 0.0) / k;
+    const double zsh = a.skm && sk ? mean : 0.0;
+    if (lane < k) {
+      rx[lane] = coord_fast(zx);
+      ry[lane] = coord_fast(zy);
+      sp[lane] = zl - zsh;
+      sp[kNebRows + lane] = 1.0;
+      for (int qd = 1; qd < p; ++qd)
+        sp[(1 + qd) * kNebRows + lane] =
+            a.stn_drift[(int64_t)s * a.m + (qd - 1)];
+    }
+    const VgFast &vf = vfs[t];
+    const double sill = a.vgs[t].sill_sum;
+    bool bounded = true;
+    for (int qd = 0; qd < vf.n; ++qd)
+      if (vf.type[qd] == SPK_VG_RNG) bounded = false;
+    const int r0 = k + 1 + P1, NC = NR - r0;
+    for (int i0 = 0; i0 < np; i0 += NC) {
+      const int nc = min(NC, np - i0);
+      // the cells' rows
+      const int ic = lane - r0;
+      const int ci = __shfl(cme, min(max(i0 + ic, 0), 63), 64);
+      const bool mine = ic >= 0 && ic < nc;
+      double x = 0.0, y = 0.0;
+      if (mine) {
+        x = a.cx[ci];
+        y = a.cy[ci];
+      }
+      if (lane >= k && lane < NR) {
+        rx[lane] = coord_fast(x);
+        ry[lane] = coord_fast(y);
+      }
+      __syncthreads();
+      // ---- entries, in the register layout
+      neb_d4 acc[NBR][NBC];
+      double bx[NBR], by[NBR];
+#pragma unroll
+      for (int I = 0; I < NBR; ++I) {
+        bx[I] = rx[16 * I + c];
+        by[I] = ry[16 * I + c];
+      }
+      double c0 = sk ? 0.0 : sill;
+      // f(dx, dy) for every entry of the blocks at and below the diagonal
+      auto fill = [&](auto f) {
+#pragma unroll
+        for (int J = 0; J < NBC; ++J)
+#pragma unroll
+          for (int r = 0; r < 4; ++r) {
+            // columns beyond the stations hold numbers that nothing reads
+            if (J + 1 == NBC && r > 0 && 16 * J + 4 * r >= k) continue;
+            const int col = 16 * J + 4 * r + g;
+            const double sx_ = rx[col], sy_ = ry[col];
+#pragma unroll
+            for (int I = J; I < NBR; ++I)
+              acc[I][J][r] = f(bx[I] - sx_, by[I] - sy_);
+          }
+      };
+      VgOne o;
+      int one = vg_one_of(vf, o);
+      // entries <= min_vg_val become zero (pyx:217): with min_vg_val <= 0
+      // and nonnegative sills that changes nothing
+      if (!(a.mvg <= 0.0 && o.s >= 0.0 && o.nug >= 0.0)) one = -1;
+      const double sl = o.s, off = sk ? 0.0 : c0 - o.nug - o.s;
+      double dmaxc = off + sl;  // the largest diagonal entry
+      if (one == SPK_VG_EXP) {
+        fill([&](double dx, double dy) {
+          return fma(sl, exp2_neg(dist_fast(dx, dy) * o.c1), off);
+        });
+      } else if (one == SPK_VG_GAU) {
+        fill([&](double dx, double dy) {
+          return fma(sl, exp2_neg(fma(dx, dx, dy * dy) * o.c1), off);
+        });
+      } else if (one == SPK_VG_SPH) {
+        const double qr = 1.0 / o.r, top = off + sl;
+        fill([&](double dx, double dy) {
+          const double h = dist_fast(dx, dy) * qr;
+          const double v = h < 1.0 ? h : h >= 1.0 ? 1.0 : h;  // NaN stays NaN
+          return fma(sl * v, fma(v * v, 0.5, -1.5), top);
+        });
+      } else {
+        // several components, unbounded models, a positive min_vg_val: the
+        // distances first, then one evaluation in a loop
+        fill([&](double dx, double dy) { return dist_fast(dx, dy); });
+#pragma unroll
+        for (int J = 0; J < NBC; ++J)
+#pragma unroll
+          for (int I = J; I < NBR; ++I) {
+            if (16 * J >= k) continue;
+#pragma unroll
+            for (int r = 0; r < 4; ++r) T[r * 64 + lane] = acc[I][J][r];
+#pragma unroll 1
+            for (int r = 0; r < 4; ++r) {
+              const double v =
+                  vg_simple_entry(vf, T[r * 64 + lane], sk ? 1 : 0, a.mvg);
+              T[r * 64 + lane] = sk || !bounded ? v : c0 - v;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[I][J][r] = T[r * 64 + lane];
+          }
+        if (!sk && !bounded) {
+          double mx = 0.0;
+#pragma unroll
+          for (int J = 0; J < NBC; ++J)
+#pragma unroll
+            for (int I = J; I < NBR; ++I)
+#pragma unroll
+              for (int r = 0; r < 4; ++r)
+                if (16 * I + c < k && 16 * J + g + 4 * r < k)
+                  mx = fmax(mx, fabs(acc[I][J][r]));
+          c0 = 2.0 * wave_max(mx) + fabs(sill);
+#pragma unroll
+          for (int J = 0; J < NBC; ++J)
+#pragma unroll
+            for (int I = J; I < NBR; ++I)
+#pragma unroll
+              for (int r = 0; r < 4; ++r) acc[I][J][r] = c0 - acc[I][J][r];
+        }
+        double dg = 0.0;
+#pragma unroll
+        for (int J = 0; J < NBC; ++J)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (c == g + 4 * r && 16 * J + c < k)
+              dg = fmax(dg, acc[J][J][r]);
+        dmaxc = wave_max(dg);
+      }
+      // rows of values and border, their columns.  (The lane and k go
+      // through an empty asm here and below so that the many comparisons
+      // with them are not made beforehand, kept and spilled.)
+      int co = c, go = g, ko = k;
+      asm volatile("" : "+v"(co), "+v"(go), "+s"(ko));
+#pragma unroll
+      for (int I = 0; I < NBR; ++I) {
+        if (16 * I + 15 < ko || 16 * I >= ko + 1 + P1) continue;
+        const int row = 16 * I + co;
+        const bool special = row >= ko && row < ko + 1 + P1;
+#pragma unroll
+        for (int J = 0; J < NBC && J <= I; ++J)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            if (special)
+              acc[I][J][r] = sp[(row - ko) * kNebRows + 16 * J + go + 4 * r];
+      }
+#pragma unroll
+      for (int J = 0; J < NBC; ++J)
+#pragma unroll
+        for (int r = 0; r < 4; ++r) {
+          if (16 * J + 4 * r + 3 < ko || 16 * J + 4 * r >= ko + 1 + P1)
+            continue;
+          const int col = 16 * J + 4 * r + go;
+#pragma unroll
+          for (int I = J; I < NBR; ++I)
+            if (col >= ko && col < ko + 1 + P1) acc[I][J][r] = 0.0;
+        }
+      // ---- Cholesky sweep, 16 columns at a time
+      double pmin = INFINITY, ylast = 0.0, yu = 0.0, yy = 0.0, yf[PA];
+#pragma unroll
+      for (int qd = 0; qd < PA; ++qd) yf[qd] = 0.0;
+#pragma unroll
+      for (int J = 0; J < NBC; ++J) {
+        asm volatile("" : "+s"(ko));
+        if (16 * J >= ko + 1 + P1) break;
+        __syncthreads();  // T's readers are done
+#pragma unroll
+        for (int I = J; I < NBR; ++I)
+#pragma unroll
+          for (int r = 0; r < 4; ++r)
+            T[(16 * I + c) * kNebLd + g + 4 * r] = acc[I][J][r];
+        __syncthreads();
+        // lane i: row i of the panel (rows above it and unused rows hold
+        // leftovers that nothing reads)
+        double2 v2[8];
+        double2 *row2 = reinterpret_cast<double2 *>(T + lane * kNebLd);
+#pragma unroll
+        for (int e = 0; e < 8; ++e) v2[e] = row2[e];
+        double v[16];
+#pragma unroll
+        for (int e = 0; e < 8; ++e) {
+          v[2 * e] = v2[e].x;
+          v[2 * e + 1] = v2[e].y;
+        }
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          if (16 * J + j >= ko) break;
+          const double piv = bcast(v[j], 16 * J + j);
+          pmin = fmin(pmin, piv);
+          // 1 / sqrt(piv), one step of third order from 5e-8; NaN for
+          // pivots that are not positive and finite, and then for all
+          // later ones
+          double y = __builtin_amdgcn_rsq(piv);
+          const double e = fma(-piv * y, y, 1.0);
+          y = fma(y * e, fma(e, 0.375, 0.5), y);
+          ylast = y;
+          const double l = v[j] * y;
+          v[j] = l;
+#pragma unroll
+          for (int i = j + 1; i < 16; ++i)
+            v[i] = fma(-l, bcast(l, 16 * J + i), v[i]);
+          yy = fma(l, l, yy);
+        }
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          row2[e] = make_double2(v[2 * e], v[2 * e + 1]);
+        // the products with u and G whose columns are in this panel
+        const double *row = T + lane * kNebLd - 16 * J;
+        if (ko >= 16 * J && ko < 16 * J + 16) yu = -row[ko];
+#pragma unroll
+        for (int qd = 0; qd < PA; ++qd) {
+          const int col = ko + 1 + qd;
+          if (qd < P1 && col >= 16 * J && col < 16 * J + 16) yf[qd] = -row[col];
+        }
+        if (J + 1 == NBC || 16 * (J + 1) >= ko + 1 + P1) continue;
+        __syncthreads();
+        // operands: lane (c, g) takes columns 4 g .. 4 g + 3 of row c
+        double fr[NBR][4];
+#pragma unroll
+        for (int I = J + 1; I < NBR; ++I) {
+          const double2 *f2 = reinterpret_cast<const double2 *>(
+              T + (16 * I + c) * kNebLd + 4 * g);
+          const double2 f0 = f2[0], f1 = f2[1];
+          fr[I][0] = f0.x;
+          fr[I][1] = f0.y;
+          fr[I][2] = f1.x;
+          fr[I][3] = f1.y;
+        }
+        // stations end inside this panel, the products' columns in the next
+        if (16 * J + 16 > ko)
+#pragma unroll
+          for (int I = J + 1; I < NBR; ++I)
+#pragma unroll
+            for (int kk = 0; kk < 4; ++kk)
+              if (16 * J + 4 * g + kk >= ko) fr[I][kk] = 0.0;
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+#pragma unroll
+          for (int J2 = J + 1; J2 < NBC; ++J2) {
+            const double ng = -fr[J2][kk];
+#pragma unroll
+            for (int I = J2; I < NBR; ++I)
+              acc[I][J2] = __builtin_amdgcn_mfma_f64_16x16x4f64(
+                  ng, fr[I][kk], acc[I][J2], 0, 0, 0);
+          }
+      }
+      // condition estimate max diag(C) / min pivot (a lower bound of the
+      // condition number); sets beyond 1e10 take the pseudo-inverse as the
+      // reference computes it
+      const double kap = dmaxc / pmin;
+      bool ok = ylast == ylast && pmin > 0.0;
+      double beta[PA];
+      double bsc = 0.0;
+      if (ok && kap <= 1e10 && p > 0) {
+        double B[PA][PA], gu[PA];
+        for (int i = 0; i < p; ++i) {
+          gu[i] = bcast(yu, k + 1 + i);
+          for (int j = 0; j <= i; ++j) B[i][j] = bcast(yf[j], k + 1 + i);
+        }
+        bsc = B[0][0];
+        ok = neb_beta<PA>(p, B, gu, beta);
+      }
+      if (!ok || !(kap <= 1e10)) {
+        if (lane == 0) a.fail_list[atomicAdd(a.fail_cnt, 1)] = ch;
+        break;
+      }
+      if (lane == 0 && i0 == 0) atomicMax(&a.skappa[t], dbits(kap));
+      if (mine) {
+        double e;
+        if (sk) {
+          if (a.skm) {
+            e = mean + yu;
+          } else if (neb_close1(yf[0])) {
+            e = yu;
+          } else {
+            // the sum test fails: nearest station of the set
+            // (interp/steps.py:418-427)
+            double bd = INFINITY;
+            int bj = 0;
+            for (int j = 0; j < k; ++j) {
+              const double d = dist2(x, y, rx[j], ry[j]);
+              if (d < bd) {
+                bd = d;
+                bj = j;
+              }
+            }
+            e = sp[bj];  // zsh is zero here
+          }
+        } else {
+          e = yu + beta[0] * (1.0 - yf[0]);
+          for (int qd = 1; qd < p; ++qd)
+            e += (a.cell_drift[(int64_t)(qd - 1) * a.C + ci] - yf[qd]) *
+                 beta[qd];
+        }
+        a.est[(int64_t)t * a.C + ci] = e;
+        if (a.want_var && a.var)
+          a.var[(int64_t)t * a.C + ci] =
+              c0 - yy + (yf[0] - 1.0) * (yf[0] - 2.0) / bsc;
+      }
+      __syncthreads();  // rx and ry are read
+    }
+  }
+}
+
+// Column blocks for sets of K stations.
+static inline int neb_col_blocks(int K, int p) {
+  return (int)ceil_div(K + neb_extra(p), 16);
+}
+
+template <int PT>
+static void neb_mfma_launch(int nbc, dim3 grid, hipStream_t st,
+                            const NebArgs &a, const VgFast *vf) {
+  auto k = nbc == 1 ? k_neb_mfma<1, PT>
+                    : nbc == 2 ? k_neb_mfma<2, PT>
+                               : nbc == 3 ? k_neb_mfma<3, PT>
+                                          : k_neb_mfma<4, PT>;
+  hipLaunchKernelGGL(k, grid, dim3(64), 0, st, a, vf);
 }
 
 // ---- pseudo-inverse fallback ----------------------------------------------------
@@ -1453,6 +1878,13 @@ int spk_interp_neb_steps_dev(spk_ctx *ctx, const spk_problem *prob,
         ph = ph || v.type[qd] == SPK_VG_POW || v.type[qd] == SPK_VG_HOL;
   }
   const int lds_krige = neb_lds_doubles(K, p) * 8;
+  // sets on the matrix cores where four cells or more fit in their rows
+  // and no model needs pow or sin
+  const int nbc = neb_col_blocks(K, p);
+  const bool mf = krig && !ph && nbc <= 4 &&
+                  K + neb_extra(p) + 4 <= 16 * neb_row_blocks(nbc);
+  VgFast *vf = nullptr;
+  if (mf) SPK_TRY(ws_get(ctx, "neb_vf", S * sizeof(VgFast), (void **)&vf));
   int hbad = 0;
   for (int64_t t0 = 0; t0 < T; t0 += S) {
     const int Sb = (int)std::min<int64_t>(S, T - t0);
@@ -1519,12 +1951,21 @@ int spk_interp_neb_steps_dev(spk_ctx *ctx, const spk_problem *prob,
     a.fail_list = flist;
     a.fail_cnt = fcnt;
     a.bad = bad;
+    if (mf) {
+      hipLaunchKernelGGL(k_neb_vf, dim3((unsigned)ceil_div(Sb, 64)), dim3(64),
+                         0, sm, gb, Sb, vf);
+      SPK_TRY(check_launch("k_neb_vf"));
+    }
     {
       ProfScope ps(ctx, "neb_krige");
       const unsigned grid =
           (unsigned)std::max<int64_t>(1, std::min<int64_t>(tot, 16384));
       const dim3 g(grid), b(64);
-      if (!krig)
+      if (mf && method == SPK_M_EDK)
+        neb_mfma_launch<kMaxP>(nbc, g, sm, a, vf);
+      else if (mf)
+        neb_mfma_launch<1>(nbc, g, sm, a, vf);
+      else if (!krig)
         hipLaunchKernelGGL((k_neb_krige<0, false, false>), g, b, lds_krige,
                            sm, a);
       else if (method == SPK_M_OK && ph)

@@ -114,6 +114,36 @@ def test_other_methods_match_oracle(gpu, method):
     assert v is None
 
 
+@pytest.mark.parametrize('method', ['OK', 'SK', 'EDK'])
+@pytest.mark.parametrize('n_nebs', [2, 13, 14, 15, 16, 29, 30, 31, 45, 46, 47,
+                                    48, 54, 55, 58, 60])
+def test_set_sizes_match_oracle(gpu, method, n_nebs):
+    """Set sizes around the 16-row blocks of the chunk kernel and its limit,
+    with one-model, two-model, linear and unbounded variograms.  The
+    covariance matrices' condition numbers stay below 1e4 (the Gaussian
+    model's with a range of 12 km near the station spacing; 3e7 at 50 km), so
+    k 2^-53 cond is below 1e-10; EDK's border adds a factor."""
+    case = list(_case(n=90, side=6, T=8, seed=n_nebs))
+    v = [float(x.split()[0]) * 10.0 for x in case[5]]
+    case[5][4] = f'{0.6 * v[4]!r} Sph(2e4) + {0.4 * v[4]!r} Exp(7e4)'
+    case[5][5] = f'{0.1 * v[5]!r} Nug(0.0) + {0.9 * v[5]!r} Gau(1.2e4)'
+    if method != 'EDK':
+        # (with a drift the linear model, not positive definite in the plane,
+        # gives bordered matrices with condition numbers of 3e6 and more)
+        case[5][6] = f'{0.2 * v[6]!r} Nug(0.0) + {0.8 * v[6]!r} Lin(5e4)'
+    if method == 'OK':
+        # (for EDK in metres the condition number is 2e11)
+        case[5][7] = f'{v[7]!r} Rng(1.0)'
+    if method == 'EDK' and n_nebs < 4:
+        pytest.skip('two stations do not determine mean and drift')
+    e, var, info, f64, prb = _run(gpu, case, method, 'nrst', n_nebs, thr=0.0)
+    scale = np.nanmax(np.abs(case[4]))
+    _close(e, f64[method], scale, {'EDK': 1e-8}.get(method, 1e-9), method)
+    if method == 'OK':
+        _close(var, f64['EST_VARS_OK'], np.nanmax(f64['EST_VARS_OK']), 1e-8,
+               'var')
+
+
 def test_edk_reproduces_the_drift(gpu):
     """Values that are a linear function of the drift are reproduced at
     every cell (the weights sum to one and reproduce the drift)."""
