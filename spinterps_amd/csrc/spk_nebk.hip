@@ -200,7 +200,7 @@ __global__ void k_neb_mask(const double *__restrict__ vals, int64_t n,
     out[i] = keep[i % N] ? vals[i] : NAN;
 }
 
-// ---- Z order of the cells ----------------------------------------------------
+// ---- order of the cells along a Hilbert curve ----------------------------------------------------
 // One workgroup: the bounding box of the cells, bb = (x0, x1, y0, y1).
 __global__ __launch_bounds__(1024) void k_neb_bbox(
     const double *__restrict__ cx, const double *__restrict__ cy, int64_t C,
@@ -230,38 +230,47 @@ __global__ __launch_bounds__(1024) void k_neb_bbox(
   }
 }
 
-__device__ inline unsigned spread16(unsigned v) {
-  v &= 0xffffu;
-  v = (v | (v << 8)) & 0x00ff00ffu;
-  v = (v | (v << 4)) & 0x0f0f0f0fu;
-  v = (v | (v << 2)) & 0x33333333u;
-  v = (v | (v << 1)) & 0x55555555u;
-  return v;
+// Position of (x, y), 16 bits each, on the Hilbert curve: quadrant by
+// quadrant, the curve inside each turned or mirrored.
+__device__ inline unsigned hilbert16(unsigned x, unsigned y) {
+  unsigned d = 0;
+  for (int b = 15; b >= 0; --b) {
+    const unsigned qx = (x >> b) & 1u, qy = (y >> b) & 1u;
+    d = (d << 2) | ((3u * qx) ^ qy);
+    if (!qy) {
+      const unsigned m = qx ? 0xffffu : 0u, u = x ^ m;
+      x = y ^ m;
+      y = u;
+    }
+  }
+  return d;
 }
 
-// code[c]: coordinates quantised to 16 bits over the bounding box and
-// interleaved (Z order); id[c] = c.
-__global__ void k_neb_morton(const double *__restrict__ cx,
+// code[c]: coordinates quantised to 16 bits over the bounding box, along the
+// Hilbert curve; id[c] = c.  (Along the Z order a tile of 64 consecutive cells
+// that crosses a quadrant's edge spans the domain: too many candidates to
+// stage.  Of 10.4 ms for 13 selections over 250 000 cells the device was
+// busy for 3.8, the rest waited for such tiles.)
+__global__ void k_neb_curve(const double *__restrict__ cx,
                              const double *__restrict__ cy, int64_t C,
                              const double *__restrict__ bb,
                              unsigned *__restrict__ code,
                              int32_t *__restrict__ id) {
   const double x0 = bb[0], y0 = bb[2];
   const double wx = bb[1] - x0, wy = bb[3] - y0;
-  const double sx = wx > 0.0 ? 65535.0 / wx : 0.0;
-  const double sy = wy > 0.0 ? 65535.0 / wy : 0.0;
+  const double w = fmax(wx, wy), sc = w > 0.0 ? 65535.0 / w : 0.0;
   for (int64_t c = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; c < C;
        c += (int64_t)gridDim.x * blockDim.x) {
-    const double fx = fmin(fmax((cx[c] - x0) * sx, 0.0), 65535.0);
-    const double fy = fmin(fmax((cy[c] - y0) * sy, 0.0), 65535.0);
-    code[c] = spread16((unsigned)fx) | (spread16((unsigned)fy) << 1);
+    const double fx = fmin(fmax((cx[c] - x0) * sc, 0.0), 65535.0);
+    const double fy = fmin(fmax((cy[c] - y0) * sc, 0.0), 65535.0);
+    code[c] = hilbert16((unsigned)fx, (unsigned)fy);
     id[c] = (int32_t)c;
   }
 }
 
 // ---- nrst selection ----------------------------------------------------------
 // grid (ceil(C / 64), S), 256 threads.  Tile i holds cells perm[64 i ..
-// 64 i + 63], consecutive in Z order, so a tile is a compact patch.  For
+// 64 i + 63], consecutive along the curve, so a tile is a compact patch.  For
 // the tile's bounding box
 // (centre c, half diagonal h) the block finds a T with at least k active
 // stations within T of c; the k nearest of any cell x of the tile then lie
@@ -600,13 +609,22 @@ __global__ void k_neb_mark(const unsigned long long *__restrict__ key,
                            int kfix, int64_t total, int32_t *__restrict__ gs) {
   for (int64_t p = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; p < total;
        p += (int64_t)gridDim.x * blockDim.x) {
-    bool nw = (p % C) == 0 || key[p] != key[p - 1];
+    const unsigned t = (unsigned)p / (unsigned)C;  // both below 2^31
+    bool nw = p == (int64_t)t * C || key[p] != key[p - 1];
     if (!nw) {
-      const int64_t t = p / C;
       const int k = neb_set_size(K, kfix, sc[t].n);
       const int32_t *a = nb + (t * C + cell[p]) * K;
       const int32_t *b = nb + (t * C + cell[p - 1]) * K;
-      for (int r = 0; r < k && !nw; ++r) nw = a[r] != b[r];
+      // eight entries at a time, their loads in flight together
+      for (int r = 0; r < k && !nw; r += 8) {
+        int diff = 0;
+#pragma unroll
+        for (int u = 0; u < 8; ++u) {
+          const int e = min(r + u, k - 1);
+          diff |= a[e] ^ b[e];
+        }
+        nw = diff != 0;
+      }
     }
     gs[p] = nw ? (int32_t)p : 0;
   }
@@ -1784,7 +1802,7 @@ int spk_interp_neb_steps_dev(spk_ctx *ctx, const spk_problem *prob,
     }
   }
   int *h_cnt = static_cast<int *>(ctx->h_sc);
-  // cells in Z order: the nrst selection tiles
+  // cells along the curve: the nrst selection tiles
   int32_t *perm, *mid;
   unsigned *mcode;
   double *bbd;
@@ -1841,9 +1859,9 @@ int spk_interp_neb_steps_dev(spk_ctx *ctx, const spk_problem *prob,
 
   if (sel == SPK_NEB_NRST) {
     hipLaunchKernelGGL(k_neb_bbox, dim3(1), dim3(1024), 0, sm, cx, cy, C, bbd);
-    hipLaunchKernelGGL(k_neb_morton, g1(C), dim3(256), 0, sm, cx, cy, C,
+    hipLaunchKernelGGL(k_neb_curve, g1(C), dim3(256), 0, sm, cx, cy, C,
                        (const double *)bbd, mcode, mid);
-    SPK_TRY(check_launch("k_neb_morton"));
+    SPK_TRY(check_launch("k_neb_curve"));
     size_t b = tmp_bytes;
     SPK_HIP(hipcub::DeviceRadixSort::SortPairs(tmp, b, mcode, mcode + C, mid,
                                                perm, (int)C, 0, 32, sm));

@@ -196,6 +196,18 @@ def test_singular_sets_use_the_pseudo_inverse(gpu):
     assert info[0] & _lib.ST_PINV and info[0] & _lib.ST_ILLCOND
 
 
+@pytest.mark.parametrize('n_nebs,n_pies', [(1, 1), (9, 1), (24, 3), (24, 24),
+                                           (40, 33), (64, 64), (50, 2)])
+def test_pie_sector_counts(gpu, n_nebs, n_pies):
+    """Sector counts around the powers of two that split the wavefront; sets
+    of the wrong stations would be off by far more than rounding."""
+    case = list(_case(n=150, side=7))
+    case[4][2] = case[4][0]
+    e, _, info, f64, prb = _run(gpu, case, 'IDW', 'pie', n_nebs, n_pies,
+                                thr=0.0)
+    _close(e, f64['IDW'], np.nanmax(np.abs(case[4])), 1e-12, 'IDW')
+
+
 def test_pie_with_too_few_stations_is_refused(gpu):
     from spinterps_amd.interp.steps import DeviceProblem, interp_neb_steps
     sx, sy, cx, cy, z, vgs, _, _ = _case()
