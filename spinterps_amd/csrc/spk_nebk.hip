@@ -1141,7 +1141,7 @@ __global__ __launch_bounds__(64) void k_neb_krige(NebArgs a) {
 // conflicts in both layouts.
 //
 // Bound: FP64 VALU issue (entries and panels; the products of the blocks are
-// a tenth).  12 steps x 250 000 cells, 1 000 stations, 50 per set: 6.4 ms; 24.6
+// a tenth).  12 steps x 250 000 cells, 1 000 stations, 50 per set: 6.2 ms; 24.6
 // with k_neb_krige, which factorises a packed triangle in LDS by columns with
 // two LDS reads per multiply-add, and substitutes for four cells at a time.
 // That kernel keeps what does not fit here: sets of more than 58 stations,
@@ -1165,7 +1165,9 @@ __global__ void k_neb_vf(const spk_vg *__restrict__ vgs, int S,
 __host__ __device__ inline int neb_extra(int p) { return 1 + (p > 0 ? p : 1); }
 
 template <int NBC, int PT>
-__global__ __launch_bounds__(64, 2) void k_neb_mfma(
+// Small sets wait for loads more than they compute: 3 waves per SIMD (8 steps x
+// 9 797 cells, 24 per set: 722 -> 404 us); the others would spill.
+__global__ __launch_bounds__(64, NBC > 2 ? 2 : 3) void k_neb_mfma(
     NebArgs a, const VgFast *__restrict__ vfs) {
   constexpr int PA = PT > 0 ? PT : 1;
   constexpr int NBR = neb_row_blocks(NBC), NR = 16 * NBR;
@@ -1183,6 +1185,8 @@ __global__ __launch_bounds__(64, 2) void k_neb_mfma(
     const int k = q.k, t = q.t;
     const int np = (int)(q.p1 - q.p0);  // at most kNebChunk
     __syncthreads();  // the previous chunk's readers are done
+    const unsigned long long seen = __hip_atomic_load(
+        &a.skappa[t], __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
     const int cme = lane < np ? a.cells[q.p0 + lane] : 0;
     const int32_t *list =
         a.nb + ((int64_t)t * a.C + bcast_i(cme, 0)) * a.K;
@@ -1198,8 +1202,11 @@ __global__ __launch_bounds__(64, 2) void k_neb_mfma(
       zl = a.zact[(int64_t)t * a.ldz + pos];
     }
     if (neb_no_system(a, q, lane, np, cme, zl)) continue;
+    // the values less their mean: OK and EDK do not depend on a constant
+    // (the weights sum to one), and rounding then scales with the
+    // deviations; SK's weights do not
     const double mean = wave_sum(lane < k ? zl : 0.0) / k;
-    const double zsh = a.skm && sk ? mean : 0.0;
+    const double zsh = sk && !a.skm ? 0.0 : mean;
     if (lane < k) {
       rx[lane] = coord_fast(zx);
       ry[lane] = coord_fast(zy);
@@ -1461,7 +1468,10 @@ __global__ __launch_bounds__(64, 2) void k_neb_mfma(
         if (lane == 0) a.fail_list[atomicAdd(a.fail_cnt, 1)] = ch;
         break;
       }
-      if (lane == 0 && i0 == 0) atomicMax(&a.skappa[t], dbits(kap));
+      // the step's largest estimate, mostly known already: an atomic per chunk
+      // on the few steps' addresses took longer than the chunks
+      if (lane == 0 && i0 == 0 && dbits(kap) > seen)
+        atomicMax(&a.skappa[t], dbits(kap));
       if (mine) {
         double e;
         if (sk) {
@@ -1484,7 +1494,7 @@ __global__ __launch_bounds__(64, 2) void k_neb_mfma(
             e = sp[bj];  // zsh is zero here
           }
         } else {
-          e = yu + beta[0] * (1.0 - yf[0]);
+          e = mean + (yu + beta[0] * (1.0 - yf[0]));
           for (int qd = 1; qd < p; ++qd)
             e += (a.cell_drift[(int64_t)(qd - 1) * a.C + ci] - yf[qd]) *
                  beta[qd];
