@@ -862,14 +862,15 @@ def neb_leg(args, log):
            'steps_ill_conditioned': int(np.sum((info & 16) != 0)),
            'roofline': {'bound': 'mfma', 'achieved': ach, 'peak': 78.6,
                         'unit': 'TFLOP/s', 'frac': ach / 78.6,
-                        'kernel': 'k_neb_krige (per group: covariance '
-                                  'system, Cholesky and inverse in LDS; per '
-                                  'cell: dual-form estimate and variance)',
+                        'kernel': 'k_neb_mfma (per group: stations, values, '
+                                  'border and cells as the rows of one '
+                                  'matrix, Cholesky sweep over the '
+                                  'stations\' columns)',
                         'note': 'achieved: the reference\'s per-cell '
                                 '2 (k+1)^2 + 4 (k+1) flops over the '
                                 'kernel\'s time (factorisations not '
-                                'counted); the kernel runs on the FP64 '
-                                'vector units, latency-bound in LDS'}}
+                                'counted); the kernel is bound by FP64 '
+                                'vector issue'}}
     if not args.no_cpu:
         from scipy.spatial import cKDTree
         from threadpoolctl import threadpool_limits
