@@ -65,7 +65,8 @@ __global__ void k_recenter(const double *__restrict__ sx,
                            const double *__restrict__ cy, int64_t C, double ox,
                            double oy, double *__restrict__ osx,
                            double *__restrict__ osy, double *__restrict__ ocx,
-                           double *__restrict__ ocy) {
+                           double *__restrict__ ocy, int *__restrict__ zero) {
+  if (zero && blockIdx.x == 0 && threadIdx.x == 0) *zero = 0;
   for (int64_t i = blockIdx.x * (int64_t)blockDim.x + threadIdx.x; i < N + C;
        i += (int64_t)gridDim.x * blockDim.x) {
     if (i < N) {
@@ -79,12 +80,13 @@ __global__ void k_recenter(const double *__restrict__ sx,
 }
 
 int recenter(hipStream_t st, const spk_problem *prob, double *sx, double *sy,
-             double *cx, double *cy) {
+             double *cx, double *cy, int *zero) {
   const int64_t N = prob->n_stns, C = cx ? prob->n_cells : 0;
   const int64_t g = std::min<int64_t>(ceil_div(N + C, 256), 65536);
   hipLaunchKernelGGL(k_recenter, dim3((unsigned)g), dim3(256), 0, st,
                      prob->stn_x, prob->stn_y, N, prob->cell_x, prob->cell_y,
-                     C, prob->origin_x, prob->origin_y, sx, sy, cx, cy);
+                     C, prob->origin_x, prob->origin_y, sx, sy, cx, cy,
+                     zero);
   return check_launch("k_recenter");
 }
 
@@ -1402,8 +1404,8 @@ using namespace spk;
 // (interp/steps.py:285-313, and its special steps :280-283): the kernels
 // of spk_interp_steps_dev and spk_idw_steps_noalloc_dev.  sx.. cy are the
 // re-centred coordinates; idx [S x N], zact [S x ldz], sc [S] and bad [1]
-// are the caller's scratch.  The weight-sum flag is cleared by a fill
-// kernel, and read back at the end (the reference asserts, steps.py:305).
+// are the caller's scratch.  The weight-sum flag, cleared by the caller
+// (recenter), is read back at the end (the reference asserts, steps.py:305).
 static int idw_nnb_steps(spk_ctx *ctx, const spk_opts *opts, int64_t T,
                          int64_t N, int64_t C, const double *vals,
                          const double *sx, const double *sy,
@@ -1413,7 +1415,6 @@ static int idw_nnb_steps(spk_ctx *ctx, const spk_opts *opts, int64_t T,
                          double *kappa) {
   hipStream_t sm = ctx->stream;
   const int method = opts->method;
-  hipLaunchKernelGGL(k_fill_int, dim3(1), dim3(64), 0, sm, bad, 1, 0);
   for (int64_t t0 = 0; t0 < T; t0 += S) {
     const int Sb = (int)std::min<int64_t>(S, T - t0);
     double *eb = est + t0 * C;
@@ -1425,7 +1426,8 @@ static int idw_nnb_steps(spk_ctx *ctx, const spk_opts *opts, int64_t T,
       ProfScope ps(ctx, "idw_nnb");
       if (method == SPK_M_IDW) {
         SPK_TRY(idw_steps(sm, sx, sy, N, vals + t0 * N, Sb, sc, idx, zact,
-                          ldz, cx, cy, C, opts->idw_exp, eb, bad));
+                          ldz, cx, cy, C, opts->idw_exp, eb, bad, info + t0,
+                          kappa ? kappa + t0 : nullptr));
       } else {
         hipLaunchKernelGGL(k_nnb, dim3((unsigned)ceil_div(C, 256), Sb),
                            dim3(256), 0, sm, sx, sy, idx, N, zact, ldz, sc,
@@ -1433,11 +1435,11 @@ static int idw_nnb_steps(spk_ctx *ctx, const spk_opts *opts, int64_t T,
         hipLaunchKernelGGL(k_special, dim3((unsigned)ceil_div(C, 256), Sb),
                            dim3(256), 0, sm, sx, sy, idx, N, zact, ldz, sc,
                            cx, cy, C, eb, (double *)nullptr);
+        hipLaunchKernelGGL(k_status_out, dim3((unsigned)ceil_div(Sb, 256)),
+                           dim3(256), 0, sm, sc, Sb, info + t0,
+                           kappa ? kappa + t0 : nullptr);
       }
     }
-    hipLaunchKernelGGL(k_status_out, dim3((unsigned)ceil_div(Sb, 256)),
-                       dim3(256), 0, sm, sc, Sb, info + t0,
-                       kappa ? kappa + t0 : nullptr);
     SPK_TRY(check_launch("idw/nnb"));
   }
   int hbad = 0;
@@ -1599,7 +1601,9 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
   sy = sx + N;
   SPK_TRY(ws_get(ctx, "cell_xy", 2 * C * sizeof(double), (void **)&cx));
   cy = cx + C;
-  SPK_TRY(recenter(sm, prob, sx, sy, cx, cy));
+  int *bad = nullptr;  // IDW: the weight-sum flag
+  if (!krig) SPK_TRY(ws_get(ctx, "bad", 64, (void **)&bad));
+  SPK_TRY(recenter(sm, prob, sx, sy, cx, cy, bad));
   const int64_t ldz = round_up(N, 64);
   const int p = method == SPK_M_OK ? 1 : method == SPK_M_EDK ? 1 + m : 0;
   const int64_t ld = round_up(N + (p > 0 ? p : 1), 64);
@@ -1616,8 +1620,6 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
     int32_t *idx;
     double *zact;
     StepSc *sc;
-    int *bad;
-    SPK_TRY(ws_get(ctx, "bad", 64, (void **)&bad));
     SPK_TRY(ws_get(ctx, "idx0", S * N * sizeof(int32_t), (void **)&idx));
     SPK_TRY(ws_get(ctx, "zact0", S * ldz * sizeof(double), (void **)&zact));
     SPK_TRY(ws_get(ctx, "sc0", S * sizeof(StepSc), (void **)&sc));
@@ -2537,7 +2539,7 @@ int spk_idw_steps_noalloc_dev(spk_ctx *ctx, const spk_problem *prob,
   StepSc *sc = reinterpret_cast<StepSc *>(base + kNaOffSc);
   const int64_t ldz = round_up(N, 64);  // <= kNaMaxStns
   hipStream_t sm = ctx->stream;
-  SPK_TRY(recenter(sm, prob, sx, sy, cx, cy));
+  SPK_TRY(recenter(sm, prob, sx, sy, cx, cy, bad));
   return idw_nnb_steps(ctx, opts, T, N, C, vals, sx, sy, cx, cy, idx, zact,
                        ldz, sc, std::min<int64_t>(T, kNaSteps), bad, est,
                        info, kappa);

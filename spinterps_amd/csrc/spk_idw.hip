@@ -86,7 +86,8 @@ __device__ inline double idw_weight(double s2, double p, int p2) {
 
 // grid (ceil(C / (32 NW)), ceil(S / BS)), 64 NW threads; vals [S x N] the
 // launch's steps (NaN = no value), sc [S] their records (k_compact), est
-// [S x C].  Special steps (one station, mean fill) are filled here too; a
+// [S x C]; info and kappa (may be null) [S] are the steps' status words and
+// condition estimates.  Special steps (one station, mean fill) are filled here too; a
 // step without stations is left alone (interp/steps.py:280-283, 325-331).
 template <int BS, int NW, int KIND>
 __global__ __launch_bounds__(64 * NW, 2) void k_idw_mfma(
@@ -95,7 +96,8 @@ __global__ __launch_bounds__(64 * NW, 2) void k_idw_mfma(
     const int32_t *__restrict__ idx, const double *__restrict__ zact,
     int64_t ldz, const double *__restrict__ cx, const double *__restrict__ cy,
     int64_t C, double p, int p2, double *__restrict__ est,
-    int *__restrict__ bad) {
+    int *__restrict__ bad, int32_t *__restrict__ info,
+    double *__restrict__ kappa) {
   constexpr int NT = 64 * NW, BC = 32 * NW, KC = 16, TS = BS / 16;
   constexpr int AL = BS * KC / NT;          // values per thread and chunk
   __shared__ double Ws[2][KC][BC + 16];     // W[station][cell]
@@ -112,6 +114,11 @@ __global__ __launch_bounds__(64 * NW, 2) void k_idw_mfma(
   const bool have = gc < C;
   const double x = have ? cx[gc] : 0.0, y = have ? cy[gc] : 0.0;
   if (tid < BC) coinc[tid] = 0;
+  if (blockIdx.x == 0)
+    for (int u = tid; u < BS && t0 + u < S; u += NT) {
+      info[t0 + u] = sc[t0 + u].status | sc[t0 + u].flags;
+      if (kappa) kappa[t0 + u] = sc[t0 + u].kappa;
+    }
   idw_d4 acc[2][TS][2];  // [num/den][step tile][cell tile]
 #pragma unroll
   for (int q = 0; q < 2; ++q)
@@ -267,7 +274,7 @@ static void idw_launch(hipStream_t st, const double *sx, const double *sy,
                        int64_t N, const double *vals, int S, const StepSc *sc,
                        const int32_t *idx, const double *zact, int64_t ldz,
                        const double *cx, const double *cy, int64_t C, double p,
-                       double *est, int *bad) {
+                       double *est, int *bad, int32_t *info, double *kappa) {
   const double pp = 2.0 * p;
   const int p2 = pp >= 1.0 && pp <= 16.0 && pp == floor(pp) ? (int)pp : 0;
   auto k = p2 == 4 ? k_idw_mfma<BS, NW, 0>
@@ -275,13 +282,14 @@ static void idw_launch(hipStream_t st, const double *sx, const double *sy,
   hipLaunchKernelGGL(k, dim3((unsigned)ceil_div(C, 32 * NW),
                              (unsigned)ceil_div(S, BS)),
                      dim3(64 * NW), 0, st, sx, sy, N, vals, S, sc, idx, zact,
-                     ldz, cx, cy, C, p, p2, est, bad);
+                     ldz, cx, cy, C, p, p2, est, bad, info, kappa);
 }
 
 int idw_steps(hipStream_t st, const double *sx, const double *sy, int64_t N,
               const double *vals, int S, const StepSc *sc, const int32_t *idx,
               const double *zact, int64_t ldz, const double *cx,
-              const double *cy, int64_t C, double p, double *est, int *bad) {
+              const double *cy, int64_t C, double p, double *est, int *bad,
+              int32_t *info, double *kappa) {
   auto go = [&](int t0, int n) {
     const int64_t ct = ceil_div(C, 128);
     auto l = ct * ceil_div(n, 64) >= 512 && n > 48
@@ -293,7 +301,8 @@ int idw_steps(hipStream_t st, const double *sx, const double *sy, int64_t N,
                        : ct * ceil_div(n, 16) >= 512 ? idw_launch<16, 4>
                                                      : idw_launch<16, 1>;
     l(st, sx, sy, N, vals + t0 * N, n, sc + t0, idx + t0 * N, zact + t0 * ldz,
-      ldz, cx, cy, C, p, est + t0 * C, bad);
+      ldz, cx, cy, C, p, est + t0 * C, bad, info + t0,
+      kappa ? kappa + t0 : nullptr);
   };
   const int full = S / 64 * 64;
   if (full > 0) go(0, full);

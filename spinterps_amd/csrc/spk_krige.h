@@ -66,7 +66,8 @@ struct StepSc {
 int idw_steps(hipStream_t st, const double *sx, const double *sy, int64_t N,
               const double *vals, int S, const StepSc *sc, const int32_t *idx,
               const double *zact, int64_t ldz, const double *cx,
-              const double *cy, int64_t C, double p, double *est, int *bad);
+              const double *cy, int64_t C, double p, double *est, int *bad,
+              int32_t *info, double *kappa);
 
 // ---- batched estimates (spk_est.hip) -----------------------------------------
 // What the cell kernels read of one active station of a step, in one cache
@@ -236,9 +237,10 @@ int minv_steps(hipStream_t st, const double *Li, int64_t ld, int64_t stride,
                StepSc *sc, const int32_t *idx, int64_t N,
                const double *stn_drift, int m, int method, double *M,
                double *T0, const spk_vg *vgs, double min_vg_val, int S);
-// The problem's stations and (cx not null) cells less its origin.
+// The problem's stations and (cx not null) cells less its origin; clears the
+// flag `zero` where given.
 int recenter(hipStream_t st, const spk_problem *prob, double *sx, double *sy,
-             double *cx, double *cy);
+             double *cx, double *cy, int *zero = nullptr);
 __global__ void k_status_out(const StepSc *sc, int S, int32_t *info,
                              double *kappa);
 // Spatially compact order of the cells (Morton keys over the bounding box,
