@@ -786,8 +786,11 @@ __global__ __launch_bounds__(256, 3) void k_kgen(
   const int tid = threadIdx.x;
   const int64_t c = blockIdx.x * (int64_t)256 + tid;
   const bool valid = c < Cs;
-  const double x = valid ? coord_fast(cx[c]) : 0.0;
-  const double y = valid ? coord_fast(cy[c]) : 0.0;
+  double x = valid ? cx[c] : 0.0, y = valid ? cy[c] : 0.0;
+  if (vg_bounded(vgs[sl])) {
+    x = coord_fast(x);
+    y = coord_fast(y);
+  }
   if (tid == 0) {
     vg_fast_init(vgs[sl], vf);
     n_slots = 0;
@@ -838,8 +841,8 @@ __global__ __launch_bounds__(256, 3) void k_kgen(
     const int ns = n_slots;
     if (tid < ns) {
       const int g = my[slot_j[tid]];
-      stx[tid] = coord_fast(sx[g]);
-      sty[tid] = coord_fast(sy[g]);
+      stx[tid] = coord_stn(sx[g]);
+      sty[tid] = coord_stn(sy[g]);
     }
     __syncthreads();
     // J: the cell's kJ nearest stations among the table (ascending)

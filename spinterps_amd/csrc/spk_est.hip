@@ -17,12 +17,12 @@ __global__ __launch_bounds__(256) void k_stn_rec(
   const int j = blockIdx.x * 256 + threadIdx.x;
   const int n = sc[s].n;
   if (j >= (n + 15) / 16 * 16) return;
-  StnRec r = {1e140, 1e140, 0.0, 0.0, 0.0, {0.0, 0.0, 0.0}};
+  StnRec r = {kFarCoord, kFarCoord, 0.0, 0.0, 0.0, {0.0, 0.0, 0.0}};
   if (j < n) {
     const int g = idx[(int64_t)s * N + j];
     const double *v = V + (int64_t)s * ldv + j;  // alpha, w, dalpha: ld apart
-    r.x = coord_fast(sx[g]);
-    r.y = coord_fast(sy[g]);
+    r.x = coord_stn(sx[g]);
+    r.y = coord_stn(sy[g]);
     r.alpha = v[0];
     r.w = v[ld];
     r.dalpha = v[2 * ld];
@@ -86,7 +86,9 @@ __global__ __launch_bounds__(256) void k_est(
   const int64_t c = blockIdx.x * (int64_t)256 + tid;
   const bool valid = c < Cs;
   const double xr = valid ? cx[c] : 0.0, yr = valid ? cy[c] : 0.0;
-  const double x = coord_fast(xr), y = coord_fast(yr);
+  const bool bounded = vg_bounded(vgs[sl]);
+  const double x = bounded ? coord_fast(xr) : xr;
+  const double y = bounded ? coord_fast(yr) : yr;
   const StnRec *rec = recs + sl * rec_stride(N);
   const bool sk = method == SPK_M_SK;
   const double c0 = stp->c0;

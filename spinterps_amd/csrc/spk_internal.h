@@ -155,12 +155,26 @@ __host__ __device__ inline double dist2(double x1, double y1, double x2,
   return sqrt(s);
 }
 
-// A coordinate for dist_fast: infinite ones (a station or cell beyond every
-// range) become so large that every bounded model is at its sill and the
-// square stays finite; NaN stays NaN.
+// A cell's coordinate for dist_fast, whose sum of squares has to stay finite.
+// A magnitude above 1e140 (a nodata marker, an infinite cell), beyond every
+// range, becomes one in [1e140, 2e140] by the order of the magnitudes' bits:
+// equal coordinates stay equal, others stay so far apart that every bounded
+// model is at its sill, as with dist2's infinite distances.  NaN stays NaN.
+// Unbounded models need the coordinate itself (vg_bounded): their values at
+// such distances are not finite.
 __device__ inline double coord_fast(double x) {
-  return isinf(x) ? copysign(1e140, x) : x;
+  const double a = fabs(x);
+  if (!(a > 1e140)) return x;
+  const long long d = __double_as_longlong(a) - __double_as_longlong(1e140);
+  return copysign(fma((double)d, 3.97e121, 1e140), x);
 }
+// A station's: an infinite one has no distance to itself, so that no system
+// with it can be solved; it stays out of the finite distances.
+__device__ inline double coord_stn(double x) {
+  return isinf(x) ? NAN : coord_fast(x);
+}
+// Both coordinates of a record out of every range of every cell and station.
+constexpr double kFarCoord = 8e140;
 
 // dist2's value for the cell kernels' inner loops: sqrt(s) from the
 // hardware's reciprocal square root (relative error 5e-8) and two coupled
@@ -189,7 +203,13 @@ __device__ inline double dist_fast(double dx, double dy) {
 // exp(); NaN stays NaN.
 __device__ inline double exp2_neg(double y) {
   const double k = rint(y);
-  const double f = y - k;
+  double f;
+  {
+    // (not fused with the caller's product: beyond 2^52, where y is an integer,
+    // the remainder of the exact product would be anything but small)
+#pragma clang fp contract(off)
+    f = y - k;
+  }
   double p = 4.4558179083360645e-10;
   p = fma(p, f, 7.074194297288521e-09);
   p = fma(p, f, 1.0178057087733941e-07);
@@ -436,7 +456,7 @@ __host__ __device__ inline bool vg_simple(const spk_vg &vg) {
 
 // True when every component is bounded by its sill, so that
 // c0 = sum of sills turns the semivariogram matrix into a covariance.
-inline bool vg_bounded(const spk_vg &vg) {
+__host__ __device__ inline bool vg_bounded(const spk_vg &vg) {
   for (int k = 0; k < vg.n; ++k) {
     const int t = vg.type[k];
     if (t == SPK_VG_RNG || t == SPK_VG_POW || t == SPK_VG_HOL) return false;

@@ -1208,8 +1208,8 @@ __global__ __launch_bounds__(64, NBC > 2 ? 2 : 3) void k_neb_mfma(
     const double mean = wave_sum(lane < k ? zl : 0.0) / k;
     const double zsh = sk && !a.skm ? 0.0 : mean;
     if (lane < k) {
-      rx[lane] = coord_fast(zx);
-      ry[lane] = coord_fast(zy);
+      rx[lane] = coord_stn(zx);
+      ry[lane] = coord_stn(zy);
       sp[lane] = zl - zsh;
       sp[kNebRows + lane] = 1.0;
       for (int qd = 1; qd < p; ++qd)
@@ -1234,8 +1234,8 @@ __global__ __launch_bounds__(64, NBC > 2 ? 2 : 3) void k_neb_mfma(
         y = a.cy[ci];
       }
       if (lane >= k && lane < NR) {
-        rx[lane] = coord_fast(x);
-        ry[lane] = coord_fast(y);
+        rx[lane] = bounded ? coord_fast(x) : x;
+        ry[lane] = bounded ? coord_fast(y) : y;
       }
       __syncthreads();
       // ---- entries, in the register layout

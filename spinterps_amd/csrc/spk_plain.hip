@@ -58,7 +58,7 @@ __global__ __launch_bounds__(256) void k_plain_rhs(
   const int32_t *my = idx + (int64_t)s * N + j0;
   if (tid < kPlainStn && j0 + tid < n) {
     const int g = my[tid];
-    st[tid] = double2{coord_fast(sx[g]), coord_fast(sy[g])};
+    st[tid] = double2{coord_stn(sx[g]), coord_stn(sy[g])};
   }
   if (tid == kPlainStn) {
     vg = vgs[s];

@@ -697,3 +697,55 @@ def test_factor_panels_edges(gpu, n):
                                        atol=1e-9 * np.abs(vals[t, a]).mean())
             np.testing.assert_allclose(var[t], v, rtol=1e-9,
                                        atol=1e-9 * np.abs(v).mean())
+
+
+@pytest.mark.parametrize('vg', ['2.0 Exp(30000.0)', '0.1 Nug(0.0) + 2.0 Sph(30000.0)',
+                                '0.3 Nug(0.0) + 2.0 Gau(4000.0)',
+                                '0.5 Sph(9e3) + 0.5 Exp(3e4)'])
+@pytest.mark.parametrize('method', ['OK', 'EDK', 'SKM', 'SK'])
+def test_coordinates_beyond_every_range(gpu, method, vg):
+    """A station or a cell whose coordinate's square overflows (a nodata
+    marker, an infinite cell) is uncorrelated with the rest, as one at
+    1e9 m, where the models are at their sill to the last bit."""
+    from spinterps_amd.interp.steps import (DeviceProblem, interp_neb_steps,
+                                            interp_steps)
+    rng = np.random.default_rng(11)
+    n, cells = 70, 300
+    sx, sy = rng.uniform(0, 1e5, n), rng.uniform(0, 1e5, n)
+    cx, cy = rng.uniform(0, 1e5, cells), rng.uniform(0, 1e5, cells)
+    # (the drift by position, finite everywhere)
+    sd = (sx / 1e5 + np.sin(sy / 2e4))[:, None]
+    cd = (cx / 1e5 + np.sin(cy / 2e4))[None]
+    vals = rng.gamma(2.0, 3.0, (2, n))
+    vals[1, 3] = np.nan
+
+    def run(far, far2, cell):
+        x, y, gx, gy = sx.copy(), sy.copy(), cx.copy(), cy.copy()
+        x[5], y[5], y[7] = far, 0.3 * far, far2
+        gx[9], gy[11] = cell
+        prob = DeviceProblem(x, y, gx, gy, sd if method == 'EDK' else None,
+                             cd if method == 'EDK' else None)
+        out = []
+        for prec in ('fp64', 'fp64b', 'mixed'):
+            e, v, _ = interp_steps(prob, vals, [vg] * 2, method,
+                                   precision=prec)
+            out += [e.cpu().numpy()] + ([] if v is None else [v.cpu().numpy()])
+        if np.isfinite(cell).all() and max(cell) < 1e150:
+            # (every sector's nearest stations, the far ones among them)
+            e, v, _ = interp_neb_steps(prob, vals, [vg] * 2, method,
+                                       neb_sel_mthd='pie', n_nebs=48,
+                                       n_pies=6)
+            out += [e.cpu().numpy()] + ([] if v is None else [v.cpu().numpy()])
+        return out
+
+    for far, cell in ((1.7e308, (1e9, 1e9)), (1.3e154, (1e9, 1e9)),
+                      (1e9, (1.7e308, np.inf))):
+        want = run(1e9, 2e9, (1e9, 1e9))
+        got = run(far, far * 0.9 if far > 1e9 else 2e9, cell)
+        # (SK's fallback takes the nearest station, another one for far cells)
+        at = np.setdiff1d(np.arange(cells), (9, 11) if method == 'SK' else ())
+        for g, w in zip(got, want):
+            g, w = g[:, at], w[:, at]
+            assert np.isfinite(w).all()
+            np.testing.assert_allclose(g, w, rtol=0,
+                                       atol=1e-9 * np.abs(w).max())
