@@ -197,10 +197,14 @@ __device__ inline double dist_fast(double dx, double dy) {
   return fma(fma(-g, g, s), h, g);
 }
 
-// 2^y for finite y <= 0: the nearest integer goes to the exponent, the rest
-// f (|f| <= 1/2) through a degree-11 Chebyshev interpolant of 2^f (largest
-// relative error 2e-17).  15 instructions, without the range tests of
-// exp(); NaN stays NaN.
+// 2^y for y <= 0: the nearest integer goes to the exponent, the rest f
+// (|f| <= 1/2) through a degree-11 Chebyshev interpolant of 2^f (largest
+// relative error 2e-17), without the range tests of exp(); NaN stays NaN.
+// BOUND: the integer is bounded for its conversion, in one instruction on its
+// upper word, which orders negative numbers by magnitude.  Ordinary input
+// needs it: Exp(0.001) at 1 000 km has y = -4e9.  Without BOUND y has to be
+// above -2^31 and no NaN.
+template <bool BOUND = true>
 __device__ inline double exp2_neg(double y) {
   const double k = rint(y);
   double f;
@@ -222,7 +226,16 @@ __device__ inline double exp2_neg(double y) {
   p = fma(p, f, 0.24022650695910158);
   p = fma(p, f, 0.6931471805599453);
   p = fma(p, f, 1.0);
-  return ldexp(p, (int)k);
+  double kc = k;
+  if (BOUND) {
+    const unsigned long long b = (unsigned long long)__double_as_longlong(k);
+    // [-0, -2^30] and both signs of NaN
+    const unsigned hi =
+        min(max((unsigned)(b >> 32), 0x80000000u), 0xc1d00000u);
+    kc = __longlong_as_double(
+        (long long)(((unsigned long long)hi << 32) | (unsigned)b));
+  }
+  return ldexp(p, (int)kc);
 }
 constexpr double kLog2e = 1.4426950408889634;
 

@@ -727,12 +727,12 @@ __global__ __launch_bounds__(256) void k_de_energy(
     // (the bound keeps a range of zero, -inf, out of exp2_neg)
     const double c = (-3.0 / rg) * kLog2e, top = nug + sl;
     acc = de_sum(h, g, b0, b1, [&](double hb, double gb) {
-      return fma(sl, exp2_neg(fmax(hb * c, -1100.0)), gb - top);
+      return fma(sl, exp2_neg<false>(fmax(hb * c, -1100.0)), gb - top);
     });
   } else if (others == 1 && ty == SPK_VG_GAU) {
     const double c = (-3.0 / (rg * rg)) * kLog2e, top = nug + sl;
     acc = de_sum(h, g, b0, b1, [&](double hb, double gb) {
-      return fma(sl, exp2_neg(fmax((hb * hb) * c, -1100.0)), gb - top);
+      return fma(sl, exp2_neg<false>(fmax((hb * hb) * c, -1100.0)), gb - top);
     });
   } else if (others == 1 && ty == SPK_VG_SPH) {
     const double c = 1.0 / rg;

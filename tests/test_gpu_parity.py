@@ -749,3 +749,25 @@ def test_coordinates_beyond_every_range(gpu, method, vg):
             assert np.isfinite(w).all()
             np.testing.assert_allclose(g, w, rtol=0,
                                        atol=1e-9 * np.abs(w).max())
+
+
+@pytest.mark.parametrize('precision', ['fp64', 'fp64b', 'mixed'])
+def test_ranges_far_below_the_distances(gpu, precision):
+    """Exponents of -4e9 and beyond (a range of 1 mm, and one clamped to 1e-5,
+    at distances up to 1 000 km): the models are at their sill and the
+    estimate is the stations' mean, as the oracle has it."""
+    from spinterps_amd.interp.steps import DeviceProblem, interp_steps
+    rng = np.random.default_rng(3)
+    n = 37
+    sx, sy = rng.uniform(0, 1e6, n), rng.uniform(0, 1e6, n)
+    cx, cy = rng.uniform(0, 1e6, 300), rng.uniform(0, 1e6, 300)
+    vals = rng.gamma(2.0, 3.0, (4, n))
+    vgs = ['2.0 Exp(0.001)', '2.0 Gau(0.001)',
+           '0.5 Nug(0.0) + 2.0 Exp(0.00000001)', '1.0 Exp(0.001) + 1.0 Gau(1.0)']
+    est, var, info = interp_steps(DeviceProblem(sx, sy, cx, cy), vals, vgs,
+                                  'OK', precision=precision)
+    _, ref, _ = O.interp_all(sx, sy, cx, cy, vals, vgs, [('OK', 'OK', None)])
+    assert not (info.cpu().numpy() & (4 | 8 | 16 | 128)).any()
+    np.testing.assert_allclose(est.cpu().numpy(), ref['OK'], rtol=1e-11)
+    np.testing.assert_allclose(var.cpu().numpy(), ref['EST_VARS_OK'],
+                               rtol=1e-11)
