@@ -2155,13 +2155,18 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
             ProfScope ps(ctx, "gemm_plain_f64");
             // k depth per LDS stage 8, 16 or 32 (the same products in the
             // same order); a tuning run takes the first 1 024 cell tiles
-            // of the group's largest system
+            // of the group's largest system, step tstep (-1: every step of
+            // that size is one the kernel skips, and nothing is timed)
+            int tstep = -1;
+            for (int s = s0; s < s0 + ns; ++s)
+              if (h_sc[s].n == nm &&
+                  (h_sc[s].status == 0 || h_sc[s].status == SPK_ST_FAILED))
+                tstep = s;
             auto run = [&](int v, bool timing) -> int {
               int s1 = s0, n1 = ns;
               int64_t cr = cn;
               if (timing) {
-                for (int s = s0; s < s0 + ns; ++s)
-                  if (h_sc[s].n == nm) s1 = s;
+                s1 = tstep;
                 n1 = 1;
                 cr = std::min<int64_t>(cn, 1024 * 128);
               }
@@ -2178,12 +2183,7 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
                   (const int *)nullptr);
               return check_launch("k_plain_gemm");
             };
-            // a group without a system to contract is not timed
-            bool any = false;
-            for (int s = s0; s < s0 + ns; ++s)
-              any = any || (h_sc[s].n == nm && (h_sc[s].status == 0 ||
-                                                h_sc[s].status == SPK_ST_FAILED));
-            if (any)
+            if (tstep >= 0)
               SPK_TRY(tune_launch(ctx, "gemm_plain_f64",
                                   (int)ceil_div(nm + p, 1024), sm, 3, 0, run));
             else

@@ -96,3 +96,34 @@ def test_tuning_arguments_checked(gpu):
         ctx.force_variant('gemm_plain_f64', 3)
     with pytest.raises(AssertionError):
         _lib.check(_lib.lib().spk_ctx_set_tuning(ctx.h, 7))
+
+
+def test_tuning_times_a_step_with_a_system(gpu):
+    """Of the steps with the most stations the one that is timed has a
+    system: with the last of them below the threshold (mean-filled, no
+    kernel runs), the times are those of the same call without it."""
+    from spinterps_amd import _lib
+    from spinterps_amd.interp.steps import DeviceProblem
+    rng = np.random.default_rng(2)
+    n = 1000
+    g = np.linspace(0, 1e5, 300)
+    gx, gy = np.meshgrid(g, g)
+    prob = DeviceProblem(*rng.uniform(0, 1e5, (2, n)), gx.ravel(), gy.ravel())
+    vals = rng.gamma(2.0, 5.0, (2, n))
+    vgs = ['0.5 Nug(0.0) + 9.0 Exp(30000.0)'] * 2
+    fill = vals.copy()
+    fill[1] *= 1e-3
+    own, ms = _lib._ctxs.get(0), []
+    try:
+        for v in (vals, fill):
+            _lib._ctxs[0] = _lib.Context(0)
+            from spinterps_amd.interp.steps import interp_steps
+            interp_steps(prob, v, vgs, 'OK', min_var_thr=1.0)
+            ms.append([r[3] for r in _lib._ctxs[0].tuning_report()
+                       if r[0] == 'gemm_plain_f64'])
+    finally:
+        _lib._ctxs[0] = own
+        if own is None:
+            del _lib._ctxs[0]
+    # 1.5 ms and more each; empty launches take a few microseconds
+    assert min(ms[1][0]) > 0.5 * min(ms[0][0]), ms
