@@ -208,6 +208,14 @@ def test_idw_block_shapes(gpu, steps, side, p):
             got[t][at], ref, rtol=(2 * N + 8 * p + 40) * 2.0 ** -53)
 
 
+@pytest.mark.parametrize('steps,side', [(64, 31), (70, 31), (129, 5)])
+def test_idw_many_steps_few_cells(gpu, steps, side):
+    """More steps than a block of 64 on a grid that leaves the device idle:
+    one launch."""
+    for p in (2.0, 2.3):
+        test_idw_block_shapes(gpu, steps, side, p)
+
+
 @pytest.mark.parametrize('precision', ['fp64', 'fp64b', 'mixed'])
 def test_ok_small_all_precisions(gpu, precision):
     from spinterps_amd.interp.steps import DeviceProblem, interp_steps
