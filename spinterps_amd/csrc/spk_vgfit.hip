@@ -70,7 +70,8 @@ __global__ void k_pair_unpack(const unsigned long long *__restrict__ key,
 // exclusive scan, then the list; the distance clip and the bins follow.
 // One workgroup per step that walked all pairs by itself took 7.2 ms for 24
 // steps of 1 500 stations (1.1 million pairs), bound by its serial chain of
-// loads; this split takes 0.56 ms.
+// loads; this split takes 0.56 ms.  Steps of few pairs take all passes in one
+// workgroup (k_evg_small).
 constexpr int kEvgChunk = 4096;
 
 // Active pairs of one chunk: bit u of the result is set when pair
@@ -127,17 +128,15 @@ __global__ __launch_bounds__(256) void k_evg_scan(int64_t *__restrict__ cnt,
   if (threadIdx.x == 0) act[blockIdx.x] = base;
 }
 
-// grid (chunks, steps): the active pairs in their order.
-__global__ __launch_bounds__(256) void k_evg_list(
-    const int32_t *__restrict__ pi, const int32_t *__restrict__ pj, int64_t M,
-    const double *__restrict__ vals, int64_t N,
-    const int64_t *__restrict__ cnt, int32_t *__restrict__ list) {
+// The chunk's active pairs in their order, from list[base] on, by the
+// workgroup; returns how many.
+__device__ inline int evg_list(const int32_t *pi, const int32_t *pj,
+                               const double *z, int64_t b0, int64_t M,
+                               int64_t base, int32_t *L) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-  const int64_t b0 = (int64_t)blockIdx.x * kEvgChunk;
-  const unsigned m =
-      evg_active(pi, pj, vals + (int64_t)blockIdx.y * N, b0, M);
-  int32_t *L = list + (int64_t)blockIdx.y * M;
+  const unsigned m = evg_active(pi, pj, z, b0, M);
   __shared__ int wcnt[kEvgChunk / 64];  // active pairs per run of 64
+  __shared__ int total;
 #pragma unroll
   for (int u = 0; u < kEvgChunk / 256; ++u) {
     const unsigned long long bm = __ballot((m >> u) & 1u);
@@ -152,10 +151,9 @@ __global__ __launch_bounds__(256) void k_evg_list(
       if (lane >= w) x += o;
     }
     wcnt[lane] = x - v;
+    if (lane == 63) total = x;
   }
   __syncthreads();
-  const int64_t base =
-      cnt[(int64_t)blockIdx.y * gridDim.x + blockIdx.x];
 #pragma unroll
   for (int u = 0; u < kEvgChunk / 256; ++u) {
     const bool act = (m >> u) & 1u;
@@ -164,6 +162,18 @@ __global__ __launch_bounds__(256) void k_evg_list(
       L[base + wcnt[u * 4 + wave] + __popcll(bm & ((1ull << lane) - 1ull))] =
           (int32_t)(b0 + threadIdx.x + 256 * u);
   }
+  return total;
+}
+
+// grid (chunks, steps)
+__global__ __launch_bounds__(256) void k_evg_list(
+    const int32_t *__restrict__ pi, const int32_t *__restrict__ pj, int64_t M,
+    const double *__restrict__ vals, int64_t N,
+    const int64_t *__restrict__ cnt, int32_t *__restrict__ list) {
+  evg_list(pi, pj, vals + (int64_t)blockIdx.y * N,
+           (int64_t)blockIdx.x * kEvgChunk, M,
+           cnt[(int64_t)blockIdx.y * gridDim.x + blockIdx.x],
+           list + (int64_t)blockIdx.y * M);
 }
 
 // First position p in [0, hi) of a step's ascending active distances with
@@ -197,95 +207,136 @@ __device__ inline int64_t evg_first(const double *pd, const int32_t *L,
   return lo;
 }
 
-// One wave per step: the distance clip (vgs.py:597-659), argmin
-// |d - mdr max| (first occurrence) over the sorted active distances, and
-// the number of bins.  keep[step]: pairs kept.
+// The distance clip (vgs.py:597-659) of a step with `base` active pairs:
+// argmin |d - mdr max| (first occurrence) over their sorted distances.  Run
+// by one wave; every lane returns the pairs kept.
+__device__ inline int64_t evg_clip(const double *pd, const int32_t *L,
+                                   int64_t base, double mdr) {
+  if (base <= 0) return base;
+  const double act_max = pd[L[base - 1]];
+  const double md = act_max * mdr;
+  const int64_t lo = evg_first(pd, L, base, md, true);
+  int64_t idx;
+  if (lo == 0) {
+    idx = 0;
+  } else if (lo == base) {
+    idx = base - 1;
+  } else {
+    const double da = md - pd[L[lo - 1]], db = pd[L[lo]] - md;
+    idx = (da <= db) ? lo - 1 : lo;
+  }
+  // first occurrence of that distance value
+  idx = evg_first(pd, L, idx, pd[L[idx]], false);
+  double clip_ul = pd[L[idx]];
+  if (!(clip_ul - md > 0)) clip_ul = md;
+  // keep d < clip_ul
+  return idx != base - 1 ? evg_first(pd, L, base, clip_ul, false) : base;
+}
+__device__ inline int evg_nbins(int64_t keep, int nk, int max_bins) {
+  return (int)min((keep + nk - 1) / nk, (int64_t)max_bins);
+}
+
+// One wave per step.  keep[step]: pairs kept.
 __global__ __launch_bounds__(64) void k_evg_clip(
     const double *__restrict__ pd, int64_t M, double mdr, int nk,
     int max_bins, const int32_t *__restrict__ list,
     const int64_t *__restrict__ act, int64_t *__restrict__ keep_out,
     int32_t *__restrict__ nbins) {
   const int s = blockIdx.x;
-  const int32_t *L = list + (int64_t)s * M;
-  const int64_t base = act[s];
-  int64_t keep = base;
-  if (base > 0) {
-    const double act_max = pd[L[base - 1]];
-    const double md = act_max * mdr;
-    const int64_t lo = evg_first(pd, L, base, md, true);
-    int64_t idx;
-    if (lo == 0) {
-      idx = 0;
-    } else if (lo == base) {
-      idx = base - 1;
-    } else {
-      const double da = md - pd[L[lo - 1]], db = pd[L[lo]] - md;
-      idx = (da <= db) ? lo - 1 : lo;
-    }
-    // first occurrence of that distance value
-    idx = evg_first(pd, L, idx, pd[L[idx]], false);
-    double clip_ul = pd[L[idx]];
-    if (!(clip_ul - md > 0)) clip_ul = md;
-    // keep d < clip_ul
-    if (idx != base - 1) keep = evg_first(pd, L, base, clip_ul, false);
-  }
+  const int64_t keep = evg_clip(pd, list + (int64_t)s * M, act[s], mdr);
   if (threadIdx.x == 0) {
     keep_out[s] = keep;
-    nbins[s] = (int)min((keep + nk - 1) / nk, (int64_t)max_bins);
+    nbins[s] = evg_nbins(keep, nk, max_bins);
   }
 }
 
-// grid (ceil(max bins / 256), steps): one thread per bin, its pairs summed
-// in their order.
+// Bin b of a step with `keep` kept pairs, summed in their order by one thread.
+__device__ inline void evg_bin(const int32_t *pi, const int32_t *pj,
+                               const double *pd, const double *z,
+                               const int32_t *L, int64_t keep, int nk,
+                               int classic, int b, double *bh, double *bg,
+                               int32_t *bn) {
+  const int64_t p0 = (int64_t)b * nk;
+  const int cntb = (int)min((int64_t)nk, keep - p0);
+  double sd = 0.0, sr = 0.0;
+  for (int q = 0; q < cntb; ++q) {
+    const int32_t e = L[p0 + q];
+    sd += pd[e];
+    sr += sqrt(fabs(z[pi[e]] - z[pj[e]]));
+  }
+  double g;
+  if (!classic) {
+    // vgs.py:414-422
+    const double t = sr / cntb;
+    const double t4 = (t * t) * (t * t);
+    g = (t4 / (0.457 + (0.494 / cntb))) / 2.0;
+  } else {
+    // vgs.py:399-412: median of squared differences (insertion sort)
+    double v[64];
+    const int c2 = cntb < 64 ? cntb : 64;
+    for (int q = 0; q < c2; ++q) {
+      const int32_t e = L[p0 + q];
+      const double dz = z[pi[e]] - z[pj[e]];
+      double key = dz * dz;
+      int w2 = q - 1;
+      while (w2 >= 0 && v[w2] > key) {
+        v[w2 + 1] = v[w2];
+        --w2;
+      }
+      v[w2 + 1] = key;
+    }
+    g = (c2 & 1) ? v[c2 / 2] : 0.5 * (v[c2 / 2 - 1] + v[c2 / 2]);
+  }
+  bh[b] = sd / cntb;
+  bg[b] = g;
+  bn[b] = cntb;
+}
+
+// grid (ceil(max bins / 256), steps)
 __global__ __launch_bounds__(256) void k_evg_bins(
     const int32_t *__restrict__ pi, const int32_t *__restrict__ pj,
     const double *__restrict__ pd, int64_t M, const double *__restrict__ vals,
     int64_t N, int nk, int classic, int max_bins,
-    const int32_t *__restrict__ list, const int64_t *__restrict__ keep_in,
+    const int32_t *__restrict__ list, const int64_t *__restrict__ keep,
     const int32_t *__restrict__ nbins, double *__restrict__ bh,
     double *__restrict__ bg, int32_t *__restrict__ bn) {
   const int s = blockIdx.y;
-  const double *z = vals + (int64_t)s * N;
-  const int32_t *L = list + (int64_t)s * M;
-  const int64_t keep = keep_in[s];
-  const int nb = nbins[s];
   const int b = blockIdx.x * 256 + threadIdx.x;
-  if (b < nb) {
-    const int64_t p0 = (int64_t)b * nk;
-    const int cntb = (int)min((int64_t)nk, keep - p0);
-    double sd = 0.0, sr = 0.0;
-    for (int q = 0; q < cntb; ++q) {
-      const int32_t e = L[p0 + q];
-      sd += pd[e];
-      sr += sqrt(fabs(z[pi[e]] - z[pj[e]]));
-    }
-    double g;
-    if (!classic) {
-      // vgs.py:414-422
-      const double t = sr / cntb;
-      const double t4 = (t * t) * (t * t);
-      g = (t4 / (0.457 + (0.494 / cntb))) / 2.0;
-    } else {
-      // vgs.py:399-412: median of squared differences (insertion sort)
-      double v[64];
-      const int c2 = cntb < 64 ? cntb : 64;
-      for (int q = 0; q < c2; ++q) {
-        const int32_t e = L[p0 + q];
-        const double dz = z[pi[e]] - z[pj[e]];
-        double key = dz * dz;
-        int w2 = q - 1;
-        while (w2 >= 0 && v[w2] > key) {
-          v[w2 + 1] = v[w2];
-          --w2;
-        }
-        v[w2 + 1] = key;
-      }
-      g = (c2 & 1) ? v[c2 / 2] : 0.5 * (v[c2 / 2 - 1] + v[c2 / 2]);
-    }
-    bh[(int64_t)s * max_bins + b] = sd / cntb;
-    bg[(int64_t)s * max_bins + b] = g;
-    bn[(int64_t)s * max_bins + b] = cntb;
+  const int64_t o = (int64_t)s * max_bins;
+  if (b < nbins[s])
+    evg_bin(pi, pj, pd, vals + (int64_t)s * N, list + (int64_t)s * M, keep[s],
+            nk, classic, b, bh + o, bg + o, bn + o);
+}
+
+// All passes of a step in one workgroup, for few pairs (kEvgSmall chunks): a
+// step's passes are then shorter than their launches.  grid (steps)
+constexpr int kEvgSmall = 4;
+__global__ __launch_bounds__(256) void k_evg_small(
+    const int32_t *pi, const int32_t *pj, const double *pd, int64_t M,
+    const double *vals, int64_t N, double mdr, int nk, int classic,
+    int max_bins, int32_t *list, double *bh, double *bg, int32_t *bn,
+    int32_t *nbins) {
+  const int s = blockIdx.x;
+  const double *z = vals + (int64_t)s * N;
+  int32_t *L = list + (int64_t)s * M;
+  __shared__ int64_t keep_s;
+  int64_t base = 0;
+  for (int64_t b0 = 0; b0 < M; b0 += kEvgChunk) {
+    base += evg_list(pi, pj, z, b0, M, base, L);
+    __syncthreads();  // the chunk's counts are read, its list is written
   }
+  if (threadIdx.x < 64) {
+    const int64_t keep = evg_clip(pd, L, base, mdr);
+    if (threadIdx.x == 0) {
+      keep_s = keep;
+      nbins[s] = evg_nbins(keep, nk, max_bins);
+    }
+  }
+  __syncthreads();
+  const int64_t keep = keep_s, o = (int64_t)s * max_bins;
+  const int nb = evg_nbins(keep, nk, max_bins);
+  for (int b = threadIdx.x; b < nb; b += 256)
+    evg_bin(pi, pj, pd, z, L, keep, nk, classic, b, bh + o, bg + o, bn + o);
 }
 
 // ---- differential evolution ----------------------------------------------------
@@ -1108,6 +1159,14 @@ int spk_vgfit_evg_dev(spk_ctx *ctx, const int32_t *pi, const int32_t *pj,
   for (int64_t t0 = 0; t0 < T; t0 += S) {
     const int Sb = (int)std::min<int64_t>(S, T - t0);
     const double *v = vals + t0 * N;
+    if (nch <= kEvgSmall) {
+      hipLaunchKernelGGL(k_evg_small, dim3(Sb), dim3(256), 0, ctx->stream, pi,
+                         pj, pd, M, v, N, mdr, nk, classic, max_bins, list,
+                         bin_h + t0 * max_bins, bin_g + t0 * max_bins,
+                         bin_n + t0 * max_bins, nbins + t0);
+      SPK_TRY(check_launch("k_evg"));
+      continue;
+    }
     hipLaunchKernelGGL(k_evg_count, dim3(nch, Sb), dim3(256), 0, ctx->stream,
                        pi, pj, M, v, N, cnt);
     hipLaunchKernelGGL(k_evg_scan, dim3(Sb), dim3(256), 0, ctx->stream, cnt,

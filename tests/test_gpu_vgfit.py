@@ -259,3 +259,30 @@ def test_de_captured_matches_eager(gpu):
         np.testing.assert_array_equal(nit2.cpu().numpy(), nit.cpu().numpy())
         np.testing.assert_allclose(fun2.cpu().numpy(), fun.cpu().numpy(),
                                    rtol=1e-11)
+
+
+@pytest.mark.parametrize('evg', ['robust', 'classic'])
+@pytest.mark.parametrize('n', [2, 24, 91, 92, 181, 182])
+def test_bins_few_pairs(gpu, n, evg):
+    """Steps whose passes run in one workgroup (up to 4 chunks of 4 096
+    pairs: 181 stations) and beyond, with missing values and a step without
+    any, against the oracle."""
+    from spinterps_amd.variograms.fitvgs import BatchVariogramFitter
+    rng = np.random.default_rng(n)
+    x, y = rng.uniform(0, 2e5, n), rng.uniform(0, 2e5, n)
+    vals = rng.gamma(2.0, 3.0, (3, n))
+    vals[1, rng.choice(n, n // 3, replace=False)] = np.nan
+    vals[2] = np.nan
+    f = BatchVariogramFitter(x, y)
+    bh, bg, bn, nb = (a.cpu().numpy() for a in f.empirical(vals, 0.5, 50, evg))
+    assert nb[2] == 0
+    for t in (0, 1):
+        ok = ~np.isnan(vals[t])
+        if ok.sum() < 2:
+            continue
+        ref = V.empirical(x[ok], y[ok], vals[t][ok], 0.5, 50, evg)
+        k = nb[t]
+        assert k == len(ref)
+        np.testing.assert_array_equal(bn[t, :k], ref[:, 2])
+        np.testing.assert_allclose(bh[t, :k], ref[:, 0], rtol=1e-12)
+        np.testing.assert_allclose(bg[t, :k], ref[:, 1], rtol=1e-12)
