@@ -410,23 +410,119 @@ __device__ inline void set_own(double (&a)[kDeOwn], int k, double v) {
     if (j == k) a[j] = v;
 }
 
-__device__ double de_energy(const double *x, const double *lb,
-                            const double *ub, const int *types, int ncomp,
-                            const double *h, const double *g, int nb) {
-  // the parameters are formed where they are used: an array of them,
-  // indexed by the component, would live in scratch memory
+// The parts of an energy's sum: max(64, ceil(bins / 16)) bins each.
+constexpr int kDeSplit = 16;
+constexpr int kDeMinBins = 64;
+
+__host__ __device__ inline int de_part_bins(int nb) {
+  const int l = (nb + kDeSplit - 1) / kDeSplit;
+  return l < kDeMinBins ? kDeMinBins : l;
+}
+
+// Bounds of component c's (range, sill) of candidate cd (vgs.py:735-757).
+__device__ inline void de_bounds(const int32_t *cd, int c, double h0,
+                                 double g0, double v, double range_ub,
+                                 double *lb, double *ub) {
+  if (cd[1 + c] == SPK_VG_POW) {
+    lb[0] = 1e-5;
+    ub[0] = 2.0;
+    lb[1] = 1e-5;
+    ub[1] = 2.0 * v;
+  } else if (cd[5] && c == 0) {
+    lb[0] = ub[0] = h0;
+    lb[1] = ub[1] = g0;
+  } else {
+    lb[0] = h0;
+    ub[0] = range_ub;
+    lb[1] = 1e-5;
+    ub[1] = 2.0 * v;
+  }
+}
+
+// sum over bins [b0, b1) of the squares of res(h, g)
+template <typename F>
+__device__ inline double de_sum(const double *__restrict__ h,
+                                const double *__restrict__ g, int b0, int b1,
+                                F res) {
   double acc = 0.0;
-  for (int b = 0; b < nb; ++b) {
-    const double hb = h[b];
-    double v = 0.0;
-    for (int c = 0; c < ncomp; ++c) {
-      const int d = 2 * c;
-      const double rg = lb[d] + x[d] * (ub[d] - lb[d]);
-      const double sl = lb[d + 1] + x[d + 1] * (ub[d + 1] - lb[d + 1]);
-      v += fit_model(types[c], hb, rg, sl);
+#pragma unroll 4
+  for (int b = b0; b < b1; ++b) {
+    const double d = res(h[b], g[b]);
+    acc = fma(d, d, acc);
+  }
+  return acc;
+}
+
+// The components of a candidate: `others` besides the constant ones (nuggets),
+// of which component `one` (of model ty) if it is the only one.
+struct DeCand {
+  int n, one, others, ty;
+};
+__device__ inline DeCand de_cand(const int32_t *cd) {
+  DeCand q = {cd[0], -1, 0, SPK_VG_NUG};
+  for (int c = 0; c < q.n; ++c)
+    if (cd[1 + c] != SPK_VG_NUG) {
+      q.one = c;
+      q.ty = cd[1 + c];
+      ++q.others;
     }
-    const double r = g[b] - v;
-    acc += r * r;
+  return q;
+}
+
+// An energy's share of bins [b0, b1) of a step whose bins are h and g: the
+// squared residuals (vgs.py:661-678) of member x between lb and ub (de_bounds,
+// in LDS).  Both evolutions below add the same parts in the same order, so that
+// a step's result does not depend on which of them takes it.  The model's value
+// is rounded before it is subtracted: a step of one bin converges when every
+// member meets it to the last bit (about 250 generations; with the residual
+// formed in one operation it never did, and took 10 000).
+__device__ inline double de_part(const DeCand &dc, const int32_t *cd,
+                                 const double *x,
+                                 const double *lb, const double *ub,
+                                 const double *__restrict__ h,
+                                 const double *__restrict__ g, int b0, int b1) {
+#pragma clang fp contract(off)
+  const int ncomp = dc.n, one = dc.one, others = dc.others, ty = dc.ty;
+  double acc;
+  double nug = 0.0, rg = 1.0, sl = 0.0;
+  auto par = [&](int d) { return fma(x[d], ub[d] - lb[d], lb[d]); };
+  for (int c = 0; c < ncomp; ++c) {
+    if (cd[1 + c] == SPK_VG_NUG) {
+      nug += par(2 * c + 1);
+    } else if (c == one) {
+      rg = par(2 * c);
+      sl = par(2 * c + 1);
+    }
+  }
+  if (others == 0) {
+    acc = de_sum(h, g, b0, b1, [&](double, double gb) { return gb - nug; });
+  } else if (others == 1 && ty == SPK_VG_EXP) {
+    // (the bound keeps a range of zero, -inf, out of exp2_neg)
+    const double c = (-3.0 / rg) * kLog2e, top = nug + sl;
+    acc = de_sum(h, g, b0, b1, [&](double hb, double gb) {
+      return gb - fma(-sl, exp2_neg<false>(fmax(hb * c, -1100.0)), top);
+    });
+  } else if (others == 1 && ty == SPK_VG_GAU) {
+    const double c = (-3.0 / (rg * rg)) * kLog2e, top = nug + sl;
+    acc = de_sum(h, g, b0, b1, [&](double hb, double gb) {
+      return gb - fma(-sl, exp2_neg<false>(fmax((hb * hb) * c, -1100.0)), top);
+    });
+  } else if (others == 1 && ty == SPK_VG_SPH) {
+    const double c = 1.0 / rg;
+    acc = de_sum(h, g, b0, b1, [&](double hb, double gb) {
+      const double u = fmin(hb * c, 1.0);  // the sill at h >= r
+      return gb - fma(sl, u * fma(u * u, -0.5, 1.5), nug);
+    });
+  } else {
+    acc = 0.0;
+    for (int b = b0; b < b1; ++b) {
+      const double hb = h[b];
+      double y = 0.0;
+      for (int c = 0; c < ncomp; ++c)
+        y += fit_model(cd[1 + c], hb, par(2 * c), par(2 * c + 1));
+      const double r = g[b] - y;
+      acc = fma(r, r, acc);
+    }
   }
   return acc;
 }
@@ -497,7 +593,7 @@ __device__ inline int blk_argmin(const double (&en)[kDeOwn], int P,
 // One workgroup per (step, candidate).  cand[c]: {ncomp, type[4],
 // fixed_first}; with fixed_first the first component's (range, sill) are
 // pinned to the step's first bin (h0, g0), vgs.py:735-739.
-__global__ __launch_bounds__(256) void k_de(
+__global__ __launch_bounds__(256, 3) void k_de(
     const double *__restrict__ bh, const double *__restrict__ bg,
     const int32_t *__restrict__ nbins, int max_bins,
     const double *__restrict__ var, const int32_t *__restrict__ cand,
@@ -522,7 +618,6 @@ __global__ __launch_bounds__(256) void k_de(
   double *trial = pop + (int64_t)pcap * ds;
   int *perm = (int *)trial;  // start only, before the first trial
   __shared__ double lb[kDeMaxD], ub[kDeMaxD];
-  __shared__ int types[4];
   __shared__ double red[4];
   __shared__ double redv[4];
   __shared__ int redi[4];
@@ -537,26 +632,9 @@ __global__ __launch_bounds__(256) void k_de(
     }
     return;
   }
-  if (tid == 0) {
-    const double v = var[s];
-    for (int c = 0; c < ncomp; ++c) {
-      types[c] = cd[1 + c];
-      if (types[c] == SPK_VG_POW) {
-        lb[2 * c] = 1e-5;
-        ub[2 * c] = 2.0;
-        lb[2 * c + 1] = 1e-5;
-        ub[2 * c + 1] = 2.0 * v;
-      } else if (cd[5] && c == 0) {
-        lb[0] = ub[0] = h[0];
-        lb[1] = ub[1] = g[0];
-      } else {
-        lb[2 * c] = h[0];
-        ub[2 * c] = range_ub;
-        lb[2 * c + 1] = 1e-5;
-        ub[2 * c + 1] = 2.0 * v;
-      }
-    }
-  }
+  if (tid == 0)
+    for (int c = 0; c < ncomp; ++c)
+      de_bounds(cd, c, h[0], g[0], var[s], range_ub, lb + 2 * c, ub + 2 * c);
   Rng rng(mix64(seed ^ mix64(((unsigned long long)s << 20) ^
                              ((unsigned long long)ci << 8) ^ tid)));
   __syncthreads();
@@ -596,12 +674,20 @@ __global__ __launch_bounds__(256) void k_de(
     }
     __syncthreads();
   }
+  const int len = de_part_bins(nb);
+  const DeCand dc = de_cand(cd);
+  auto energy = [&](const double *x) {
+    double e = 0.0;
+    for (int b0 = 0; b0 < nb; b0 += len)
+      e += de_part(dc, cd, x, lb, ub, h, g, b0, min(nb, b0 + len));
+    return e;
+  };
   double en[kDeOwn], trial_e[kDeOwn];
 #pragma unroll
   for (int k = 0; k < kDeOwn; ++k) en[k] = trial_e[k] = 0.0;
   for (int k = 0; tid + 256 * k < P; ++k) {
     const int i = tid + 256 * k;
-    set_own(en, k, de_energy(&pop[i * ds], lb, ub, types, ncomp, h, g, nb));
+    set_own(en, k, energy(&pop[i * ds]));
   }
   __syncthreads();
   int nit = 0;
@@ -629,7 +715,7 @@ __global__ __launch_bounds__(256) void k_de(
         }
         tr[d] = v;
       }
-      set_own(trial_e, k, de_energy(tr, lb, ub, types, ncomp, h, g, nb));
+      set_own(trial_e, k, energy(tr));
     }
     __syncthreads();
 #pragma unroll
@@ -682,47 +768,6 @@ __global__ __launch_bounds__(256) void k_de(
 // per generation of the day's 430 million model values.  The random streams, the order of the draws and the
 // selection are k_de's; an energy's sum over bins is taken in kDeSplit
 // parts, whose bounds depend on the step's bins only.
-constexpr int kDeSplit = 16;
-constexpr int kDeMinBins = 64;
-
-__host__ __device__ inline int de_part_bins(int nb) {
-  const int l = (nb + kDeSplit - 1) / kDeSplit;
-  return l < kDeMinBins ? kDeMinBins : l;
-}
-
-// Bounds of component c's (range, sill) of candidate cd (vgs.py:735-757).
-__device__ inline void de_bounds(const int32_t *cd, int c, double h0,
-                                 double g0, double v, double range_ub,
-                                 double *lb, double *ub) {
-  if (cd[1 + c] == SPK_VG_POW) {
-    lb[0] = 1e-5;
-    ub[0] = 2.0;
-    lb[1] = 1e-5;
-    ub[1] = 2.0 * v;
-  } else if (cd[5] && c == 0) {
-    lb[0] = ub[0] = h0;
-    lb[1] = ub[1] = g0;
-  } else {
-    lb[0] = h0;
-    ub[0] = range_ub;
-    lb[1] = 1e-5;
-    ub[1] = 2.0 * v;
-  }
-}
-
-// sum over bins [b0, b1) of (g - c - s f(h))^2, f per model
-template <typename F>
-__device__ inline double de_sum(const double *__restrict__ h,
-                                const double *__restrict__ g, int b0, int b1,
-                                F res) {
-  double acc = 0.0;
-#pragma unroll 4
-  for (int b = b0; b < b1; ++b) {
-    const double d = res(h[b], g[b]);
-    acc = fma(d, d, acc);
-  }
-  return acc;
-}
 
 // One wave: 64 members of one candidate over one chunk of its step's bins.
 // grid (waves / 4, candidates); q = step * ncand + candidate within the
@@ -738,8 +783,15 @@ __global__ __launch_bounds__(256) void k_de_energy(
   if (done[q]) return;
   const int s = q / ncand, ci = q - s * ncand;
   const int32_t *cd = cand + ci * 6;
-  const int ncomp = cd[0], P = de_pop(popmul, 2 * ncomp);
+  const int P = de_pop(popmul, 2 * cd[0]);
   const int nb = nbins[s];
+  const double *h = bh + (int64_t)s * max_bins;
+  const double *g = bg + (int64_t)s * max_bins;
+  __shared__ double lb[kDeMaxD], ub[kDeMaxD];
+  if ((int)threadIdx.x < cd[0])
+    de_bounds(cd, threadIdx.x, h[0], g[0], var[s], range_ub,
+              lb + 2 * threadIdx.x, ub + 2 * threadIdx.x);
+  __syncthreads();
   const int mgs = (P + 63) / 64;
   const int wv = __builtin_amdgcn_readfirstlane(
       (int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
@@ -747,65 +799,9 @@ __global__ __launch_bounds__(256) void k_de_energy(
   const int len = de_part_bins(nb);
   const int b0 = ch * len, b1 = min(nb, b0 + len);
   if (ch >= kDeSplit || b0 >= b1) return;
-  const double *h = bh + (int64_t)s * max_bins;
-  const double *g = bg + (int64_t)s * max_bins;
   const int i = mg * 64 + (int)(threadIdx.x & 63);
   const double *x = mem + ((int64_t)q * pcap + min(i, P - 1)) * ds;
-  double acc;
-  // the constant (nugget) components and the one other component
-  int one = -1, others = 0;
-  for (int c = 0; c < ncomp; ++c)
-    if (cd[1 + c] != SPK_VG_NUG) {
-      one = c;
-      ++others;
-    }
-  const int ty = one >= 0 ? cd[1 + one] : SPK_VG_NUG;
-  double nug = 0.0, rg = 1.0, sl = 0.0;
-  for (int c = 0; c < ncomp; ++c) {
-    double lb[2], ub[2];
-    de_bounds(cd, c, h[0], g[0], var[s], range_ub, lb, ub);
-    const double cs = lb[1] + x[2 * c + 1] * (ub[1] - lb[1]);
-    if (cd[1 + c] == SPK_VG_NUG) {
-      nug += cs;
-    } else if (c == one) {
-      rg = lb[0] + x[2 * c] * (ub[0] - lb[0]);
-      sl = cs;
-    }
-  }
-  if (others == 0) {
-    acc = de_sum(h, g, b0, b1, [&](double, double gb) { return gb - nug; });
-  } else if (others == 1 && ty == SPK_VG_EXP) {
-    // (the bound keeps a range of zero, -inf, out of exp2_neg)
-    const double c = (-3.0 / rg) * kLog2e, top = nug + sl;
-    acc = de_sum(h, g, b0, b1, [&](double hb, double gb) {
-      return fma(sl, exp2_neg<false>(fmax(hb * c, -1100.0)), gb - top);
-    });
-  } else if (others == 1 && ty == SPK_VG_GAU) {
-    const double c = (-3.0 / (rg * rg)) * kLog2e, top = nug + sl;
-    acc = de_sum(h, g, b0, b1, [&](double hb, double gb) {
-      return fma(sl, exp2_neg<false>(fmax((hb * hb) * c, -1100.0)), gb - top);
-    });
-  } else if (others == 1 && ty == SPK_VG_SPH) {
-    const double c = 1.0 / rg;
-    acc = de_sum(h, g, b0, b1, [&](double hb, double gb) {
-      const double u = fmin(hb * c, 1.0);  // the sill at h >= r
-      return fma(-sl, u * fma(u * u, -0.5, 1.5), gb - nug);
-    });
-  } else {
-    acc = 0.0;
-    for (int b = b0; b < b1; ++b) {
-      const double hb = h[b];
-      double v = 0.0;
-      for (int c = 0; c < ncomp; ++c) {
-        double lb[2], ub[2];
-        de_bounds(cd, c, h[0], g[0], var[s], range_ub, lb, ub);
-        v += fit_model(cd[1 + c], hb, lb[0] + x[2 * c] * (ub[0] - lb[0]),
-                       lb[1] + x[2 * c + 1] * (ub[1] - lb[1]));
-      }
-      const double r = g[b] - v;
-      acc += r * r;
-    }
-  }
+  const double acc = de_part(de_cand(cd), cd, x, lb, ub, h, g, b0, b1);
   if (i < P) part[((int64_t)q * kDeSplit + ch) * pcap + i] = acc;
 }
 
@@ -1305,13 +1301,39 @@ static int de_launch(spk_ctx *ctx, const double *bin_h, const double *bin_g,
     ds = std::max(ds, D);
     pcap = std::max(pcap, de_pop(popmul, D));
   }
-  if (!stream_capturing(ctx->stream))
-    return de_device(ctx, bin_h, bin_g, nbins, max_bins, var, T, dc, n_cands,
-                     maxiter, popmul, tol, range_ub, seed, init, spread, pcap,
-                     ds, params, fun, nit);
-  // captured launches cannot be followed by host reads: one workgroup per
-  // (step, candidate) evolves by itself
+  // Few bins: one workgroup per (step, candidate) evolves it by itself.  A
+  // generation then takes 5 us and, per bin, component and 256 members, 0.05 us
+  // (eight times that for pow and sin); over the whole device it takes 20 to
+  // 50 us for its launches and the host's look, and 0.03 to 0.1 us per pair.
+  // The line is the best fit to 184 calls of 1 to 600 bins and 2 to 22 000
+  // pairs.  One step x 7 candidates of Sph, Exp and Gau, ms by the one and the
+  // other: 12 stations (1 bin) 1.1 and 5.4, 60 (21 bins) 0.90 and 1.31, 130
+  // (120 bins) 2.4 and 1.7; 200 steps: 2.6 and 17, 2.0 and 4.4, 5.2 and 6.2.
+  // Both give the same bits.  Captured launches cannot be followed by host
+  // reads and take the first form.
   const size_t lds = de_lds_bytes(pcap, ds);
+  const int64_t pairs = T * n_cands;
+  int64_t work = 0;  // of the slowest candidate, per bin
+  for (int c = 0; c < n_cands; ++c) {
+    const int32_t *cd = cands + c * 6;
+    int64_t w = 0;
+    for (int k = 0; k < cd[0]; ++k)
+      w += cd[1 + k] == SPK_VG_POW || cd[1 + k] == SPK_VG_HOL ? 8 : 1;
+    work = std::max(work, w * ceil_div(de_pop(popmul, 2 * cd[0]), 256));
+  }
+  auto few = [&](int64_t nb) { return nb * work <= 500 + pairs / 3; };
+  if (!stream_capturing(ctx->stream) && !few(max_bins)) {
+    std::vector<int32_t> h_nb(T);
+    SPK_TRY(d2h(ctx, h_nb.data(), nbins, (size_t)T * 4));
+    if (!few(*std::max_element(h_nb.begin(), h_nb.end()))) {
+      const int rc = de_device(ctx, bin_h, bin_g, nbins, max_bins, var, T, dc,
+                               n_cands, maxiter, popmul, tol, range_ub, seed,
+                               init, spread, pcap, ds, params, fun, nit);
+      // without the memory for its populations, the form that needs none
+      if (rc != SPK_ENOMEM) return rc;
+      (void)hipGetLastError();
+    }
+  }
   if (lds > 64 * 1024)
     SPK_HIP(hipFuncSetAttribute((const void *)k_de,
                                 hipFuncAttributeMaxDynamicSharedMemorySize,

@@ -286,3 +286,39 @@ def test_bins_few_pairs(gpu, n, evg):
         np.testing.assert_array_equal(bn[t, :k], ref[:, 2])
         np.testing.assert_allclose(bh[t, :k], ref[:, 0], rtol=1e-12)
         np.testing.assert_allclose(bg[t, :k], ref[:, 1], rtol=1e-12)
+
+
+def test_few_bins_and_many_give_the_same_bits(gpu):
+    """Few bins evolve in one workgroup per candidate, many over the whole
+    device: whichever takes a step, the result is the same to the last bit
+    (here the whole device is chosen for the call by a step with many bins,
+    the workgroup for the small steps alone and while capturing), and a fit of
+    one bin, which never converges, takes no launch per generation."""
+    import time
+    import torch
+    from spinterps_amd.variograms.fitvgs import BatchVariogramFitter
+    rng = np.random.default_rng(5)
+    n = 150
+    x, y = rng.uniform(0, 2e5, n), rng.uniform(0, 2e5, n)
+    vals = rng.gamma(2.0, 3.0, (4, n))
+    for t, k in ((0, 9), (1, 14), (2, 25)):
+        vals[t, k:] = np.nan
+    f = BatchVariogramFitter(x, y)
+    kw = dict(mdr=0.5, nk=20, perm_r_list=[1, 2], fit_vgs=['all'],
+              fil_nug_vg='Nug', range_ub=2e5, opt_iters=40, seed=3,
+              min_vld_stns=2, return_details=True)
+    for t, lo, hi in ((0, 1, 3), (1, 2, 5), (2, 8, 12)):
+        _, det = f.fit(vals[[t, 3]], **kw)
+        _, one = f.fit(vals[[t]], **kw)
+        nb = det['bins'][3].cpu().numpy()
+        assert lo <= nb[0] <= hi and nb[1] > 100, nb
+        # (the random streams are keyed on the step's place in the call)
+        for k in ('params', 'fun', 'nit'):
+            np.testing.assert_array_equal(one[k][0], det[k][0])
+    kw.update(opt_iters=10000, nk=50, fit_vgs=['Sph', 'Exp', 'Gau'])
+    f.fit(vals[:1], **kw)
+    torch.cuda.synchronize()
+    t0 = time.perf_counter()
+    _, det = f.fit(vals[:1], **kw)
+    # 1.2 ms; 200 ms with launches for each of up to 10 000 generations
+    assert time.perf_counter() - t0 < 0.05, det['nit']
