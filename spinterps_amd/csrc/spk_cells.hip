@@ -1764,7 +1764,7 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
   if (Cs < C) Cs = std::max<int64_t>(256, Cs / 256 * 256);
   if (Cs > C) Cs = C;
   const int64_t ldk = round_up(Cs, 128);
-  const int gsteps =
+  int gsteps =
       batched ? 1
               : (int)std::max<int64_t>(
                     1, std::min<int64_t>(S, plain_budget / (rowsR * ldk * 8)));
@@ -1797,10 +1797,17 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
     SPK_TRY(ws_get(ctx, "dual_ds", S * kDualSc * 8, (void **)&dual_ds));
   }
   if (!batched) {
-    SPK_TRY(ws_get(ctx, "R", (size_t)gsteps * rowsR * ldk * 8, (void **)&R));
-    SPK_TRY(ws_get(ctx, "qplain",
-                   (size_t)gsteps * 3 * ceil_div(N + p, 64) * ldk * 8,
-                   (void **)&qplain));
+    // (several steps where the memory allows, one as ever)
+    for (;; gsteps = (gsteps + 1) / 2) {
+      int rc = ws_get(ctx, "R", (size_t)gsteps * rowsR * ldk * 8, (void **)&R);
+      if (rc == SPK_OK)
+        rc = ws_get(ctx, "qplain",
+                    (size_t)gsteps * 3 * ceil_div(N + p, 64) * ldk * 8,
+                    (void **)&qplain);
+      if (rc == SPK_OK) break;
+      if (rc != SPK_ENOMEM || gsteps == 1) return rc;
+      (void)hipGetLastError();
+    }
   } else if (want_var) {
     // FP64 buffer for the batched FP64 path and for the steps the mixed
     // path promotes to FP64 (SPK_ST_FP64VAR)
