@@ -959,8 +959,10 @@ __global__ __launch_bounds__(256, 3) void k_kgen(
   // distance: h >= r (spherical), h c1 <= -61 (exponential) or h^2 c1 <= -61
   // (Gaussian), where 2^y < 2^-54 so that 1 - 2^y rounds to 1.  A
   // sub-chunk of 16 stations whose bounding box is that far from every cell
-  // of the block (the gap measured by dist2 itself, so that by monotone
-  // rounding no cell-station distance the loop computes is below it), and
+  // of the block (the gap by dist2, whose sum of squares, by monotone
+  // rounding, no cell-station pair's is below; the loop's root, dist_fast,
+  // ends with a Newton step from a relative error of 4e-15 and is within two
+  // units in the last place of dist2's, for which 1e-15 of r is allowed), and
   // whose staged c0 - G entries against the block's slot stations are all
   // 0, gives k = 0 and delta = 0 exactly for every cell: it adds nothing to
   // the estimate, its delta chunk stays unmarked in the chunk map, and it is
@@ -1048,7 +1050,7 @@ __global__ __launch_bounds__(256, 3) void k_kgen(
           const double D = dist2(gx, gy, 0.0, 0.0);
           bool far;
           if (one == SPK_VG_SPH)
-            far = D >= vo.r;
+            far = D >= vo.r * (1.0 + 1e-15);
           else if (one == SPK_VG_EXP)
             far = D * vo.c1 <= -61.0;
           else
