@@ -1,7 +1,7 @@
 // Cell-side kernels of the step interpolation and the batch driver behind
 // spk_interp_steps_dev.
 //
-//  k_gemm<..>    W = L^-1 K, q = |W|^2 per cell (variance term) on FP32
+//  k_gemm        W = L^-1 K, q = |W|^2 per cell (variance term) on FP32
 //                MFMA
 //  k_tri64       the same contraction in FP64, 128 x 128 tiles
 //  k_nearest     each cell's nearest active station (batched variance)
@@ -26,20 +26,6 @@ namespace spk {
 
 typedef double d4_t __attribute__((ext_vector_type(4)));
 typedef float f4_t __attribute__((ext_vector_type(4)));
-
-template <typename T>
-struct Mfma;
-// Result row held in slot r by lane group g = lane / 16 (column lane % 16):
-// f64 16x16x4 interleaves rows (g + 4 r), f32 16x16x4 keeps blocks (4 g + r)
-// (checked on gfx950 against a host matmul).
-template <>
-struct Mfma<float> {
-  using V = f4_t;
-  __device__ static inline V op(float a, float b, V c) {
-    return __builtin_amdgcn_mfma_f32_16x16x4f32(a, b, c, 0, 0, 0);
-  }
-  __device__ static constexpr int row(int g, int r) { return 4 * g + r; }
-};
 
 // |sum of weights - 1| of a cell above which the plain path flags the step
 // SPK_ST_ILLCOND (the sum is exactly one for OK / EDK).  On hourly steps
@@ -92,32 +78,23 @@ int recenter(hipStream_t st, const spk_problem *prob, double *sx, double *sy,
 
 // ---- MFMA contraction --------------------------------------------------------
 // W = L^-1 delta, |W|^2 per cell and 64-row block, on FP32 operands
-// (SPK_P_MIXED_F32, and SPK_P_MIXED above 8 192 rows).  Block tile: 64 rows x 128 cells, k in chunks of BK, 256 threads = 4 waves;
-// wave w owns cells [32 w, 32 w + 32) of the tile over all 64 rows as 4 x 2
-// MFMA 16x16 tiles, so the per-cell row reductions of the epilogue need no
-// cross-wave step.  The next k chunk is loaded into registers while the
-// current one is multiplied out of LDS (two LDS buffers, one barrier per
-// chunk).  A is column-major [P x P] (lda), B row-major [P x ldb cells];
+// (SPK_P_MIXED_F32, and SPK_P_MIXED above 8 192 rows).  Block tile: 64 rows x
+// 128 cells, k in chunks of 16, 256 threads = 4 waves; wave w owns cells
+// [32 w, 32 w + 32) of the tile over all 64 rows as 4 x 2 MFMA 16x16 tiles, so
+// the per-cell row reductions of the epilogue need no cross-wave step.  The
+// next two k chunks are loaded into registers while the current one is
+// multiplied out of LDS (two LDS buffers, one barrier per chunk), which covers
+// an L2 miss.  A is column-major [P x P] (lda), B row-major [P x ldb cells];
 // ldb is a multiple of 128 and every 128-cell tile lies inside it.
 // MFMA 16x16x4 operand layout: lane l supplies A[l % 16][l / 16] and
-// B[l / 16][l % 16]; the result row in slot r is Mfma<T>::row(l / 16, r).
-template <typename T>
-struct Vec4;
-template <>
-struct Vec4<float> {
-  using type = float4;
-};
-
-template <typename T, int BK>
+// B[l / 16][l % 16]; the result row in slot r is 4 (l / 16) + r.
 __global__ __launch_bounds__(256, 3) void k_gemm(
-    const T *__restrict__ A, int64_t lda, int64_t strideA,
-    const T *__restrict__ B, int64_t ldb, int64_t strideB,
-    const StepSc *__restrict__ sc, int64_t ldab, int64_t Cs, int sel,
+    const float *__restrict__ A, int64_t lda, int64_t strideA,
+    const float *__restrict__ B, int64_t ldb, int64_t strideB,
+    const StepSc *__restrict__ sc, int64_t ldab, int64_t Cs,
     double *__restrict__ qpart, int nrb, const uint8_t *__restrict__ nzb,
     int64_t nzk, unsigned long long *__restrict__ nexec) {
-  using MF = Mfma<T>;
-  using V = typename MF::V;
-  constexpr int BM = 64, BN = 128;
+  constexpr int BM = 64, BN = 128, BK = 16, VW = 4;
   // grid (row blocks, cell tiles, steps), one row block per block;
   // blocks on the same XCD (linear id mod 8) take consecutive row blocks of
   // one cell tile so that the tile's K rows stay in that XCD's L2.
@@ -125,61 +102,48 @@ __global__ __launch_bounds__(256, 3) void k_gemm(
   int lin = blockIdx.x + blockIdx.y * gridDim.x;
   if ((G & 7) == 0) lin = (lin & 7) * (G >> 3) + (lin >> 3);
   const int rbi = lin % gridDim.x, cti = lin / gridDim.x;
-  constexpr int VW = 16 / sizeof(T);         // elements per 16-byte load
-  // row padding: FP32 rows 16 banks apart, so the four 16-lane groups of a
+  // row padding: rows 16 banks apart, so the four 16-lane groups of a
   // 32-bit LDS read (one row each) fall on distinct banks
-  constexpr int PAD = sizeof(T) == 4 ? 16 : VW;
+  constexpr int PAD = 16;
   constexpr int A_LD = BM * BK / VW / 256;   // vector loads per thread
   constexpr int B_LD = BN * BK / VW / 256;
-  static_assert(A_LD >= 1 && B_LD >= 1, "tile too small");
-  using VT = typename Vec4<T>::type;
   const int sl = blockIdx.z;
-  const StepSc st = sc[sl];
-  if (st.status) return;
-  // sel 1: only the FP32 steps (neither SPK_ST_FP64VAR nor SPK_ST_INT8VAR),
-  // sel 2: only steps with SPK_ST_FP64VAR
-  if (sel == 1 && (st.flags & (SPK_ST_FP64VAR | SPK_ST_INT8VAR))) return;
-  if (sel == 2 && !(st.flags & SPK_ST_FP64VAR)) return;
-  const int n = st.n;
-  const int P = n;
+  const int n = sc[sl].n;
+  // the steps on FP32 operands (neither SPK_ST_FP64VAR nor SPK_ST_INT8VAR)
+  if (sc[sl].status ||
+      (sc[sl].flags & (SPK_ST_FP64VAR | SPK_ST_INT8VAR)))
+    return;
   const int64_t c0 = cti * (int64_t)BN;
-  if (c0 >= Cs) return;
-  const int r_lo = rbi * BM;
-  if (r_lo >= P) return;
-  const int r_hi = min(P, r_lo + BM);
+  const int r0 = rbi * BM;
+  if (c0 >= Cs || r0 >= n) return;
   A += (int64_t)sl * strideA;
   B += (int64_t)sl * strideB;
-  __shared__ __align__(16) T As[2][BK][BM + PAD];
-  __shared__ __align__(16) T Bs[2][BK][BN + PAD];
+  __shared__ __align__(16) float As[2][BK][BM + PAD];
+  __shared__ __align__(16) float Bs[2][BK][BN + PAD];
   __shared__ int s_list[256];  // nonzero chunks (with a chunk map)
   __shared__ int s_cnt[4];
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int li = lane & 15, lg = lane >> 4;
-
-  double acc_v[2] = {0.0, 0.0};
-
-  // register stages of the next chunks' tiles; the FP32 contraction keeps
-  // two chunks in flight, which covers an L2 miss behind the chunk being
-  // multiplied
-  constexpr bool PF2 = sizeof(T) == 4;
-  VT ra[A_LD], rb[B_LD], ra2[PF2 ? A_LD : 1], rb2[PF2 ? B_LD : 1];
-  // A tile element group q: rows r..r+VW-1 of column k
-  auto load_tiles = [&](auto &ra, auto &rb, int r0, int k0, int kend) {
+  const int kend = min(n, r0 + BM);
+  // register stages of the next two chunks' tiles
+  float4 ra[A_LD], rb[B_LD], ra2[A_LD], rb2[B_LD];
+  // A tile element group q: rows r..r+3 of column k
+  auto load_tiles = [&](auto &ra, auto &rb, int k0) {
 #pragma unroll
     for (int q = 0; q < A_LD; ++q) {
       const int e = tid + q * 256;
       const int r = (e % (BM / VW)) * VW, k = e / (BM / VW);
       const int gk = k0 + k;
       if (gk < kend) {
-        ra[q] = *reinterpret_cast<const VT *>(A + (r0 + r) +
-                                              (int64_t)gk * lda);
-        // rows beyond P are never used but may hold stale values
-        T *v = reinterpret_cast<T *>(&ra[q]);
+        ra[q] = *reinterpret_cast<const float4 *>(A + (r0 + r) +
+                                                  (int64_t)gk * lda);
+        // rows beyond n are never used but may hold stale values
+        float *v = reinterpret_cast<float *>(&ra[q]);
 #pragma unroll
         for (int u = 0; u < VW; ++u)
-          if (r0 + r + u >= P) v[u] = T(0);
+          if (r0 + r + u >= n) v[u] = 0.f;
       } else {
-        ra[q] = VT{};
+        ra[q] = float4{};
       }
     }
 #pragma unroll
@@ -188,9 +152,10 @@ __global__ __launch_bounds__(256, 3) void k_gemm(
       const int c = (e % (BN / VW)) * VW, k = e / (BN / VW);
       const int gk = k0 + k;
       if (gk < kend)
-        rb[q] = *reinterpret_cast<const VT *>(B + (int64_t)gk * ldb + c0 + c);
+        rb[q] = *reinterpret_cast<const float4 *>(B + (int64_t)gk * ldb + c0 +
+                                                  c);
       else
-        rb[q] = VT{};
+        rb[q] = float4{};
     }
   };
   auto store_tiles = [&](const auto &ra, const auto &rb, int buf) {
@@ -198,147 +163,109 @@ __global__ __launch_bounds__(256, 3) void k_gemm(
     for (int q = 0; q < A_LD; ++q) {
       const int e = tid + q * 256;
       const int r = (e % (BM / VW)) * VW, k = e / (BM / VW);
-      *reinterpret_cast<VT *>(&As[buf][k][r]) = ra[q];
+      *reinterpret_cast<float4 *>(&As[buf][k][r]) = ra[q];
     }
 #pragma unroll
     for (int q = 0; q < B_LD; ++q) {
       const int e = tid + q * 256;
       const int c = (e % (BN / VW)) * VW, k = e / (BN / VW);
-      *reinterpret_cast<VT *>(&Bs[buf][k][c]) = rb[q];
+      *reinterpret_cast<float4 *>(&Bs[buf][k][c]) = rb[q];
     }
   };
-
-  // FP32 MFMA sums are added in FP64 after every chunk (BK products), or
-  // for the FP32 contraction after every second chunk (2 BK products)
-  constexpr bool ACC64 = sizeof(T) == 4;
-  for (int r0 = r_lo; r0 < r_hi; r0 += BM) {
-    V acc[4][2];
-    double acc64[ACC64 ? 4 : 1][2][4];
+  // FP32 MFMA sums go to FP64 after every second chunk (32 products)
+  f4_t acc[4][2];
+  double acc64[4][2][4];
 #pragma unroll
-    for (int a = 0; a < 4; ++a)
+  for (int a = 0; a < 4; ++a)
 #pragma unroll
-      for (int b = 0; b < 2; ++b) acc[a][b] = V{0, 0, 0, 0};
-    if (ACC64) {
+    for (int b = 0; b < 2; ++b) {
+      acc[a][b] = f4_t{0, 0, 0, 0};
 #pragma unroll
-      for (int a = 0; a < (ACC64 ? 4 : 1); ++a)
-#pragma unroll
-        for (int b = 0; b < 2; ++b)
-#pragma unroll
-          for (int r = 0; r < 4; ++r) acc64[a][b][r] = 0.0;
+      for (int r = 0; r < 4; ++r) acc64[a][b][r] = 0.0;
     }
-    const int kend = min(P, r0 + BM);
-    int nch = (kend + BK - 1) / BK;
-    // with a map of the 16-row chunks of delta that hold a nonzero
-    // value in this cell tile: only those chunks are multiplied (a zero
-    // chunk adds exactly nothing)
-    const bool skip = BK == 16 && nzb != nullptr && nch <= 256;
-    if (skip) {
-      const uint8_t *nz = nzb + ((int64_t)sl * gridDim.y + cti) * nzk;
-      const bool f = tid < nch && nz[tid] != 0;
-      const unsigned long long bm = __ballot(f);
-      if (lane == 0) s_cnt[wave] = __popcll(bm);
-      __syncthreads();
-      int off = 0;
-      for (int w2 = 0; w2 < wave; ++w2) off += s_cnt[w2];
-      if (f) s_list[off + __popcll(bm & ((1ull << lane) - 1ull))] = tid;
-      const int tot = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
-      __syncthreads();
-      nch = tot;
-    }
-    // executed chunks, counted when profiling
-    if (nexec && tid == 0)
-      atomicAdd(nexec, (unsigned long long)nch);
-    auto kchunk = [&](int ch) { return skip ? s_list[ch] * BK : ch * BK; };
-    // multiply chunk ch out of LDS buffer ch & 1 (FP32: then add to FP64)
-    auto mma_chunk = [&](int buf, bool zs = true, bool fl = true) {
+  int nch = (kend + BK - 1) / BK;
+  // with a map of the 16-row chunks of delta that hold a nonzero
+  // value in this cell tile: only those chunks are multiplied (a zero
+  // chunk adds exactly nothing)
+  const bool skip = nzb != nullptr && nch <= 256;
+  if (skip) {
+    const uint8_t *nz = nzb + ((int64_t)sl * gridDim.y + cti) * nzk;
+    const bool f = tid < nch && nz[tid] != 0;
+    const unsigned long long bm = __ballot(f);
+    if (lane == 0) s_cnt[wave] = __popcll(bm);
+    __syncthreads();
+    int off = 0;
+    for (int w2 = 0; w2 < wave; ++w2) off += s_cnt[w2];
+    if (f) s_list[off + __popcll(bm & ((1ull << lane) - 1ull))] = tid;
+    const int tot = s_cnt[0] + s_cnt[1] + s_cnt[2] + s_cnt[3];
+    __syncthreads();
+    nch = tot;
+  }
+  // executed chunks, counted when profiling
+  if (nexec && tid == 0) atomicAdd(nexec, (unsigned long long)nch);
+  auto kchunk = [&](int ch) { return skip ? s_list[ch] * BK : ch * BK; };
+  // multiply a chunk out of LDS buffer buf: the first of a pair starts from
+  // zero, the last adds the pair's sums to FP64
+  auto mma_chunk = [&](int buf, bool first, bool last) {
 #pragma unroll
-      for (int kk = 0; kk < BK / 4; ++kk) {
-        const int ka = kk * 4 + lg;
-        T af[4], bf[2];
+    for (int kk = 0; kk < BK / 4; ++kk) {
+      const int ka = kk * 4 + lg;
+      float af[4], bf[2];
 #pragma unroll
-        for (int ti = 0; ti < 4; ++ti) af[ti] = As[buf][ka][ti * 16 + li];
+      for (int ti = 0; ti < 4; ++ti) af[ti] = As[buf][ka][ti * 16 + li];
+#pragma unroll
+      for (int tj = 0; tj < 2; ++tj)
+        bf[tj] = Bs[buf][ka][wave * 32 + tj * 16 + li];
+#pragma unroll
+      for (int ti = 0; ti < 4; ++ti)
 #pragma unroll
         for (int tj = 0; tj < 2; ++tj)
-          bf[tj] = Bs[buf][ka][wave * 32 + tj * 16 + li];
-        // FP32 chunk sums start from zero (the previous chunk's went to FP64)
-#pragma unroll
-        for (int ti = 0; ti < 4; ++ti)
-#pragma unroll
-          for (int tj = 0; tj < 2; ++tj)
-            acc[ti][tj] = MF::op(af[ti], bf[tj],
-                                 ACC64 && zs && kk == 0 ? V{0, 0, 0, 0}
-                                                        : acc[ti][tj]);
-      }
-      if (ACC64 && fl) {
-#pragma unroll
-        for (int ti = 0; ti < (ACC64 ? 4 : 1); ++ti)
-#pragma unroll
-          for (int tj = 0; tj < 2; ++tj) {
-#pragma unroll
-            for (int r = 0; r < 4; ++r)
-              acc64[ti][tj][r] += (double)acc[ti][tj][r];
-          }
-      }
-    };
-    load_tiles(ra, rb, r0, nch > 0 ? kchunk(0) : 0, kend);
-    __syncthreads();  // previous row block's readers are done with LDS
-    store_tiles(ra, rb, 0);
-    if constexpr (PF2) {
-      // stage ra holds chunk ch + 1 on entry to chunk ch, even ch
-      if (nch > 1) load_tiles(ra, rb, r0, kchunk(1), kend);
-      __syncthreads();
-      auto step = [&](int ch, auto &la, auto &lb, const auto &sa,
-                      const auto &sb) {
-        if (ch + 2 < nch) load_tiles(la, lb, r0, kchunk(ch + 2), kend);
-        // FP32 sums of two chunks (32 products) start from zero and then
-        // go to FP64
-        mma_chunk(ch & 1, (ch & 1) == 0, (ch & 1) || ch + 1 >= nch);
-        if (ch + 1 < nch) store_tiles(sa, sb, (ch & 1) ^ 1);
-        __syncthreads();
-      };
-      for (int ch = 0; ch < nch; ch += 2) {
-        step(ch, ra2, rb2, ra, rb);
-        if (ch + 1 < nch) step(ch + 1, ra, rb, ra2, rb2);
-      }
-    } else {
-      __syncthreads();
-      for (int ch = 0; ch < nch; ++ch) {
-        if (ch + 1 < nch) load_tiles(ra, rb, r0, kchunk(ch + 1), kend);
-        mma_chunk(ch & 1);
-        if (ch + 1 < nch) store_tiles(ra, rb, (ch & 1) ^ 1);
-        __syncthreads();
-      }
+          acc[ti][tj] = __builtin_amdgcn_mfma_f32_16x16x4f32(
+              af[ti], bf[tj],
+              first && kk == 0 ? f4_t{0, 0, 0, 0} : acc[ti][tj], 0, 0, 0);
     }
-    // epilogue for this row block
+    if (last) {
 #pragma unroll
-    for (int tj = 0; tj < 2; ++tj) {
-      const int64_t col = c0 + wave * 32 + tj * 16 + li;
-      if (col >= Cs) continue;
+      for (int ti = 0; ti < 4; ++ti)
 #pragma unroll
-      for (int ti = 0; ti < 4; ++ti) {
+        for (int tj = 0; tj < 2; ++tj)
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int row = r0 + ti * 16 + MF::row(lg, r);
-          const double v = ACC64 ? acc64[ACC64 ? ti : 0][tj][r]
-                                 : (double)acc[ti][tj][r];
-          if (row < n) acc_v[tj] += v * v;
-        }
-      }
+          for (int r = 0; r < 4; ++r)
+            acc64[ti][tj][r] += (double)acc[ti][tj][r];
     }
+  };
+  load_tiles(ra, rb, nch > 0 ? kchunk(0) : 0);
+  store_tiles(ra, rb, 0);
+  // stage ra holds chunk ch + 1 on entry to chunk ch, even ch
+  if (nch > 1) load_tiles(ra, rb, kchunk(1));
+  __syncthreads();
+  auto step = [&](int ch, auto &la, auto &lb, const auto &sa,
+                  const auto &sb) {
+    if (ch + 2 < nch) load_tiles(la, lb, kchunk(ch + 2));
+    mma_chunk(ch & 1, (ch & 1) == 0, (ch & 1) || ch + 1 >= nch);
+    if (ch + 1 < nch) store_tiles(sa, sb, (ch & 1) ^ 1);
+    __syncthreads();
+  };
+  for (int ch = 0; ch < nch; ch += 2) {
+    step(ch, ra2, rb2, ra, rb);
+    if (ch + 1 < nch) step(ch + 1, ra, rb, ra2, rb2);
   }
-  // the four lane groups of a wave share each column
-#pragma unroll
-  for (int tj = 0; tj < 2; ++tj) {
-    acc_v[tj] += __shfl_xor(acc_v[tj], 16, 64);
-    acc_v[tj] += __shfl_xor(acc_v[tj], 32, 64);
-  }
-  if (lg != 0) return;
+  // this row block's share of |L^-1 delta|^2, per cell
 #pragma unroll
   for (int tj = 0; tj < 2; ++tj) {
     const int64_t col = c0 + wave * 32 + tj * 16 + li;
-    // this row block's share of |L^-1 delta|^2
-    if (col < Cs)
-      qpart[((int64_t)sl * nrb + rbi) * ldab + col] = acc_v[tj];
+    double v = 0.0;
+#pragma unroll
+    for (int ti = 0; ti < 4; ++ti)
+#pragma unroll
+      for (int r = 0; r < 4; ++r)
+        if (r0 + ti * 16 + 4 * lg + r < n)
+          v += acc64[ti][tj][r] * acc64[ti][tj][r];
+    // the four lane groups of a wave share each column
+    v += __shfl_xor(v, 16, 64);
+    v += __shfl_xor(v, 32, 64);
+    if (lg == 0 && col < Cs)
+      qpart[((int64_t)sl * nrb + rbi) * ldab + col] = v;
   }
 }
 
@@ -2311,9 +2238,9 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
         } else if (mixed) {
           ProfScope ps(ctx, "gemm_tri_f32");
           // k chunks of 16: FP32 sums of 32 products, 3 waves per SIMD
-          hipLaunchKernelGGL((k_gemm<float, 16>), grid, dim3(256), 0, sm,
+          hipLaunchKernelGGL(k_gemm, grid, dim3(256), 0, sm,
                              q.L32, ld, strideM, (const float *)K32, ldk,
-                             ld * ldk, q.sc, ldk, cn, 1, qpart, nrb,
+                             ld * ldk, q.sc, ldk, cn, qpart, nrb,
                              (const uint8_t *)nzb, nzk,
                              prof_of(ctx).on ? prof_of(ctx).work : nullptr);
         }
@@ -2328,7 +2255,7 @@ static int interp_steps_impl(spk_ctx *ctx, const spk_problem *prob,
                              (const double *)K64, ldk, ld * ldk, q.sc, cn,
                              qpart, ldk, nrb, mixed ? 2 : 0, Sb);
         }
-        SPK_TRY(check_launch("k_gemm<tri>"));
+        SPK_TRY(check_launch("k_gemm"));
         {
           ProfScope ps(ctx, "var_reduce");
           hipLaunchKernelGGL(k_var_reduce, dim3((unsigned)ceil_div(cn, 256), Sb),
