@@ -1359,7 +1359,8 @@ __global__ __launch_bounds__(64, NBC > 2 ? 2 : 3) void k_neb_mfma(
           for (int I = J; I < NBR; ++I)
             if (col >= ko && col < ko + 1 + P1) acc[I][J][r] = 0.0;
         }
-      // ---- Cholesky sweep, 16 columns at a time
+      // ---- Cholesky sweep, 16 columns at a time; |y|^2 by half panels (its
+      // rounding goes into the variance, most of which it cancels)
       double pmin = INFINITY, ylast = 0.0, yu = 0.0, yy = 0.0, yf[PA];
 #pragma unroll
       for (int qd = 0; qd < PA; ++qd) yf[qd] = 0.0;
@@ -1386,6 +1387,7 @@ __global__ __launch_bounds__(64, NBC > 2 ? 2 : 3) void k_neb_mfma(
           v[2 * e] = v2[e].x;
           v[2 * e + 1] = v2[e].y;
         }
+        double yp = 0.0;
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
           if (16 * J + j >= ko) break;
@@ -1403,8 +1405,13 @@ __global__ __launch_bounds__(64, NBC > 2 ? 2 : 3) void k_neb_mfma(
 #pragma unroll
           for (int i = j + 1; i < 16; ++i)
             v[i] = fma(-l, bcast(l, 16 * J + i), v[i]);
-          yy = fma(l, l, yy);
+          yp = fma(l, l, yp);
+          if (j == 7) {
+            yy += yp;
+            yp = 0.0;
+          }
         }
+        yy += yp;
 #pragma unroll
         for (int e = 0; e < 8; ++e)
           row2[e] = make_double2(v[2 * e], v[2 * e + 1]);
