@@ -730,32 +730,47 @@ __device__ inline bool neb_no_system(const NebArgs &a, const NebChunk &q,
 }
 
 // beta = B^-1 g by Cholesky of the p x p matrix B; false where B is not
-// positive definite.
+// positive definite.  The loops run over PA with tests on p: indexed by
+// variables, the arrays would live in scratch memory.
 template <int PA>
 __device__ inline bool neb_beta(int p, double (&B)[PA][PA],
                                 const double (&g)[PA], double (&beta)[PA]) {
-  for (int j = 0; j < p; ++j) {
-    double d = B[j][j];
-    for (int l = 0; l < j; ++l) d -= B[j][l] * B[j][l];
-    if (!(d > 0.0) || !isfinite(d)) return false;
-    B[j][j] = sqrt(d);
-    for (int i = j + 1; i < p; ++i) {
-      double s = B[i][j];
-      for (int l = 0; l < j; ++l) s -= B[i][l] * B[j][l];
-      B[i][j] = s / B[j][j];
+  bool ok = true;
+#pragma unroll
+  for (int j = 0; j < PA; ++j)
+    if (j < p) {
+      double d = B[j][j];
+#pragma unroll
+      for (int l = 0; l < j; ++l) d -= B[j][l] * B[j][l];
+      ok = ok && d > 0.0 && isfinite(d);
+      B[j][j] = sqrt(d);
+#pragma unroll
+      for (int i = j + 1; i < PA; ++i)
+        if (i < p) {
+          double s = B[i][j];
+#pragma unroll
+          for (int l = 0; l < j; ++l) s -= B[i][l] * B[j][l];
+          B[i][j] = s / B[j][j];
+        }
     }
-  }
-  for (int i = 0; i < p; ++i) {
-    double s = g[i];
-    for (int l = 0; l < i; ++l) s -= B[i][l] * beta[l];
-    beta[i] = s / B[i][i];
-  }
-  for (int i = p - 1; i >= 0; --i) {
-    double s = beta[i];
-    for (int l = i + 1; l < p; ++l) s -= B[l][i] * beta[l];
-    beta[i] = s / B[i][i];
-  }
-  return true;
+#pragma unroll
+  for (int i = 0; i < PA; ++i)
+    if (i < p) {
+      double s = g[i];
+#pragma unroll
+      for (int l = 0; l < i; ++l) s -= B[i][l] * beta[l];
+      beta[i] = s / B[i][i];
+    }
+#pragma unroll
+  for (int i = PA - 1; i >= 0; --i)
+    if (i < p) {
+      double s = beta[i];
+#pragma unroll
+      for (int l = i + 1; l < PA; ++l)
+        if (l < p) s -= B[l][i] * beta[l];
+      beta[i] = s / B[i][i];
+    }
+  return ok;
 }
 
 // One 64-thread workgroup per chunk (grid-stride over the chunks).  Lane j
@@ -1167,7 +1182,7 @@ __host__ __device__ inline int neb_extra(int p) { return 1 + (p > 0 ? p : 1); }
 template <int NBC, int PT>
 // Small sets wait for loads more than they compute: 3 waves per SIMD (8 steps x
 // 9 797 cells, 24 per set: 722 -> 404 us); the others would spill.
-__global__ __launch_bounds__(64, NBC > 2 ? 2 : 3) void k_neb_mfma(
+__global__ __launch_bounds__(64, NBC > 2 || PT > 2 ? 2 : 3) void k_neb_mfma(
     NebArgs a, const VgFast *__restrict__ vfs) {
   constexpr int PA = PT > 0 ? PT : 1;
   constexpr int NBR = neb_row_blocks(NBC), NR = 16 * NBR;
@@ -1464,9 +1479,12 @@ __global__ __launch_bounds__(64, NBC > 2 ? 2 : 3) void k_neb_mfma(
       double bsc = 0.0;
       if (ok && kap <= 1e10 && p > 0) {
         double B[PA][PA], gu[PA];
-        for (int i = 0; i < p; ++i) {
-          gu[i] = bcast(yu, k + 1 + i);
-          for (int j = 0; j <= i; ++j) B[i][j] = bcast(yf[j], k + 1 + i);
+#pragma unroll
+        for (int i = 0; i < PA; ++i) {
+          const int r = min(k + 1 + i, 63);
+          gu[i] = bcast(yu, r);
+#pragma unroll
+          for (int j = 0; j <= i; ++j) B[i][j] = bcast(yf[j], r);
         }
         bsc = B[0][0];
         ok = neb_beta<PA>(p, B, gu, beta);
@@ -1502,9 +1520,11 @@ __global__ __launch_bounds__(64, NBC > 2 ? 2 : 3) void k_neb_mfma(
           }
         } else {
           e = mean + (yu + beta[0] * (1.0 - yf[0]));
-          for (int qd = 1; qd < p; ++qd)
-            e += (a.cell_drift[(int64_t)(qd - 1) * a.C + ci] - yf[qd]) *
-                 beta[qd];
+#pragma unroll
+          for (int qd = 1; qd < PA; ++qd)
+            if (qd < p)
+              e += (a.cell_drift[(int64_t)(qd - 1) * a.C + ci] - yf[qd]) *
+                   beta[qd];
         }
         a.est[(int64_t)t * a.C + ci] = e;
         if (a.want_var && a.var)
@@ -1996,7 +2016,12 @@ int spk_interp_neb_steps_dev(spk_ctx *ctx, const spk_problem *prob,
       const unsigned grid =
           (unsigned)std::max<int64_t>(1, std::min<int64_t>(tot, 16384));
       const dim3 g(grid), b(64);
-      if (mf && method == SPK_M_EDK)
+      // (one drift in a kernel of its own: 8 steps x 2 500 cells, 10 per set,
+      // 166 us; with room for kMaxP border columns, which kept them in scratch
+      // memory, 389)
+      if (mf && method == SPK_M_EDK && p <= 2)
+        neb_mfma_launch<2>(nbc, g, sm, a, vf);
+      else if (mf && method == SPK_M_EDK)
         neb_mfma_launch<kMaxP>(nbc, g, sm, a, vf);
       else if (mf)
         neb_mfma_launch<1>(nbc, g, sm, a, vf);

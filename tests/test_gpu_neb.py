@@ -144,6 +144,49 @@ def test_set_sizes_match_oracle(gpu, method, n_nebs):
                'var')
 
 
+@pytest.mark.parametrize('method,drifts', [('OK', 0), ('SK', 0), ('SKM', 0),
+                                           ('EDK', 1), ('EDK', 2),
+                                           ('EDK', 3), ('EDK', 7)])
+@pytest.mark.parametrize('n_nebs', [40, 47, 54, 58])
+def test_chunks_of_many_cells(gpu, method, drifts, n_nebs):
+    """One set for all cells: chunks of 64, 64 and 41 cells, which take one
+    chunk kernel or the other by their groups of cells (one-model and
+    two-model variograms in calls of their own), against the exact solution
+    of the same systems.  Covariance matrices of condition 1e4 and less, the
+    drifts of order one: k 2^-53 cond is below 1e-10, 1e-9 with the border."""
+    from spinterps_amd.interp.steps import DeviceProblem, interp_neb_steps
+    rng = np.random.default_rng(n_nebs)
+    n = n_nebs
+    sx, sy = rng.uniform(0, 1e5, n), rng.uniform(0, 1e5, n)
+    g = np.arange(13) * 8e3 + 1e3
+    cx, cy = [a.ravel() for a in np.meshgrid(g, g)]
+    m = drifts
+
+    def drift(x, y):
+        return np.stack([np.sin((x + k * y) / (2e4 + 5e3 * k))
+                         for k in range(m)])
+    z = rng.gamma(2.0, 5.0, (2, n))
+    for vgs in (['0.5 Nug(0.0) + 9.0 Exp(30000.0)', '9.0 Sph(40000.0)'],
+                ['4.0 Sph(20000.0) + 5.0 Exp(60000.0)', '9.0 Sph(40000.0)']):
+        sd, cd = (drift(sx, sy).T.copy(), drift(cx, cy)) if m else (None, None)
+        prob = DeviceProblem(sx, sy, cx, cy, sd, cd)
+        e, v, info = interp_neb_steps(prob, z, vgs, method,
+                                      neb_sel_mthd='nrst', n_nebs=n)
+        for t in range(2):
+            assert not int(info[t]) & (_lib.ST_PINV | _lib.ST_ILLCOND)
+            dd = O.dists_2d(sx, sy, sx, sy)
+            rd = O.dists_2d(cx, cy, sx, sy)
+            if method == 'SK':
+                K, R = O.krig_system('SK', vgs[t], dd, rd, None, None, 0.0)
+                ref, var = O.krige_solve(K, R, z[t], rd, False)[:2]
+            else:
+                ref, var, _ = O.krige_exact(method, vgs[t], dd, rd, z[t], sd,
+                                            cd, want_var=method == 'OK')
+            _close(e[t].cpu().numpy(), ref, np.abs(z).max(), 1e-9, method)
+            if method == 'OK':
+                _close(v[t].cpu().numpy(), var, var.max(), 1e-9, 'var')
+
+
 def test_variance_rounding(gpu):
     """The variance c0 - |y|^2 + ... of sets of 50 against long double: with
     |y|^2 summed by eights its error is 4.7e-16 of the variances' size (term by
