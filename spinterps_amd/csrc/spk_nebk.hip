@@ -673,6 +673,9 @@ struct NebArgs {
   int64_t total;
   int method, want_var, skm;
   double thr, mvg, idw_exp;
+  // k_neb_mfma takes the chunks whose cells fit mf_groups groups of its
+  // mf_rows rows, k_neb_krige the others (mf_rows 0: all)
+  int mf_rows, mf_groups;
   double *est, *var;  // [S x C] of the batch
   int *sflags;
   unsigned long long *skappa;
@@ -705,6 +708,13 @@ __device__ inline NebChunk neb_chunk(const NebArgs &a, int ch, int nch) {
   q.n = a.sc[q.t].n;
   q.k = neb_set_size(a.K, a.kfix, q.n);
   return q;
+}
+
+// Whether chunk q is k_neb_mfma's (p border columns).
+__device__ inline bool neb_on_mfma(const NebArgs &a, const NebChunk &q,
+                                   int p) {
+  const int cells = a.mf_rows - (q.k + 1 + (p > 0 ? p : 1));
+  return (int)(q.p1 - q.p0) <= cells * a.mf_groups;
 }
 
 // Chunks that need no system (kriging): a single station, its value
@@ -807,6 +817,7 @@ __global__ __launch_bounds__(64) void k_neb_krige(NebArgs a) {
   for (int ch = blockIdx.x; ch < nch; ch += gridDim.x) {
     const NebChunk q = neb_chunk(a, ch, nch);
     if (q.n <= 0) continue;
+    if (KRIG && a.mf_rows && neb_on_mfma(a, q, p)) continue;
     const int k = q.k, t = q.t;
     const int np = (int)(q.p1 - q.p0);  // at most kNebChunk
     double *eo = a.est + (int64_t)t * a.C;
@@ -1159,8 +1170,9 @@ __global__ __launch_bounds__(64) void k_neb_krige(NebArgs a) {
 // a tenth).  12 steps x 250 000 cells, 1 000 stations, 50 per set: 6.2 ms; 24.6
 // with k_neb_krige, which factorises a packed triangle in LDS by columns with
 // two LDS reads per multiply-add, and substitutes for four cells at a time.
-// That kernel keeps what does not fit here: sets of more than 58 stations,
-// Pow and Hol models, and the methods without a system.
+// That kernel keeps what does not fit here (sets of more than 58 stations, Pow
+// and Hol models, the methods without a system) and chunks of many groups of
+// cells (neb_on_mfma).
 constexpr int kNebRows = 64;
 // Row blocks of 16 for nbc column blocks (stations, values, border).
 __host__ __device__ constexpr int neb_row_blocks(int nbc) {
@@ -1196,7 +1208,7 @@ __global__ __launch_bounds__(64, NBC > 2 || PT > 2 ? 2 : 3) void k_neb_mfma(
   const bool sk = a.method == SPK_M_SK;
   for (int ch = blockIdx.x; ch < nch; ch += gridDim.x) {
     const NebChunk q = neb_chunk(a, ch, nch);
-    if (q.n <= 0) continue;
+    if (q.n <= 0 || !neb_on_mfma(a, q, p)) continue;
     const int k = q.k, t = q.t;
     const int np = (int)(q.p1 - q.p0);  // at most kNebChunk
     __syncthreads();  // the previous chunk's readers are done
@@ -1922,22 +1934,46 @@ int spk_interp_neb_steps_dev(spk_ctx *ctx, const spk_problem *prob,
   const int kfix = sel == SPK_NEB_PIE ? 1 : 0;
   // Pow or Hol components anywhere in the call: the kernel variant with
   // pow and sin (they cost registers, and so occupancy, when compiled in)
-  bool ph = false;
+  bool ph = false, one = true;
   if (krig) {
     std::vector<spk_vg> hv((size_t)T);
     SPK_HIP(hipMemcpyAsync(hv.data(), vgs, T * sizeof(spk_vg),
                            hipMemcpyDeviceToHost, sm));
     SPK_HIP(hipStreamSynchronize(sm));
-    for (const spk_vg &v : hv)
-      for (int qd = 0; qd < v.n && qd < SPK_VG_MAX; ++qd)
-        ph = ph || v.type[qd] == SPK_VG_POW || v.type[qd] == SPK_VG_HOL;
+    for (const spk_vg &v : hv) {
+      int nugs = 0, models = 0;
+      for (int qd = 0; qd < v.n && qd < SPK_VG_MAX; ++qd) {
+        const int ty = v.type[qd];
+        ph = ph || ty == SPK_VG_POW || ty == SPK_VG_HOL;
+        nugs += ty == SPK_VG_NUG;
+        models += ty == SPK_VG_SPH || ty == SPK_VG_EXP || ty == SPK_VG_GAU;
+      }
+      one = one && models == 1 && nugs + models == v.n && nugs <= 1;
+    }
+    one = one && opts->min_vg_val <= 0.0;
   }
   const int lds_krige = neb_lds_doubles(K, p) * 8;
-  // sets on the matrix cores where four cells or more fit in their rows
-  // and no model needs pow or sin
+  // Sets on the matrix cores where four cells or more fit in their rows
+  // and no model needs pow or sin.  k_neb_mfma sweeps the stations' columns
+  // once per group of cells, k_neb_krige factorises once per chunk and then
+  // takes little per cell where no variance is wanted.  10 000 chunks of 64
+  // cells, 54 stations (8 groups; with a drift 10), ms:
+  //                                k_neb_mfma      k_neb_krige
+  //   one model, variance          0.79            1.70
+  //   one model, estimates         0.79 (1.12)     0.81 (1.00)
+  //   several models, variance     1.51            1.74
+  //   several models, estimates    1.51 (2.03)     0.86 (1.04)
+  // The first is ahead at any number of groups (16: 1.62 and 1.94), the
+  // others up to 8, 9 and 4; a chunk of more goes to k_neb_krige.
   const int nbc = neb_col_blocks(K, p);
-  const bool mf = krig && !ph && nbc <= 4 &&
-                  K + neb_extra(p) + 4 <= 16 * neb_row_blocks(nbc);
+  const int mrows = 16 * neb_row_blocks(nbc);
+  const bool mf =
+      krig && !ph && nbc <= 4 && K + neb_extra(p) + 4 <= mrows;
+  const bool nvar = !(opts->want_var && method == SPK_M_OK && var);
+  const int mgroups = one ? (nvar ? 8 : kNebChunk) : (nvar ? 4 : 9);
+  // whether a chunk can have more groups
+  const bool both =
+      mf && mgroups * (mrows - K - neb_extra(p)) < kNebChunk;
   VgFast *vf = nullptr;
   if (mf) SPK_TRY(ws_get(ctx, "neb_vf", S * sizeof(VgFast), (void **)&vf));
   int hbad = 0;
@@ -2006,6 +2042,8 @@ int spk_interp_neb_steps_dev(spk_ctx *ctx, const spk_problem *prob,
     a.fail_list = flist;
     a.fail_cnt = fcnt;
     a.bad = bad;
+    a.mf_rows = mf ? mrows : 0;
+    a.mf_groups = mgroups;
     if (mf) {
       hipLaunchKernelGGL(k_neb_vf, dim3((unsigned)ceil_div(Sb, 64)), dim3(64),
                          0, sm, gb, Sb, vf);
@@ -2016,6 +2054,47 @@ int spk_interp_neb_steps_dev(spk_ctx *ctx, const spk_problem *prob,
       const unsigned grid =
           (unsigned)std::max<int64_t>(1, std::min<int64_t>(tot, 16384));
       const dim3 g(grid), b(64);
+      // where both kernels have chunks, k_neb_krige's run beside the others
+      // on the second stream: one after the other, the latency of a second
+      // launch is what a small call is made of (one step x 2 500 cells of 50
+      // per set, two models: 523 us by k_neb_krige, 664 by both in turn, 552)
+      hipStream_t sk = sm;
+      if (both) {
+        if (!ctx->aux_stream)
+          SPK_HIP(hipStreamCreateWithFlags(&ctx->aux_stream,
+                                           hipStreamNonBlocking));
+        for (int e = 0; e < 2; ++e)
+          if (!ctx->ev[e])
+            SPK_HIP(hipEventCreateWithFlags(&ctx->ev[e],
+                                            hipEventDisableTiming));
+        sk = ctx->aux_stream;
+        SPK_HIP(hipEventRecord(ctx->ev[0], sm));
+        SPK_HIP(hipStreamWaitEvent(sk, ctx->ev[0], 0));
+      }
+      if (mf && !both) {
+        // every chunk is k_neb_mfma's
+      } else if (!krig) {
+        hipLaunchKernelGGL((k_neb_krige<0, false, false>), g, b, lds_krige,
+                           sk, a);
+      } else if (method == SPK_M_OK && ph) {
+        hipLaunchKernelGGL((k_neb_krige<1, true, true>), g, b, lds_krige, sk,
+                           a);
+      } else if (method == SPK_M_OK) {
+        hipLaunchKernelGGL((k_neb_krige<1, false, true>), g, b, lds_krige, sk,
+                           a);
+      } else if (method == SPK_M_EDK && ph) {
+        hipLaunchKernelGGL((k_neb_krige<kMaxP, true, true>), g, b, lds_krige,
+                           sk, a);
+      } else if (method == SPK_M_EDK) {
+        hipLaunchKernelGGL((k_neb_krige<kMaxP, false, true>), g, b,
+                           lds_krige, sk, a);
+      } else if (ph) {
+        hipLaunchKernelGGL((k_neb_krige<0, true, true>), g, b, lds_krige, sk,
+                           a);
+      } else {
+        hipLaunchKernelGGL((k_neb_krige<0, false, true>), g, b, lds_krige, sk,
+                           a);
+      }
       // (one drift in a kernel of its own: 8 steps x 2 500 cells, 10 per set,
       // 166 us; with room for kMaxP border columns, which kept them in scratch
       // memory, 389)
@@ -2025,27 +2104,10 @@ int spk_interp_neb_steps_dev(spk_ctx *ctx, const spk_problem *prob,
         neb_mfma_launch<kMaxP>(nbc, g, sm, a, vf);
       else if (mf)
         neb_mfma_launch<1>(nbc, g, sm, a, vf);
-      else if (!krig)
-        hipLaunchKernelGGL((k_neb_krige<0, false, false>), g, b, lds_krige,
-                           sm, a);
-      else if (method == SPK_M_OK && ph)
-        hipLaunchKernelGGL((k_neb_krige<1, true, true>), g, b, lds_krige, sm,
-                           a);
-      else if (method == SPK_M_OK)
-        hipLaunchKernelGGL((k_neb_krige<1, false, true>), g, b, lds_krige, sm,
-                           a);
-      else if (method == SPK_M_EDK && ph)
-        hipLaunchKernelGGL((k_neb_krige<kMaxP, true, true>), g, b, lds_krige,
-                           sm, a);
-      else if (method == SPK_M_EDK)
-        hipLaunchKernelGGL((k_neb_krige<kMaxP, false, true>), g, b,
-                           lds_krige, sm, a);
-      else if (ph)
-        hipLaunchKernelGGL((k_neb_krige<0, true, true>), g, b, lds_krige, sm,
-                           a);
-      else
-        hipLaunchKernelGGL((k_neb_krige<0, false, true>), g, b, lds_krige, sm,
-                           a);
+      if (both) {
+        SPK_HIP(hipEventRecord(ctx->ev[1], sk));
+        SPK_HIP(hipStreamWaitEvent(sm, ctx->ev[1], 0));
+      }
       SPK_TRY(check_launch("k_neb_krige"));
     }
     SPK_TRY(read_cnt());
