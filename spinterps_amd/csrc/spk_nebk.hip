@@ -408,8 +408,10 @@ __global__ __launch_bounds__(256) void k_neb_nrst(
       // bisection on the distance until exactly k lie at or below it
       // (count(<= lo) < k <= count(<= hi)); a near tie that stops it falls
       // back to the exact order on (distance, position) below
-      double lo = -1.0, hi = dmax, thr = -1.0;
-      for (int it = 0; it < 64; ++it) {
+      // (exactly k candidates, which no bisection below dmax finds, are all
+      // taken)
+      double lo = -1.0, hi = dmax, thr = m == k ? dmax : -1.0;
+      for (int it = 0; it < 64 && thr < 0.0; ++it) {
         const double mid = 0.5 * (lo + hi);
         if (!(mid > lo && mid < hi)) break;
         int cnt = 0;

@@ -231,6 +231,27 @@ def test_variance_rounding(gpu):
     assert rel < 5.0e-16, rel
 
 
+@pytest.mark.parametrize('k', [1, 3, 8])
+def test_tiles_of_exactly_k_candidates(gpu, k):
+    """Tiles of cells that no more than k stations can reach: all are taken
+    (clusters of k stations far apart, the cells of a cluster around it)."""
+    from spinterps_amd.interp.steps import DeviceProblem, interp_neb_steps
+    rng = np.random.default_rng(k)
+    ox, oy = np.meshgrid(np.arange(4) * 1e6, np.arange(4) * 1e6)
+    sx = (ox.ravel()[:, None] + rng.uniform(0, 1e3, (16, k))).ravel()
+    sy = (oy.ravel()[:, None] + rng.uniform(0, 1e3, (16, k))).ravel()
+    cx = (ox.ravel()[:, None] + rng.uniform(0, 1e3, (16, 64))).ravel()
+    cy = (oy.ravel()[:, None] + rng.uniform(0, 1e3, (16, 64))).ravel()
+    z = rng.gamma(2.0, 5.0, (1, sx.size))
+    e, _, _ = interp_neb_steps(DeviceProblem(sx, sy, cx, cy), z, None, 'IDW',
+                               neb_sel_mthd='nrst', n_nebs=k)
+    d = np.hypot(cx[:, None] - sx, cy[:, None] - sy)
+    at = np.argsort(d, axis=1)[:, :k]
+    w = 1.0 / np.take_along_axis(d, at, 1) ** 2
+    ref = (w * z[0][at]).sum(1) / w.sum(1)
+    np.testing.assert_allclose(e[0].cpu().numpy(), ref, rtol=1e-12)
+
+
 def test_edk_reproduces_the_drift(gpu):
     """Values that are a linear function of the drift are reproduced at
     every cell (the weights sum to one and reproduce the drift)."""
