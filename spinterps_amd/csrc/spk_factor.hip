@@ -180,28 +180,18 @@ __device__ inline f4d_t mfma64(double a, double b, f4d_t c) {
   return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
 }
 
-// c0 of every step (grid (steps)).
-__global__ __launch_bounds__(256) void k_chol_c0(const double *__restrict__ A,
-                                                 int64_t ld, int64_t strideA,
-                                                 StepSc *__restrict__ sc,
-                                                 const spk_vg *__restrict__ vgs) {
-  const int s = blockIdx.x;
-  if (sc[s].status) return;
-  const int n = sc[s].n;
-  const double *As = A + (int64_t)s * strideA;
+// c0 of one step, by the workgroup; every thread returns it.
+__device__ inline double chol_c0(const double *As, int64_t ld, int n,
+                                 const spk_vg &vg) {
   const int tid = threadIdx.x;
   __shared__ double red[256];
-  const spk_vg &vg = vgs[s];
   bool bounded = true;
   for (int k = 0; k < vg.n; ++k) {
-    const int ty = vg.type[k];
-    if (ty == SPK_VG_RNG || ty == SPK_VG_POW || ty == SPK_VG_HOL)
+    const int t = vg.type[k];
+    if (t == SPK_VG_RNG || t == SPK_VG_POW || t == SPK_VG_HOL)
       bounded = false;
   }
-  if (bounded) {
-    if (tid == 0) sc[s].c0 = vg.sill_sum;
-    return;
-  }
+  if (bounded) return vg.sill_sum;
   double mx = 0.0;
   for (int64_t e = tid; e < (int64_t)n * n; e += 256) {
     const int i = (int)(e % n), j = (int)(e / n);
@@ -213,7 +203,19 @@ __global__ __launch_bounds__(256) void k_chol_c0(const double *__restrict__ A,
     if (tid < w) red[tid] = fmax(red[tid], red[tid + w]);
     __syncthreads();
   }
-  if (tid == 0) sc[s].c0 = 2.0 * red[0] + fabs(vg.sill_sum);
+  return 2.0 * red[0] + fabs(vg.sill_sum);
+}
+
+// c0 of every step (grid (steps)).
+__global__ __launch_bounds__(256) void k_chol_c0(const double *__restrict__ A,
+                                                 int64_t ld, int64_t strideA,
+                                                 StepSc *__restrict__ sc,
+                                                 const spk_vg *__restrict__ vgs) {
+  const int s = blockIdx.x;
+  if (sc[s].status) return;
+  const double c0 =
+      chol_c0(A + (int64_t)s * strideA, ld, sc[s].n, vgs[s]);
+  if (threadIdx.x == 0) sc[s].c0 = c0;
 }
 
 // A <- c0 - A on the lower triangle; grid (column groups, steps), block x
@@ -244,11 +246,12 @@ __device__ inline double lane_value(double v, int src) {
 // multipliers by readlane, no barrier inside), then all waves update the
 // columns to their right.  Bound by the chain of 64 reciprocal square roots;
 // 32 columns with three barriers each took 24 us, 64 now 22 us.
-// grid (steps)
-__global__ __launch_bounds__(256) void k_chol_diag(double *__restrict__ A,
-                                                   int64_t ld, int64_t strideA,
-                                                   StepSc *__restrict__ sc,
-                                                   int k0) {
+// SHIFT: the whole of a system of at most 64 rows, c0 and the shift
+// included.  grid (steps)
+template <bool SHIFT>
+__global__ __launch_bounds__(256) void k_chol_diag(
+    double *__restrict__ A, int64_t ld, int64_t strideA,
+    StepSc *__restrict__ sc, const spk_vg *__restrict__ vgs, int k0) {
   const int s = blockIdx.x;
   if (sc[s].status) return;
   const int n = sc[s].n;
@@ -259,11 +262,19 @@ __global__ __launch_bounds__(256) void k_chol_diag(double *__restrict__ A,
   __shared__ double D[64][65];  // D[column][row]
   __shared__ int fail;
   if (tid == 0) fail = 0;
+  double c0 = 0.0;
+  if (SHIFT) {
+    c0 = chol_c0(As, ld, n, vgs[s]);
+    if (tid == 0) sc[s].c0 = c0;
+  }
   for (int e = tid; e < 64 * 64; e += 256) {
     const int i = e & 63, j = e >> 6;
-    D[j][i] = (i < jb && j < jb && i >= j)
-                  ? As[(k0 + i) + (int64_t)(k0 + j) * ld]
-                  : (i == j ? 1.0 : 0.0);
+    double v = i == j ? 1.0 : 0.0;
+    if (i < jb && j < jb && i >= j) {
+      v = As[(k0 + i) + (int64_t)(k0 + j) * ld];
+      if (SHIFT) v = c0 - v;
+    }
+    D[j][i] = v;
   }
   __syncthreads();
   for (int b = 0; b < jb; b += 16) {
@@ -311,17 +322,18 @@ __global__ __launch_bounds__(256) void k_chol_diag(double *__restrict__ A,
 // wave: 16 unknowns at a time in registers, first reduced by the earlier ones
 // (kept in LDS, as many FMAs as 16-byte broadcasts of L allow), then solved
 // among themselves.  Lt[q][c] = L[c][q], dinv[c] = 1 / L[c][c], a(c) the
-// lane's right-hand side, done(c, x) takes the results.  The loops over the
+// lane's right-hand side, done(c, x) takes the results, for the unknowns
+// below `rows` (and those of its last block of 16).  The loops over the
 // blocks stay rolled: fully unrolled, with all 64 unknowns in registers, the
 // 35 KB of code took 50 to 78 us per launch, bound by instruction fetch; this
 // takes 18 to 33.
 template <typename A, typename D>
 __device__ inline void wave_fwd_subst(const double (*Lt)[64],
                                       const double *dinv, double (*Xs)[64],
-                                      A a, D done) {
+                                      int rows, A a, D done) {
   const int lane = threadIdx.x & 63;
 #pragma unroll 1
-  for (int b = 0; b < 64; b += 16) {
+  for (int b = 0; b < rows; b += 16) {
     double x[16];
 #pragma unroll
     for (int c = 0; c < 16; ++c) x[c] = a(b + c);
@@ -373,7 +385,7 @@ __global__ __launch_bounds__(64) void k_chol_solve(double *__restrict__ A,
   const double *in = As + min(r, n - 1) + (int64_t)k0 * ld;
   double *out = As + r + (int64_t)k0 * ld;
   wave_fwd_subst(
-      Lt, dinv, Xs, [&](int c) { return in[(int64_t)c * ld]; },
+      Lt, dinv, Xs, 64, [&](int c) { return in[(int64_t)c * ld]; },
       [&](int c, double x) {
         if (r < n) out[(int64_t)c * ld] = x;
       });
@@ -439,6 +451,13 @@ __global__ __launch_bounds__(256, 2) void k_chol_trail(double *__restrict__ A,
 
 int chol_steps(hipStream_t st, double *A, int64_t ld, int64_t stride,
                StepSc *sc, const spk_vg *vgs, int shift, int64_t N, int S) {
+  // systems of one panel in one launch here and below: a one-step call with
+  // 3 stations and its variance takes 220 us, 241 with five launches more
+  if (shift && N <= 64) {
+    hipLaunchKernelGGL(k_chol_diag<true>, dim3(S), dim3(256), 0, st, A, ld,
+                       stride, sc, vgs, 0);
+    return check_launch("k_chol");
+  }
   if (shift) {
     hipLaunchKernelGGL(k_chol_c0, dim3(S), dim3(256), 0, st,
                        (const double *)A, ld, stride, sc, vgs);
@@ -447,8 +466,8 @@ int chol_steps(hipStream_t st, double *A, int64_t ld, int64_t stride,
                        0, st, A, ld, stride, (const StepSc *)sc);
   }
   for (int k0 = 0; k0 < N; k0 += 64) {
-    hipLaunchKernelGGL(k_chol_diag, dim3(S), dim3(256), 0, st, A, ld, stride,
-                       sc, k0);
+    hipLaunchKernelGGL(k_chol_diag<false>, dim3(S), dim3(256), 0, st, A, ld,
+                       stride, sc, vgs, k0);
     const int64_t nt = ceil_div(N - k0, 64) - 1;
     if (nt <= 0) break;
     hipLaunchKernelGGL(k_chol_solve, dim3((unsigned)nt, S), dim3(64), 0, st, A,
@@ -499,7 +518,7 @@ __global__ __launch_bounds__(64) void k_trtri_diag(
   dinv[lane] = 1.0 / Lt[lane][lane];
   __syncthreads();
   wave_fwd_subst(
-      Lt, dinv, Xc, [&](int c) { return lane == c ? 1.0 : 0.0; },
+      Lt, dinv, Xc, rn, [&](int c) { return lane == c ? 1.0 : 0.0; },
       [&](int c, double x) {
         T[c & 15][lane] = x;
         if ((c & 15) != 15) return;
@@ -647,7 +666,9 @@ int trtri_steps(hipStream_t st, const double *L, double *X, int64_t ld,
                 int64_t stride, const StepSc *sc, int64_t N, int S) {
   const dim3 g((unsigned)ceil_div(N, 64), S);
   hipLaunchKernelGGL(k_trtri_diag, g, dim3(64), 0, st, L, X, ld, stride, sc);
-  hipLaunchKernelGGL(k_trtri_cols, g, dim3(256), 0, st, L, X, ld, stride, sc);
+  if (N > 64)  // one diagonal block is the whole inverse
+    hipLaunchKernelGGL(k_trtri_cols, g, dim3(256), 0, st, L, X, ld, stride,
+                       sc);
   return check_launch("k_trtri");
 }
 
@@ -1246,28 +1267,15 @@ __global__ void k_dual_fin(StepSc *__restrict__ sc, int m, int method,
 // inverse [[-P, Q], [Q^T, B^-1 - c0 e0 e0^T]], written to M (ld rows).
 // SK has no constraint rows: M = Cinv.
 // Launches over (tiles or row blocks, steps): k_minv_tiles, k_minv_w,
-// k_minv_mid, k_minv_fin (minv_steps).  One workgroup per step for all of it
+// k_minv_mid, k_minv_fin (minv_steps; systems of one tile: k_minv_small).  One workgroup per step for all of it
 // took 11.8 ms for systems of 900 rows; the four take 0.24 ms for seven.
 
 // Cinv[i, j] = sum over k >= i of Li[k, i] Li[k, j], a 64 x 64 tile (bi >=
 // bj) per workgroup and its mirror image, on FP64 MFMA (32 x 32 per wave).
 // Both operands are read down columns of Li and kept by columns in LDS (36
 // doubles apart).  grid (tiles of the lower triangle, steps)
-__global__ __launch_bounds__(256, 2) void k_minv_tiles(
-    const double *__restrict__ Li, int64_t ld, int64_t stride,
-    const StepSc *__restrict__ sc, double *__restrict__ M) {
-  const int s = blockIdx.y;
-  if (sc[s].status) return;
-  const int n = sc[s].n;
-  const int nb = (n + 63) / 64;
-  const int t = blockIdx.x;
-  if (t >= nb * (nb + 1) / 2) return;
-  int bi = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
-  while (bi * (bi + 1) / 2 > t) --bi;
-  while ((bi + 1) * (bi + 2) / 2 <= t) ++bi;
-  const int bj = t - bi * (bi + 1) / 2;
-  const double *L = Li + (int64_t)s * stride;
-  double *Ms = M + (int64_t)s * stride;
+__device__ inline void minv_tile(const double *L, int64_t ld, int n, int bi,
+                                 int bj, double *Ms) {
   const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
   const int li = lane & 15, lg = lane >> 4;
   const int wi = (wave & 1) * 32, wj = (wave >> 1) * 32;
@@ -1332,22 +1340,28 @@ __global__ __launch_bounds__(256, 2) void k_minv_tiles(
         }
       }
 }
+__global__ __launch_bounds__(256, 2) void k_minv_tiles(
+    const double *__restrict__ Li, int64_t ld, int64_t stride,
+    const StepSc *__restrict__ sc, double *__restrict__ M) {
+  const int s = blockIdx.y;
+  if (sc[s].status) return;
+  const int n = sc[s].n;
+  const int nb = (n + 63) / 64;
+  const int t = blockIdx.x;
+  if (t >= nb * (nb + 1) / 2) return;
+  int bi = (int)((sqrt(8.0 * t + 1.0) - 1.0) * 0.5);
+  while (bi * (bi + 1) / 2 > t) --bi;
+  while ((bi + 1) * (bi + 2) / 2 <= t) ++bi;
+  minv_tile(Li + (int64_t)s * stride, ld, n, bi, t - bi * (bi + 1) / 2,
+            M + (int64_t)s * stride);
+}
 
 // W = Cinv F (columns 0 .. p-1 of the step's work area T0), 64 rows per
 // workgroup, each wave a quarter of the columns; grid (ceil(n_max / 64),
 // steps)
-__global__ __launch_bounds__(256) void k_minv_w(
-    const double *__restrict__ M, int64_t ld, int64_t stride,
-    const StepSc *__restrict__ sc, const int32_t *__restrict__ idx, int64_t N,
-    const double *__restrict__ stn_drift, int m, int p,
-    double *__restrict__ T0, int64_t ldt) {
-  const int s = blockIdx.y;
-  if (sc[s].status) return;
-  const int n = sc[s].n;
-  const int i0 = blockIdx.x * 64;
-  if (i0 >= n) return;
-  const double *Ms = M + (int64_t)s * stride;
-  const int32_t *my = idx + (int64_t)s * N;
+__device__ inline void minv_w(const double *Ms, int64_t ld, int n, int i0,
+                              const int32_t *my, const double *stn_drift,
+                              int m, int p, double *W, int64_t ldt) {
   const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
   const int i = min(i0 + lane, n - 1);
   __shared__ double red[kMaxP][4][64];
@@ -1366,27 +1380,34 @@ __global__ __launch_bounds__(256) void k_minv_w(
 #pragma unroll
   for (int r = 0; r < kMaxP; ++r) red[r][wave][lane] = acc[r];
   __syncthreads();
-  double *W = T0 + (int64_t)s * ldt * kT0Cols;
   for (int r = wave; r < p; r += 4)
     if (i0 + lane < n)
       W[i0 + lane + (int64_t)r * ldt] = red[r][0][lane] + red[r][1][lane] +
                                         red[r][2][lane] + red[r][3][lane];
 }
+__global__ __launch_bounds__(256) void k_minv_w(
+    const double *__restrict__ M, int64_t ld, int64_t stride,
+    const StepSc *__restrict__ sc, const int32_t *__restrict__ idx, int64_t N,
+    const double *__restrict__ stn_drift, int m, int p,
+    double *__restrict__ T0, int64_t ldt) {
+  const int s = blockIdx.y;
+  if (sc[s].status) return;
+  const int n = sc[s].n;
+  const int i0 = blockIdx.x * 64;
+  if (i0 >= n) return;
+  minv_w(M + (int64_t)s * stride, ld, n, i0, idx + (int64_t)s * N, stn_drift,
+         m, p, T0 + (int64_t)s * ldt * kT0Cols, ldt);
+}
 
 // The condition estimate max diag(Cinv) max diag(C), then B = F^T W, its
 // inverse (M's corner) and Q = W B^-1 (columns p .. 2p-1 of T0); grid
 // (steps)
-__global__ __launch_bounds__(256) void k_minv_mid(
-    double *__restrict__ M, int64_t ld, int64_t stride,
-    StepSc *__restrict__ sc, const int32_t *__restrict__ idx, int64_t N,
-    const double *__restrict__ stn_drift, int m, int method, int p,
-    double *__restrict__ T0, int64_t ldt, const spk_vg *__restrict__ vgs,
-    double min_vg_val) {
-  const int s = blockIdx.x;
-  if (sc[s].status) return;
-  const int n = sc[s].n;
-  double *Ms = M + (int64_t)s * stride;
-  const int32_t *my = idx + (int64_t)s * N;
+__device__ inline void minv_mid(double *Ms, int64_t ld, StepSc *st,
+                                const int32_t *my, const double *stn_drift,
+                                int m, int method, int p, double *W,
+                                int64_t ldt, const spk_vg &vg,
+                                double min_vg_val) {
+  const int n = st->n;
   const int tid = threadIdx.x;
   __shared__ double red[256];
   double mx = 0.0;
@@ -1398,16 +1419,14 @@ __global__ __launch_bounds__(256) void k_minv_mid(
     __syncthreads();
   }
   if (tid == 0) {
-    const spk_vg &vg = vgs[s];
     const double cii = (method == SPK_M_SK)
                            ? vg_entry(vg, 0.0, 1, min_vg_val)
-                           : sc[s].c0 - vg_entry(vg, 0.0, 0, min_vg_val);
+                           : st->c0 - vg_entry(vg, 0.0, 0, min_vg_val);
     const double kap = red[0] * fabs(cii);
-    sc[s].kappa = kap;
-    sc[s].flags = (kap <= 1e12) ? 0 : SPK_ST_ILLCOND;
+    st->kappa = kap;
+    st->flags = (kap <= 1e12) ? 0 : SPK_ST_ILLCOND;
   }
   if (method == SPK_M_SK) return;
-  double *W = T0 + (int64_t)s * ldt * kT0Cols;
   __shared__ double Bs[kMaxP * kMaxP], Bi[kMaxP * kMaxP];
   for (int e = tid >> 6; e < p * p; e += 4) {
     const int a = e / p, b = e % p;
@@ -1432,21 +1451,26 @@ __global__ __launch_bounds__(256) void k_minv_mid(
   if (tid < p * p) {
     const int a = tid / p, b = tid % p;
     Ms[(n + a) + (int64_t)(n + b) * ld] =
-        Bi[a * p + b] - ((a == 0 && b == 0) ? sc[s].c0 : 0.0);
+        Bi[a * p + b] - ((a == 0 && b == 0) ? st->c0 : 0.0);
   }
+}
+__global__ __launch_bounds__(256) void k_minv_mid(
+    double *__restrict__ M, int64_t ld, int64_t stride,
+    StepSc *__restrict__ sc, const int32_t *__restrict__ idx, int64_t N,
+    const double *__restrict__ stn_drift, int m, int method, int p,
+    double *__restrict__ T0, int64_t ldt, const spk_vg *__restrict__ vgs,
+    double min_vg_val) {
+  const int s = blockIdx.x;
+  if (sc[s].status) return;
+  minv_mid(M + (int64_t)s * stride, ld, sc + s, idx + (int64_t)s * N,
+           stn_drift, m, method, p, T0 + (int64_t)s * ldt * kT0Cols, ldt,
+           vgs[s], min_vg_val);
 }
 
 // M <- -(Cinv - Q W^T) and the border rows; grid (column groups, steps),
 // block x takes columns x, x + gridDim.x, ...
-__global__ __launch_bounds__(256) void k_minv_fin(
-    double *__restrict__ M, int64_t ld, int64_t stride,
-    const StepSc *__restrict__ sc, int p, const double *__restrict__ T0,
-    int64_t ldt) {
-  const int s = blockIdx.y;
-  if (sc[s].status) return;
-  const int n = sc[s].n;
-  double *Ms = M + (int64_t)s * stride;
-  const double *W = T0 + (int64_t)s * ldt * kT0Cols;
+__device__ inline void minv_fin(double *Ms, int64_t ld, int n, int p,
+                                const double *W, int64_t ldt) {
   const double *Q = W + (int64_t)p * ldt;
   for (int j = blockIdx.x; j < n; j += gridDim.x) {
     for (int i = threadIdx.x; i < n; i += 256) {
@@ -1463,6 +1487,37 @@ __global__ __launch_bounds__(256) void k_minv_fin(
     }
   }
 }
+__global__ __launch_bounds__(256) void k_minv_fin(
+    double *__restrict__ M, int64_t ld, int64_t stride,
+    const StepSc *__restrict__ sc, int p, const double *__restrict__ T0,
+    int64_t ldt) {
+  const int s = blockIdx.y;
+  if (sc[s].status) return;
+  minv_fin(M + (int64_t)s * stride, ld, sc[s].n, p,
+           T0 + (int64_t)s * ldt * kT0Cols, ldt);
+}
+
+// All of it for systems of one tile (n <= 64); grid (1, steps)
+__global__ __launch_bounds__(256, 2) void k_minv_small(
+    const double *Li, int64_t ld, int64_t stride, StepSc *sc,
+    const int32_t *idx, int64_t N, const double *stn_drift, int m, int method,
+    int p, double *M, double *T0, int64_t ldt, const spk_vg *vgs,
+    double min_vg_val) {
+  const int s = blockIdx.y;
+  if (sc[s].status) return;
+  const int n = sc[s].n;
+  double *Ms = M + (int64_t)s * stride;
+  double *W = T0 + (int64_t)s * ldt * kT0Cols;
+  const int32_t *my = idx + (int64_t)s * N;
+  minv_tile(Li + (int64_t)s * stride, ld, n, 0, 0, Ms);
+  __syncthreads();
+  if (p > 0) minv_w(Ms, ld, n, 0, my, stn_drift, m, p, W, ldt);
+  __syncthreads();
+  minv_mid(Ms, ld, sc + s, my, stn_drift, m, method, p, W, ldt, vgs[s],
+           min_vg_val);
+  __syncthreads();
+  if (p > 0) minv_fin(Ms, ld, n, p, W, ldt);
+}
 
 int minv_steps(hipStream_t st, const double *Li, int64_t ld, int64_t stride,
                StepSc *sc, const int32_t *idx, int64_t N,
@@ -1470,6 +1525,12 @@ int minv_steps(hipStream_t st, const double *Li, int64_t ld, int64_t stride,
                double *T0, const spk_vg *vgs, double min_vg_val, int S) {
   const int64_t nb = ceil_div(N, 64);
   const int p = method == SPK_M_SK ? 0 : method == SPK_M_EDK ? 1 + m : 1;
+  if (N <= 64) {
+    hipLaunchKernelGGL(k_minv_small, dim3(1, S), dim3(256), 0, st, Li, ld,
+                       stride, sc, idx, N, stn_drift, m, method, p, M, T0, ld,
+                       vgs, min_vg_val);
+    return check_launch("k_minv");
+  }
   hipLaunchKernelGGL(k_minv_tiles, dim3((unsigned)(nb * (nb + 1) / 2), S),
                      dim3(256), 0, st, Li, ld, stride, (const StepSc *)sc, M);
   if (p > 0)

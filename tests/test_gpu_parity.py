@@ -779,3 +779,48 @@ def test_ranges_far_below_the_distances(gpu, precision):
     np.testing.assert_allclose(est.cpu().numpy(), ref['OK'], rtol=1e-11)
     np.testing.assert_allclose(var.cpu().numpy(), ref['EST_VARS_OK'],
                                rtol=1e-11)
+
+
+@pytest.mark.parametrize('n', [2, 17, 63, 64, 65])
+@pytest.mark.parametrize('method', ['OK', 'EDK', 'SKM'])
+def test_small_systems_in_one_launch(gpu, n, method):
+    """Systems of at most 64 rows, factorised, inverted and bordered in one
+    launch each, and of 65: bounded models and, for OK, the unbounded ones
+    whose shift is found from the matrix, against the exact solution (or the
+    oracle, for the power model and the plain distances)."""
+    from spinterps_amd.interp.steps import DeviceProblem, interp_steps
+    if method == 'EDK' and n < 4:
+        pytest.skip('two stations do not determine mean and drift')
+    rng = np.random.default_rng(n)
+    sx, sy = rng.uniform(0, 1e5, n), rng.uniform(0, 1e5, n)
+    cx, cy = rng.uniform(0, 1e5, 50), rng.uniform(0, 1e5, 50)
+    sd = (sx / 1e5 + np.sin(sy / 2e4))[:, None]
+    cd = (cx / 1e5 + np.sin(cy / 2e4))[None]
+    vgs = ['0.1 Nug(0.0) + 0.9 Sph(30000.0)', '1.2 Exp(20000.0)',
+           '0.5 Sph(9e3) + 0.5 Exp(3e4)']
+    if method == 'OK':
+        vgs += ['0.5 Pow(1.2)', '1.0 Rng(1.0)']
+    vals = rng.gamma(2.0, 3.0, (len(vgs), n))
+    if n > 5:
+        vals[1, : n // 3] = np.nan
+    prob = DeviceProblem(sx, sy, cx, cy, sd if method == 'EDK' else None,
+                         cd if method == 'EDK' else None)
+    est, var, info = interp_steps(prob, vals, vgs, method)
+    est = est.cpu().numpy()
+    assert not (info.cpu().numpy() & (4 | 8 | 16 | 128)).any()
+    for t, vg in enumerate(vgs):
+        a = ~np.isnan(vals[t])
+        z = vals[t, a]
+        dd = O.dists_2d(sx[a], sy[a], sx[a], sy[a])
+        rd = O.dists_2d(cx, cy, sx[a], sy[a])
+        if 'Pow' in vg or 'Rng' in vg:
+            K, R = O.krig_system('OK', vg, dd, rd, None, None, 0.0)
+            ref, v = O.krige_solve(K, R, z, rd, True)[:2]
+        else:
+            ref, v, _ = O.krige_exact(method, vg, dd, rd, z, sd[a], cd,
+                                      want_var=method == 'OK')
+        np.testing.assert_allclose(est[t], ref, rtol=0,
+                                   atol=1e-9 * np.abs(z).mean())
+        if method == 'OK':
+            np.testing.assert_allclose(var[t].cpu().numpy(), v, rtol=1e-9,
+                                       atol=1e-9 * np.abs(v).mean())
