@@ -142,6 +142,11 @@ def test_set_sizes_match_oracle(gpu, method, n_nebs):
     if method == 'OK':
         _close(var, f64['EST_VARS_OK'], np.nanmax(f64['EST_VARS_OK']), 1e-8,
                'var')
+    # solved by the sweep itself, not by the pseudo-inverse that takes the
+    # chunks it rejects (and that agrees with the oracle anyway); the linear
+    # model is not positive definite in the plane, some of its sets fail
+    for t in (0, 1, 4, 5) + ((6,) if method == 'EDK' else ()):
+        assert not info[t] & (_lib.ST_PINV | _lib.ST_ILLCOND), (t, info[t])
 
 
 @pytest.mark.parametrize('method,drifts', [('OK', 0), ('SK', 0), ('SKM', 0),
