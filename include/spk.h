@@ -375,11 +375,15 @@ int spk_vgfit_evg_dev(spk_ctx *ctx, const int32_t *pi, const int32_t *pj,
  * sill) per component; fun, nit: device [T x n_cands].  range_ub is the
  * upper range bound (1e9 in vgs.py:747); popmul 50 and tol 0.01 are the
  * reference's settings.  A candidate with D = 2 n_comp parameters evolves
- * min(popmul D^2, 800) members.  All candidates' trials of a generation are
- * evaluated over the whole device, and the host reads every few generations
- * which pairs still evolve (the call returns when the last has converged);
- * on a stream that is being captured each pair evolves in one workgroup
- * instead, with the same random streams. */
+ * min(popmul D^2, 800) members.  With many
+ * bins all candidates' trials of a generation are evaluated over the whole
+ * device, and the host reads every few generations which pairs still evolve:
+ * the call blocks until the last has converged, and the context keeps up to
+ * 0.44 GB of workspace for it (162 to 213 KB for each of at most 2 048 pairs
+ * at a time).  With few bins, without the memory for that, or on a stream that
+ * is being captured, each pair evolves in one workgroup, without a workspace
+ * (the call may still wait for the stream once, to read the bin counts).  Both
+ * give the same bits. */
 int spk_vgfit_de_dev(spk_ctx *ctx, const double *bin_h, const double *bin_g,
                      const int32_t *nbins, int max_bins, const double *var,
                      int64_t T, const int32_t *cands, int n_cands, int maxiter,
@@ -413,9 +417,10 @@ int spk_vgfit_de_seeded_dev(spk_ctx *ctx, const double *bin_h,
  * normal from a counter-based generator keyed on (seed, t, station rank).
  * out [T x N]: NaN at masked stations.  info [T]: SPK_ST_* (FAILED when
  * the Cholesky failed; the step's row stays NaN).  Returns SPK_EARG on a
- * context that has run spk_vgfit_pairs_dev: that call order stalled on the
- * GPU with no cause found, so it is refused (simulate first, or use a
- * second context). */
+ * context that has run spk_vgfit_pairs_dev: the first runs of that
+ * call order went silent, on a lock of the Python wrapper that no longer
+ * blocks; the order has not been run since and stays refused (simulate first,
+ * or use a second context). */
 int spk_simulate_fields_dev(spk_ctx *ctx, const spk_problem *prob, int64_t T,
                             const double *mask_vals, const spk_vg *vgs,
                             const double *means, uint64_t seed, double *out,

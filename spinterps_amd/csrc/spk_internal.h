@@ -59,8 +59,9 @@ struct spk_ctx {
   int n_marks = 0;
   std::vector<double> last_ms;
   // set by spk_vgfit_pairs_dev: spk_simulate_fields_dev refuses to run on
-  // a context that has sorted station pairs (that order stalled with no
-  // cause found; simulations before any pair sort are unaffected)
+  // a context that has sorted station pairs (that order went silent, on a
+  // lock of the Python wrapper that no longer blocks; it has not been run
+  // since, and stays refused)
   bool pairs_sorted = false;
   // pseudo-inverse fallback of failed steps: a rocBLAS handle (rocSOLVER
   // eigendecompositions and the reassembly GEMM) and pinned host copies

@@ -183,8 +183,8 @@ __global__ void k_assemble(const double *sx, const double *sy,
                            double *Gfull);
 // C = c0 - G (shift) or A as it is, then the Cholesky factor in the lower
 // triangle, of S systems of at most N rows: k_chol_c0, k_chol_shift, then
-// per 64-wide panel k_chol_diag, k_chol_solve, k_chol_trail.  N <= ld, ld a
-// multiple of 64.
+// per 64-wide panel k_chol_diag, k_chol_solve, k_chol_trail (with a shift and
+// at most 64 rows k_chol_diag alone).  N <= ld, ld a multiple of 64.
 int chol_steps(hipStream_t st, double *A, int64_t ld, int64_t stride,
                StepSc *sc, const spk_vg *vgs, int shift, int64_t N, int S);
 // X = L^-1 of the same systems

@@ -498,9 +498,9 @@ int spk_simulate_fields_dev(spk_ctx *ctx, const spk_problem *prob, int64_t T,
   if (ctx->pairs_sorted)
     return set_error(SPK_EARG,
                      "field simulation after a station-pair sort on the same "
-                     "context is disabled (that order stalled on the GPU with "
-                     "no cause found): simulate first, or use another "
-                     "context");
+                     "context is disabled (that order has not been run since "
+                     "a lock that stalled it was mended): simulate first, or "
+                     "use another context");
   if (T <= 0) return SPK_OK;
   SPK_HIP(hipSetDevice(ctx->device));
   hipStream_t sm = ctx->stream;

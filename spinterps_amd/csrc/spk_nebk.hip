@@ -19,11 +19,12 @@
 //   k_neb_mfma     one wavefront per chunk: stations, values, border and
 //                  cells as the rows of one matrix, Cholesky sweep over the
 //                  stations' columns, results from dot products of rows
-//   k_neb_krige    the same chunks, where that matrix has too few rows, and
-//                  the methods without a system: factor in LDS, dual-form
-//                  vectors, then every cell of the chunk
+//   k_neb_krige    the same chunks, where that matrix has too few rows or
+//                  the chunk too many cells for it, and the methods without a
+//                  system: factor in LDS, dual-form vectors, then every cell
+//                  of the chunk
 //   k_neb_pinv_*   chunks whose Cholesky fails (or whose condition estimate
-//                  exceeds 1e14) are solved as the reference solves every
+//                  exceeds 1e10) are solved as the reference solves every
 //                  group: pinv of the bordered system (rocSOLVER eigen-
 //                  decomposition, numpy's cutoff), lambda = pinv(K) rhs
 //                  per cell and the sum test
@@ -200,7 +201,7 @@ __global__ void k_neb_mask(const double *__restrict__ vals, int64_t n,
     out[i] = keep[i % N] ? vals[i] : NAN;
 }
 
-// ---- order of the cells along a Hilbert curve ----------------------------------------------------
+// ---- order of the cells along a Hilbert curve --------------------------------
 // One workgroup: the bounding box of the cells, bb = (x0, x1, y0, y1).
 __global__ __launch_bounds__(1024) void k_neb_bbox(
     const double *__restrict__ cx, const double *__restrict__ cy, int64_t C,

@@ -1196,8 +1196,8 @@ static bool stream_capturing(hipStream_t st) {
 }
 
 // The evolution over the whole device (k_de_energy, k_de_step) in batches
-// of at most kDeBatch (step, candidate) pairs, whose scratch is 150 KB
-// (two components) to 260 KB each.  The host reads the pairs still
+// of at most kDeBatch (step, candidate) pairs, whose scratch is 162 KB
+// (two components) to 213 KB (four) each.  The host reads the pairs still
 // evolving every kDePoll generations (fits take 1 to 45).
 constexpr int kDeBatch = 2048;
 constexpr int kDePoll = 4;

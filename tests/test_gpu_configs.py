@@ -256,7 +256,8 @@ def test_stress_subset_flags(gpu):
 
 def test_simulate_after_pair_sort_refused(gpu):
     """A context that has sorted station pairs refuses to simulate fields
-    (that order stalled once with no cause found); nothing is launched.
+    (that order went silent before the wrapper's lock was mended, and has not
+    been run since); nothing is launched.
     Uses a context of its own so the shared one is unaffected."""
     import ctypes
 
