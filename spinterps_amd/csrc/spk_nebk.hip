@@ -270,14 +270,23 @@ __global__ void k_neb_curve(const double *__restrict__ cx,
 }
 
 // ---- nrst selection ----------------------------------------------------------
+// A distance of the order below: one that overflows or is no number counts as
+// the largest finite one (ties by position), so that it stays below the
+// infinity of an empty slot and every set has k entries.
+__device__ inline double neb_dist(double x, double y, double sx, double sy) {
+  return fmin(dist2(x, y, sx, sy), 0x1.fffffffffffffp+1023);
+}
+
 // grid (ceil(C / 64), S), 256 threads.  Tile i holds cells perm[64 i ..
 // 64 i + 63], consecutive along the curve, so a tile is a compact patch.  For
 // the tile's bounding box
 // (centre c, half diagonal h) the block finds a T with at least k active
 // stations within T of c; the k nearest of any cell x of the tile then lie
 // within T + 2h of c (r_k(x) <= r_k(c) + h, and |s - c| <= |s - x| + h),
-// so only those candidates are staged.  Each cell's selection is exact:
-// the k smallest (distance, position) pairs, distances as in pyx:141.
+// so only those candidates are staged (and all whose distance from c does not
+// compare: a tile with a cell at infinity stages every station).  Each cell's
+// selection is exact: the k smallest (distance, position) pairs, distances as
+// in pyx:141 where they are finite.
 // Output: nb[(t C + c) K + r] the r-th selected position into the step's
 // active list, ascending; key = step << 56 | hash of the set; cell = c.
 __global__ __launch_bounds__(256) void k_neb_nrst(
@@ -364,7 +373,7 @@ __global__ __launch_bounds__(256) void k_neb_nrst(
       x = sx[my[j]];
       y = sy[my[j]];
       const double dx = x - xc, dy = y - yc;
-      f = (dx * dx + dy * dy) <= R2;
+      f = !((dx * dx + dy * dy) > R2);
     }
     const unsigned long long bal = __ballot(f);
     __syncthreads();  // wcnt of the previous round is read
@@ -401,7 +410,7 @@ __global__ __launch_bounds__(256) void k_neb_nrst(
         const int q = s * 64 + lane;
         dv[s] = INFINITY;
         if (s < ns && q < m) {
-          dv[s] = dist2(x, y, cand_x[q], cand_y[q]);
+          dv[s] = neb_dist(x, y, cand_x[q], cand_y[q]);
           dmax = fmax(dmax, dv[s]);
         }
       }
@@ -496,7 +505,7 @@ __global__ __launch_bounds__(256) void k_neb_nrst(
         double bd = INFINITY;
         int bi = 0x7fffffff;
         for (int j = lane; j < n; j += 64) {
-          const double d = dist2(x, y, sx[my[j]], sy[my[j]]);
+          const double d = neb_dist(x, y, sx[my[j]], sy[my[j]]);
           if (lex_less(cd, ci, d, j) && lex_less(d, j, bd, bi)) {
             bd = d;
             bi = j;

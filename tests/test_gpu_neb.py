@@ -257,6 +257,39 @@ def test_tiles_of_exactly_k_candidates(gpu, k):
     np.testing.assert_allclose(e[0].cpu().numpy(), ref, rtol=1e-12)
 
 
+@pytest.mark.parametrize('n,k', [(71, 30), (51, 50), (65, 64), (701, 20)])
+def test_cells_without_finite_distances(gpu, n, k):
+    """Cells at infinity, beyond 1e154 or without a coordinate beside others in
+    a tile: their sets are the first k active stations, the others' results
+    are as without them (some of many candidates, all of exactly k, more sets
+    than fit the sweep, more candidates than are staged)."""
+    from spinterps_amd.interp.steps import (DeviceProblem, interp_neb_steps,
+                                            interp_steps)
+    rng = np.random.default_rng(n + k)
+    sx, sy = rng.uniform(0, 1e5, n), rng.uniform(0, 1e5, n)
+    cx, cy = rng.uniform(0, 1e5, 200), rng.uniform(0, 1e5, 200)
+    z = rng.gamma(2.0, 3.0, (1, n))
+    z[0, 2] = np.nan
+    vg = ['0.1 Nug(0.0) + 2.0 Sph(60000.0)']
+    fx, fy = cx.copy(), cy.copy()
+    fx[9], fy[11], fy[70], fx[130] = 1.7e308, np.inf, 1e200, np.nan
+
+    def run(x, y):
+        e, v, _ = interp_neb_steps(DeviceProblem(sx, sy, x, y), z, vg, 'OK',
+                                   neb_sel_mthd='nrst', n_nebs=k)
+        return e.cpu().numpy()[0], v.cpu().numpy()[0]
+
+    want, got = run(cx, cy), run(fx, fy)
+    own = np.setdiff1d(np.arange(200), (9, 11, 70, 130))
+    first = np.setdiff1d(np.arange(n), (2,))[:k]
+    e, v, _ = interp_steps(
+        DeviceProblem(sx[first], sy[first], np.array([1e9]), np.array([1e9])),
+        z[:, first], vg, 'OK')
+    for g, w, f in zip(got, want, (e.cpu().numpy(), v.cpu().numpy())):
+        np.testing.assert_allclose(g[own], w[own], rtol=1e-11)
+        np.testing.assert_allclose(g[[9, 11, 70]], f[0, 0], rtol=1e-11)
+
+
 def test_edk_reproduces_the_drift(gpu):
     """Values that are a linear function of the drift are reproduced at
     every cell (the weights sum to one and reproduce the drift)."""
